@@ -1,4 +1,4 @@
-"""Compiles the HIP sources of the attention library for gfx950 into ``flame_amd/lib``.
+"""Compiles the HIP sources of the attention library for gfx950, and the native host module, into ``flame_amd/lib``.
 
 ``python -m flame_amd.build`` (or ``build_lib()``) cross-compiles with hipcc; no GPU is needed.
 """
@@ -63,6 +63,27 @@ def build_lib(verbose: bool = False, extra=()) -> str:
 
 
 
+HOST_LIB_PATH = os.path.join(LIB_DIR, "_flame_torch_host.so")
+
+
+def build_host(verbose: bool = False) -> str:
+    """The native host module (csrc/torch_host.cpp): a CPython extension on torch's C++ API, no device code."""
+    import sysconfig
+
+    import torch
+    os.makedirs(LIB_DIR, exist_ok=True)
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+           sysconfig.get_paths()["include"]]
+    libs = ["c10", "c10_hip", "torch", "torch_cpu", "torch_hip", "torch_python"]
+    lib_dir = os.path.join(root, "lib")
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-Wall", "-Wno-unused-function",
+          *(f"-isystem{d}" for d in inc), os.path.join(CSRC, "torch_host.cpp"), "-o", HOST_LIB_PATH, f"-L{lib_dir}",
+          *(f"-l{name}" for name in libs), f"-Wl,-rpath,{lib_dir}"], verbose)
+    return HOST_LIB_PATH
+
+
 PROBE_LIB_PATH = os.path.join(LIB_DIR, "libflame_mfma_probe.so")
 
 
@@ -76,4 +97,5 @@ def build_probe(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     print(build_lib(verbose=True, extra=sys.argv[1:]))
+    print(build_host(verbose=True))
     print(build_probe(verbose=True))

@@ -1,12 +1,16 @@
-"""ctypes binding of ``libflame_attn_hip.so`` (the C ABI declared in ``include/flame_attn.h``).
+"""Binding of ``libflame_attn_hip.so`` (the C ABI declared in ``include/flame_attn.h``).
 
 Tensors are torch CUDA(HIP) tensors used purely as device-memory handles: the library receives raw
-pointers, element strides and the current HIP stream.  There is no CPU path: if the shared library
+pointers, element strides and the current HIP stream.  The attention, Sage, input-preparation and FP8 calls go
+through the native host module (``csrc/torch_host.cpp``: unpacking, allocation and the call in C++), the others
+through ctypes.  There is no CPU path: if the shared library
 is missing or a call fails, an exception is raised.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -34,6 +38,24 @@ def lib() -> ctypes.CDLL:
                 f"{LIB_PATH} is missing: build it with `python -m flame_amd.build` (hipcc, gfx950)")
         _lib = ctypes.CDLL(LIB_PATH)
     return _lib
+
+
+_host = None
+HOST_PATH = os.path.join(_HERE, "lib", "_flame_torch_host.so")
+
+
+def host():
+    """The native host module, bound to the library that lib() opened."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise FileNotFoundError(f"{HOST_PATH} is missing: build it with `python -m flame_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("_flame_torch_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_flame_torch_host", loader))
+        loader.exec_module(mod)
+        mod.bind(lib()._handle, FlameAttnError)
+        _host = mod
+    return _host
 
 
 def _i64x4(vals):
@@ -71,46 +93,12 @@ def fwd_workspace_bytes(B, H, Sq, Sk, D) -> int:
 def attn_fwd(q, k, v, scale, causal=False, kv_len=None, mask=None, want_lse=True, out=None, lse_out=None, workspace=None):
     """O, LSE = flame_attn_fwd_bf16(...).  q [B,H,Sq,D], k/v [B,H,Sk,D] bf16, D stride 1.
     `workspace` (uint8 device tensor): flame_attn_fwd_ws_bf16 instead, which may use it."""
-    B, H, Sq, D = q.shape
-    Sk = k.shape[2]
-    o = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device) if out is None else out
-    lse = lse_out if lse_out is not None else (torch.empty((B * H, Sq), dtype=torch.float32, device=q.device) if want_lse else None)
-    ms = _mask_strides(mask, B, H, Sq, Sk)
-    args = (_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), B, H, Sq, Sk, D, ctypes.c_float(scale),
-            _i64x4(q.stride()), _i64x4(k.stride()), _i64x4(v.stride()), _i64x4(o.stride()),
-            *(ctypes.c_int64(0) for _ in range(5)),
-            int(bool(causal)), _ptr(kv_len), _ptr(mask), ms)
-    if workspace is None:
-        fn, rc = "flame_attn_fwd_bf16", lib().flame_attn_fwd_bf16(*args, _stream())
-    else:
-        fn, rc = "flame_attn_fwd_ws_bf16", lib().flame_attn_fwd_ws_bf16(
-            *args, _ptr(workspace), ctypes.c_size_t(workspace.numel()), _stream())
-    if rc != 0:
-        raise FlameAttnError(fn, rc)
-    return o, lse
+    return host().attn_fwd(q, k, v, scale, causal, kv_len, mask, want_lse, out, lse_out, workspace)
 
 
 def attn_fwd_bias(q, k, v, scale, bias, mask=None, want_lse=True):
     """softmax(scale * Q K^T + bias) V.  bias: fp32 or bf16 [B|1, H|1, Sq, Sk] (inference only)."""
-    B, H, Sq, D = q.shape
-    Sk = k.shape[2]
-    assert bias.dim() == 4 and bias.dtype in (torch.float32, torch.bfloat16)
-    full = (B, H, Sq, Sk)
-    bst = []
-    for ax in range(4):
-        assert bias.shape[ax] in (1, full[ax]), "bias is not broadcastable to [B,H,Sq,Sk]"
-        bst.append(0 if (bias.shape[ax] == 1 and full[ax] != 1) else bias.stride(ax))
-    o = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
-    lse = torch.empty((B * H, Sq), dtype=torch.float32, device=q.device) if want_lse else None
-    rc = lib().flame_attn_fwd_bias_bf16(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), B, H, Sq, Sk, D, ctypes.c_float(scale),
-        _i64x4(q.stride()), _i64x4(k.stride()), _i64x4(v.stride()), _i64x4(o.stride()),
-        *(ctypes.c_int64(0) for _ in range(5)),
-        _ptr(bias), 1 if bias.dtype == torch.float32 else 0, _i64x4(bst),
-        _ptr(mask), _mask_strides(mask, B, H, Sq, Sk), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_attn_fwd_bias_bf16", rc)
-    return o, lse
+    return host().attn_fwd_bias(q, k, v, scale, bias, mask, want_lse)
 
 
 def bwd_workspace_bytes(B, H, Sq, D) -> int:
@@ -122,29 +110,8 @@ def bwd_workspace_bytes(B, H, Sq, D) -> int:
 def attn_bwd(q, k, v, o, do, lse, scale, causal=False, kv_len=None, mask=None, workspace=None, grads=None):
     """dQ, dK, dV = flame_attn_bwd_bf16(...).  `workspace`: uint8 device tensor of at least
     bwd_workspace_bytes(...) bytes (allocated here when omitted)."""
-    B, H, Sq, D = q.shape
-    Sk = k.shape[2]
-    need = bwd_workspace_bytes(B, H, Sq, D)
-    if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    if grads is None:
-        dq = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
-        dk = torch.empty((B, H, Sk, D), dtype=torch.bfloat16, device=q.device)
-        dv = torch.empty((B, H, Sk, D), dtype=torch.bfloat16, device=q.device)
-    else:
-        dq, dk, dv = grads
-    ms = _mask_strides(mask, B, H, Sq, Sk)
-    rc = lib().flame_attn_bwd_bf16(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv),
-        B, H, Sq, Sk, D, ctypes.c_float(scale),
-        _i64x4(q.stride()), _i64x4(k.stride()), _i64x4(v.stride()), _i64x4(o.stride()),
-        _i64x4(do.stride()), _i64x4(dq.stride()), _i64x4(dk.stride()), _i64x4(dv.stride()),
-        *(ctypes.c_int64(0) for _ in range(9)),
-        int(bool(causal)), _ptr(kv_len), _ptr(mask), ms,
-        _ptr(workspace), ctypes.c_size_t(workspace.numel()), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_attn_bwd_bf16", rc)
-    return dq, dk, dv
+    dq, dk, dv = grads if grads is not None else (None, None, None)
+    return host().attn_bwd(q, k, v, o, do, lse, scale, causal, kv_len, mask, workspace, dq, dk, dv)
 
 
 def attn_bwd_noalloc(q, k, v, o, do, lse, scale, grads, causal=False, kv_len=None, mask=None):
@@ -219,50 +186,13 @@ def sage_quant(q, k, smooth_k=True, want_ks=False):
     Returns dict(qi8, ki8, sq, sk, kmean[, ks]): int8 [B,H,S,D], fp32 [B,H,nblk], fp32 [B,H,D]; with
     want_ks also the smoothed bf16 K that was quantised.  For head dims other than 64 and 128 the library writes
     rows of sage_row_elems(D) elements, zero beyond D: the tensors returned are the [..., :D] views of those."""
-    B, H, Sq, D = q.shape
-    Sk = k.shape[2]
-    dev = q.device
-    Dp = sage_row_elems(D)
-    out = dict(
-        qi8=torch.empty((B, H, Sq, Dp), dtype=torch.int8, device=dev)[..., :D],
-        ki8=torch.empty((B, H, Sk, Dp), dtype=torch.int8, device=dev)[..., :D],
-        sq=torch.empty((B, H, -(-Sq // 128)), dtype=torch.float32, device=dev),
-        sk=torch.empty((B, H, -(-Sk // 64)), dtype=torch.float32, device=dev),
-        kmean=torch.empty((B, H, Dp), dtype=torch.float32, device=dev)[..., :D])
-    if want_ks:
-        out["ks"] = torch.empty((B, H, Sk, Dp), dtype=torch.bfloat16, device=dev)[..., :D]
-    rc = lib().flame_sage_quant_qk_int8_ks(
-        _ptr(q), _ptr(k), B, H, Sq, Sk, D, _i64x4(q.stride()), _i64x4(k.stride()),
-        ctypes.c_int64(0), ctypes.c_int64(0), int(bool(smooth_k)),
-        _ptr(out["qi8"]), _ptr(out["ki8"]), _ptr(out["sq"]), _ptr(out["sk"]), _ptr(out["kmean"]),
-        _ptr(out.get("ks")), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_sage_quant_qk_int8_ks", rc)
-    return out
+    return host().sage_quant(q, k, smooth_k, want_ks, sage_row_elems(q.shape[3]))
 
 
 def sage_fwd(qz, v, scale, causal=False, kv_len=None, want_lse=False, out=None, bias=None):
     """O (and LSE) from quantised operands `qz` (the dict returned by sage_quant) and bf16 V.
     bias: additive fp32 or bf16 [B|1, H|1, Sq, Sk] on the scaled logits (-inf excludes), or None."""
-    B, H, Sq, D = qz["qi8"].shape
-    Sk = qz["ki8"].shape[2]
-    o = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=v.device) if out is None else out
-    lse = torch.empty((B * H, Sq), dtype=torch.float32, device=v.device) if want_lse else None
-    bst, bdt = None, 1
-    if bias is not None:
-        assert bias.dim() == 4 and bias.dtype in (torch.float32, torch.bfloat16)
-        full = (B, H, Sq, Sk)
-        st = []
-        for ax in range(4):
-            assert bias.shape[ax] in (1, full[ax]), "bias is not broadcastable to [B,H,Sq,Sk]"
-            st.append(0 if (bias.shape[ax] == 1 and full[ax] != 1) else bias.stride(ax))
-        bst, bdt = _i64x4(st), (1 if bias.dtype == torch.float32 else 0)
-    rc = lib().flame_sage_attn_fwd_bias_int8(
-        _ptr(qz["qi8"]), _ptr(qz["ki8"]), _ptr(qz["sq"]), _ptr(qz["sk"]), _ptr(v), _ptr(o), _ptr(lse),
-        B, H, Sq, Sk, D, ctypes.c_float(scale), _i64x4(v.stride()), _i64x4(o.stride()),
-        ctypes.c_int64(0), ctypes.c_int64(0), int(bool(causal)), _ptr(kv_len), _ptr(bias), bdt, bst, _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_sage_attn_fwd_bias_int8", rc)
+    o, lse = host().sage_fwd(qz["qi8"], qz["ki8"], qz["sq"], qz["sk"], v, scale, causal, kv_len, want_lse, out, bias)
     return (o, lse) if want_lse else o
 
 
@@ -271,25 +201,7 @@ def prep_rmsnorm_rope(x_bnhd, weight=None, cos=None, sin=None, eps=1e-6, apply_n
 
     x_bnhd: bf16 [B,N,H,D] (any B/N/H strides); weight: bf16 [D] or None; cos/sin: [N,D/2] fp32 or
     bf16, or None.  Returns a contiguous bf16 [B,H,N,D] tensor."""
-    B, N, H, D = x_bnhd.shape
-    xv = x_bnhd.permute(0, 2, 1, 3)                       # logical [B,H,N,D] view of the same memory
-    if out is None:
-        out = torch.empty((B, H, N, D), dtype=torch.bfloat16, device=x_bnhd.device)
-    tdt = 0
-    if cos is not None:
-        if cos.dtype != sin.dtype or cos.shape != sin.shape or tuple(cos.shape) != (N, D // 2):
-            raise ValueError("cos/sin must both be [N, D/2] of one dtype")
-        if not (cos.is_contiguous() and sin.is_contiguous()):
-            raise ValueError("cos/sin must be contiguous")
-        tdt = 1 if cos.dtype == torch.float32 else 0
-    rc = lib().flame_attn_prep_rmsnorm_rope_bf16(
-        _ptr(xv), _ptr(weight) if weight is not None else None,
-        _ptr(cos) if cos is not None else None, _ptr(sin) if sin is not None else None, tdt,
-        _ptr(out), B, H, N, D, ctypes.c_float(eps), int(bool(apply_norm)),
-        _i64x4(xv.stride()), _i64x4(out.stride()), ctypes.c_int64(0), ctypes.c_int64(0), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_attn_prep_rmsnorm_rope_bf16", rc)
-    return out
+    return host().prep_rmsnorm_rope(x_bnhd, weight, cos, sin, eps, apply_norm, out)
 
 
 # ---------------------------------------------------------------- element-wise primitives on score tiles
@@ -368,24 +280,12 @@ def tile_dropout(probs, p, seed):
 # ---------------------------------------------------------------- FP8 form of offloaded activations
 def bf16_to_fp8(x, inv_scale, out=None):
     """out[i] = fp8_e4m3(float(x[i]) * inv_scale) (uint8), flame_bf16_to_fp8; x is any contiguous bf16 tensor."""
-    assert x.dtype == torch.bfloat16 and x.is_contiguous()
-    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device) if out is None else out
-    assert out.dtype == torch.uint8 and out.is_contiguous() and out.numel() == x.numel()
-    rc = lib().flame_bf16_to_fp8(_ptr(x), _ptr(out), ctypes.c_float(inv_scale), ctypes.c_size_t(x.numel()), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_bf16_to_fp8", rc)
-    return out
+    return host().fp8(x, inv_scale, out, True)
 
 
 def fp8_to_bf16(codes, scale, out=None):
     """out[i] = bf16(float(fp8(codes[i])) * scale), flame_fp8_to_bf16."""
-    assert codes.dtype == torch.uint8 and codes.is_contiguous()
-    out = torch.empty(codes.shape, dtype=torch.bfloat16, device=codes.device) if out is None else out
-    assert out.dtype == torch.bfloat16 and out.is_contiguous() and out.numel() == codes.numel()
-    rc = lib().flame_fp8_to_bf16(_ptr(codes), _ptr(out), ctypes.c_float(scale), ctypes.c_size_t(codes.numel()), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_fp8_to_bf16", rc)
-    return out
+    return host().fp8(codes, scale, out, False)
 
 
 # ---------------------------------------------------------------- dropout of the probabilities
@@ -393,42 +293,13 @@ def attn_fwd_dropout(q, k, v, scale, dropout_p, dropout_seed, causal=False, kv_l
                      draw_chunk_q=0, draw_chunk_kv=0):
     """O, LSE = flame_attn_fwd_dropout_tiled_bf16(...): the kept set of the reference's autograd_v4 operator for this
     seed; draw_chunk_q / draw_chunk_kv: the tiles it draws over when it is chunked (0 = the whole axis)."""
-    B, H, Sq, D = q.shape
-    Sk = k.shape[2]
-    o = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device) if out is None else out
-    lse = torch.empty((B * H, Sq), dtype=torch.float32, device=q.device)
-    rc = lib().flame_attn_fwd_dropout_tiled_bf16(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), B, H, Sq, Sk, D, ctypes.c_float(scale),
-        _i64x4(q.stride()), _i64x4(k.stride()), _i64x4(v.stride()), _i64x4(o.stride()),
-        *(ctypes.c_int64(0) for _ in range(5)),
-        int(bool(causal)), _ptr(kv_len), _ptr(mask), _mask_strides(mask, B, H, Sq, Sk),
-        ctypes.c_float(dropout_p), ctypes.c_uint64(dropout_seed & (2 ** 64 - 1)), int(draw_chunk_q), int(draw_chunk_kv), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_attn_fwd_dropout_tiled_bf16", rc)
-    return o, lse
+    return host().attn_fwd_dropout(q, k, v, scale, dropout_p, dropout_seed, causal, kv_len, mask, out, draw_chunk_q, draw_chunk_kv)
 
 
 def attn_bwd_dropout(q, k, v, o, do, lse, scale, dropout_p, dropout_seed, causal=False, kv_len=None, mask=None, workspace=None,
                      draw_chunk_q=0, draw_chunk_kv=0):
-    B, H, Sq, D = q.shape
-    Sk = k.shape[2]
-    if workspace is None:
-        workspace = torch.empty(bwd_workspace_bytes(B, H, Sq, D), dtype=torch.uint8, device=q.device)
-    dq = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
-    dk = torch.empty((B, H, Sk, D), dtype=torch.bfloat16, device=q.device)
-    dv = torch.empty((B, H, Sk, D), dtype=torch.bfloat16, device=q.device)
-    rc = lib().flame_attn_bwd_dropout_tiled_bf16(
-        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv),
-        B, H, Sq, Sk, D, ctypes.c_float(scale),
-        _i64x4(q.stride()), _i64x4(k.stride()), _i64x4(v.stride()), _i64x4(o.stride()),
-        _i64x4(do.stride()), _i64x4(dq.stride()), _i64x4(dk.stride()), _i64x4(dv.stride()),
-        *(ctypes.c_int64(0) for _ in range(9)),
-        int(bool(causal)), _ptr(kv_len), _ptr(mask), _mask_strides(mask, B, H, Sq, Sk),
-        ctypes.c_float(dropout_p), ctypes.c_uint64(dropout_seed & (2 ** 64 - 1)), int(draw_chunk_q), int(draw_chunk_kv),
-        _ptr(workspace), ctypes.c_size_t(workspace.numel()), _stream())
-    if rc != 0:
-        raise FlameAttnError("flame_attn_bwd_dropout_tiled_bf16", rc)
-    return dq, dk, dv
+    return host().attn_bwd_dropout(q, k, v, o, do, lse, scale, dropout_p, dropout_seed, causal, kv_len, mask, workspace, draw_chunk_q,
+                                   draw_chunk_kv)
 
 
 def materialised_workspace_bytes(B, H, Sq, Sk, D, Dv, backward) -> int:
