@@ -340,6 +340,12 @@ __device__ __forceinline__ void dma16u(const void* gbase_wave_uniform, uint32_t 
     dma16u(gbase_wave_uniform, lane_byte_off, lds_addr(lds_dst));
 }
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0) only
+// at most N of this wavefront's vector memory operations are still outstanding (they complete in order)
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit field");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 
 // Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by linear id.  Remap the id
 // so that XCD x works on the contiguous range [x*total/8, (x+1)*total/8) of tiles: all tiles of one

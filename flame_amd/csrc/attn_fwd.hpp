@@ -37,6 +37,11 @@ struct FwdParams {
     int dv;              // real head dim of V and O, likewise
     float scale;
     MaskArgs m;
+    // Key split (the key-sharing forward and the one for head dims above 128): key_splits workgroups share a query tile, each walks a contiguous slice of its key tiles and leaves a
+    // normalised fp32 partial output with its log-sum-exp; fwd_merge_kernel combines them.
+    int key_splits = 1;          // 1: O and LSE are written directly
+    float* part_o = nullptr;     // [key_splits][B*H*Sq][dv]
+    float* part_lse = nullptr;   // [key_splits][B*H*Sq], natural log, -inf for a slice without an attended key
 };
 
 template <int D>
@@ -50,15 +55,17 @@ struct FwdTile {
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;   // copies per wave and tensor
 };
 
-// VECMASK (with HASMASK): the only exclusions besides key lengths and the causal flag come from a keep-mask
-// whose rows are contiguous and 16-byte aligned, Sk is a multiple of the tile and there is no bias; the
-// general exclusion code (per-element loads, bias) is then not compiled in, which frees the registers
-// that made the general masked kernel spill.
+// What a forward kernel excludes besides keys past the key length and, with the causal flag, past the query.
+enum FwdExcl : int {
+    kExNone = 0,
+    kExRows16 = 1,       // uint8 keep-mask, rows contiguous and 16-byte aligned, Sk a multiple of the tile, no bias
+    kExGeneral = 2,      // any keep-mask and / or bias, one element at a time
+};
+
 // DROPOUT: the probabilities that multiply V are dropped and rescaled element by element (drop_factor); the row sums,
 // and with them the log-sum-exp, stay those of the undropped softmax.
-template <int D, bool HASMASK, int NW, bool VECMASK = false, bool DROPOUT = false>
+template <int D, int EXCL, int NW, bool DROPOUT = false>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const FwdParams p) {
-    static_assert(!VECMASK || HASMASK, "VECMASK is a special case of HASMASK");
     using T = FwdTile<D>;
     constexpr int BN = T::BN, RS = T::RS;
     constexpr int BM = 32 * NW;  // query rows per workgroup
@@ -68,9 +75,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     constexpr int NDMA = T::DMA_PER_WAVE * 4 / NW;
     constexpr int PD = 4;        // LDS read-ahead depth, in fragments
     // Tile t lives in stage t % 2; K runs 2 tiles and V 1 tile ahead of use, one barrier per step.
-    // (Measured: four stages with deeper prefetch, or a barrier only every second step, are slower.)
-    constexpr int NSTAGE = 2;
-    constexpr int KD = NSTAGE / 2 + 1, VD = NSTAGE / 2;      // prefetch distances, in tiles
+    // (Measured: four stages with counted waits, or a barrier only every second step, are not faster, not even for a
+    // workgroup that has its compute unit to itself: the step is bound by instruction issue, not by the copies.)
+    constexpr int KD = 2, VD = 1;
     static_assert((2 * DC) % PD == 0 && (4 * DB) % PD == 0, "read-ahead depth must divide the fragment counts");
     static_assert(2 * DC == 16 || 2 * DC == 8, "softmax slicing assumes 16 or 8 logit MFMAs per tile");
 
@@ -88,35 +95,24 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 32;
+    const int qi = qw0 + n;                           // this lane's query
 
     const uint16_t* qbase = p.q + b * p.qs.b + hh * p.qs.h;
     const uint16_t* kbase = p.k + b * p.ks.b + hh * p.ks.h;
     const uint16_t* vbase = p.v + b * p.vs.b + hh * p.vs.h;
-    uint16_t* obase = p.o + b * p.os.b + hh * p.os.h;
 
     int klimit = p.Sk;
     if (p.m.kv_len) klimit = min(klimit, max(p.m.kv_len[b], 0));
     int kend = klimit;
     if (p.m.causal) kend = min(kend, q0 + BM);
     const int n_tiles = (kend + BN - 1) / BN;
-    const uint8_t* mbase = (HASMASK && p.m.mask) ? mask_head_base(p.m, b, hh) : nullptr;
-    const char* bbase = (HASMASK && p.m.bias)
+    const uint8_t* mbase = (EXCL != kExNone && p.m.mask) ? mask_head_base(p.m, b, hh) : nullptr;
+    const char* bbase = (EXCL == kExGeneral && p.m.bias)
                             ? static_cast<const char*>(p.m.bias) + (b * p.m.bb + hh * p.m.bh) * (p.m.bias_f32 ? 4 : 2)
                             : nullptr;
 
-    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d
-    bf16x8 qf[DC];
-    {
-        const int row = qw0 + n;
-        const bool ok = row < p.Sq;
-        const uint16_t* rp = qbase + (int64_t)row * p.qs.n + 8 * h;
-#pragma unroll
-        for (int dc = 0; dc < DC; ++dc) qf[dc] = __builtin_bit_cast(bf16x8, ldg16(rp + 16 * dc, ok && 16 * dc + 8 * h < p.d));
-    }
-
-    // ---- asynchronous tile copies.  K(t) and V(t) live in stage t&1.  Full tiles: uniform tile base
-    //      + a per-lane 32-bit byte offset that never changes; ragged tiles clamp their rows into the
-    //      attended range.
+    // ---- asynchronous tile copies.  Full tiles: uniform tile base + a per-lane 32-bit byte offset that never changes;
+    //      ragged tiles clamp their rows into the attended range.
     const uint32_t lds0 = lds_addr(lds);
     const int dma_row_in = lane / GPR;                       // row inside one 1 KiB copy
     const int dma_gran = lane % GPR;                         // physical granule written by this lane
@@ -129,19 +125,21 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
         v_lane_off[i] = 2u * (uint32_t)(row * (int)p.vs.n + src_granule(c, p.dv) * 8);
     }
     auto dst_of = [&](int t, int which, int i) {             // LDS byte address of copy i of this wave
-        return lds0 + 2u * (uint32_t)((t & (NSTAGE - 1)) * T::STAGE_ELEMS + which * T::TILE_ELEMS + (wave * NDMA + i) * 512);
+        return lds0 + 2u * (uint32_t)((t & 1) * T::STAGE_ELEMS + which * T::TILE_ELEMS + (wave * NDMA + i) * 512);
     };
-    auto issue_ragged = [&](const uint16_t* base, int64_t row_stride, int t, int which) {
+    // any tile: rows past the attended range re-read the last attended key, which lies `over` rows further up
+    const int dma_row0 = wave * NDMA * T::ROWS_PER_DMA + dma_row_in;
+    auto issue_any = [&](const uint16_t* base, int64_t row_stride, const uint32_t (&lane_off)[NDMA], int t, int which) {
+        const uint16_t* tb = base + (int64_t)t * BN * row_stride;
+        const int row_max = klimit - 1 - t * BN;             // not negative for a tile that is walked
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
-            const int row = (wave * NDMA + i) * T::ROWS_PER_DMA + dma_row_in;
-            const int key = min(t * BN + row, klimit - 1);   // tail rows re-read the last attended key
-            const int c = src_granule(dma_gran ^ swz<D>(row), which ? p.dv : p.d);
-            dma16(base + (int64_t)key * row_stride + c * 8, dst_of(t, which, i));
+            const int over = max(dma_row0 + i * T::ROWS_PER_DMA - row_max, 0);
+            dma16u(tb, lane_off[i] - 2u * (uint32_t)(over * (int)row_stride), dst_of(t, which, i));
         }
     };
-    auto issue_k = [&](int t) { issue_ragged(kbase, p.ks.n, t, 0); };
-    auto issue_v = [&](int t) { issue_ragged(vbase, p.vs.n, t, 1); };
+    auto issue_k = [&](int t) { issue_any(kbase, p.ks.n, k_lane_off, t, 0); };
+    auto issue_v = [&](int t) { issue_any(vbase, p.vs.n, v_lane_off, t, 1); };
     auto issue_full_kv = [&](int tk, int tv) {               // K tile tk and V tile tv, both full
         const uint16_t* kt = kbase + (int64_t)tk * BN * p.ks.n;
         const uint16_t* vt = vbase + (int64_t)tv * BN * p.vs.n;
@@ -151,6 +149,21 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             dma16u(vt, v_lane_off[i], dst_of(tv, 1, i));
         }
     };
+    // the first tiles are on their way before anything else is loaded: on short walks their round trip is the run time
+#pragma unroll
+    for (int i = 0; i < KD; ++i) {
+        if (i < n_tiles) issue_k(i);
+        if (i < VD && i < n_tiles) issue_v(i);
+    }
+
+    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d
+    bf16x8 qf[DC];
+    {
+        const bool ok = qi < p.Sq;
+        const uint16_t* rp = qbase + (int64_t)qi * p.qs.n + 8 * h;
+#pragma unroll
+        for (int dc = 0; dc < DC; ++dc) qf[dc] = __builtin_bit_cast(bf16x8, ldg16(rp + 16 * dc, ok && 16 * dc + 8 * h < p.d));
+    }
 
     // ---- per-lane LDS read offsets (elements), constant over the key loop
     int koff[DC];          // K fragment: row 32*kb + n, logical granule 2*dc + h
@@ -166,11 +179,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             voff[half][db] = row * RS + (((4 * db + 2 * tr_g16 + ((tr_r & 3) >> 1)) ^ swz<D>(row)) << 3) + 4 * (tr_r & 1);
     }
     auto k_frag = [&](int t, int i) {       // fragment i = (dc, kb) of K(t)
-        const uint16_t* ks = lds + (t & (NSTAGE - 1)) * T::STAGE_ELEMS;
+        const uint16_t* ks = lds + (t & 1) * T::STAGE_ELEMS;
         return *reinterpret_cast<const bf16x8*>(ks + koff[i >> 1] + 32 * (i & 1) * RS);
     };
     auto v_frag = [&](int t, int i) {       // fragment i = (cc, db) of V(t)^T
-        const uint16_t* vs = lds + (t & (NSTAGE - 1)) * T::STAGE_ELEMS + T::TILE_ELEMS;
+        const uint16_t* vs = lds + (t & 1) * T::STAGE_ELEMS + T::TILE_ELEMS;
         const int cc = i / DB, db = i % DB;
         const u32x2 lo = lds_read_tr16(vs + voff[0][db] + 16 * cc * RS);
         const u32x2 hi = lds_read_tr16(vs + voff[1][db] + 16 * cc * RS);
@@ -191,30 +204,34 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     constexpr int NS = 2 * DC;     // logit MFMAs per tile
     constexpr int NP = 4 * DB;     // PV MFMAs per tile
     constexpr int EPS = 32 / NS;   // logits handled per softmax slice
+    constexpr int MPS = 32 / NP;   // logits handled per maximum-scan slice
 
     // flat index (mod 2^32) of this lane's query row in the [B*H, Sq, Sk] probability tensor
-    const uint32_t drop_qi = (uint32_t)(qw0 + n);
+    const uint32_t drop_qi = (uint32_t)qi;
     (void)drop_qi;
-    // exclusions of tile t: ragged tail / key length, causal, explicit keep-mask
-    auto apply_mask = [&](f32x16 (&s)[2], int t) {
-        const int qi = qw0 + n;
-        if constexpr (VECMASK) {
-            MaskRow64 mrow;
+    // Exclusions of a tile.  The ragged tail / key length and the causal diagonal are one comparison per element with a
+    // per-lane limit (excl_elem, threaded into the maximum scan); a keep-mask row is fetched when the step begins; the
+    // general mask and bias are applied in one go (excl_general).
+    int lim = 0;                   // keys of the tile below it attend, counted from 4h
+    MaskRow64 mrow;
+    auto excl_begin = [&](int t) {
+        const int limit = (p.m.causal ? min(klimit, qi + 1) : klimit) - t * BN;
+        lim = limit - 4 * h;
+        if constexpr (EXCL == kExRows16) {
+            // folded into the mask bytes where they cut the tile: the per-element test is then the mask byte alone
             mrow.load(mbase + (int64_t)min(qi, p.Sq - 1) * p.m.sq + t * BN);
-            // the key length and the causal diagonal cut few tiles: there they are folded into the mask bytes,
-            // so that the per-element test is the mask byte alone
-            const int lim = (p.m.causal ? min(klimit, qi + 1) : klimit) - t * BN;
-            if (__any(lim < BN)) mrow.restrict_to(lim);
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[kb][r] = mrow.keep(kb, r, h) ? s[kb][r] : -INFINITY;
-            return;
+            if (__any(limit < BN)) mrow.restrict_to(limit);
         }
+    };
+    auto excl_elem = [&](f32x16 (&s)[2], int idx) {
+        const int kb = idx >> 4, r = idx & 15;
+        if constexpr (EXCL == kExRows16) s[kb][r] = mrow.keep(kb, r, h) ? s[kb][r] : -INFINITY;
+        if constexpr (EXCL == kExNone) s[kb][r] = 32 * kb + 8 * (r >> 2) + (r & 3) >= lim ? -INFINITY : s[kb][r];
+    };
+    auto excl_general = [&](f32x16 (&s)[2], int t) {
         // a lane's 64 keep-mask bytes of the tile in four 16-byte loads where the layout allows it (each
         // lane owns a query row, so byte loads would touch one cache line per lane and element)
-        const bool vec_mask = HASMASK && mbase && p.m.rows16 && t * BN + BN <= p.Sk;
-        MaskRow64 mrow;
+        const bool vec_mask = mbase && p.m.rows16 && t * BN + BN <= p.Sk;
         if (vec_mask) mrow.load(mbase + (int64_t)min(qi, p.Sq - 1) * p.m.sq + t * BN);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -223,18 +240,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 const int key = t * BN + 32 * kb + acc_row(r, h);
                 bool drop = (key >= klimit) | ((p.m.causal != 0) & (key > qi));     // bitwise: selects, not branches
                 float val = s[kb][r];
-                if (HASMASK) {
-                    if (vec_mask) drop = drop || !mrow.keep(kb, r, h);
-                    else if (mbase && !drop && qi < p.Sq) drop = !mask_attends(p.m, mbase, (int64_t)qi * p.m.sq + (int64_t)key * p.m.sk);
-                    if (bbase) {      // scale * (s + bias / scale) = scale * s + bias
-                        float bv = 0.f;
-                        if (!drop && qi < p.Sq) {
-                            const int64_t e = (int64_t)qi * p.m.bq + (int64_t)key * p.m.bk;
-                            bv = p.m.bias_f32 ? reinterpret_cast<const float*>(bbase)[e]
-                                              : __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(bbase)[e] << 16);
-                        }
-                        val = fmaf(bv, p.m.inv_scale, val);
+                if (vec_mask) drop = drop || !mrow.keep(kb, r, h);
+                else if (mbase && !drop && qi < p.Sq) drop = !mask_attends(p.m, mbase, (int64_t)qi * p.m.sq + (int64_t)key * p.m.sk);
+                if (bbase) {      // scale * (s + bias / scale) = scale * s + bias
+                    float bv = 0.f;
+                    if (!drop && qi < p.Sq) {
+                        const int64_t e = (int64_t)qi * p.m.bq + (int64_t)key * p.m.bk;
+                        bv = p.m.bias_f32 ? reinterpret_cast<const float*>(bbase)[e]
+                                          : __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(bbase)[e] << 16);
                     }
+                    val = fmaf(bv, p.m.inv_scale, val);
                 }
                 s[kb][r] = drop ? -INFINITY : val;   // select, not a divergent store
             }
@@ -265,15 +280,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     };
 
     // One step: P(t) from the logits in `cur`, logits of tile t+1 into `nxt`, O += P(t) V(t).
-    // FAST: tile t+1 needs no exclusions and K(t+KD), V(t+VD) are full tiles (straight-line copies and
-    // the interleaved instruction stream).  Otherwise every decision is taken at run time and the
-    // phases run one after the other.
-    auto step = [&](auto fast_tag, f32x16 (&cur)[2], f32x16 (&nxt)[2], int t) {
-        constexpr bool FAST = decltype(fast_tag)::value;
-        const bool has_next = FAST || t + 1 < n_tiles;
-        if (FAST) {
+    // COPY: K(t+KD) and V(t+VD) exist and are full tiles (straight-line copies); else decided at run time.
+    // NEXT: 0 = tile t+1 needs no exclusions, 1 = it does, 2 = tile t is the last one.
+    auto step = [&](auto copy_tag, auto next_tag, f32x16 (&cur)[2], f32x16 (&nxt)[2], int t) {
+        constexpr bool COPY = decltype(copy_tag)::value;
+        constexpr int NEXT = decltype(next_tag)::value;
+        if constexpr (COPY) {
             issue_full_kv(t + KD, t + VD);
-        } else {
+        } else if constexpr (NEXT != 2) {
             if (t + KD < n_tiles) issue_k(t + KD);
             if (t + VD < n_tiles) issue_v(t + VD);
         }
@@ -303,8 +317,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 }
             }
         };
-
-        if (FAST) {
+        if constexpr (NEXT == 2) {
+#pragma unroll
+            for (int i = 0; i < PD; ++i) {
+                fb[i] = v_frag(t, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int j = 0; j < NS; ++j) exp_slice(j);
+            l_run += rsum0 + rsum1;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                oacc[i % DB] = mfma32(fb[i % PD], pf[i / DB], oacc[i % DB]);
+                if (i + PD < NP) fb[i % PD] = v_frag(t, i + PD);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            if (NEXT == 1) excl_begin(t + 1);
             // ---- S(t+1)^T = K(t+1) Q^T between the exponentials of tile t
             zero_tile(nxt);
 #pragma unroll
@@ -328,13 +357,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 __builtin_amdgcn_sched_barrier(0);
             }
             l_run += rsum0 + rsum1;
+            if (NEXT == 1 && EXCL == kExGeneral) excl_general(nxt, t + 1);
             // ---- O^T += V(t)^T P(t)^T between the row-maximum scan of tile t+1
-            float tmax = nxt[0][0];
-            constexpr int MPS = 32 / NP;
+            float tmax = -INFINITY;
             auto max_slice = [&](int i) {
 #pragma unroll
                 for (int e = 0; e < MPS; e += 2) {
                     const int idx = MPS * i + e;
+                    if (NEXT == 1) {
+                        excl_elem(nxt, idx);
+                        excl_elem(nxt, idx + 1);
+                    }
                     tmax = fmaxf(fmaxf(tmax, nxt[idx >> 4][idx & 15]), nxt[(idx + 1) >> 4][(idx + 1) & 15]);
                 }
             };
@@ -352,69 +385,30 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 __builtin_amdgcn_sched_barrier(0);
             }
             fold_max(tmax);
-        } else {
-            if (has_next) {
-                zero_tile(nxt);
-#pragma unroll
-                for (int i = 0; i < PD; ++i) {
-                    fb[i] = k_frag(t + 1, i);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int i = 0; i < NS; ++i) {
-                    nxt[i & 1] = mfma32(fb[i % PD], qf[i >> 1], nxt[i & 1]);
-                    if (i + PD < NS) fb[i % PD] = k_frag(t + 1, i + PD);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                apply_mask(nxt, t + 1);
-            }
-#pragma unroll
-            for (int j = 0; j < NS; ++j) exp_slice(j);
-            l_run += rsum0 + rsum1;
-#pragma unroll
-            for (int i = 0; i < PD; ++i) {
-                fb[i] = v_frag(t, i);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-#pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                oacc[i % DB] = mfma32(fb[i % PD], pf[i / DB], oacc[i % DB]);
-                if (i + PD < NP) fb[i % PD] = v_frag(t, i + PD);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (has_next) {
-                float tmax = nxt[0][0];
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, nxt[kb][r]);
-                fold_max(tmax);
-            }
+            wait_vm0();          // the copies issued by this step have landed
+            __syncthreads();     // ... for every wave, and everyone is done reading this step's tiles
         }
-        wait_vm0();          // the copies issued by this step have landed
-        __syncthreads();     // ... for every wave, and everyone is done reading this step's tiles
     };
 
-    // Tiles [0, n_full) need no exclusions for any query of the workgroup; the rest (ragged tail, causal
+    // Tiles below t_clean need no exclusions for any query of the workgroup; the rest (ragged tail, causal
     // diagonal, or everything under an explicit mask) carry per-element exclusions.
-    int n_full = HASMASK ? 0 : klimit / BN;
-    if (p.m.causal) n_full = min(n_full, (q0 + 1) / BN);
-    n_full = min(n_full, n_tiles);
+    int t_clean = EXCL != kExNone ? 0 : klimit / BN;
+    if (p.m.causal) t_clean = min(t_clean, (q0 + 1) / BN);
+    t_clean = min(t_clean, n_tiles);
 
     f32x16 sa[2], sb[2];
     if (n_tiles > 0) {
-        // prologue: the first KD tiles of K and VD tiles of V land; logits and maximum of tile 0
-#pragma unroll
-        for (int i = 0; i < KD; ++i) {
-            if (i < n_tiles) issue_k(i);
-            if (i < VD && i < n_tiles) issue_v(i);
-        }
         wait_vm0();
         __syncthreads();
+        if (t_clean == 0) excl_begin(0);
         zero_tile(sa);
 #pragma unroll
         for (int i = 0; i < NS; ++i) sa[i & 1] = mfma32(k_frag(0, i), qf[i >> 1], sa[i & 1]);
-        if (n_full < 1) apply_mask(sa, 0);
+        if (t_clean == 0) {
+            if (EXCL == kExGeneral) excl_general(sa, 0);
+#pragma unroll
+            for (int idx = 0; idx < 32; ++idx) excl_elem(sa, idx);
+        }
         float tmax = sa[0][0];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -423,41 +417,90 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
         fold_max(tmax);
         __syncthreads();     // every wave has read K(0) before step 0 starts overwriting it
 
-        // step t is FAST when t + KD < n_full; an even number of them keeps `sa` the current tile
-        const int n_fast = max(0, n_full - KD) & ~1;
+        using Yes = std::true_type;
+        using No = std::false_type;
+        using Clean = std::integral_constant<int, 0>;
+        using Cut = std::integral_constant<int, 1>;
+        using Last = std::integral_constant<int, 2>;
+        // Two steps per trip, so that `sa` is the current tile when t is even; where the number of steps of
+        // one kind is odd, the pair that mixes kinds runs as the more general one.
         int t = 0;
-        for (; t < n_fast; t += 2) {
-            step(std::true_type{}, sa, sb, t);
-            step(std::true_type{}, sb, sa, t + 1);
+        if (EXCL == kExNone) {
+            const int copy_end = t_clean - KD;              // steps below it copy two full tiles
+            for (; t + 1 < copy_end; t += 2) {
+                step(Yes{}, Clean{}, sa, sb, t);
+                step(Yes{}, Clean{}, sb, sa, t + 1);
+            }
+            for (; t + 2 < t_clean; t += 2) {
+                step(No{}, Clean{}, sa, sb, t);
+                step(No{}, Clean{}, sb, sa, t + 1);
+            }
         }
-        for (; t < n_tiles; t += 2) {
-            step(std::false_type{}, sa, sb, t);
-            if (t + 1 < n_tiles) step(std::false_type{}, sb, sa, t + 1);
+        if (EXCL != kExNone) {
+            const int copy_end = min(n_tiles, klimit / BN) - KD;
+            for (; t + 1 < copy_end; t += 2) {
+                step(Yes{}, Cut{}, sa, sb, t);
+                step(Yes{}, Cut{}, sb, sa, t + 1);
+            }
+        }
+        for (; t + 2 < n_tiles; t += 2) {
+            step(No{}, Cut{}, sa, sb, t);
+            step(No{}, Cut{}, sb, sa, t + 1);
+        }
+        if (t + 1 < n_tiles) {
+            step(No{}, Cut{}, sa, sb, t);
+            step(No{}, Last{}, sb, sa, t + 1);
+        } else {
+            step(No{}, Last{}, sa, sb, t);
         }
     }
 
     // ---- epilogue
-    {
-        const int row = qw0 + n;
+    if (qi < p.Sq) {
         const float l = l_run + xhalf(l_run);
         const float inv = l > 0.f ? 1.0f / l : 0.f;
-        if (row < p.Sq) {
-            uint16_t* orow = obase + (int64_t)row * p.os.n;
+        uint16_t* orow = p.o + b * p.os.b + hh * p.os.h + (int64_t)qi * p.os.n;
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const f32x16& a = oacc[db];
-                    u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv),
-                               pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
-                    if (32 * db + 8 * g + 4 * h < p.dv) *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * g + 4 * h) = w;
-                }
-            if (p.lse && h == 0) {
-                const float v = l > 0.f ? (m_run * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
-                p.lse[(int64_t)bh * p.Sq + row] = v;
+            for (int g = 0; g < 4; ++g) {
+                const f32x16& a = oacc[db];
+                u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv),
+                           pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
+                if (32 * db + 8 * g + 4 * h < p.dv) *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * g + 4 * h) = w;
             }
+        if (p.lse && h == 0) p.lse[(int64_t)bh * p.Sq + qi] = l > 0.f ? (m_run * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
+    }
+}
+
+// Combines the partial outputs of a key split: LSE = log sum_s exp(LSE_s), O = sum_s exp(LSE_s - LSE) O_s.  One lane
+// per query row and 4 output columns.
+static __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p) {
+    const int groups = p.dv >> 2;
+    const int64_t rows = (int64_t)p.B * p.H * p.Sq;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= rows * groups) return;
+    const int64_t row = idx / groups;
+    const int g = (int)(idx % groups);
+    float m = -INFINITY;
+    for (int s = 0; s < p.key_splits; ++s) m = fmaxf(m, p.part_lse[s * rows + row]);
+    float sum = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (m != -INFINITY) {
+        for (int s = 0; s < p.key_splits; ++s) {
+            const float w = expf(p.part_lse[s * rows + row] - m);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(p.part_o + (s * rows + row) * p.dv + 4 * g);
+            sum += w;
+            acc[0] = fmaf(w, v[0], acc[0]); acc[1] = fmaf(w, v[1], acc[1]);
+            acc[2] = fmaf(w, v[2], acc[2]); acc[3] = fmaf(w, v[3], acc[3]);
         }
     }
+    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+    const int64_t bh = row / p.Sq, qi = row % p.Sq;
+    uint16_t* orow = p.o + (bh / p.H) * p.os.b + (bh % p.H) * p.os.h + qi * p.os.n;
+    const u32x2 w = {pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv)};
+    *reinterpret_cast<u32x2*>(orow + 4 * g) = w;
+    if (p.lse && g == 0) p.lse[row] = sum > 0.f ? m + logf(sum) : -INFINITY;
 }
 
 // ------------------------------------------------------------------- forward, 256-query workgroups

@@ -41,22 +41,13 @@ struct FwdBigDTile {
     static constexpr int COPIES_PER_WAVE = NC * 8 / NW;        // 1 KiB copies (4 rows of one chunk) per tensor and wave
 };
 
-// A problem with few query tiles leaves most compute units idle; then key_splits workgroups share a query tile, each
-// walks a contiguous slice of its key tiles and writes a normalised fp32 partial output with its log-sum-exp, and
-// fwd_bigd_merge_kernel combines them (the partial sums of flash decoding).
-struct FwdBigDParams : FwdParams {
-    int key_splits;      // 1: no split, O and LSE are written directly
-    float* part_o;       // [key_splits][B*H*Sq][dv]
-    float* part_lse;     // [key_splits][B*H*Sq], natural log, -inf for a slice without an attended key
-};
-
 // the other of the two LDS stages, as a constant where the stage is one
 template <int P>
 __device__ constexpr std::integral_constant<int, 1 - P> other_stage(std::integral_constant<int, P>) { return {}; }
 __device__ inline int other_stage(int stage) { return stage ^ 1; }
 
 template <int NC, bool SPLIT, int NW>
-__global__ __launch_bounds__(64 * NW) void fwd_bigd_kernel(const FwdBigDParams p) {
+__global__ __launch_bounds__(64 * NW) void fwd_bigd_kernel(const FwdParams p) {
     using T = FwdBigDTile<NC, SPLIT, NW>;
     constexpr int BN = T::BN, BM = T::BM, NDB = T::NDB;
     constexpr int NCP = T::COPIES_PER_WAVE;
@@ -406,36 +397,6 @@ __global__ __launch_bounds__(64 * NW) void fwd_bigd_kernel(const FwdBigDParams p
                 }
         if (p.lse && h == 0 && db0 == 0) p.lse[(int64_t)bh * p.Sq + qi] = lse_val;
     }
-}
-
-// Combines the partial outputs of a key split: LSE = log sum_s exp(LSE_s), O = sum_s exp(LSE_s - LSE) O_s.  One lane
-// per query row and 4 output columns.
-__global__ __launch_bounds__(256) void fwd_bigd_merge_kernel(const FwdBigDParams p) {
-    const int groups = p.dv >> 2;
-    const int64_t rows = (int64_t)p.B * p.H * p.Sq;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= rows * groups) return;
-    const int64_t row = idx / groups;
-    const int g = (int)(idx % groups);
-    float m = -INFINITY;
-    for (int s = 0; s < p.key_splits; ++s) m = fmaxf(m, p.part_lse[s * rows + row]);
-    float sum = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (m != -INFINITY) {
-        for (int s = 0; s < p.key_splits; ++s) {
-            const float w = expf(p.part_lse[s * rows + row] - m);
-            const f32x4 v = *reinterpret_cast<const f32x4*>(p.part_o + (s * rows + row) * p.dv + 4 * g);
-            sum += w;
-            acc[0] = fmaf(w, v[0], acc[0]); acc[1] = fmaf(w, v[1], acc[1]);
-            acc[2] = fmaf(w, v[2], acc[2]); acc[3] = fmaf(w, v[3], acc[3]);
-        }
-    }
-    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-    const int64_t bh = row / p.Sq, qi = row % p.Sq;
-    uint16_t* orow = p.o + (bh / p.H) * p.os.b + (bh % p.H) * p.os.h + qi * p.os.n;
-    const u32x2 w = {pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv)};
-    *reinterpret_cast<u32x2*>(orow + 4 * g) = w;
-    if (p.lse && g == 0) p.lse[row] = sum > 0.f ? m + logf(sum) : -INFINITY;
 }
 
 }  // namespace fattn

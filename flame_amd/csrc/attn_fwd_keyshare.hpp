@@ -1,0 +1,233 @@
+// Forward for problems with few query tiles: a few new rows of a decoder against the keys and values of all earlier ones,
+// or short and few sequences in general.  A workgroup takes 32 queries of one (batch, head) and its four wavefronts share
+// the keys: each walks every fourth 32-key tile on its own (own LDS stages, no barrier in the loop), with the copies of
+// its next tile always in flight, and the four partial softmaxes meet in LDS at the end.  Against fwd_kernel (128 queries
+// per workgroup, every wavefront walks all keys) a problem becomes four times as many workgroups with a quarter of the
+// walk, which is what a grid that does not fill the chip needs; K and V are read four times as often, from L2 mostly.
+// With one query tile the kernel is bound by reading K and V once; all 32 query columns of the MFMAs are computed whatever
+// Sq is, the matrix cores being far from busy then.  Where even these workgroups leave compute units idle the keys are
+// split over workgroups as well (FwdParams::key_splits) and fwd_merge_kernel combines the slices.
+#pragma once
+#include "attn_fwd.hpp"
+
+namespace fattn {
+
+template <int D>
+struct FwdKeyShareTile {
+    static constexpr int BQ = 32, BN = 32, NW = 4, NSTAGE = 2;
+    static constexpr int TILE_ELEMS = BN * D;                          // K or V
+    static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;
+    static constexpr int WAVE_ELEMS = NSTAGE * STAGE_ELEMS;            // a wavefront's own stages
+    static constexpr int ROWS_PER_DMA = 1024 / (D * 2);
+    static constexpr int NDMA = BN / ROWS_PER_DMA;                     // copies per tile and tensor
+    static constexpr int O_STRIDE = D + 4;                             // floats; row stride of the partial outputs in LDS
+    static constexpr int ML_FLOATS = NW * BQ * 2;                      // per wavefront and query: maximum and sum
+    static constexpr int LDS_BYTES = NW * WAVE_ELEMS * 2 + ML_FLOATS * 4;
+    static_assert(BQ * O_STRIDE * 4 <= WAVE_ELEMS * 2, "a wavefront's partial output fits its stages");
+};
+
+// DROPOUT as in fwd_kernel.
+template <int D, bool DROPOUT>
+__global__ __launch_bounds__(256) void fwd_keyshare_kernel(const FwdParams p) {
+    using T = FwdKeyShareTile<D>;
+    constexpr int BN = T::BN, NW = T::NW, DC = D / 16, DB = D / 32, GPR = D / 8, NDMA = T::NDMA;
+
+    extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, h = lane >> 5;
+
+    const int n_qt = (p.Sq + T::BQ - 1) / T::BQ;
+    const int all = xcd_remap(blockIdx.x, gridDim.x);            // the workgroups of a (batch, head) share an L2
+    const int slice = all % p.key_splits, wg = all / p.key_splits;
+    const int bh = wg / n_qt, qi = (wg % n_qt) * T::BQ + n, q0 = (wg % n_qt) * T::BQ;     // qi: this lane's query
+    const int b = bh / p.H, hh = bh % p.H;
+    const uint16_t* qbase = p.q + b * p.qs.b + hh * p.qs.h;
+    const uint16_t* kbase = p.k + b * p.ks.b + hh * p.ks.h;
+    const uint16_t* vbase = p.v + b * p.vs.b + hh * p.vs.h;
+
+    int klimit = p.Sk;
+    if (p.m.kv_len) klimit = min(klimit, max(p.m.kv_len[b], 0));
+    int kend = klimit;
+    if (p.m.causal) kend = min(kend, q0 + T::BQ);
+    const int n_tiles_all = (kend + BN - 1) / BN;
+    const int per = (n_tiles_all + p.key_splits - 1) / p.key_splits;
+    const int t_lo = slice * per, t_hi = min(n_tiles_all, t_lo + per);
+
+    // ---- tile copies: this wavefront's tiles are t_lo + wave, + NW, ...; its j-th lives in stage j % 2
+    uint16_t* const own = lds + wave * T::WAVE_ELEMS;
+    const uint32_t lds0 = lds_addr(own);
+    const int row_in = lane / GPR, gran = lane % GPR;
+    uint32_t k_lane_off[NDMA], v_lane_off[NDMA];                // bytes
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+        const int row = i * T::ROWS_PER_DMA + row_in;
+        const int c = gran ^ swz<D>(row);
+        k_lane_off[i] = 2u * (uint32_t)(row * (int)p.ks.n + src_granule(c, p.d) * 8);
+        v_lane_off[i] = 2u * (uint32_t)(row * (int)p.vs.n + src_granule(c, p.dv) * 8);
+    }
+    auto issue_tile = [&](int t, int stage) {
+        const uint16_t* kt = kbase + (int64_t)t * BN * p.ks.n;
+        const uint16_t* vt = vbase + (int64_t)t * BN * p.vs.n;
+        const uint32_t dst = lds0 + 2u * (uint32_t)(stage * T::STAGE_ELEMS);
+        const int row_max = klimit - 1 - t * BN;                 // not negative for a tile that is walked
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) {      // rows past the attended range re-read the last attended key, `over` rows further up
+            const int over = max(i * T::ROWS_PER_DMA + row_in - row_max, 0);
+            dma16u(kt, k_lane_off[i] - 2u * (uint32_t)(over * (int)p.ks.n), dst + 1024u * i);
+        }
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) {
+            const int over = max(i * T::ROWS_PER_DMA + row_in - row_max, 0);
+            dma16u(vt, v_lane_off[i] - 2u * (uint32_t)(over * (int)p.vs.n), dst + 2u * T::TILE_ELEMS + 1024u * i);
+        }
+    };
+
+    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d
+    bf16x8 qf[DC];
+    {
+        const uint16_t* rp = qbase + (int64_t)qi * p.qs.n + 8 * h;
+#pragma unroll
+        for (int dc = 0; dc < DC; ++dc) qf[dc] = __builtin_bit_cast(bf16x8, ldg16(rp + 16 * dc, qi < p.Sq && 16 * dc + 8 * h < p.d));
+    }
+    // before the first copies: the compiler's wait for these loads must not become one for the copies behind them
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) asm volatile("" : "+v"(qf[dc]));
+    int t = t_lo + wave;
+    if (t < t_hi) issue_tile(t, 0);
+
+    int koff[DC];
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) koff[dc] = n * D + (((2 * dc + h) ^ swz<D>(n)) << 3);
+    const int tr_r = lane & 15, tr_g16 = (lane >> 4) & 1;
+    int voff[2][DB];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const int row = 4 * h + (tr_r >> 2) + 8 * half;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            voff[half][db] = row * D + (((4 * db + 2 * tr_g16 + ((tr_r & 3) >> 1)) ^ swz<D>(row)) << 3) + 4 * (tr_r & 1);
+    }
+
+    const float c_log2 = p.scale * kLog2e;
+    float m_run = -INFINITY, l_run = 0.f;          // both halves of a wave hold the same maximum, each its own part of the sum
+    f32x16 oacc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
+
+    for (int j = 0; t < t_hi; t += NW, ++j) {
+        const int stage = j & 1;
+        if (t + NW < t_hi) {
+            issue_tile(t + NW, stage ^ 1);
+            wait_vm<2 * NDMA>();                   // this tile has landed, the next one is in flight
+        } else {
+            wait_vm0();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const uint16_t* ks = own + stage * T::STAGE_ELEMS;
+        const uint16_t* vs = ks + T::TILE_ELEMS;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+        for (int dc = 0; dc < DC; ++dc) s = mfma32(*reinterpret_cast<const bf16x8*>(ks + koff[dc]), qf[dc], s);
+        const int lim = (p.m.causal ? min(klimit, qi + 1) : klimit) - t * BN - 4 * h;
+        if (__any(lim < BN))
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) >= lim ? -INFINITY : s[r];
+        float tmax = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
+        tmax = fmaxf(tmax, xhalf(tmax));
+        if (__any(tmax > m_run)) {
+            const float m_new = fmaxf(m_run, tmax);
+            const float m_to = (m_new == -INFINITY) ? 0.f : m_new;
+            const float alpha = exp2_fast((m_run - m_to) * c_log2);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+        }
+        const float msc = ((m_run == -INFINITY) ? 0.f : m_run) * c_log2;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s[r] = exp2_fast(fmaf(s[r], c_log2, -msc));
+            l_run += s[r];
+            if constexpr (DROPOUT)
+                s[r] *= drop_factor_at(p.m, (uint32_t)bh, (uint32_t)qi, (uint32_t)(t * BN + acc_row(r, h)), (uint32_t)p.Sq, (uint32_t)p.Sk);
+        }
+        bf16x8 pf[2];
+        pf[0] = pack8(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]);
+        pf[1] = pack8(s[8], s[9], s[10], s[11], s[12], s[13], s[14], s[15]);
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const u32x2 lo = lds_read_tr16(vs + voff[0][db] + 16 * cc * D);
+                const u32x2 hi = lds_read_tr16(vs + voff[1][db] + 16 * cc * D);
+                const u32x4 u = {lo[0], lo[1], hi[0], hi[1]};
+                oacc[db] = mfma32(__builtin_bit_cast(bf16x8, u), pf[cc], oacc[db]);
+            }
+        // the copies of the tile after the next overwrite this stage: its reads have returned (their MFMAs were issued)
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lds_reads<0>();
+    }
+
+    // ---- the four wavefronts' partial softmaxes meet: unnormalised O, maximum and sum of every query row
+    float* ml = reinterpret_cast<float*>(lds + NW * T::WAVE_ELEMS);             // [wave][query][maximum, sum]
+    {
+        const float l = l_run + xhalf(l_run);
+        float* orow = reinterpret_cast<float*>(own) + n * T::O_STRIDE;
+        if (qi < p.Sq) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<f32x4*>(orow + 32 * db + 8 * g + 4 * h) =
+                        f32x4{oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2], oacc[db][4 * g + 3]};
+            if (h == 0) {
+                ml[(wave * T::BQ + n) * 2] = m_run;
+                ml[(wave * T::BQ + n) * 2 + 1] = l;
+            }
+        }
+    }
+    __syncthreads();
+    const int groups = p.dv >> 2;                  // columns in fours
+    const int64_t rows = (int64_t)p.B * p.H * p.Sq;
+    for (int idx = tid; idx < min(T::BQ, p.Sq - q0) * groups; idx += 256) {
+        const int row = idx / groups, g = idx % groups;
+        float m = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) m = fmaxf(m, ml[(w * T::BQ + row) * 2]);
+        const float m_to = (m == -INFINITY) ? 0.f : m;
+        float l = 0.f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float a = exp2_fast((ml[(w * T::BQ + row) * 2] - m_to) * c_log2);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(lds + w * T::WAVE_ELEMS) + row * T::O_STRIDE + 4 * g);
+            l = fmaf(a, ml[(w * T::BQ + row) * 2 + 1], l);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = fmaf(a, v[i], acc[i]);
+        }
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        const float lse = l > 0.f ? (m * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
+        const int64_t r = (int64_t)bh * p.Sq + q0 + row;
+        if (p.key_splits > 1) {
+            *reinterpret_cast<f32x4*>(p.part_o + ((int64_t)slice * rows + r) * p.dv + 4 * g) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+            if (g == 0) p.part_lse[(int64_t)slice * rows + r] = lse;
+        } else {
+            uint16_t* orow = p.o + b * p.os.b + hh * p.os.h + (int64_t)(q0 + row) * p.os.n;
+            *reinterpret_cast<u32x2*>(orow + 4 * g) = u32x2{pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv)};
+            if (p.lse && g == 0) p.lse[r] = lse;
+        }
+    }
+}
+
+}  // namespace fattn

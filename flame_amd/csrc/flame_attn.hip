@@ -22,6 +22,7 @@
 #include "attn_bwd.hpp"
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
+#include "attn_fwd_keyshare.hpp"
 #include "prep.hpp"
 #include "sage.hpp"
 #include "plan_cache.hpp"
@@ -102,24 +103,50 @@ struct ScopedKernelTimer {
     }
 };
 
-template <int D, bool HASMASK, int NW, bool VECMASK = false>
+// the kernel's dynamic LDS size, set once per kernel (idempotent, so a benign race at worst repeats the call)
+int set_lds(const void* kern, int bytes, std::atomic<bool>& done) {
+    if (done.load(std::memory_order_relaxed)) return FLAME_ATTN_OK;
+    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return (int)e;
+    done.store(true, std::memory_order_relaxed);
+    return FLAME_ATTN_OK;
+}
+
+// combines the slices of a key split (p.key_splits > 1)
+void launch_fwd_merge(const FwdParams& p, hipStream_t s) {
+    const int64_t lanes = (int64_t)p.B * p.H * p.Sq * (p.dv / 4);
+    hipLaunchKernelGGL(fwd_merge_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, p);
+}
+
+template <int D, int EXCL, int NW, bool DROPOUT = false>
 int launch_fwd(const FwdParams& p, hipStream_t s) {
     using T = FwdTile<D>;
     constexpr int BM = 32 * NW;
-    static bool attr_done = false;   // idempotent, so a benign race at worst repeats the call
-    auto kern = fwd_kernel<D, HASMASK, NW, VECMASK>;
-    if (!attr_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        attr_done = true;
-    }
-    const int64_t n_qt = (p.Sq + BM - 1) / BM;
-    const int64_t grid = n_qt * p.B * p.H;
+    static std::atomic<bool> lds_set{false};
+    auto kern = fwd_kernel<D, EXCL, NW, DROPOUT>;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
+    const int64_t grid = (int64_t)((p.Sq + BM - 1) / BM) * p.B * p.H;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), T::LDS_BYTES, s, p);
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
+template <int D, bool DROPOUT>
+int launch_fwd_keyshare(const FwdParams& p, hipStream_t s) {
+    using T = FwdKeyShareTile<D>;
+    static std::atomic<bool> lds_set{false};
+    auto kern = fwd_keyshare_kernel<D, DROPOUT>;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
+    const int64_t grid = (int64_t)((p.Sq + T::BQ - 1) / T::BQ) * p.B * p.H * p.key_splits;
+    if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    {
+        ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, s, p);
+        if (p.key_splits > 1) launch_fwd_merge(p, s);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -352,7 +379,7 @@ inline int bigd_key_splits(int64_t query_tile_wgs, int Sk) {
 
 // queries per workgroup of the big-head-dim forward the library launches for head dim D
 inline int bigd_query_tile(int D) { return D <= 256 ? 128 : 64; }
-inline size_t bigd_partials_bytes(int key_splits, int64_t rows, int dv) { return (size_t)key_splits * rows * (dv + 1) * sizeof(float); }
+inline size_t partials_bytes(int key_splits, int64_t rows, int dv) { return (size_t)key_splits * rows * (dv + 1) * sizeof(float); }
 
 template <int NC, int NW>
 int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc) {
@@ -366,12 +393,9 @@ int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc)
         if (e != hipSuccess) return (int)e;
         attr_done = true;
     }
-    FwdBigDParams p;
-    static_cast<FwdParams&>(p) = fp;
+    FwdParams p = fp;
     const int64_t grid0 = (int64_t)((p.Sq + T::BM - 1) / T::BM) * p.B * p.H;
     p.key_splits = bigd_key_splits(grid0, p.Sk);
-    p.part_o = nullptr;
-    p.part_lse = nullptr;
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
     static_assert(T::BM == (NC <= 2 ? 128 : 64), "bigd_query_tile must name this kernel's query tile");
     std::unique_lock<std::mutex> enqueue(lib_scratch_enqueue_mutex(), std::defer_lock);
@@ -381,11 +405,11 @@ int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc)
         // behind the reference-named entry points, which take the library's per-(device, stream) buffer
         void* ws = nullptr;
         if (sc.ws && aligned16(sc.ws)) {
-            while (p.key_splits > 1 && bigd_partials_bytes(p.key_splits, rows, p.dv) > sc.bytes) --p.key_splits;
+            while (p.key_splits > 1 && partials_bytes(p.key_splits, rows, p.dv) > sc.bytes) --p.key_splits;
             ws = sc.ws;
         } else if (sc.library) {
             enqueue.lock();          // held until both kernels are enqueued
-            const int rc = lib_scratch_get(bigd_partials_bytes(p.key_splits, rows, p.dv), s, &ws);
+            const int rc = lib_scratch_get(partials_bytes(p.key_splits, rows, p.dv), s, &ws);
             if (rc == FLAME_ATTN_ERR_UNSUPPORTED) p.key_splits = 1;      // under a capture and nothing allocated yet: unsplit
             else if (rc) return rc;
         } else {
@@ -401,10 +425,7 @@ int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc)
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), T::LDS_BYTES, s, p);
-        if (p.key_splits > 1) {
-            const int64_t lanes = rows * (p.dv / 4);
-            hipLaunchKernelGGL(fwd_bigd_merge_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, p);
-        }
+        if (p.key_splits > 1) launch_fwd_merge(p, s);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -414,27 +435,6 @@ int launch_fwd_bigd(const FwdParams& p, hipStream_t s, const FwdScratch& sc) { r
 
 // Dropout of the probabilities: the 128-query forward and dQ kernels and the dK/dV kernel in their DROPOUT
 // instantiations, without the split of the last round; HASMASK: the general kernels for an explicit mask or bias.
-template <int D, bool HASMASK>
-int launch_fwd_dropout(const FwdParams& p, hipStream_t s) {
-    using T = FwdTile<D>;
-    static bool attr_done = false;
-    auto kern = fwd_kernel<D, HASMASK, 4, false, true>;
-    if (!attr_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        attr_done = true;
-    }
-    const int64_t grid = (int64_t)((p.Sq + 127) / 128) * p.B * p.H;
-    if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
-    {
-        ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, s, p);
-    }
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
-}
-
 template <int D, bool HASMASK>
 int launch_bwd_dropout(const BwdParams& p, hipStream_t s) {
     using T = BwdTile<D>;
@@ -825,6 +825,39 @@ int flame_sage_attn_fwd_bias_int8(const void* Qi8, const void* Ki8, const void* 
 
 }  // extern "C"
 
+// fwd_keyshare_kernel instead of fwd_kernel (head dims up to 128, nothing excluded but by causal flag and key lengths): a
+// few query rows, or 128-query workgroups on at most a quarter of the compute units, so that four times as many still run
+// in one round.  Measured with 32 such workgroups, D = 128: 62 -> 31 us at 4096 keys, 20 -> 16 us at 1024; with 128 of
+// them 35 -> 51 us (each K / V tile is fetched four times as often, and a step then waits for it).
+static bool fwd_rule_keyshare(int64_t bh, int N_q) {
+    return N_q <= 32 || (int64_t)((N_q + 127) / 128) * bh * 4 <= device_cu_count();
+}
+
+// ... and the workgroups that share the keys of one of its query tiles: the least of an estimate in microseconds.  Every
+// round of the chip costs a start and its steps, all of K and V take at least the time of reading them, a split one merge
+// launch and the traffic of its fp32 partials.  (The constants were measured; one row against 4097 keys of 64 heads,
+// D = 128: 39 / 27 / 27 / 32 us with 1 / 2 / 4 / 8 slices.)
+static int fwd_key_splits(int64_t bh, int N_q, int N_kv, int DP) {
+    if (!fwd_rule_keyshare(bh, N_q)) return 1;
+    const int64_t wgs = (int64_t)((N_q + 31) / 32) * bh;
+    const int64_t slots = device_cu_count() * (DP == 64 ? 2 : 1);             // LDS: two workgroups per compute unit at D = 64
+    const int steps = (N_kv + 127) / 128;
+    const double step_us = DP == 64 ? 0.8 : 1.1, start_us = 2.5;
+    const double read_us = 4.0 * bh * N_kv * DP / 5.2e6;
+    double best = 1e30;
+    int best_s = 1;
+    for (int s = 1; s <= 64 && s <= (steps + 1) / 2; ++s) {
+        const int64_t rounds = (wgs * s + slots - 1) / slots;
+        const double merge_us = s == 1 ? 0.0 : 2.5 + 0.55 * s + 2.0 * s * (double)bh * N_q * DP * 4 / 8e6;
+        const double t = std::max((double)rounds * (start_us + step_us * ((steps + s - 1) / s)), read_us) + merge_us;
+        if (t < best) {
+            best = t;
+            best_s = s;
+        }
+    }
+    return best_s;
+}
+
 // the rule for the forward's query tile: 256 rows per workgroup (true) or 128
 static bool fwd_rule_wide(int B, int H, int N_q, bool has_mask_or_bias, bool has_kv_len) {
     const int64_t n256 = (N_q + 255) / 256;
@@ -903,9 +936,13 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     const bool hm = keep_mask != nullptr || bias != nullptr;
     if (dropout_p != 0.f) {
         if (!set_dropout(p.m, dropout_p, dropout_seed, draw_cq, draw_ck, N_q, N_kv)) return FLAME_ATTN_ERR_INVALID;
-        if (std::max(padded_head_dim(D), padded_head_dim(Dv)) == 128)
-            return hm ? launch_fwd_dropout<128, true>(p, s) : launch_fwd_dropout<128, false>(p, s);
-        return hm ? launch_fwd_dropout<64, true>(p, s) : launch_fwd_dropout<64, false>(p, s);
+        const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
+        // the kernel of the undropped call, so that the log-sum-exp is the same to the bit
+        if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q))
+            return DP == 128 ? launch_fwd_keyshare<128, true>(p, s) : launch_fwd_keyshare<64, true>(p, s);
+        if (DP == 128)
+            return hm ? launch_fwd<128, kExGeneral, 4, true>(p, s) : launch_fwd<128, kExNone, 4, true>(p, s);
+        return hm ? launch_fwd<64, kExGeneral, 4, true>(p, s) : launch_fwd<64, kExNone, 4, true>(p, s);
     }
     // 256-query workgroups when they neither add padding rows nor leave compute units
     // without a workgroup
@@ -918,12 +955,23 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel
     const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
     if (keep_mask != nullptr && bias == nullptr && p.m.rows16 && N_kv % 64 == 0)
-        return DP == 128 ? launch_fwd<128, true, 4, true>(p, s) : launch_fwd<64, true, 4, true>(p, s);
-    if (DP == 128)
-        return hm ? launch_fwd<128, true, 4>(p, s)
-                  : wide ? (plain ? launch_fwd_wide<128>(p, s) : launch_fwd<128, false, 8>(p, s)) : launch_fwd<128, false, 4>(p, s);
-    return hm ? launch_fwd<64, true, 4>(p, s)
-              : wide ? (plain ? launch_fwd_wide<64>(p, s) : launch_fwd<64, false, 8>(p, s)) : launch_fwd<64, false, 4>(p, s);
+        return DP == 128 ? launch_fwd<128, kExRows16, 4>(p, s) : launch_fwd<64, kExRows16, 4>(p, s);
+    if (hm) return DP == 128 ? launch_fwd<128, kExGeneral, 4>(p, s) : launch_fwd<64, kExGeneral, 4>(p, s);
+    if (wide) {
+        if (plain) return DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
+        return DP == 128 ? launch_fwd<128, kExNone, 8>(p, s) : launch_fwd<64, kExNone, 8>(p, s);
+    }
+    if (q_tile_plan == 0 && fwd_rule_keyshare((int64_t)B * H, N_q)) {
+        const int64_t rows = (int64_t)B * H * N_q;
+        if (scratch.ws) {
+            p.key_splits = fwd_key_splits((int64_t)B * H, N_q, N_kv, DP);
+            while (p.key_splits > 1 && partials_bytes(p.key_splits, rows, Dv) > scratch.bytes) --p.key_splits;
+            p.part_o = static_cast<float*>(scratch.ws);
+            p.part_lse = p.part_o + (size_t)p.key_splits * rows * Dv;
+        }
+        return DP == 128 ? launch_fwd_keyshare<128, false>(p, s) : launch_fwd_keyshare<64, false>(p, s);
+    }
+    return DP == 128 ? launch_fwd<128, kExNone, 4>(p, s) : launch_fwd<64, kExNone, 4>(p, s);
 }
 
 
@@ -946,7 +994,14 @@ size_t flame_attn_fwd_workspace_bytes(int B, int H, int N_q, int N_kv, int D) {
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !big_head_dim_ok(D)) return 0;
     const int bm = bigd_query_tile(D);
     const int ks = bigd_key_splits((int64_t)((N_q + bm - 1) / bm) * B * H, N_kv);
-    return ks > 1 ? bigd_partials_bytes(ks, (int64_t)B * H * N_q, D) : 0;
+    return ks > 1 ? partials_bytes(ks, (int64_t)B * H * N_q, D) : 0;
+}
+
+size_t flame_attn_fwd_scratch_bytes(int B, int H, int N_q, int N_kv, int D) {
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0) return 0;
+    if (!head_dim_ok(D)) return flame_attn_fwd_workspace_bytes(B, H, N_q, N_kv, D);
+    const int ks = fwd_key_splits((int64_t)B * H, N_q, N_kv, padded_head_dim(D));
+    return ks > 1 ? partials_bytes(ks, (int64_t)B * H * N_q, D) : 0;
 }
 
 int flame_attn_fwd_ws_bf16(const void* Q, const void* K, const void* V, void* O, void* LSE,

@@ -30,7 +30,7 @@ namespace {
 using at::Tensor;
 
 #define FLAME_HOST_ENTRY_POINTS(X)                                                                                      \
-    X(flame_attn_fwd_bf16) X(flame_attn_fwd_ws_bf16) X(flame_attn_fwd_workspace_bytes) X(flame_attn_fwd_bias_bf16)      \
+    X(flame_attn_fwd_bf16) X(flame_attn_fwd_ws_bf16) X(flame_attn_fwd_scratch_bytes) X(flame_attn_fwd_bias_bf16)      \
     X(flame_attn_bwd_bf16) X(flame_attn_bwd_workspace_bytes) X(flame_attn_fwd_dropout_tiled_bf16)                       \
     X(flame_attn_bwd_dropout_tiled_bf16) X(flame_attn_materialised_workspace_bytes) X(flame_attn_fwd_materialised_bf16) \
     X(flame_attn_bwd_materialised_bf16) X(flame_sage_quant_qk_int8_ks) X(flame_sage_attn_fwd_bias_int8)                 \
@@ -188,10 +188,15 @@ struct FwdOpts {
 int call_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Sizes& z, float scale, const FwdOpts& f, Tensor& o, Tensor& lse) {
     if (!o.defined()) o = empty({z.B, z.H, z.Sq, z.D}, at::kBFloat16, q);
     if (!lse.defined() && f.want_lse) lse = empty({(int64_t)z.B * z.H, z.Sq}, at::kFloat, q);
-    if (f.workspace.defined())
+    Tensor ws = f.workspace;
+    if (!ws.defined() && !f.mask.data) {       // room for the slices of a key split, where the grid would leave compute units idle
+        const size_t need = g_api.flame_attn_fwd_scratch_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
+        if (need) ws = bytes_like(need, q);
+    }
+    if (ws.defined())
         return g_api.flame_attn_fwd_ws_bf16(ptr(q), ptr(k), ptr(v), ptr(o), ptr(lse), z.B, z.H, z.Sq, z.Sk, z.D, scale, strides4(q), strides4(k),
                                             strides4(v), strides4(o), 0, 0, 0, 0, 0, f.causal, static_cast<const int32_t*>(ptr(f.kv_len)), f.mask.data,
-                                            f.mask.strides(), ptr(f.workspace), (size_t)f.workspace.numel(), stream_of(q));
+                                            f.mask.strides(), ptr(ws), (size_t)ws.numel(), stream_of(q));
     return g_api.flame_attn_fwd_bf16(ptr(q), ptr(k), ptr(v), ptr(o), ptr(lse), z.B, z.H, z.Sq, z.Sk, z.D, scale, strides4(q), strides4(k),
                                      strides4(v), strides4(o), 0, 0, 0, 0, 0, f.causal, static_cast<const int32_t*>(ptr(f.kv_len)), f.mask.data,
                                      f.mask.strides(), stream_of(q));
