@@ -60,7 +60,13 @@ enum FwdExcl : int {
     kExNone = 0,
     kExRows16 = 1,       // uint8 keep-mask, rows contiguous and 16-byte aligned, Sk a multiple of the tile, no bias
     kExGeneral = 2,      // any keep-mask and / or bias, one element at a time
+    kExBiasF32 = 3,      // an additive fp32 bias, contiguous along the keys, and no keep-mask, causal flag or key lengths
+    kExBiasBf16 = 4,     // the same in bf16
 };
+
+// four consecutive bias values, at any element's address
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 
 // DROPOUT: the probabilities that multiply V are dropped and rescaled element by element (drop_factor); the row sums,
 // and with them the log-sum-exp, stay those of the undropped softmax.
@@ -110,6 +116,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     const char* bbase = (EXCL == kExGeneral && p.m.bias)
                             ? static_cast<const char*>(p.m.bias) + (b * p.m.bb + hh * p.m.bh) * (p.m.bias_f32 ? 4 : 2)
                             : nullptr;
+
+    constexpr bool BIAS = EXCL == kExBiasF32 || EXCL == kExBiasBf16;
 
     // ---- asynchronous tile copies.  Full tiles: uniform tile base + a per-lane 32-bit byte offset that never changes;
     //      ragged tiles clamp their rows into the attended range.
@@ -223,8 +231,39 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             if (__any(limit < BN)) mrow.restrict_to(limit);
         }
     };
+    // Bias: every lane needs 64 (of its half: 32) consecutive values of its query's row, four at a time, so a group of four
+    // is one 16-byte (bf16: 8-byte) load; group j of the next tile is requested at the j-th eighth of the logit phase, when
+    // the exponentials have freed the registers it takes, and added in the j-th eighth of the PV phase.
+    // (B=1 H=64 S=512 D=64, fp32: one load per element 62 us, this 24 us; 84 MB move, 18 us at the rate of a copy.)
+    using BiasGroup = typename std::conditional<EXCL == kExBiasF32, f32x4_any, u16x4_any>::type;
+    using BiasElem = typename std::conditional<EXCL == kExBiasF32, float, uint16_t>::type;
+    BiasGroup bg[BIAS ? 8 : 1];
+    const BiasElem* brow = nullptr;
+    if constexpr (BIAS)
+        brow = static_cast<const BiasElem*>(p.m.bias) + b * p.m.bb + hh * p.m.bh + (int64_t)min(qi, p.Sq - 1) * p.m.bq + 4 * h;
+    auto bias_request = [&](auto ragged_tag, int t, int j) {
+        if constexpr (BIAS) {
+            const int key = t * BN + 8 * j;          // of half 0
+            if constexpr (!decltype(ragged_tag)::value) {
+                bg[j] = *reinterpret_cast<const BiasGroup*>(brow + key);
+            } else {                                 // ragged tail: nothing past the row is read, keys past the end get -inf
+                const int last = p.Sk - 1 - 4 * h;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const BiasElem v = brow[min(key + e, last)];
+                    bg[j][e] = key + e > last ? (EXCL == kExBiasF32 ? (BiasElem)-INFINITY : (BiasElem)0xff80u) : v;
+                }
+            }
+        }
+    };
     auto excl_elem = [&](f32x16 (&s)[2], int idx) {
         const int kb = idx >> 4, r = idx & 15;
+        if constexpr (BIAS) {     // scale * (s + bias / scale) = scale * s + bias
+            float v;
+            if constexpr (EXCL == kExBiasF32) v = bg[idx >> 2][idx & 3];
+            else v = __uint_as_float((uint32_t)bg[idx >> 2][idx & 3] << 16);
+            s[kb][r] = fmaf(v, p.m.inv_scale, s[kb][r]);
+        }
         if constexpr (EXCL == kExRows16) s[kb][r] = mrow.keep(kb, r, h) ? s[kb][r] : -INFINITY;
         if constexpr (EXCL == kExNone) s[kb][r] = 32 * kb + 8 * (r >> 2) + (r & 3) >= lim ? -INFINITY : s[kb][r];
     };
@@ -334,6 +373,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             }
         } else {
             if (NEXT == 1) excl_begin(t + 1);
+            const std::integral_constant<bool, NEXT == 1> ragged_tag{};
             // ---- S(t+1)^T = K(t+1) Q^T between the exponentials of tile t
             zero_tile(nxt);
 #pragma unroll
@@ -349,9 +389,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             for (int i = 0; i < NS; i += 2) {
                 nxt[1] = mfma32(fb[(i + 1) % PD], qf[i >> 1], nxt[1]);
                 exp_slice(i);
+                if (BIAS && i % (NS / 8) == 0) bias_request(ragged_tag, t + 1, i / (NS / 8));
                 __builtin_amdgcn_sched_barrier(0);
                 nxt[0] = mfma32(fb[i % PD], qf[i >> 1], nxt[0]);
                 exp_slice(i + 1);
+                if (BIAS && (i + 1) % (NS / 8) == 0) bias_request(ragged_tag, t + 1, (i + 1) / (NS / 8));
                 fb[i % PD] = frag_of(i + PD);
                 fb[(i + 1) % PD] = frag_of(i + 1 + PD);
                 __builtin_amdgcn_sched_barrier(0);
@@ -364,7 +406,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
 #pragma unroll
                 for (int e = 0; e < MPS; e += 2) {
                     const int idx = MPS * i + e;
-                    if (NEXT == 1) {
+                    if (NEXT == 1 || BIAS) {
                         excl_elem(nxt, idx);
                         excl_elem(nxt, idx + 1);
                     }
@@ -392,7 +434,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
 
     // Tiles below t_clean need no exclusions for any query of the workgroup; the rest (ragged tail, causal
     // diagonal, or everything under an explicit mask) carry per-element exclusions.
-    int t_clean = EXCL != kExNone ? 0 : klimit / BN;
+    int t_clean = (EXCL == kExNone || BIAS) ? klimit / BN : 0;
     if (p.m.causal) t_clean = min(t_clean, (q0 + 1) / BN);
     t_clean = min(t_clean, n_tiles);
 
@@ -401,10 +443,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
         wait_vm0();
         __syncthreads();
         if (t_clean == 0) excl_begin(0);
+        if constexpr (BIAS)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) bias_request(std::true_type{}, 0, j);
         zero_tile(sa);
 #pragma unroll
         for (int i = 0; i < NS; ++i) sa[i & 1] = mfma32(k_frag(0, i), qf[i >> 1], sa[i & 1]);
-        if (t_clean == 0) {
+        if (t_clean == 0 || BIAS) {
             if (EXCL == kExGeneral) excl_general(sa, 0);
 #pragma unroll
             for (int idx = 0; idx < 32; ++idx) excl_elem(sa, idx);
@@ -425,7 +470,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
         // Two steps per trip, so that `sa` is the current tile when t is even; where the number of steps of
         // one kind is odd, the pair that mixes kinds runs as the more general one.
         int t = 0;
-        if (EXCL == kExNone) {
+        if (EXCL == kExNone || BIAS) {
             const int copy_end = t_clean - KD;              // steps below it copy two full tiles
             for (; t + 1 < copy_end; t += 2) {
                 step(Yes{}, Clean{}, sa, sb, t);
@@ -436,7 +481,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 step(No{}, Clean{}, sb, sa, t + 1);
             }
         }
-        if (EXCL != kExNone) {
+        if (EXCL != kExNone && !BIAS) {
             const int copy_end = min(n_tiles, klimit / BN) - KD;
             for (; t + 1 < copy_end; t += 2) {
                 step(Yes{}, Cut{}, sa, sb, t);

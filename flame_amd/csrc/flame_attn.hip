@@ -956,6 +956,11 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
     if (keep_mask != nullptr && bias == nullptr && p.m.rows16 && N_kv % 64 == 0)
         return DP == 128 ? launch_fwd<128, kExRows16, 4>(p, s) : launch_fwd<64, kExRows16, 4>(p, s);
+    // a bias alone, its rows contiguous: loaded in fours
+    if (bias != nullptr && keep_mask == nullptr && !causal && kv_len == nullptr && p.m.bk == 1) {
+        if (p.m.bias_f32) return DP == 128 ? launch_fwd<128, kExBiasF32, 4>(p, s) : launch_fwd<64, kExBiasF32, 4>(p, s);
+        return DP == 128 ? launch_fwd<128, kExBiasBf16, 4>(p, s) : launch_fwd<64, kExBiasBf16, 4>(p, s);
+    }
     if (hm) return DP == 128 ? launch_fwd<128, kExGeneral, 4>(p, s) : launch_fwd<64, kExGeneral, 4>(p, s);
     if (wide) {
         if (plain) return DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
