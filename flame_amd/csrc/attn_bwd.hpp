@@ -56,6 +56,7 @@ struct BwdParams {
     int d;                // real head dim: a multiple of 8, at most the compiled D
     float scale;
     MaskArgs m;
+    int key_mask = 0;     // m.mask is the same for every query: kernels without the general mask code serve it
     unsigned long long* phase_cycles;   // profiling aid: per-phase cycle sums of wave 0 of every workgroup, or null
 };
 
@@ -114,7 +115,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     const int n_kt = (p.Sk + BN - 1) / BN;
     int wg, part = 0, nparts = 1;
     if (p.n_whole < 0) {
-        wg = p.m.kv_len ? xcd_remap_heads(block, nblocks, n_kt) : xcd_remap(block, nblocks);
+        wg = p.m.kv_len || p.key_mask ? xcd_remap_heads(block, nblocks, n_kt) : xcd_remap(block, nblocks);
     } else if (block < p.n_whole) {
         wg = xcd_remap(block, p.n_whole);
     } else {          // the split key blocks come last in dispatch order and fill the final, partial round
@@ -140,10 +141,26 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     if (p.m.kv_len) klimit = min(klimit, max(p.m.kv_len[b], 0));
     const uint8_t* mbase = HASMASK ? mask_head_base(p.m, b, hh) : nullptr;
 
+    // A keep-mask of keys is a key length with holes: a lane owns one key, so its P and dS need no test, and the columns of
+    // the excluded keys are zeroed before the store.  Two loads per wavefront tell whether any of the 128 keys is attended.
+    bool dead = false;
+    uint64_t any_alive = ~0ull;
+    if (!HASMASK && p.key_mask) {
+        const uint8_t* kmask = mask_head_base(p.m, b, hh);
+        bool alive[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int kk = k0 + 64 * u + lane;
+            alive[u] = kk < klimit && mask_attends(p.m, kmask, (int64_t)min(kk, p.Sk - 1) * p.m.sk);
+        }
+        const uint64_t b0 = __ballot(alive[0]), b1 = __ballot(alive[1]);
+        any_alive = b0 | b1;
+        dead = ((((wave & 2) ? b1 : b0) >> (32 * (wave & 1) + n)) & 1ull) == 0;
+    }
     const int n_qt = (p.Sq + BM - 1) / BM;
     int qt_begin = p.m.causal ? (k0 / BM) : 0;
-    if (k0 >= klimit || (p.m.causal && k0 >= p.Sq)) {
-        // Nothing attends to these keys (past the key length, or past the last query under the causal flag):
+    if (k0 >= klimit || any_alive == 0 || (p.m.causal && k0 >= p.Sq)) {
+        // Nothing attends to these keys (past the key length, masked, or past the last query under the causal flag):
         // dK = dV = 0, written at once.  Padded batches launch many such workgroups; they must not cost a
         // prologue each.
         f32x16 zero[D / 32];
@@ -672,7 +689,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
             }
         return;
     }
-    if (key >= klimit) {          // nothing attends to this lane's key
+    if (key >= klimit || dead) {  // nothing attends to this lane's key
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -770,11 +787,10 @@ struct BwdDqTile {
 
 // NW wavefronts of 32 queries each per workgroup, two per SIMD (the library instantiates NW = 4; problems
 // that fill 256-query workgroups go to bwd_dq_wide_kernel below).
-// VECMASK (with HASMASK): the keep-mask rows are contiguous and 16-byte aligned and Sk is a multiple of the
-// tile, so the per-element mask loads are not compiled in and the kernel fits two workgroups per unit again.
-template <int D, bool HASMASK, int NW, bool VECMASK = false, bool DROPOUT = false>
-__global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
-    static_assert(!VECMASK || HASMASK, "VECMASK is a special case of HASMASK");
+// EXCL: see there.  Only the general form compiles per-element mask loads in; the others fit two workgroups per unit.
+template <int D, int EXCL, int NW, bool DROPOUT = false>
+__global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
+    constexpr bool HASMASK = EXCL == kExRows16 || EXCL == kExGeneral, VECMASK = EXCL == kExRows16, KEYS = EXCL == kExKeys;
     using T = BwdDqTile<D>;
     constexpr int BM = 32 * NW, BN = T::BN, RS = T::RS;
     constexpr int DC = D / 16;
@@ -789,7 +805,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.m.kv_len || KEYS ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
     const int b = bh / p.H, hh = bh % p.H;
@@ -805,8 +821,20 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1
     if (p.m.kv_len) klimit = min(klimit, max(p.m.kv_len[b], 0));
     int kend = klimit;
     if (p.m.causal) kend = min(kend, q0 + BM);
-    const int n_tiles = (kend + BN - 1) / BN;
-    const uint8_t* mbase = HASMASK ? mask_head_base(p.m, b, hh) : nullptr;
+    int n_tiles = (kend + BN - 1) / BN;
+    const uint8_t* mbase = HASMASK || KEYS ? mask_head_base(p.m, b, hh) : nullptr;
+    // KEYS: step t of the walk takes tile tile_of(t) (elsewhere the two are the same number)
+    KeyTiles kt;
+    if constexpr (KEYS) {
+        kt.build(reinterpret_cast<char*>(lds) + T::LDS_BYTES, klimit, NW, [&](int key) {
+            return key < klimit && mask_attends(p.m, mbase, (int64_t)min(key, p.Sk - 1) * p.m.sk);
+        });
+        n_tiles = kt.n_tiles;
+    }
+    auto tile_of = [&](int t) {
+        if constexpr (KEYS) return kt.tile(t);
+        else return t;
+    };
 
     // ---- Q and dO fragments (B operands: column = query, 8 consecutive d), per-query scalars
     const int qrow = qw0 + n;
@@ -863,22 +891,24 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1
         return lds0 + 2u * (uint32_t)(buf * T::STAGE_ELEMS + which * T::TILE_ELEMS + (wave * NDMA + i) * 512);
     };
     auto issue_tile = [&](int t, int buf) {
+        const int tile = tile_of(t);
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
             const int row = (wave * NDMA + i) * T::ROWS_PER_DMA + dma_row_in;
-            const int key = min(t * BN + row, klimit - 1);   // tail rows re-read the last attended key
+            const int key = min(tile * BN + row, klimit - 1);   // tail rows re-read the last attended key
             const int c = src_granule(dma_gran ^ swz<D>(row), p.d);
             dma16(kbase + (int64_t)key * p.ks.n + c * 8, dst_of(buf, 0, i));
             dma16(vbase + (int64_t)key * p.vs.n + c * 8, dst_of(buf, 1, i));
         }
     };
     auto issue_full_tile = [&](int t, int buf) {
-        const uint16_t* kt = kbase + (int64_t)t * BN * p.ks.n;
-        const uint16_t* vt = vbase + (int64_t)t * BN * p.vs.n;
+        const int tile = tile_of(t);
+        const uint16_t* ktile = kbase + (int64_t)tile * BN * p.ks.n;
+        const uint16_t* vtile = vbase + (int64_t)tile * BN * p.vs.n;
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
-            dma16u(kt, k_lane_off[i], dst_of(buf, 0, i));
-            dma16u(vt, v_lane_off[i], dst_of(buf, 1, i));
+            dma16u(ktile, k_lane_off[i], dst_of(buf, 0, i));
+            dma16u(vtile, v_lane_off[i], dst_of(buf, 1, i));
         }
     };
 
@@ -926,7 +956,13 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1
         else if (t + 1 < n_tiles) issue_tile(t + 1, buf ^ 1);
         const uint16_t* ks = lds + buf * T::STAGE_ELEMS;
         const uint16_t* vs = ks + T::TILE_ELEMS;
-        const int key0 = t * BN;
+        const int key0 = t * BN;      // (not KEYS)
+        uint32_t keep_bits[2] = {0u, 0u};
+        if constexpr (KEYS && MASKED) {
+            const uint64_t w = kt.bits[kt.tile(t)];
+            keep_bits[0] = (uint32_t)w >> (4 * h);
+            keep_bits[1] = (uint32_t)(w >> 32) >> (4 * h);
+        }
 
         // operand fetch f of the tile, in consumption order
         constexpr int NROW = 4 * DC;                // row-read fragments: S(0), dP(0), S(1), dP(1)
@@ -970,6 +1006,8 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1
             float pr = exp2_fast(fmaf(sacc[kb][r], c_log2, -lse2));
             if constexpr (VECMASK) {
                 pr = mrow.keep(kb, r, h) ? pr : 0.f;
+            } else if constexpr (KEYS && MASKED) {
+                pr = keep_bits[kb] & (1u << (8 * (r >> 2) + (r & 3))) ? pr : 0.f;
             } else if (MASKED) {
                 const int key = key0 + 32 * kb + acc_row(r, h);
                 bool drop = (key >= klimit) | ((p.m.causal != 0) & (key > qrow));     // bitwise: selects, not branches
@@ -1049,7 +1087,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && (!HASMASK || VECMASK)) ? 2 : 1
         __syncthreads();
     };
 
-    int n_full = HASMASK ? 0 : klimit / BN;
+    int n_full = HASMASK ? 0 : KEYS ? kt.n_whole : klimit / BN;
     if (p.m.causal) n_full = min(n_full, (q0 + 1) / BN);
     n_full = min(n_full, n_tiles);
     using IM = std::integral_constant<int, -1>;

@@ -482,4 +482,65 @@ __device__ __forceinline__ const uint8_t* mask_head_base(const MaskArgs& m, int 
     return m.mask + (b * m.sb + hh * m.sh) * (m.mask_mode == kMaskU8 ? 1 : 2);
 }
 
+// What a kernel whose lanes own queries excludes besides keys past the key length and, with the causal flag, past the query.
+enum Excl : int {
+    kExNone = 0,
+    kExRows16 = 1,       // uint8 keep-mask, rows contiguous and 16-byte aligned, Sk a multiple of the tile, no bias
+    kExGeneral = 2,      // any keep-mask and / or bias, one element at a time
+    kExBiasF32 = 3,      // (forward) an additive fp32 bias, contiguous along the keys, and no keep-mask, causal flag or key lengths
+    kExBiasBf16 = 4,     // (forward) the same in bf16
+    kExKeys = 5,         // a keep-mask that is the same for every query (a padded batch), no causal flag
+};
+
+// The 64-key tiles that a keep-mask of keys leaves anything of, in LDS: the tiles attended whole first, then the others
+// (the order of the tiles is irrelevant to the sums), and the 64 keep bits of every tile.  A padded batch walks the
+// attended part of its sequences only, and nearly all of that without a test per element.
+struct KeyTiles {
+    static constexpr int kMaxTiles = 1024;            // 65536 keys: 10 KiB
+    static __host__ __device__ int lds_bytes(int n_all) { return (n_all * 10 + 8 + 15) / 16 * 16; }
+    uint64_t* bits;      // [n_all]
+    uint32_t* counts;    // whole tiles, cut tiles
+    uint16_t* list;      // [n_all]: whole tiles from the front, cut ones from the back
+    int n_all, n_whole, n_tiles;
+
+    // keep(key): does this key attend (false past the end)?  Every thread of the workgroup calls this; ends with a barrier.
+    template <class F>
+    __device__ __forceinline__ void build(void* lds, int n_keys, int nw, F&& keep) {
+        n_all = (n_keys + 63) / 64;
+        bits = static_cast<uint64_t*>(lds);
+        counts = reinterpret_cast<uint32_t*>(bits + n_all);
+        list = reinterpret_cast<uint16_t*>(counts + 2);
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll 4
+        for (int t = wave; t < n_all; t += nw) {
+            const uint64_t b = __ballot(keep(t * 64 + lane));
+            if (lane == 0) bits[t] = b;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            int whole = 0, cut = 0;
+            for (int t0 = 0; t0 < n_all; t0 += 64) {
+                const uint64_t b = t0 + lane < n_all ? bits[t0 + lane] : 0ull;
+                const bool is_whole = b == ~0ull, is_cut = b != 0ull && !is_whole;
+                const uint64_t mw = __ballot(is_whole), mc = __ballot(is_cut), below = (1ull << lane) - 1ull;
+                if (is_whole) list[whole + __popcll(mw & below)] = (uint16_t)(t0 + lane);
+                if (is_cut) list[n_all - 1 - (cut + __popcll(mc & below))] = (uint16_t)(t0 + lane);
+                whole += __popcll(mw);
+                cut += __popcll(mc);
+            }
+            if (lane == 0) {
+                counts[0] = (uint32_t)whole;
+                counts[1] = (uint32_t)cut;
+            }
+        }
+        __syncthreads();
+        n_whole = __builtin_amdgcn_readfirstlane(counts[0]);
+        n_tiles = n_whole + __builtin_amdgcn_readfirstlane(counts[1]);
+    }
+    // the j-th tile of the walk
+    __device__ __forceinline__ int tile(int j) const {
+        return __builtin_amdgcn_readfirstlane(list[j < n_whole ? j : n_all - 1 - (j - n_whole)]);
+    }
+};
+
 }  // namespace fattn

@@ -55,15 +55,6 @@ struct FwdTile {
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;   // copies per wave and tensor
 };
 
-// What a forward kernel excludes besides keys past the key length and, with the causal flag, past the query.
-enum FwdExcl : int {
-    kExNone = 0,
-    kExRows16 = 1,       // uint8 keep-mask, rows contiguous and 16-byte aligned, Sk a multiple of the tile, no bias
-    kExGeneral = 2,      // any keep-mask and / or bias, one element at a time
-    kExBiasF32 = 3,      // an additive fp32 bias, contiguous along the keys, and no keep-mask, causal flag or key lengths
-    kExBiasBf16 = 4,     // the same in bf16
-};
-
 // four consecutive bias values, at any element's address
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint16_t u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
@@ -95,7 +86,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.m.kv_len || EXCL == kExKeys ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
     const int b = bh / p.H, hh = bh % p.H;
@@ -111,12 +102,25 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     if (p.m.kv_len) klimit = min(klimit, max(p.m.kv_len[b], 0));
     int kend = klimit;
     if (p.m.causal) kend = min(kend, q0 + BM);
-    const int n_tiles = (kend + BN - 1) / BN;
+    int n_tiles = (kend + BN - 1) / BN;
     const uint8_t* mbase = (EXCL != kExNone && p.m.mask) ? mask_head_base(p.m, b, hh) : nullptr;
     const char* bbase = (EXCL == kExGeneral && p.m.bias)
                             ? static_cast<const char*>(p.m.bias) + (b * p.m.bb + hh * p.m.bh) * (p.m.bias_f32 ? 4 : 2)
                             : nullptr;
 
+    // KEYS: step t of the walk takes tile tile_of(t) (elsewhere the two are the same number); stages go by the step
+    constexpr bool KEYS = EXCL == kExKeys;
+    KeyTiles kt;
+    if constexpr (KEYS) {
+        kt.build(reinterpret_cast<char*>(lds) + T::LDS_BYTES, klimit, NW, [&](int key) {
+            return key < klimit && mask_attends(p.m, mbase, (int64_t)min(key, p.Sk - 1) * p.m.sk);
+        });
+        n_tiles = kt.n_tiles;
+    }
+    auto tile_of = [&](int t) {
+        if constexpr (KEYS) return kt.tile(t);
+        else return t;
+    };
     constexpr bool BIAS = EXCL == kExBiasF32 || EXCL == kExBiasBf16;
 
     // ---- asynchronous tile copies.  Full tiles: uniform tile base + a per-lane 32-bit byte offset that never changes;
@@ -138,8 +142,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     // any tile: rows past the attended range re-read the last attended key, which lies `over` rows further up
     const int dma_row0 = wave * NDMA * T::ROWS_PER_DMA + dma_row_in;
     auto issue_any = [&](const uint16_t* base, int64_t row_stride, const uint32_t (&lane_off)[NDMA], int t, int which) {
-        const uint16_t* tb = base + (int64_t)t * BN * row_stride;
-        const int row_max = klimit - 1 - t * BN;             // not negative for a tile that is walked
+        const int tile = tile_of(t);
+        const uint16_t* tb = base + (int64_t)tile * BN * row_stride;
+        const int row_max = klimit - 1 - tile * BN;          // not negative for a tile that is walked
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
             const int over = max(dma_row0 + i * T::ROWS_PER_DMA - row_max, 0);
@@ -149,12 +154,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     auto issue_k = [&](int t) { issue_any(kbase, p.ks.n, k_lane_off, t, 0); };
     auto issue_v = [&](int t) { issue_any(vbase, p.vs.n, v_lane_off, t, 1); };
     auto issue_full_kv = [&](int tk, int tv) {               // K tile tk and V tile tv, both full
-        const uint16_t* kt = kbase + (int64_t)tk * BN * p.ks.n;
-        const uint16_t* vt = vbase + (int64_t)tv * BN * p.vs.n;
+        const uint16_t* ktile = kbase + (int64_t)tile_of(tk) * BN * p.ks.n;
+        const uint16_t* vtile = vbase + (int64_t)tile_of(tv) * BN * p.vs.n;
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
-            dma16u(kt, k_lane_off[i], dst_of(tk, 0, i));
-            dma16u(vt, v_lane_off[i], dst_of(tv, 1, i));
+            dma16u(ktile, k_lane_off[i], dst_of(tk, 0, i));
+            dma16u(vtile, v_lane_off[i], dst_of(tv, 1, i));
         }
     };
     // the first tiles are on their way before anything else is loaded: on short walks their round trip is the run time
@@ -222,7 +227,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     // general mask and bias are applied in one go (excl_general).
     int lim = 0;                   // keys of the tile below it attend, counted from 4h
     MaskRow64 mrow;
+    uint32_t keep_bits[2];         // KEYS: of this lane's half, key block by key block
     auto excl_begin = [&](int t) {
+        if constexpr (KEYS) {
+            const uint64_t w = kt.bits[kt.tile(t)];
+            keep_bits[0] = (uint32_t)w >> (4 * h);
+            keep_bits[1] = (uint32_t)(w >> 32) >> (4 * h);
+        }
         const int limit = (p.m.causal ? min(klimit, qi + 1) : klimit) - t * BN;
         lim = limit - 4 * h;
         if constexpr (EXCL == kExRows16) {
@@ -264,6 +275,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             else v = __uint_as_float((uint32_t)bg[idx >> 2][idx & 3] << 16);
             s[kb][r] = fmaf(v, p.m.inv_scale, s[kb][r]);
         }
+        if constexpr (KEYS) s[kb][r] = keep_bits[kb] & (1u << (8 * (r >> 2) + (r & 3))) ? s[kb][r] : -INFINITY;
         if constexpr (EXCL == kExRows16) s[kb][r] = mrow.keep(kb, r, h) ? s[kb][r] : -INFINITY;
         if constexpr (EXCL == kExNone) s[kb][r] = 32 * kb + 8 * (r >> 2) + (r & 3) >= lim ? -INFINITY : s[kb][r];
     };
@@ -434,7 +446,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
 
     // Tiles below t_clean need no exclusions for any query of the workgroup; the rest (ragged tail, causal
     // diagonal, or everything under an explicit mask) carry per-element exclusions.
-    int t_clean = (EXCL == kExNone || BIAS) ? klimit / BN : 0;
+    int t_clean = KEYS ? kt.n_whole : (EXCL == kExNone || BIAS) ? klimit / BN : 0;
     if (p.m.causal) t_clean = min(t_clean, (q0 + 1) / BN);
     t_clean = min(t_clean, n_tiles);
 
@@ -470,7 +482,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
         // Two steps per trip, so that `sa` is the current tile when t is even; where the number of steps of
         // one kind is odd, the pair that mixes kinds runs as the more general one.
         int t = 0;
-        if (EXCL == kExNone || BIAS) {
+        if (EXCL == kExNone || BIAS || KEYS) {
             const int copy_end = t_clean - KD;              // steps below it copy two full tiles
             for (; t + 1 < copy_end; t += 2) {
                 step(Yes{}, Clean{}, sa, sb, t);
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 step(No{}, Clean{}, sb, sa, t + 1);
             }
         }
-        if (EXCL != kExNone && !BIAS) {
+        if (EXCL == kExRows16 || EXCL == kExGeneral) {
             const int copy_end = min(n_tiles, klimit / BN) - KD;
             for (; t + 1 < copy_end; t += 2) {
                 step(Yes{}, Cut{}, sa, sb, t);

@@ -49,6 +49,11 @@ int check_view(const void* base, const int64_t* st, int64_t off) {
 
 Strides mk(const int64_t* st) { return Strides{st[0], st[1], st[2]}; }
 
+// a keep-mask that is the same for every query
+bool keys_only(const MaskArgs& m, int N_q, int N_kv) {
+    return m.mask && (m.sq == 0 || N_q == 1) && !m.causal && (N_kv + 63) / 64 <= KeyTiles::kMaxTiles;
+}
+
 // FLAME_ATTN_WG_WAVES=4 forces 128-query workgroups in the forward and dQ kernels (read once per process)
 int wg_waves_override() {
     static const int value = [] {
@@ -124,12 +129,14 @@ int launch_fwd(const FwdParams& p, hipStream_t s) {
     constexpr int BM = 32 * NW;
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_kernel<D, EXCL, NW, DROPOUT>;
-    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
+    constexpr bool KEYS = EXCL == kExKeys;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
+    const int lds = T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
     const int64_t grid = (int64_t)((p.Sq + BM - 1) / BM) * p.B * p.H;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), T::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), lds, s, p);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -221,8 +228,9 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     using TQ = BwdDqTile<D>;
     static bool attr_done = false;
     auto kern = bwd_dkdv_kernel<D, HASMASK, TIMING>;
-    auto kern_dq = bwd_dq_kernel<D, HASMASK, 4>;
-    auto kern_dqv = bwd_dq_kernel<D, true, 4, true>;                 // keep-mask with vector-loadable rows over whole tiles
+    auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4>;
+    auto kern_dqk = bwd_dq_kernel<D, kExKeys, 4>;                    // keep-mask of keys
+    auto kern_dqv = bwd_dq_kernel<D, kExRows16, 4>;                  // keep-mask with vector-loadable rows over whole tiles
     auto kern_kvv = bwd_dkdv_kernel<D, true, false, true>;           // ... whose tiles travel through LDS
     using TW = BwdDqWideTile<D>;
     auto kern_dqw = bwd_dq_wide_kernel<D>;                           // 256-query workgroups, builds without a keep-mask only
@@ -236,6 +244,11 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqw),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, TW::LDS_BYTES);
         if (e != hipSuccess) return (int)e;
+        if (!HASMASK) {
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqk), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    TQ::LDS_BYTES + KeyTiles::lds_bytes(KeyTiles::kMaxTiles));
+            if (e != hipSuccess) return (int)e;
+        }
         if (HASMASK) {
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqv),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
@@ -252,7 +265,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     const int64_t n256 = (p.Sq + 255) / 256;
     // (with key lengths the walks differ in length and the longest ones set the time: unless the units fill two
     // rounds, twice as many workgroups of half the size finish sooner)
-    const bool wide = !HASMASK && n256 * 256 <= ((int64_t)(p.Sq + 127) / 128) * 128 && n256 * p.B * p.H >= device_cu_count() &&
+    const bool wide = !HASMASK && !p.key_mask && n256 * 256 <= ((int64_t)(p.Sq + 127) / 128) * 128 && n256 * p.B * p.H >= device_cu_count() &&
                       !(p.m.kv_len && n256 * p.B * p.H < 2 * device_cu_count()) && wg_waves_override() != 4;
     const int64_t n_qt = wide ? n256 : (p.Sq + TQ::BM - 1) / TQ::BM;
     const int64_t grid_dq = n_qt * p.B * p.H;
@@ -314,6 +327,8 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);
         if (wide) hipLaunchKernelGGL(kern_dqw, dim3((unsigned)grid_dq), dim3(256), TW::LDS_BYTES, s, p);
+        else if (!HASMASK && p.key_mask)
+            hipLaunchKernelGGL(kern_dqk, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
         else if (HASMASK && p.m.rows16 && p.Sk % TQ::BN == 0) hipLaunchKernelGGL(kern_dqv, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
         else hipLaunchKernelGGL(kern_dq, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
     }
@@ -328,7 +343,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         const int cus = device_cu_count();
         const int64_t rem = grid % cus;
         const int64_t n_qtiles = (p.Sq + T::BM - 1) / T::BM;
-        const bool uniform = !HASMASK && !p.m.causal && !p.m.kv_len;
+        const bool uniform = !HASMASK && !p.key_mask && !p.m.causal && !p.m.kv_len;
         if (uniform && grid > cus && rem > 0 && 2 * rem <= cus && n_qtiles >= 16 && p.split_ws) {
             int parts = (int)std::min<int64_t>(cus / rem, 4);
             const size_t room = p.split_ws_bytes / bwd_split_slot_bytes(D);
@@ -441,7 +456,7 @@ int launch_bwd_dropout(const BwdParams& p, hipStream_t s) {
     using TQ = BwdDqTile<D>;
     static bool attr_done = false;
     auto kern = bwd_dkdv_kernel<D, HASMASK, false, false, true>;
-    auto kern_dq = bwd_dq_kernel<D, HASMASK, 4, false, true>;
+    auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, true>;
     if (!attr_done) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
@@ -594,6 +609,8 @@ static int attn_bwd_impl(const void* Q, const void* K, const void* V, const void
         if (padded_head_dim(D) == 128) return keep_mask ? launch_bwd_dropout<128, true>(p, s) : launch_bwd_dropout<128, false>(p, s);
         return keep_mask ? launch_bwd_dropout<64, true>(p, s) : launch_bwd_dropout<64, false>(p, s);
     }
+    p.key_mask = keys_only(p.m, N_q, N_kv) ? 1 : 0;
+    if (p.key_mask) keep_mask = nullptr;           // served by the kernels without the general mask code
     if (padded_head_dim(D) == 128) return keep_mask ? launch_bwd<128, true>(p, s) : launch_bwd<128, false>(p, s);
     return keep_mask ? launch_bwd<64, true>(p, s) : launch_bwd<64, false>(p, s);
 }
@@ -952,8 +969,11 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     else if (q_tile_plan == 256 && !hm) wide = true;
     // ... as 4 wavefronts of 64 queries when nothing is excluded at all, else as 8 wavefronts of 32
     const bool plain = !causal && kv_len == nullptr && N_kv % 64 == 0;
-    // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel
     const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
+    // a keep-mask of keys: the walk takes the attended tiles only (up to what their list holds)
+    if (keep_mask != nullptr && bias == nullptr && keys_only(p.m, N_q, N_kv))
+        return DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
+    // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel
     if (keep_mask != nullptr && bias == nullptr && p.m.rows16 && N_kv % 64 == 0)
         return DP == 128 ? launch_fwd<128, kExRows16, 4>(p, s) : launch_fwd<64, kExRows16, 4>(p, s);
     // a bias alone, its rows contiguous: loaded in fours
