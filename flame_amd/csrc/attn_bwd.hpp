@@ -75,26 +75,29 @@ struct BwdTile {
     // with a keep-mask staged through LDS: [3 x (64 queries x 128 keys) mask bytes] behind the rest
     static constexpr int MASK_STAGE_BYTES = BM * BN;
     static constexpr int LDS_BYTES_VECMASK = LDS_BYTES + NSTAGE * MASK_STAGE_BYTES;
+    // kDropRows64: the generator's word of every query row at each wavefront's first key, behind the rest
+    static constexpr int LDS_BYTES_DROP = LDS_BYTES + 4 * BM * 4;
     static constexpr int ROWS_PER_DMA = 1024 / (D * 2);
     static constexpr int DMA_PER_WAVE = BM / ROWS_PER_DMA / 4;    // 1 KiB copies per wave and tensor
 };
 
 template <int D>
 __device__ __forceinline__ void dkdv_store(const BwdParams& p, const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32],
-                                           int b, int hh, int krow, int h);
+                                           int b, int hh, int krow, int h, float dv_scale = 1.0f);
 
 // VECMASK (with HASMASK): the keep-mask rows are contiguous and 16-byte aligned, Sq is a multiple of 64, Sk
 // of 128, and there is no causal flag.  The 64 x 128 mask bytes of a step then travel to LDS with the step's other copies (two more
 // 1 KiB copies per wavefront) and every lane reads the bytes of its key a few elements ahead of use,
 // instead of fetching 32 bytes from global memory into 32 registers at the start of every step; with the
 // registers back, the walk runs the same straight-line steps as the unmasked one.
-// DROPOUT: dV takes the dropped and rescaled probabilities, dP = f (dO V^T) with the same factor f (drop_factor), and
+// DROP (DropMode): dV takes the dropped and rescaled probabilities, dP = f (dO V^T) with the same factor f (drop_factor), and
 // -delta is added per element instead of seeding the dP accumulators.
 // block / nblocks: this workgroup's index in the dK/dV grid and the size of that grid (the kernel's own launch, or
 // the dK/dV part of bwd_joint_kernel's).
-template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, bool DROPOUT = false>
+template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int block, const int nblocks) {
     static_assert(!VECMASK || HASMASK, "VECMASK is a special case of HASMASK");
+    constexpr bool DROPOUT = DROP != kDropNone;
     using T = BwdTile<D>;
     constexpr int BM = T::BM, BN = T::BN, RS = T::RS;
     constexpr int DC = D / 16;     // contraction chunks over the head dim
@@ -318,6 +321,8 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
 
     const float c_log2 = p.scale * kLog2e;
     const int key = kw0 + n;
+    const uint32_t drop_lane = xorshift32((uint32_t)n);
+    (void)drop_lane;
     // VECMASK: a mask byte excludes its element when it is <= this: 0 for an attended key, 255 for one past the key length
     const uint32_t dead_thr = key >= klimit ? 0xffu : 0u;
 
@@ -436,9 +441,20 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         const uint8_t* nm_base = VECMASK ? mask_tile(qt_next) : nullptr;
         uint32_t m4[4], m4n[4];
         f32x4 nd4, nd4n;                 // DROPOUT: -delta of the same four queries
+        // kDropRows64: the index of (query, key) is the query's index at this wavefront's first key XOR the lane's n, so the 64
+        // lanes evaluate the generator for the 64 queries of the step, once, and pass the words on through LDS (a wavefront
+        // reads what it has written itself: no barrier)
+        u32x4 dw4{}, dw4n{};
+        // kDropFlat: index of the next element; the elements are visited in query order, four rows and then four of the other half
+        uint32_t drop_idx = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)(q0 + 4 * h)) * (uint32_t)p.Sk + (uint32_t)key;
+        (void)drop_idx;
+        uint32_t* const drop_words = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(lds) + T::LDS_BYTES) + wave * BM;
+        if constexpr (DROP == kDropRows64)
+            drop_words[lane] = xorshift32(p.m.drop_seed ^ (((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)(q0 + lane)) * (uint32_t)p.Sk + (uint32_t)kw0));
         auto rows_ahead = [&](int qb, int g) {
             l4n = *reinterpret_cast<const f32x4*>(rows_c + 32 * qb + 8 * g + 4 * h);
             if (DROPOUT) nd4n = *reinterpret_cast<const f32x4*>(rows_c + BM + 32 * qb + 8 * g + 4 * h);
+            if (DROP == kDropRows64) dw4n = *reinterpret_cast<const u32x4*>(drop_words + 32 * qb + 8 * g + 4 * h);
             if (VECMASK) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) m4n[t] = mask_c[(32 * qb + 8 * g + t) * BN];
@@ -461,6 +477,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
             if (t == 0) {
                 l4 = l4n;
                 if (DROPOUT) nd4 = nd4n;
+                if (DROP == kDropRows64) dw4 = dw4n;
                 if (VECMASK) {
 #pragma unroll
                     for (int u = 0; u < 4; ++u) m4[u] = m4n[u];
@@ -482,11 +499,23 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
                 }
                 pr = drop ? 0.f : pr;
             }
-            if constexpr (DROPOUT) {
+            if constexpr (DROP == kDropTiled) {
                 const uint32_t qi = (uint32_t)(q0 + 32 * qb + 8 * g + 4 * h + t);
                 const float f = drop_factor_at(p.m, (uint32_t)bh, qi, (uint32_t)key, (uint32_t)p.Sq, (uint32_t)p.Sk);
                 dpacc[qb][r] = pr * fmaf(f, dpacc[qb][r], nd4[t]);       // dS = P (f dP - delta)
                 pr *= f;                                                  // what multiplied V in the forward
+            } else if constexpr (DROPOUT) {                               // the same, dV rescaled at the end
+                uint32_t w;
+                if constexpr (DROP == kDropRows64) {
+                    w = dw4[t] ^ drop_lane;
+                } else {
+                    w = xorshift32(p.m.drop_seed ^ drop_idx);
+                    drop_idx += (t == 3 ? 5u : 1u) * (uint32_t)p.Sk;
+                    asm volatile("" : "+v"(drop_idx));       // stepped, not 32 multiples of Sk kept in registers
+                }
+                const bool kept = w >= p.m.drop_thr32;
+                dpacc[qb][r] = pr * fmaf(kept ? dpacc[qb][r] : 0.f, p.m.drop_scale, nd4[t]);
+                pr = kept ? pr : 0.f;
             }
             sacc[qb][r] = pr;
             if ((r & 7) == 7) {
@@ -698,18 +727,18 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
                 dvacc[db][r] = 0.f;
             }
     }
-    dkdv_store<D>(p, dkacc, dvacc, b, hh, kw0 + n, h);
+    dkdv_store<D>(p, dkacc, dvacc, b, hh, kw0 + n, h, DROP == kDropFlat || DROP == kDropRows64 ? p.m.drop_scale : 1.0f);
 }
 
-template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, bool DROPOUT = false>
+template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone>
 __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
-    bwd_dkdv_body<D, HASMASK, TIMING, VECMASK, DROPOUT>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_dkdv_body<D, HASMASK, TIMING, VECMASK, DROP>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // dK^T / dV^T accumulators (rows = d, column = this lane's key) -> bf16 rows of dK (scaled) and dV
 template <int D>
 __device__ __forceinline__ void dkdv_store(const BwdParams& p, const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32],
-                                           int b, int hh, int krow, int h) {
+                                           int b, int hh, int krow, int h, float dv_scale) {
     constexpr int DB = D / 32;
     if (krow < p.Sk) {
         uint16_t* dkrow = p.dk + b * p.dks.b + hh * p.dks.h + (int64_t)krow * p.dks.n;
@@ -722,7 +751,7 @@ __device__ __forceinline__ void dkdv_store(const BwdParams& p, const f32x16 (&dk
                 const f32x16& a = dkacc[db];
                 const f32x16& c = dvacc[db];
                 u32x2 wk = {pack_bf16(a[4 * g] * s, a[4 * g + 1] * s), pack_bf16(a[4 * g + 2] * s, a[4 * g + 3] * s)};
-                u32x2 wv = {pack_bf16(c[4 * g], c[4 * g + 1]), pack_bf16(c[4 * g + 2], c[4 * g + 3])};
+                u32x2 wv = {pack_bf16(c[4 * g] * dv_scale, c[4 * g + 1] * dv_scale), pack_bf16(c[4 * g + 2] * dv_scale, c[4 * g + 3] * dv_scale)};
                 if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dkrow + 32 * db + 8 * g + 4 * h) = wk;
                 if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dvrow + 32 * db + 8 * g + 4 * h) = wv;
             }
@@ -788,7 +817,7 @@ struct BwdDqTile {
 // NW wavefronts of 32 queries each per workgroup, two per SIMD (the library instantiates NW = 4; problems
 // that fill 256-query workgroups go to bwd_dq_wide_kernel below).
 // EXCL: see there.  Only the general form compiles per-element mask loads in; the others fit two workgroups per unit.
-template <int D, int EXCL, int NW, bool DROPOUT = false>
+template <int D, int EXCL, int NW, int DROP = kDropNone>
 __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
     constexpr bool HASMASK = EXCL == kExRows16 || EXCL == kExGeneral, VECMASK = EXCL == kExRows16, KEYS = EXCL == kExKeys;
     using T = BwdDqTile<D>;
@@ -957,6 +986,10 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
         const uint16_t* ks = lds + buf * T::STAGE_ELEMS;
         const uint16_t* vs = ks + T::TILE_ELEMS;
         const int key0 = t * BN;      // (not KEYS)
+        const uint32_t drop_tile = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qrow) * (uint32_t)p.Sk + (uint32_t)(key0 + 4 * h);
+        const uint32_t drop_word = DROP == kDropRows64 ? xorshift32(p.m.drop_seed ^ drop_tile) : 0u;
+        (void)drop_tile;
+        (void)drop_word;
         uint32_t keep_bits[2] = {0u, 0u};
         if constexpr (KEYS && MASKED) {
             const uint64_t w = kt.bits[kt.tile(t)];
@@ -1020,11 +1053,14 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
             sacc[kb][r] = pr;
         };
         auto ds_elem = [&](int kb, int r) {         // dS^T = P^T (dP^T - delta), packed after 8 and 16
-            if constexpr (DROPOUT) {
-                // O = (P f) V with f = 0 or 1 / (1 - p): dP = f (dO V^T), and rowsum(dP P) is still rowsum(dO O)
-                const uint32_t key = (uint32_t)(key0 + 32 * kb + acc_row(r, h));
-                const float f = drop_factor_at(p.m, (uint32_t)bh, (uint32_t)qrow, key, (uint32_t)p.Sq, (uint32_t)p.Sk);
+            // O = (P f) V with f = 0 or 1 / (1 - p): dP = f (dO V^T), and rowsum(dP P) is still rowsum(dO O)
+            const uint32_t off = 32 * kb + 8 * (r >> 2) + (r & 3);       // of the element, from drop_tile
+            if constexpr (DROP == kDropTiled) {
+                const float f = drop_factor_at(p.m, (uint32_t)bh, (uint32_t)qrow, (uint32_t)(key0 + 4 * h) + off, (uint32_t)p.Sq, (uint32_t)p.Sk);
                 dpacc[kb][r] = sacc[kb][r] * fmaf(f, dpacc[kb][r], -delta);
+            } else if constexpr (DROP != kDropNone) {
+                const uint32_t w = DROP == kDropRows64 ? drop_word ^ xorshift32(off) : xorshift32(p.m.drop_seed ^ (drop_tile + off));
+                dpacc[kb][r] = sacc[kb][r] * fmaf(w >= p.m.drop_thr32 ? dpacc[kb][r] : 0.f, p.m.drop_scale, -delta);
             } else {
                 dpacc[kb][r] = sacc[kb][r] * (dpacc[kb][r] - delta);
             }

@@ -440,6 +440,7 @@ struct MaskArgs {
     // dropout of the probabilities (kernels instantiated with DROPOUT only): see drop_factor
     uint32_t drop_seed = 0;  // low 32 bits of the seed
     uint32_t drop_thr = 0;   // ceil(p * 2^24): an element is kept when its 24-bit uniform is >= this
+    uint32_t drop_thr32 = 0; // drop_thr << 8, for the comparison with the whole 32-bit word
     float drop_scale = 1.f;  // 1 / (1 - p)
     uint32_t drop_cq = 0, drop_ck = 0;   // tiles of a chunked draw along queries and keys; drop_cq = 0: one draw over the tensor
 };
@@ -448,13 +449,27 @@ struct MaskArgs {
 // (low 32 bits): 0 or 1 / (1 - p).  The uniform is the reference's (src/rng/mod.rs:14-24, drawn over the whole
 // tensor by src/autograd_v4/ops/sdpa.rs:229-231, :604-649): u = (xorshift32(seed ^ idx) >> 8) / 2^24, kept when
 // u >= p, which in integers is (xorshift32(seed ^ idx) >> 8) >= ceil(p * 2^24).
-__device__ __forceinline__ float drop_factor(const MaskArgs& m, uint32_t idx) {
-    uint32_t s = m.drop_seed ^ idx;
+__device__ __forceinline__ constexpr uint32_t xorshift32(uint32_t s) {
     s ^= s << 13;
     s ^= s >> 17;
     s ^= s << 5;
-    return (s >> 8) >= m.drop_thr ? m.drop_scale : 0.f;
+    return s;
 }
+__device__ __forceinline__ float drop_factor(const MaskArgs& m, uint32_t idx) {
+    return (xorshift32(m.drop_seed ^ idx) >> 8) >= m.drop_thr ? m.drop_scale : 0.f;
+}
+
+// How a kernel draws.  xorshift32 is linear over GF(2): xorshift32(a ^ b) = xorshift32(a) ^ xorshift32(b).  Where the rows
+// of the probability tensor start on multiples of 64 elements (Sk % 64 == 0) the index of an element is the index of the
+// first element of its tile row XOR its offset, so one generator evaluation serves a row of a tile and every element costs
+// an XOR with a constant, a comparison and a select; the factor 1 / (1 - p) is left to the sums.  (One evaluation per
+// element, about ten vector instructions, more than doubles the vector work of the forward.)
+enum DropMode : int {
+    kDropNone = 0,
+    kDropTiled = 1,      // any draw, chunked ones among them (drop_factor_at)
+    kDropFlat = 2,       // one draw over the tensor
+    kDropRows64 = 3,     // ... whose rows start on multiples of 64 elements
+};
 
 // The same for element (bh, qi, key) when the reference's operator is chunked (src/autograd_v4/ops/sdpa.rs:180-199,
 // :444): it draws per tile of drop_cq x drop_ck (the last ones shorter) over the tile's own [B*H, q_t, k_t] tensor,
@@ -464,11 +479,7 @@ __device__ __forceinline__ float drop_factor_at(const MaskArgs& m, uint32_t bh, 
     if (m.drop_cq == 0) return drop_factor(m, (bh * Sq + qi) * Sk + key);
     const uint32_t qo = qi / m.drop_cq * m.drop_cq, ko = key / m.drop_ck * m.drop_ck;
     const uint32_t qt = min(m.drop_cq, Sq - qo), kt = min(m.drop_ck, Sk - ko);
-    uint32_t s = (m.drop_seed + ko) ^ ((bh * qt + (qi - qo)) * kt + (key - ko));
-    s ^= s << 13;
-    s ^= s >> 17;
-    s ^= s << 5;
-    return (s >> 8) >= m.drop_thr ? m.drop_scale : 0.f;
+    return (xorshift32((m.drop_seed + ko) ^ ((bh * qt + (qi - qo)) * kt + (key - ko))) >> 8) >= m.drop_thr ? m.drop_scale : 0.f;
 }
 
 // one element of an explicit mask, addressed in elements from the (batch, head) base: does it attend?

@@ -59,9 +59,9 @@ struct FwdTile {
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint16_t u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 
-// DROPOUT: the probabilities that multiply V are dropped and rescaled element by element (drop_factor); the row sums,
-// and with them the log-sum-exp, stay those of the undropped softmax.
-template <int D, int EXCL, int NW, bool DROPOUT = false>
+// DROP (DropMode): the probabilities that multiply V are dropped element by element (drop_factor) and O is rescaled; the
+// row sums, and with them the log-sum-exp, stay those of the undropped softmax.
+template <int D, int EXCL, int NW, int DROP = kDropNone>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const FwdParams p) {
     using T = FwdTile<D>;
     constexpr int BN = T::BN, RS = T::RS;
@@ -219,9 +219,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     constexpr int EPS = 32 / NS;   // logits handled per softmax slice
     constexpr int MPS = 32 / NP;   // logits handled per maximum-scan slice
 
-    // flat index (mod 2^32) of this lane's query row in the [B*H, Sq, Sk] probability tensor
-    const uint32_t drop_qi = (uint32_t)qi;
-    (void)drop_qi;
+    // DROP: flat index (mod 2^32) of this lane's first element of the row in the [B*H, Sq, Sk] probability tensor
+    const uint32_t drop_row = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qi) * (uint32_t)p.Sk + 4 * h;
+    (void)drop_row;
     // Exclusions of a tile.  The ragged tail / key length and the causal diagonal are one comparison per element with a
     // per-lane limit (excl_elem, threaded into the maximum scan); a keep-mask row is fetched when the step begins; the
     // general mask and bias are applied in one go (excl_general).
@@ -347,6 +347,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
         float rsum0 = 0.f, rsum1 = 0.f;
         bf16x8 pf[4];
         bf16x8 fb[PD];
+        const uint32_t drop_tile = drop_row + (uint32_t)(t * BN), drop_word = DROP == kDropRows64 ? xorshift32(p.m.drop_seed ^ drop_tile) : 0u;
+        (void)drop_tile;
+        (void)drop_word;
         // P(t): slice j covers logits [EPS*j, EPS*j + EPS) of the tile in (kb, r) order
         auto exp_slice = [&](int j) {
 #pragma unroll
@@ -355,9 +358,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 const float v = exp2_fast(fmaf(cur[kb][r], c_log2, -msc));
                 if (e & 1) rsum1 += v;
                 else rsum0 += v;
-                if constexpr (DROPOUT) {
-                    const uint32_t key = (uint32_t)(t * BN + 32 * kb + acc_row(r, h));
-                    cur[kb][r] = v * drop_factor_at(p.m, (uint32_t)bh, drop_qi, key, (uint32_t)p.Sq, (uint32_t)p.Sk);
+                const uint32_t off = 32 * kb + 8 * (r >> 2) + (r & 3);       // of the element, from drop_tile
+                if constexpr (DROP == kDropTiled) {
+                    cur[kb][r] = v * drop_factor_at(p.m, (uint32_t)bh, (uint32_t)qi, (uint32_t)(t * BN + 4 * h) + off, (uint32_t)p.Sq, (uint32_t)p.Sk);
+                } else if constexpr (DROP != kDropNone) {
+                    const uint32_t w = DROP == kDropRows64 ? drop_word ^ xorshift32(off) : xorshift32(p.m.drop_seed ^ (drop_tile + off));
+                    cur[kb][r] = w >= p.m.drop_thr32 ? v : 0.f;
                 } else {
                     cur[kb][r] = v;
                 }
@@ -515,7 +521,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     // ---- epilogue
     if (qi < p.Sq) {
         const float l = l_run + xhalf(l_run);
-        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        float inv = l > 0.f ? 1.0f / l : 0.f;
+        if constexpr (DROP == kDropFlat || DROP == kDropRows64) inv *= p.m.drop_scale;
         uint16_t* orow = p.o + b * p.os.b + hh * p.os.h + (int64_t)qi * p.os.n;
 #pragma unroll
         for (int db = 0; db < DB; ++db)

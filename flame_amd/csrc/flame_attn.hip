@@ -123,12 +123,12 @@ void launch_fwd_merge(const FwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL(fwd_merge_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, p);
 }
 
-template <int D, int EXCL, int NW, bool DROPOUT = false>
+template <int D, int EXCL, int NW, int DROP = kDropNone>
 int launch_fwd(const FwdParams& p, hipStream_t s) {
     using T = FwdTile<D>;
     constexpr int BM = 32 * NW;
     static std::atomic<bool> lds_set{false};
-    auto kern = fwd_kernel<D, EXCL, NW, DROPOUT>;
+    auto kern = fwd_kernel<D, EXCL, NW, DROP>;
     constexpr bool KEYS = EXCL == kExKeys;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
     const int lds = T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
@@ -448,24 +448,30 @@ int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc)
 template <int NC>
 int launch_fwd_bigd(const FwdParams& p, hipStream_t s, const FwdScratch& sc) { return launch_fwd_bigd_nw<NC, 4>(p, s, sc); }
 
-// Dropout of the probabilities: the 128-query forward and dQ kernels and the dK/dV kernel in their DROPOUT
+// how the kernels draw (after set_dropout)
+int drop_mode(const MaskArgs& m, int Sk) { return m.drop_cq != 0 ? kDropTiled : Sk % 64 == 0 ? kDropRows64 : kDropFlat; }
+
+// Dropout of the probabilities: the 128-query forward and dQ kernels and the dK/dV kernel in their DROP
 // instantiations, without the split of the last round; HASMASK: the general kernels for an explicit mask or bias.
-template <int D, bool HASMASK>
-int launch_bwd_dropout(const BwdParams& p, hipStream_t s) {
+template <int D>
+int launch_fwd_dropout(const FwdParams& p, bool has_mask, hipStream_t s) {
+    if (has_mask) return launch_fwd<D, kExGeneral, 4, kDropTiled>(p, s);
+    switch (drop_mode(p.m, p.Sk)) {
+        case kDropRows64: return launch_fwd<D, kExNone, 4, kDropRows64>(p, s);
+        case kDropFlat: return launch_fwd<D, kExNone, 4, kDropFlat>(p, s);
+        default: return launch_fwd<D, kExNone, 4, kDropTiled>(p, s);
+    }
+}
+
+template <int D, bool HASMASK, int DROP>
+int launch_bwd_drop(const BwdParams& p, hipStream_t s) {
     using T = BwdTile<D>;
     using TQ = BwdDqTile<D>;
-    static bool attr_done = false;
-    auto kern = bwd_dkdv_kernel<D, HASMASK, false, false, true>;
-    auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, true>;
-    if (!attr_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dq),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        attr_done = true;
-    }
+    static std::atomic<bool> lds_set{false}, lds_set_dq{false};
+    auto kern = bwd_dkdv_kernel<D, HASMASK, false, false, DROP>;
+    auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, DROP>;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES_DROP, lds_set)) return rc;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_dq), TQ::LDS_BYTES, lds_set_dq)) return rc;
     const int64_t grid = (int64_t)((p.Sk + T::BN - 1) / T::BN) * p.B * p.H;
     const int64_t grid_dq = (int64_t)((p.Sq + TQ::BM - 1) / TQ::BM) * p.B * p.H;
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
@@ -475,10 +481,19 @@ int launch_bwd_dropout(const BwdParams& p, hipStream_t s) {
     }
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DKDV, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES_DROP, s, p);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+template <int D>
+int launch_bwd_dropout(const BwdParams& p, bool has_mask, hipStream_t s) {
+    if (has_mask) return launch_bwd_drop<D, true, kDropTiled>(p, s);
+    switch (drop_mode(p.m, p.Sk)) {
+        case kDropRows64: return launch_bwd_drop<D, false, kDropRows64>(p, s);
+        case kDropFlat: return launch_bwd_drop<D, false, kDropFlat>(p, s);
+        default: return launch_bwd_drop<D, false, kDropTiled>(p, s);
+    }
 }
 
 // 0 <= p < 1 (src/autograd_v4/ops/sdpa.rs:110-116); fills the kernel-side description of the draw
@@ -490,6 +505,7 @@ bool set_dropout(MaskArgs& m, float dropout_p, uint64_t dropout_seed, int draw_c
     m.drop_ck = (uint32_t)ck;
     m.drop_seed = (uint32_t)dropout_seed;
     m.drop_thr = (uint32_t)ceil((double)dropout_p * 16777216.0);      // u >= p  <=>  24-bit integer >= ceil(p * 2^24)
+    m.drop_thr32 = m.drop_thr << 8;                                    // p <= 1 - 2^-24, so the 24-bit threshold fits
     const float keep = 1.0f - dropout_p;
     m.drop_scale = 1.0f / keep;
     return true;
@@ -606,8 +622,7 @@ static int attn_bwd_impl(const void* Q, const void* K, const void* V, const void
 #endif
     if (dropout_p != 0.f) {
         if (!set_dropout(p.m, dropout_p, dropout_seed, draw_cq, draw_ck, N_q, N_kv)) return FLAME_ATTN_ERR_INVALID;
-        if (padded_head_dim(D) == 128) return keep_mask ? launch_bwd_dropout<128, true>(p, s) : launch_bwd_dropout<128, false>(p, s);
-        return keep_mask ? launch_bwd_dropout<64, true>(p, s) : launch_bwd_dropout<64, false>(p, s);
+        return padded_head_dim(D) == 128 ? launch_bwd_dropout<128>(p, keep_mask != nullptr, s) : launch_bwd_dropout<64>(p, keep_mask != nullptr, s);
     }
     p.key_mask = keys_only(p.m, N_q, N_kv) ? 1 : 0;
     if (p.key_mask) keep_mask = nullptr;           // served by the kernels without the general mask code
@@ -957,9 +972,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         // the kernel of the undropped call, so that the log-sum-exp is the same to the bit
         if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q))
             return DP == 128 ? launch_fwd_keyshare<128, true>(p, s) : launch_fwd_keyshare<64, true>(p, s);
-        if (DP == 128)
-            return hm ? launch_fwd<128, kExGeneral, 4, true>(p, s) : launch_fwd<128, kExNone, 4, true>(p, s);
-        return hm ? launch_fwd<64, kExGeneral, 4, true>(p, s) : launch_fwd<64, kExNone, 4, true>(p, s);
+        return DP == 128 ? launch_fwd_dropout<128>(p, hm, s) : launch_fwd_dropout<64>(p, hm, s);
     }
     // 256-query workgroups when they neither add padding rows nor leave compute units
     // without a workgroup
