@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "attn_bwd.hpp"
+#include "attn_bwd_wide.hpp"
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
 #include "attn_fwd_keyshare.hpp"
@@ -1872,6 +1873,46 @@ size_t mat_band_row_bytes(int B, int H, int N_kv, bool backward) { return (size_
 size_t mat_fixed_bytes(int B, int H, int N_q, bool backward) { return backward ? align_up((size_t)B * H * N_q * sizeof(float), 256) : 0; }
 size_t mat_accum_bytes(int B, int H, int N_kv, int D, int Dv) { return align_up((size_t)B * H * N_kv * (size_t)(D + Dv) * sizeof(float), 256); }
 
+// The backward for head dims above 128 on kernels of its own (attn_bwd_wide.hpp): what it needs per (batch, head) slice.
+int pad128(int n) { return (n + 127) / 128 * 128; }
+size_t wide_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
+size_t wide_slice_bytes(int N_q, int N_kv) { return (size_t)pad128(N_q) * pad128(N_kv) * 4; }         // P and dS, bf16
+// as many slices at a time as 512 MiB hold (a slice above 2 GiB: not served)
+size_t wide_workspace_bytes(int B, int H, int N_q, int N_kv) {
+    const size_t slice = wide_slice_bytes(N_q, N_kv);
+    if (slice > ((size_t)2 << 30)) return 0;
+    const size_t n = std::max<size_t>(1, std::min<size_t>((size_t)B * H, ((size_t)512 << 20) / slice));
+    return wide_rows_bytes(B, H, N_q) + n * slice;
+}
+
+int launch_bwd_wide(BwdWideParams p, void* workspace, size_t bytes, hipStream_t s) {
+    static std::atomic<bool> lds_set{false};
+    if (const int rc = set_lds(reinterpret_cast<const void*>(bwd_wide_scores_kernel), BwdWideScoresTile::LDS_BYTES, lds_set)) return rc;
+    const int bh = p.B * p.H;
+    char* ws = static_cast<char*>(workspace);
+    p.ndelta = reinterpret_cast<float*>(ws);
+    p.lse2 = reinterpret_cast<float*>(ws + wide_rows_bytes(p.B, p.H, p.Sq) / 2);
+    p.sq_pad = pad128(p.Sq);
+    p.sk_pad = pad128(p.Sk);
+    const size_t slice = wide_slice_bytes(p.Sq, p.Sk), fixed = wide_rows_bytes(p.B, p.H, p.Sq);
+    const int group = (int)std::min<size_t>((size_t)bh, (bytes - fixed) / slice);
+    p.probs = reinterpret_cast<uint16_t*>(ws + fixed);
+    p.ds = p.probs + (size_t)group * p.sq_pad * p.sk_pad;
+    const int64_t n_kt = p.sk_pad / 128, n_qt = p.sq_pad / 128, n_dt = (p.d + 127) / 128;
+    const int64_t rows = (int64_t)bh * p.Sq;
+    if ((rows + 3) / 4 > 0x7fffffff || group * n_kt * n_qt > 0x7fffffff || group * (2 * n_kt + n_qt) * n_dt > 0x7fffffff)
+        return FLAME_ATTN_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(bwd_wide_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, p);
+    for (p.bh0 = 0; p.bh0 < bh; p.bh0 += group) {
+        p.n_slices = std::min(group, bh - p.bh0);
+        hipLaunchKernelGGL(bwd_wide_scores_kernel, dim3((unsigned)(p.n_slices * n_kt * n_qt)), dim3(256), BwdWideScoresTile::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(bwd_wide_products_kernel, dim3((unsigned)(p.n_slices * (2 * n_kt + n_qt) * n_dt)), dim3(256),
+                           BwdWideProductsTile::LDS_BYTES, s, p);
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
 struct MatPlan {
     int tq = 0;              // query rows per band
     bool accumulate = false; // more than one band in the backward: dK / dV are summed in fp32 and stored at the end
@@ -1944,7 +1985,8 @@ size_t flame_attn_materialised_workspace_bytes(int B, int H, int N_q, int N_kv, 
     // bands of at least 64 rows and at most 512 MiB, with the fp32 dK / dV sums a banded backward needs
     const size_t band_rows = std::max<size_t>(64, std::min<size_t>((size_t)N_q, ((size_t)512 << 20) / per_row / 16 * 16));
     const size_t banded = fixed + (bw ? mat_accum_bytes(B, H, N_kv, D, Dv) : 0) + per_row * (band_rows + 1) + 1024;
-    return std::min(whole, banded);
+    const size_t wide = bw && D == Dv && D % 8 == 0 ? wide_workspace_bytes(B, H, N_q, N_kv) : 0;
+    return std::max(std::min(whole, banded), wide);
 }
 
 static int mat_fwd_impl(const void* Q, const void* K, const void* V, void* O, void* LSE,
@@ -2043,6 +2085,30 @@ int flame_attn_bwd_materialised_bf16(const void* Q, const void* K, const void* V
         return rc;
     if (keep_mask && !mask_strides) return FLAME_ATTN_ERR_INVALID;
     if ((int64_t)B * H * N_q > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    // head dims in granules of 8, nothing excluded but by causal flag and key lengths, rows the copies can take: the wide kernels
+    if (D % 8 == 0 && Dv == D && !keep_mask && dropout_p == 0.f && workspace && aligned16(workspace) && wide_workspace_bytes(1, 1, N_q, N_kv) != 0 &&
+        workspace_bytes >= wide_rows_bytes(B, H, N_q) + wide_slice_bytes(N_q, N_kv) &&
+        !check_view(Q, q_strides, q_off) && !check_view(K, k_strides, k_off) && !check_view(V, v_strides, v_off) && !check_view(O, o_strides, o_off) &&
+        !check_view(dO, do_strides, do_off) && !check_view(dQ, dq_strides, dq_off) && !check_view(dK, dk_strides, dk_off) &&
+        !check_view(dV, dv_strides, dv_off)) {
+        BwdWideParams w{};
+        w.q = static_cast<const uint16_t*>(Q) + q_off;
+        w.k = static_cast<const uint16_t*>(K) + k_off;
+        w.v = static_cast<const uint16_t*>(V) + v_off;
+        w.o = static_cast<const uint16_t*>(O) + o_off;
+        w.dout = static_cast<const uint16_t*>(dO) + do_off;
+        w.lse = static_cast<const float*>(LSE) + lse_off;
+        w.dq = static_cast<uint16_t*>(dQ) + dq_off;
+        w.dk = static_cast<uint16_t*>(dK) + dk_off;
+        w.dv = static_cast<uint16_t*>(dV) + dv_off;
+        w.qs = mk(q_strides); w.ks = mk(k_strides); w.vs = mk(v_strides); w.os = mk(o_strides);
+        w.dos = mk(do_strides); w.dqs = mk(dq_strides); w.dks = mk(dk_strides); w.dvs = mk(dv_strides);
+        w.B = B; w.H = H; w.Sq = N_q; w.Sk = N_kv; w.d = D;
+        w.scale = scale;
+        w.kv_len = kv_len;
+        w.causal = causal ? 1 : 0;
+        return launch_bwd_wide(w, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    }
     MatPlan plan;
     if ((rc = mat_plan(workspace, workspace_bytes, B, H, N_q, N_kv, D, Dv, true, &plan))) return rc;
     void* handle = nullptr;

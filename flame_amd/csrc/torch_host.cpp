@@ -313,7 +313,7 @@ struct Sdpa : public torch::autograd::Function<Sdpa> {
         }
         Grads g;
         int rc = FLAME_ATTN_ERR_UNSUPPORTED;
-        if (!ctx->saved_data["materialised"].toBool()) rc = call_bwd(q, k, v, o, d_o, lse, z, scale, causal, Tensor(), mv, Tensor(), g);
+        if (!ctx->saved_data["materialised"].toBool() && z.D <= 128) rc = call_bwd(q, k, v, o, d_o, lse, z, scale, causal, Tensor(), mv, Tensor(), g);
         if (rc == FLAME_ATTN_ERR_UNSUPPORTED) {         // a head dim the fused forward serves and the fused backward does not
             rc = call_bwd_materialised(q, k, v, o, d_o, lse, z, scale, causal, mv, g);
             if (rc != FLAME_ATTN_OK) throw_python({"flame_attn_bwd_materialised_bf16", rc});
