@@ -37,6 +37,7 @@ struct BwdParams {
     int n_whole = -1;
     int split_parts = 1;
     int rows_ready = 0;            // -delta and lse2 are in the workspace already (bwd_rows_kernel ran): read, do not form
+    int dq_base = 0;               // the dQ launch covers the problem's workgroups from this one on (problems without exclusions only)
     int joint_n_dq = 0;            // bwd_joint_kernel: the first joint_n_dq workgroups are dQ workgroups
     float* split_ws = nullptr;
     size_t split_ws_bytes = 0;     // host side only
@@ -834,7 +835,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len || KEYS ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.m.kv_len || KEYS ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
     const int b = bh / p.H, hh = bh % p.H;

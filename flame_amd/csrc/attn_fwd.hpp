@@ -37,6 +37,7 @@ struct FwdParams {
     int dv;              // real head dim of V and O, likewise
     float scale;
     MaskArgs m;
+    int wg_base = 0;     // the launch covers the problem's workgroups from this one on (problems without exclusions only)
     // Key split (the key-sharing forward and the one for head dims above 128): key_splits workgroups share a query tile, each walks a contiguous slice of its key tiles and leaves a
     // normalised fp32 partial output with its log-sum-exp; fwd_merge_kernel combines them.
     int key_splits = 1;          // 1: O and LSE are written directly
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len || EXCL == kExKeys ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.m.kv_len || EXCL == kExKeys ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
     const int b = bh / p.H, hh = bh % p.H;

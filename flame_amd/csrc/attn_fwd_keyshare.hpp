@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256) void fwd_keyshare_kernel(const FwdParams p) {
 
     const int n_qt = (p.Sq + T::BQ - 1) / T::BQ;
     const int all = xcd_remap(blockIdx.x, gridDim.x);            // the workgroups of a (batch, head) share an L2
-    const int slice = all % p.key_splits, wg = all / p.key_splits;
+    const int slice = all % p.key_splits, wg = p.wg_base + all / p.key_splits;
     const int bh = wg / n_qt, qi = (wg % n_qt) * T::BQ + n, q0 = (wg % n_qt) * T::BQ;     // qi: this lane's query
     const int b = bh / p.H, hh = bh % p.H;
     const uint16_t* qbase = p.q + b * p.qs.b + hh * p.qs.h;

@@ -109,6 +109,20 @@ struct ScopedKernelTimer {
     }
 };
 
+// compute units of the current device (cached; 256 when the query fails)
+int device_cu_count() {
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+            cus = n;
+        else
+            cus = 256;
+    }
+    return cus;
+}
+
 // the kernel's dynamic LDS size, set once per kernel (idempotent, so a benign race at worst repeats the call)
 int set_lds(const void* kern, int bytes, std::atomic<bool>& done) {
     if (done.load(std::memory_order_relaxed)) return FLAME_ATTN_OK;
@@ -124,8 +138,9 @@ void launch_fwd_merge(const FwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL(fwd_merge_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, p);
 }
 
+// wg_count workgroups from p.wg_base on (0: all of the problem's)
 template <int D, int EXCL, int NW, int DROP = kDropNone>
-int launch_fwd(const FwdParams& p, hipStream_t s) {
+int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     using T = FwdTile<D>;
     constexpr int BM = 32 * NW;
     static std::atomic<bool> lds_set{false};
@@ -133,7 +148,7 @@ int launch_fwd(const FwdParams& p, hipStream_t s) {
     constexpr bool KEYS = EXCL == kExKeys;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
     const int lds = T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
-    const int64_t grid = (int64_t)((p.Sq + BM - 1) / BM) * p.B * p.H;
+    const int64_t grid = wg_count ? wg_count : (int64_t)((p.Sq + BM - 1) / BM) * p.B * p.H;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
@@ -144,12 +159,12 @@ int launch_fwd(const FwdParams& p, hipStream_t s) {
 }
 
 template <int D, bool DROPOUT>
-int launch_fwd_keyshare(const FwdParams& p, hipStream_t s) {
+int launch_fwd_keyshare(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     using T = FwdKeyShareTile<D>;
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_keyshare_kernel<D, DROPOUT>;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
-    const int64_t grid = (int64_t)((p.Sq + T::BQ - 1) / T::BQ) * p.B * p.H * p.key_splits;
+    const int64_t grid = (wg_count ? wg_count : (int64_t)((p.Sq + T::BQ - 1) / T::BQ) * p.B * p.H) * p.key_splits;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
@@ -162,22 +177,28 @@ int launch_fwd_keyshare(const FwdParams& p, hipStream_t s) {
 
 // 256-query workgroups, one wavefront per SIMD (builds without keep-mask / bias only)
 template <int D>
-int launch_fwd_wide(const FwdParams& p, hipStream_t s) {
+int launch_fwd_wide(FwdParams p, hipStream_t s) {
     using T = FwdWideTile<D>;
-    static bool attr_done = false;
+    static std::atomic<bool> lds_set{false};
     auto kern = fwd_wide_kernel<D>;
-    if (!attr_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        attr_done = true;
-    }
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
     const int64_t n_qt = (p.Sq + T::BM - 1) / T::BM;
-    const int64_t grid = n_qt * p.B * p.H;
-    if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    const int64_t total = n_qt * p.B * p.H, cus = device_cu_count();
+    if (8 * total > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    // A last round that would leave at least half of the compute units idle goes to smaller workgroups in a launch of its own:
+    // 32-query ones that share the keys while these fit one per unit, else 128-query ones.  (B=2 H=24 S=1536 D=128: 288
+    // units of 256 queries, 92 us as two rounds, 79 us as one round and 256 small workgroups.)
+    const int64_t rest = total % cus;
+    const bool cut = total > cus && rest > 0 && 2 * rest <= cus;
+    const int64_t count = cut ? total - rest : total;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)count), dim3(256), T::LDS_BYTES, s, p);
+    }
+    if (cut) {
+        const bool share = 8 * rest <= cus && (p.Sq + 31) / 32 == 8 * n_qt;
+        p.wg_base = (int)(count * (share ? 8 : 2));
+        return share ? launch_fwd_keyshare<D, false>(p, s, 8 * rest) : launch_fwd<D, kExNone, 4>(p, s, 2 * rest);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -204,20 +225,6 @@ bool head_dim_ok(int D) { return D > 0 && D <= 128 && D % 8 == 0; }
 // head dims served by the forward alone, in chunks of 128 (attn_fwd_bigd.hpp)
 bool big_head_dim_ok(int D) { return D > 128 && D <= 512 && D % 8 == 0; }
 int padded_head_dim(int D) { return D <= 64 ? 64 : 128; }
-
-// compute units of the current device (cached; 256 when the query fails)
-int device_cu_count() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            cus = n;
-        else
-            cus = 256;
-    }
-    return cus;
-}
 
 // backward workspace: [-delta rows][lse2 rows][fp32 partials of the split dK/dV workgroups]
 size_t bwd_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
@@ -327,7 +334,18 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     // workspace, which the dK/dV kernel stages per query tile.
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);
-        if (wide) hipLaunchKernelGGL(kern_dqw, dim3((unsigned)grid_dq), dim3(256), TW::LDS_BYTES, s, p);
+        if (wide) {
+            // a last round on at most half of the compute units: 128-query workgroups in a launch of their own (problems
+            // whose walks are all equally long)
+            const int64_t cus = device_cu_count(), rest = grid_dq % cus;
+            const bool cut = grid_dq > cus && rest > 0 && 2 * rest <= cus && !p.m.causal && !p.m.kv_len && 2 * grid_dq <= 0x7fffffff;
+            hipLaunchKernelGGL(kern_dqw, dim3((unsigned)(cut ? grid_dq - rest : grid_dq)), dim3(256), TW::LDS_BYTES, s, p);
+            if (cut) {
+                BwdParams pt = p;
+                pt.dq_base = (int)(2 * (grid_dq - rest));
+                hipLaunchKernelGGL(kern_dq, dim3((unsigned)(2 * rest)), dim3(256), TQ::LDS_BYTES, s, pt);
+            }
+        }
         else if (!HASMASK && p.key_mask)
             hipLaunchKernelGGL(kern_dqk, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
         else if (HASMASK && p.m.rows16 && p.Sk % TQ::BN == 0) hipLaunchKernelGGL(kern_dqv, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
