@@ -38,6 +38,7 @@ struct BwdParams {
     int split_parts = 1;
     int rows_ready = 0;            // -delta and lse2 are in the workspace already (bwd_rows_kernel ran): read, do not form
     int dq_base = 0;               // the dQ launch covers the problem's workgroups from this one on (problems without exclusions only)
+    int dq_parts = 1;              // workgroups that share the key walk of one 128-query tile, leaving fp32 partial sums in split_ws
     int joint_n_dq = 0;            // bwd_joint_kernel: the first joint_n_dq workgroups are dQ workgroups
     float* split_ws = nullptr;
     size_t split_ws_bytes = 0;     // host side only
@@ -122,8 +123,8 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         wg = p.m.kv_len || p.key_mask ? xcd_remap_heads(block, nblocks, n_kt) : xcd_remap(block, nblocks);
     } else if (block < p.n_whole) {
         wg = xcd_remap(block, p.n_whole);
-    } else {          // the split key blocks come last in dispatch order and fill the final, partial round
-        const int e = block - p.n_whole;
+    } else {          // the split key blocks come last in dispatch order and fill the final, partial round (or are all there is)
+        const int e = p.n_whole == 0 ? xcd_remap(block, nblocks) : block - p.n_whole;
         nparts = p.split_parts;
         wg = p.n_whole + e / nparts;
         part = e % nparts;
@@ -704,7 +705,8 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
 
     // ---- epilogue
     if (nparts > 1) {
-        // fp32 partial sums of this slice, in accumulator order: [tensor][thread][db][16]
+        // fp32 partial sums of this slice, in accumulator order: [tensor][db][group of four][thread], so that the lanes of a
+        // wavefront write, and the merge reads, 1 KiB at a time
         float* dst = p.split_ws + ((size_t)(wg - p.n_whole) * nparts + part) * (size_t)(2 * BN * D);
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -712,10 +714,9 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
             for (int g = 0; g < 4; ++g) {
                 const f32x16& a = dkacc[db];
                 const f32x16& c = dvacc[db];
-                const f32x4 wk = {a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
-                const f32x4 wv = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-                *reinterpret_cast<f32x4*>(dst + ((size_t)tid * DB + db) * 16 + 4 * g) = wk;
-                *reinterpret_cast<f32x4*>(dst + (size_t)BN * D + ((size_t)tid * DB + db) * 16 + 4 * g) = wv;
+                const size_t at = ((size_t)(db * 4 + g) * 256 + tid) * 4;
+                *reinterpret_cast<f32x4*>(dst + at) = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+                *reinterpret_cast<f32x4*>(dst + (size_t)BN * D + at) = f32x4{c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
             }
         return;
     }
@@ -759,7 +760,8 @@ __device__ __forceinline__ void dkdv_store(const BwdParams& p, const f32x16 (&dk
     }
 }
 
-// Sums the fp32 partials that the split workgroups of one key block left behind and writes dK, dV.
+// Sums the fp32 partials that the split workgroups of one key block left behind and writes dK, dV; keys that nothing attends
+// to (past the key length, masked, past the last query under the causal flag) get zeros.
 // One workgroup per (split key block, 32-wide block of d); the thread layout mirrors the accumulators.
 template <int D>
 __global__ __launch_bounds__(256) void bwd_dkdv_merge_kernel(const BwdParams p) {
@@ -779,16 +781,20 @@ __global__ __launch_bounds__(256) void bwd_dkdv_merge_kernel(const BwdParams p) 
         ak[g] = f32x4{0.f, 0.f, 0.f, 0.f};
         av[g] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    for (int part = 0; part < p.split_parts; ++part) {
-        const float* src = p.split_ws + ((size_t)sb * p.split_parts + part) * (size_t)(2 * BN * D) + ((size_t)tid * DB + db) * 16;
+    const float* src = p.split_ws + (size_t)sb * p.split_parts * (size_t)(2 * BN * D) + ((size_t)db * 4 * 256 + tid) * 4;
+#pragma unroll 2
+    for (int part = 0; part < p.split_parts; ++part, src += (size_t)(2 * BN * D)) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            ak[g] += *reinterpret_cast<const f32x4*>(src + 4 * g);
-            av[g] += *reinterpret_cast<const f32x4*>(src + (size_t)BN * D + 4 * g);
+            ak[g] += *reinterpret_cast<const f32x4*>(src + g * 1024);
+            av[g] += *reinterpret_cast<const f32x4*>(src + (size_t)BN * D + g * 1024);
         }
     }
     const int krow = kt * BN + 32 * wave + n;
     if (krow < p.Sk) {
+        bool dead = p.m.kv_len && krow >= p.m.kv_len[b];
+        if (p.key_mask && !dead) dead = !mask_attends(p.m, mask_head_base(p.m, b, hh), (int64_t)krow * p.m.sk);
+        if (p.m.causal && kt * BN >= p.Sq) dead = true;
         uint16_t* dkrow = p.dk + b * p.dks.b + hh * p.dks.h + (int64_t)krow * p.dks.n;
         uint16_t* dvrow = p.dv + b * p.dvs.b + hh * p.dvs.h + (int64_t)krow * p.dvs.n;
         const float s = p.scale;
@@ -796,6 +802,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_merge_kernel(const BwdParams p) 
         for (int g = 0; g < 4; ++g) {
             u32x2 wk = {pack_bf16(ak[g][0] * s, ak[g][1] * s), pack_bf16(ak[g][2] * s, ak[g][3] * s)};
             u32x2 wv = {pack_bf16(av[g][0], av[g][1]), pack_bf16(av[g][2], av[g][3])};
+            if (dead) wk = wv = u32x2{0u, 0u};
             if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dkrow + 32 * db + 8 * g + 4 * h) = wk;
             if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dvrow + 32 * db + 8 * g + 4 * h) = wv;
         }
@@ -835,9 +842,16 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len || KEYS ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
+    int wg, part = 0;
+    if (p.dq_parts > 1) {
+        const int all = xcd_remap(blockIdx.x, gridDim.x);
+        part = all % p.dq_parts;
+        wg = all / p.dq_parts;
+    } else {
+        wg = p.m.kv_len || KEYS ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
+    }
     int qt = wg % n_qt, bh = wg / n_qt;
-    if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
+    if (p.m.causal && !p.m.kv_len && p.dq_parts == 1) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 32;
@@ -853,7 +867,13 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
     if (p.m.causal) kend = min(kend, q0 + BM);
     int n_tiles = (kend + BN - 1) / BN;
     const uint8_t* mbase = HASMASK || KEYS ? mask_head_base(p.m, b, hh) : nullptr;
-    // KEYS: step t of the walk takes tile tile_of(t) (elsewhere the two are the same number)
+    int t_lo = 0;             // first tile of this workgroup's share of the walk
+    if (p.dq_parts > 1) {
+        const int per = (n_tiles + p.dq_parts - 1) / p.dq_parts;
+        t_lo = part * per;
+        n_tiles = min(n_tiles, t_lo + per) - t_lo;      // not positive: nothing to do
+    }
+    // step t of the walk takes tile tile_of(t)
     KeyTiles kt;
     if constexpr (KEYS) {
         kt.build(reinterpret_cast<char*>(lds) + T::LDS_BYTES, klimit, NW, [&](int key) {
@@ -863,7 +883,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
     }
     auto tile_of = [&](int t) {
         if constexpr (KEYS) return kt.tile(t);
-        else return t;
+        else return t_lo + t;
     };
 
     // ---- Q and dO fragments (B operands: column = query, 8 consecutive d), per-query scalars
@@ -986,7 +1006,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
         else if (t + 1 < n_tiles) issue_tile(t + 1, buf ^ 1);
         const uint16_t* ks = lds + buf * T::STAGE_ELEMS;
         const uint16_t* vs = ks + T::TILE_ELEMS;
-        const int key0 = t * BN;      // (not KEYS)
+        const int key0 = (t_lo + t) * BN;      // (not KEYS)
         const uint32_t drop_tile = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qrow) * (uint32_t)p.Sk + (uint32_t)(key0 + 4 * h);
         const uint32_t drop_word = DROP == kDropRows64 ? xorshift32(p.m.drop_seed ^ drop_tile) : 0u;
         (void)drop_tile;
@@ -1126,7 +1146,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
 
     int n_full = HASMASK ? 0 : KEYS ? kt.n_whole : klimit / BN;
     if (p.m.causal) n_full = min(n_full, (q0 + 1) / BN);
-    n_full = min(n_full, n_tiles);
+    n_full = min(n_full - t_lo, n_tiles);
     using IM = std::integral_constant<int, -1>;
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
@@ -1141,7 +1161,19 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
         for (; t < n_tiles; ++t) tile_step(std::true_type{}, I2{}, IM{}, t);
     }
 
-    // ---- epilogue: dQ = scale * dQ^T, bf16
+    // ---- epilogue: fp32 partial sums for bwd_dq_merge_kernel, in accumulator order: [db][group of four][thread] ...
+    if (p.dq_parts > 1) {
+        float* dst = p.split_ws + ((size_t)wg * p.dq_parts + part) * (size_t)(BM * D);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x16& a = dqacc[db];
+                *reinterpret_cast<f32x4*>(dst + ((size_t)(db * 4 + g) * 256 + tid) * 4) = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+            }
+        return;
+    }
+    // ... or dQ = scale * dQ^T, bf16
     if (qok) {
         uint16_t* dqrow = p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)qrow * p.dqs.n;
         const float s = p.scale;
@@ -1153,6 +1185,34 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
                 u32x2 w = {pack_bf16(a[4 * g] * s, a[4 * g + 1] * s), pack_bf16(a[4 * g + 2] * s, a[4 * g + 3] * s)};
                 if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dqrow + 32 * db + 8 * g + 4 * h) = w;
             }
+    }
+}
+
+// Sums the fp32 partials of the workgroups that shared a 128-query tile and writes dQ.  One workgroup per (tile, 32-wide block
+// of d); the thread layout mirrors the accumulators.
+template <int D>
+__global__ __launch_bounds__(256) void bwd_dq_merge_kernel(const BwdParams p) {
+    constexpr int BM = BwdDqTile<D>::BM, DB = D / 32;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 31, h = lane >> 5;
+    const int wg = (int)blockIdx.x / DB, db = (int)blockIdx.x % DB;
+    const int n_qt = (p.Sq + BM - 1) / BM;
+    const int bh = wg / n_qt, b = bh / p.H, hh = bh % p.H;
+    f32x4 acc[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float* src = p.split_ws + (size_t)wg * p.dq_parts * (size_t)(BM * D) + ((size_t)db * 4 * 256 + tid) * 4;
+#pragma unroll 4
+    for (int part = 0; part < p.dq_parts; ++part, src += (size_t)(BM * D)) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) acc[g] += *reinterpret_cast<const f32x4*>(src + g * 1024);
+    }
+    const int row = (wg % n_qt) * BM + 32 * wave + n;
+    if (row >= p.Sq) return;
+    uint16_t* dqrow = p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)row * p.dqs.n;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const u32x2 w = {pack_bf16(acc[g][0] * p.scale, acc[g][1] * p.scale), pack_bf16(acc[g][2] * p.scale, acc[g][3] * p.scale)};
+        if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dqrow + 32 * db + 8 * g + 4 * h) = w;
     }
 }
 

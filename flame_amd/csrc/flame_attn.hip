@@ -349,7 +349,19 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         else if (!HASMASK && p.key_mask)
             hipLaunchKernelGGL(kern_dqk, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
         else if (HASMASK && p.m.rows16 && p.Sk % TQ::BN == 0) hipLaunchKernelGGL(kern_dqv, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
-        else hipLaunchKernelGGL(kern_dq, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
+        else {
+            // query tiles on at most half of the compute units: their key walks are shared, where the steps saved outweigh the
+            // merge (about 5 us, a step being about 1 us)
+            BwdParams pq = p;
+            const int tiles = (p.Sk + TQ::BN - 1) / TQ::BN;
+            if (!HASMASK && 2 * grid_dq <= device_cu_count() && p.split_ws) {
+                int64_t parts = std::min<int64_t>(std::min<int64_t>(device_cu_count() / grid_dq, 16), tiles / 4);
+                while (parts > 1 && (size_t)(grid_dq * parts) * (TQ::BM * D * sizeof(float)) > p.split_ws_bytes) --parts;
+                if (parts > 1 && tiles - (tiles + parts - 1) / parts >= 12) pq.dq_parts = (int)parts;
+            }
+            hipLaunchKernelGGL(kern_dq, dim3((unsigned)(grid_dq * pq.dq_parts)), dim3(256), TQ::LDS_BYTES, s, pq);
+            if (pq.dq_parts > 1) hipLaunchKernelGGL(bwd_dq_merge_kernel<D>, dim3((unsigned)(grid_dq * (D / 32))), dim3(256), 0, s, pq);
+        }
     }
     // The dK/dV kernel keeps one workgroup per compute unit.  When the key blocks do not fill the last
     // round of that schedule, the blocks of the last round are split over the idle units along the query
@@ -372,6 +384,19 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
                 pk.split_parts = parts;
                 n_split = (int)rem;
                 grid_kv = pk.n_whole + rem * parts;
+            }
+        }
+        // Key blocks on at most half of the compute units (few keys or few heads): every one is split along its query walk,
+        // where the steps saved outweigh the merge (about 5 us, or 8 steps).  (B=8 H=1, 1993 queries, 64 keys, D = 64:
+        // 8 workgroups, dK/dV 30 us; 14 us with the split, backward 36.6 -> 25 us.)
+        if (!HASMASK && 2 * grid <= cus && p.split_ws) {
+            int64_t parts = std::min<int64_t>(std::min<int64_t>(cus / grid, 16), n_qtiles / 4);
+            while (parts > 1 && (size_t)(grid * parts) * bwd_split_slot_bytes(D) > p.split_ws_bytes) --parts;
+            if (parts > 1 && n_qtiles - (n_qtiles + parts - 1) / parts >= 12) {
+                pk.n_whole = 0;
+                pk.split_parts = (int)parts;
+                n_split = (int)grid;
+                grid_kv = grid * parts;
             }
         }
     }
