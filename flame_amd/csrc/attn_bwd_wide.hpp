@@ -9,11 +9,14 @@
 // are [Sq, Sk] padded to multiples of 128 (zero there), so that the products need no tests in their loops; the launcher
 // takes as many (batch, head) slices at a time as the workspace holds.  Tiles that the causal flag excludes are neither
 // formed nor read.
-// Tiles are copied global -> LDS by LDS-DMA in steps of 32 along the contraction, two stages, one barrier per step, and at
-// least two workgroups per compute unit, so that one's wait is covered by the other.  Bound by LDS traffic: a wavefront's
-// 64 x 64 tile reads 8 KiB per 8 MFMAs.
-// B=1 H=1 S=4096 D=512: library GEMMs and separate passes 246 us, this 159 us; B=3 H=2 S=640 D=512, where the
-// library's 15 calls kept the host busy, forward and backward: 615 -> 80 us.
+// Tiles of 128 rows x 64 (or 64 x 128) elements, 16 KiB each, are copied global -> LDS by LDS-DMA through a ring of five
+// (WideRing): rows of a tile are whole 128-byte cache lines, and while one pair of tiles is multiplied the next pair and half
+// of the one after are on their way.  Two workgroups per compute unit.  Bound by LDS traffic: a wavefront's 64 x 64 tile reads
+// 8 KiB and its share of the copies writes 4 KiB per 8 MFMAs.
+// B=1 H=1 S=4096 D=512: scores 54 us (0.64 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
+// stages, whose 64-byte rows fetched every line twice, and stores straight from the accumulators; 246 us for the whole
+// backward by library GEMMs and separate passes.  B=3 H=2 S=640 D=512, where the library's 15 calls kept the host busy,
+// forward and backward: 615 -> 80 us.
 #pragma once
 #include "attn_common.hpp"
 
@@ -35,7 +38,7 @@ struct BwdWideParams {
     int causal;
 };
 
-constexpr int kWideTile = 128, kWideStep = 32;
+constexpr int kWideTile = 128, kWideStep = 64;
 
 // one wavefront per query row
 static __global__ __launch_bounds__(256) void bwd_wide_rows_kernel(const BwdWideParams p) {
@@ -61,70 +64,79 @@ static __global__ __launch_bounds__(256) void bwd_wide_rows_kernel(const BwdWide
     }
 }
 
-// Rows of 32 elements (64 bytes, four granules): 16 consecutive rows reading the same granule hit 16 distinct bank groups.
-__device__ __forceinline__ constexpr int swz_row32(int row) { return (row >> 2) & 3; }
-
-// ---- P and dS.  Stage: [K | V | Q | dO] tiles of 128 rows x 32; wavefront w copies tensor w.
-struct BwdWideScoresTile {
-    static constexpr int TILE_ELEMS = kWideTile * kWideStep;
-    static constexpr int STAGE_ELEMS = 4 * TILE_ELEMS;
-    static constexpr int LDS_BYTES = 2 * STAGE_ELEMS * 2;
+// Five 16 KiB tiles ("units") in LDS, used in pairs: phase j multiplies units 2 j and 2 j + 1.  At its start unit 2 j + 2 may
+// still be on its way; then units 2 j + 3 and 2 j + 4 are requested into the slots of the pair that phase j - 1 has read.
+// Four 1 KiB copies per wavefront and unit, so that the count of outstanding copies says which units have landed.
+struct WideRing {
+    static constexpr int UNITS = 5, UNIT_ELEMS = kWideTile * kWideStep;
+    static constexpr int LDS_BYTES = UNITS * UNIT_ELEMS * 2;
+    int a = 0;                                             // slot of the first unit of the current phase
+    __device__ __forceinline__ int slot(int i) const { return a + i < UNITS ? a + i : a + i - UNITS; }
+    __device__ __forceinline__ void next() { a = slot(2); }
+    // The pair of this phase has landed for every wavefront, and every wavefront has its fragments of the previous pair.
+    // One statement, so that no access to LDS moves across it.
+    __device__ __forceinline__ static void landed(bool last) {
+        if (last) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
 };
 
+// ---- P and dS.  Units of contraction step t: 4 t = K, + 1 = Q, + 2 = V, + 3 = dO (rows of 64 elements).
 static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const BwdWideParams p) {
-    using T = BwdWideScoresTile;
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int wk = wave & 1, wq = wave >> 1;          // this wavefront's 64 keys and 64 queries of the tile
 
+    // bands of eight key tiles, query tiles across: the 64 workgroups that an XCD runs at a time share 8 + 8 tiles of rows
     const int n_kt = p.sk_pad / kWideTile, n_qt = p.sq_pad / kWideTile;
     const int wg = xcd_remap(blockIdx.x, gridDim.x);
-    const int kt = wg % n_kt, qt = (wg / n_kt) % n_qt, slice = wg / (n_kt * n_qt);
+    const int slice = wg / (n_kt * n_qt), in_slice = wg % (n_kt * n_qt);
+    const int band = in_slice / (8 * n_qt), in_band = in_slice % (8 * n_qt), width = min(8, n_kt - 8 * band);
+    const int kt = 8 * band + in_band % width, qt = in_band / width;
     const int bh = p.bh0 + slice, b = bh / p.H, hh = bh % p.H;
     const int k0 = kt * kWideTile, q0 = qt * kWideTile;
     if (p.causal && k0 > q0 + kWideTile - 1) return;       // nothing of this tile is attended, and nothing reads it
     int klimit = p.Sk;
     if (p.kv_len) klimit = min(klimit, max(p.kv_len[b], 0));
 
-    // ---- copies: 8 of 16 rows x 64 bytes per wavefront and step; rows past the end re-read the last one
-    const bool is_q = wave >= 2;
-    const Strides st = wave == 0 ? p.ks : wave == 1 ? p.vs : wave == 2 ? p.qs : p.dos;
-    const uint16_t* base = (wave == 0 ? p.k : wave == 1 ? p.v : wave == 2 ? p.q : p.dout) + b * st.b + hh * st.h;
-    const int row0 = is_q ? q0 : k0, row_max = (is_q ? p.Sq : p.Sk) - 1;
-    base += (int64_t)min(row0, row_max) * st.n;
-    const int cp_row = lane >> 2, cp_gran = lane & 3;
-    uint32_t off[8];
-    int gran[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int row = 16 * i + cp_row;
-        gran[i] = cp_gran ^ swz_row32(row);
-        off[i] = 2u * (uint32_t)(min(row, max(row_max - row0, 0)) * (int)st.n + 8 * gran[i]);
-    }
-    const uint32_t lds0 = lds_addr(lds);
-    auto issue = [&](int s, int stage) {                   // contraction step s: elements [32 s, 32 s + 32)
-        const uint32_t dst = lds0 + 2u * (uint32_t)(stage * T::STAGE_ELEMS + wave * T::TILE_ELEMS);
-        const uint16_t* src = base + kWideStep * s;
-        if (kWideStep * (s + 1) <= p.d) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dma16u(src, off[i], dst + 1024u * i);
-        } else {                                           // granules past the head dim: filler, zeroed before use
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dma16u(src, kWideStep * s + 8 * gran[i] < p.d ? off[i] : off[i] - 16u * gran[i], dst + 1024u * i);
+    // ---- copies: 16 of 8 rows x 128 bytes per unit; rows past the end re-read the last one
+    const int k_last = p.Sk - 1, q_last = p.Sq - 1, k_rows = p.Sk - k0, q_rows = p.Sq - q0;
+    const uint16_t* kbase = p.k + b * p.ks.b + hh * p.ks.h + (int64_t)min(k0, k_last) * p.ks.n;
+    const uint16_t* vbase = p.v + b * p.vs.b + hh * p.vs.h + (int64_t)min(k0, k_last) * p.vs.n;
+    const uint16_t* qbase = p.q + b * p.qs.b + hh * p.qs.h + (int64_t)min(q0, q_last) * p.qs.n;
+    const uint16_t* gbase = p.dout + b * p.dos.b + hh * p.dos.h + (int64_t)min(q0, q_last) * p.dos.n;
+    // Copy i of a unit: rows 8 (4 wave + i) + lane / 8.  The swizzle of copies 0 and 2, and of 1 and 3, is the same, so two
+    // lane offsets per tensor do where all 128 rows exist.
+    const int row0 = 32 * wave + (lane >> 3), gran0 = (lane & 7) ^ swz<64>(row0), gran1 = (lane & 7) ^ swz<64>(row0 + 8);
+    static_assert(swz<64>(0) == swz<64>(16) && swz<64>(8) == swz<64>(24) && swz<64>(7) == swz<64>(23), "the swizzle repeats every 16 rows");
+    const uint32_t lds0 = lds_addr(lds) + 4096u * (uint32_t)wave;
+    auto issue = [&](const uint16_t* base, int64_t stride, int rows, int t, int slot) {      // elements [64 t, 64 t + 64)
+        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS);
+        const uint16_t* src = base + kWideStep * t;
+        if (kWideStep * (t + 1) <= p.d && rows >= kWideTile) {
+            const uint32_t at = 2u * (uint32_t)(row0 * (int)stride + 8 * gran0), at1 = at + 16u * (uint32_t)(stride + gran1 - gran0);
+            dma16u(src, at, dst);
+            dma16u(src, at1, dst + 1024u);
+            dma16u(src + 16 * stride, at, dst + 2048u);
+            dma16u(src + 16 * stride, at1, dst + 3072u);
+        } else {                                           // rows past the end re-read the last one; granules past the head dim:
+#pragma unroll                                             // filler, zeroed in the fragments
+            for (int i = 0; i < 4; ++i) {
+                const int g = i & 1 ? gran1 : gran0;
+                dma16u(src, 2u * (uint32_t)(min(row0 + 8 * i, max(rows - 1, 0)) * (int)stride + (kWideStep * t + 8 * g < p.d ? 8 * g : 0)), dst + 1024u * i);
+            }
         }
     };
-    int foff[2][2];                                        // [chunk of 16][block of 32 rows]: elements inside a tile, for the keys
-    int goff[2][2];                                        // ... for the queries
+    // fragment of 16 contraction elements c: row, granule 2 c + h; the chunk only flips bits 4 and 5 of the offset
+    int fk[2], fq[2];
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int rk = 64 * wk + 32 * u + n, rq = 64 * wq + 32 * u + n;
-            foff[c][u] = rk * kWideStep + 8 * ((2 * c + h) ^ swz_row32(rk));
-            goff[c][u] = rq * kWideStep + 8 * ((2 * c + h) ^ swz_row32(rq));
-        }
+    for (int u = 0; u < 2; ++u) {
+        const int rk = 64 * wk + 32 * u + n, rq = 64 * wq + 32 * u + n;
+        fk[u] = rk * kWideStep + 8 * (h ^ swz<64>(rk));
+        fq[u] = rq * kWideStep + 8 * (h ^ swz<64>(rq));
+    }
 
     f32x16 s[2][2], dp[2][2];                              // [key block][query block]
 #pragma unroll
@@ -134,60 +146,67 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[kb][qb][r] = dp[kb][qb][r] = 0.f;
 
-    const int n_steps = (p.d + kWideStep - 1) / kWideStep;
-    issue(0, 0);
-    wait_vm0();
-    __syncthreads();
-    for (int t = 0; t < n_steps; ++t) {
-        const int stage = t & 1;
-        if (t + 1 < n_steps) issue(t + 1, stage ^ 1);
-        uint16_t* tile = lds + stage * T::STAGE_ELEMS;
-        if (kWideStep * (t + 1) > p.d) {                   // the last step of a head dim that is no multiple of 32
-            const u32x4 z = {0u, 0u, 0u, 0u};
-            for (int idx = tid; idx < 2 * kWideTile * 4; idx += 256) {      // granules of the Q and dO tiles
-                const int which = 2 + (idx >> 9), row = (idx >> 2) & 127, g = idx & 3;
-                if (kWideStep * t + 8 * g >= p.d)
-                    *reinterpret_cast<u32x4*>(tile + which * T::TILE_ELEMS + row * kWideStep + 8 * (g ^ swz_row32(row))) = z;
-            }
-            // K and V as well: a filler must not meet a zero as an infinity
-            for (int idx = tid; idx < 2 * kWideTile * 4; idx += 256) {
-                const int which = idx >> 9, row = (idx >> 2) & 127, g = idx & 3;
-                if (kWideStep * t + 8 * g >= p.d)
-                    *reinterpret_cast<u32x4*>(tile + which * T::TILE_ELEMS + row * kWideStep + 8 * (g ^ swz_row32(row))) = z;
-            }
-            __syncthreads();
-        }
+    auto multiply = [&](auto tail_tag, f32x16 (&acc)[2][2], int slot_k, int slot_q, int rest) {
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        const uint16_t* kt_ = lds + slot_k * WideRing::UNIT_ELEMS;
+        const uint16_t* qt_ = lds + slot_q * WideRing::UNIT_ELEMS;
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            bf16x8 kf[2], vf[2], qf[2], gf[2];
+        for (int c = 0; c < kWideStep / 16; ++c) {
+            if (TAIL && 16 * c >= rest) break;
+            bf16x8 kf[2], qf[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                kf[u] = *reinterpret_cast<const bf16x8*>(tile + foff[c][u]);
-                vf[u] = *reinterpret_cast<const bf16x8*>(tile + T::TILE_ELEMS + foff[c][u]);
-                qf[u] = *reinterpret_cast<const bf16x8*>(tile + 2 * T::TILE_ELEMS + goff[c][u]);
-                gf[u] = *reinterpret_cast<const bf16x8*>(tile + 3 * T::TILE_ELEMS + goff[c][u]);
+                kf[u] = *reinterpret_cast<const bf16x8*>(kt_ + (fk[u] ^ (16 * c)));
+                qf[u] = *reinterpret_cast<const bf16x8*>(qt_ + (fq[u] ^ (16 * c)));
+                if (TAIL && 16 * c + 8 * h >= rest) kf[u] = qf[u] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});   // both: a filler must not meet a zero as an infinity
             }
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int qb = 0; qb < 2; ++qb) {
-                    s[kb][qb] = mfma32(kf[kb], qf[qb], s[kb][qb]);
-                    dp[kb][qb] = mfma32(vf[kb], gf[qb], dp[kb][qb]);
-                }
+                for (int qb = 0; qb < 2; ++qb) acc[kb][qb] = mfma32(kf[kb], qf[qb], acc[kb][qb]);
         }
-        wait_vm0();
-        __syncthreads();
-    }
+    };
+    using Yes = std::integral_constant<bool, true>;
+    using No = std::integral_constant<bool, false>;
 
-    // ---- P and dS: a lane owns one query per block and four consecutive keys per register group
+    const int n_steps = (p.d + kWideStep - 1) / kWideStep;
+    WideRing ring;
+    issue(kbase, p.ks.n, k_rows, 0, 0);
+    issue(qbase, p.qs.n, q_rows, 0, 1);
+    issue(vbase, p.vs.n, k_rows, 0, 2);
+    for (int t = 0; t < n_steps; ++t) {
+        const bool more = t + 1 < n_steps;
+        const int rest = p.d - kWideStep * t;
+        WideRing::landed(false);                           // K and Q
+        issue(gbase, p.dos.n, q_rows, t, ring.slot(3));
+        if (more) issue(kbase, p.ks.n, k_rows, t + 1, ring.slot(4));
+        if (rest >= kWideStep) multiply(No{}, s, ring.slot(0), ring.slot(1), rest);
+        else multiply(Yes{}, s, ring.slot(0), ring.slot(1), rest);
+        ring.next();
+        WideRing::landed(!more);                           // V and dO
+        if (more) {
+            issue(qbase, p.qs.n, q_rows, t + 1, ring.slot(3));
+            issue(vbase, p.vs.n, k_rows, t + 1, ring.slot(4));
+        }
+        if (rest >= kWideStep) multiply(No{}, dp, ring.slot(0), ring.slot(1), rest);
+        else multiply(Yes{}, dp, ring.slot(0), ring.slot(1), rest);
+        ring.next();
+    }
+    __syncthreads();                                       // the tiles are no longer needed: P and dS take their place
+
+    // ---- P and dS: a lane owns one query per block and four consecutive keys per register group.  Through LDS (rows of 128
+    // keys, granules swizzled by the row), so that a store instruction writes whole cache lines: straight from the
+    // accumulators it would touch 32 of them, 16 bytes each.
     const float c_log2 = p.scale * kLog2e;
+    uint16_t* p_tile = lds;
+    uint16_t* ds_tile = lds + kWideTile * kWideTile;
+    static_assert(2 * kWideTile * kWideTile * 2 <= WideRing::LDS_BYTES, "P and dS of a tile fit where the ring was");
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-        const int qi = q0 + 64 * wq + 32 * qb + n;
+        const int rq = 64 * wq + 32 * qb + n, qi = q0 + rq;
         const bool ok = qi < p.Sq;
         const float nd = ok ? p.ndelta[(int64_t)bh * p.Sq + qi] : 0.f, l2 = ok ? p.lse2[(int64_t)bh * p.Sq + qi] : INFINITY;
         const int lim = ok ? (p.causal ? min(klimit, qi + 1) : klimit) : 0;     // keys below it are attended
-        const int64_t row = ((int64_t)slice * p.sq_pad + qi) * p.sk_pad;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -200,25 +219,30 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
                     pr[e] = key + e < lim ? x : 0.f;
                     dsv[e] = key + e < lim ? x * (dp[kb][qb][4 * g + e] + nd) : 0.f;
                 }
-                *reinterpret_cast<u32x2*>(p.probs + row + key) = u32x2{pack_bf16(pr[0], pr[1]), pack_bf16(pr[2], pr[3])};
-                *reinterpret_cast<u32x2*>(p.ds + row + key) = u32x2{pack_bf16(dsv[0], dsv[1]), pack_bf16(dsv[2], dsv[3])};
+                const int at = rq * kWideTile + 8 * ((8 * wk + 4 * kb + g) ^ (rq & 15)) + 4 * h;
+                *reinterpret_cast<u32x2*>(p_tile + at) = u32x2{pack_bf16(pr[0], pr[1]), pack_bf16(pr[2], pr[3])};
+                *reinterpret_cast<u32x2*>(ds_tile + at) = u32x2{pack_bf16(dsv[0], dsv[1]), pack_bf16(dsv[2], dsv[3])};
             }
+    }
+    __syncthreads();
+    const int64_t out0 = ((int64_t)slice * p.sq_pad + q0) * p.sk_pad + k0;
+#pragma unroll
+    for (int i = 0; i < kWideTile / 16; ++i) {
+        const int row = 16 * i + (tid >> 4), g = tid & 15;
+        const int at = row * kWideTile + 8 * (g ^ (row & 15));
+        const int64_t to = out0 + (int64_t)row * p.sk_pad + 8 * g;
+        *reinterpret_cast<u32x4*>(p.probs + to) = *reinterpret_cast<const u32x4*>(p_tile + at);
+        *reinterpret_cast<u32x4*>(p.ds + to) = *reinterpret_cast<const u32x4*>(ds_tile + at);
     }
 }
 
 // ---- The three products.  Output tile: 128 columns of the head dim x 128 rows (keys of dV and dK, queries of dQ), formed
-// transposed so that a lane owns one row.  Stage: [X | W]: X = 32 rows (contraction) x 128 columns of dO, Q or K, read
-// transposed; W = 32 x 128 of P or dS, read transposed (dV, dK), or 128 rows x 32 of dS, read along its rows (dQ).
-struct BwdWideProductsTile {
-    static constexpr int TILE_ELEMS = kWideTile * kWideStep;
-    static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;
-    static constexpr int LDS_BYTES = 2 * STAGE_ELEMS * 2;
-};
-
+// transposed so that a lane owns one row.  Units of contraction step t: 2 t = X, 64 rows (contraction) x 128 columns of dO, Q
+// or K, read transposed; 2 t + 1 = W, 64 x 128 of P or dS, read transposed (dV, dK), or 128 rows x 64 of dS, read along its
+// rows (dQ).
 template <bool DQ>
 __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const uint16_t* x, const Strides& xs, const uint16_t* w, uint16_t* out,
                                                  const Strides& outs, float mul, int slice, int mt, int dt) {
-    using T = BwdWideProductsTile;
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -235,38 +259,39 @@ __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const u
     const uint16_t* xbase = x + b * xs.b + hh * xs.h + d0;
     const uint16_t* wbase = w + (int64_t)slice * p.sq_pad * p.sk_pad + (DQ ? (int64_t)m0 * p.sk_pad : m0);
 
-    // ---- copies: X: 8 of 4 rows x 256 bytes; W the same, or (DQ) 8 of 16 rows x 64 bytes; four of the sixteen per wavefront
-    uint32_t xoff[2], woff[2];
-    int xrow[2];
+    // ---- copies: X: 16 of 4 rows x 256 bytes; W the same, or (DQ) 16 of 8 rows x 128 bytes
+    uint32_t xoff[4], woff[4];
+    int xrow[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int row = (2 * wave + i) * 4 + (lane >> 4), g = (lane & 15) ^ swz<128>(row);
+    for (int i = 0; i < 4; ++i) {
+        const int row = (4 * wave + i) * 4 + (lane >> 4), g = (lane & 15) ^ swz<128>(row);
         xrow[i] = row;
         xoff[i] = 2u * (uint32_t)(d0 + 8 * g < p.d ? 8 * g : 0);        // columns past the head dim: filler, not stored
         if (DQ) {
-            const int wr = (2 * wave + i) * 16 + (lane >> 2), wg = (lane & 3) ^ swz_row32(wr);
+            const int wr = (4 * wave + i) * 8 + (lane >> 3), wg = (lane & 7) ^ swz<64>(wr);
             woff[i] = 2u * (uint32_t)(wr * p.sk_pad + 8 * wg);
         } else {
             woff[i] = 2u * (uint32_t)(row * p.sk_pad + 8 * g);
         }
     }
-    const uint32_t lds0 = lds_addr(lds);
-    auto issue = [&](int c0, int stage) {              // contraction rows [c0, c0 + 32); past the end the last row, against zeros of W
-        const uint32_t dst = lds0 + 2u * (uint32_t)(stage * T::STAGE_ELEMS) + 2048u * (uint32_t)wave;
-        const int first = min(c0, n_con - 1);
+    const uint32_t lds0 = lds_addr(lds) + 4096u * (uint32_t)wave;
+    auto issue_x = [&](int c0, int slot) {             // contraction rows [c0, c0 + 64); past the end the last row, against zeros of W
+        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS);
+        const int first = min(c0, n_con - 1), over = n_con - 1 - first;
         const uint16_t* xsrc = xbase + (int64_t)first * xs.n;
-        const uint16_t* wsrc = wbase + (DQ ? (int64_t)c0 : (int64_t)c0 * p.sk_pad);
-        const int over = n_con - 1 - first;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            dma16u(xsrc, xoff[i] + 2u * (uint32_t)(min(xrow[i], over) * (int)xs.n), dst + 1024u * i);
-            dma16u(wsrc, woff[i], dst + 2u * T::TILE_ELEMS + 1024u * i);
-        }
+        for (int i = 0; i < 4; ++i) dma16u(xsrc, xoff[i] + 2u * (uint32_t)(min(xrow[i], over) * (int)xs.n), dst + 1024u * i);
     };
-    // fragment addresses: transposing reads of a 32 x 128 tile, 16 contraction rows per chunk
+    auto issue_w = [&](int c0, int slot) {
+        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS);
+        const uint16_t* wsrc = wbase + (DQ ? (int64_t)c0 : (int64_t)c0 * p.sk_pad);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dma16u(wsrc, woff[i], dst + 1024u * i);
+    };
+    // fragment addresses: transposing reads of a 64 x 128 tile, 16 contraction rows per chunk
     const int tr_r = lane & 15, tr_g16 = (lane >> 4) & 1;
     // (DQ: eight consecutive contraction rows per half wave, as the row reads of dS have them; else 4 h and 8 further on)
-    int xo[2][2], wo[2][2];                            // [half of the chunk][block of 32]; DQ: wo[chunk][block]
+    int xo[2][2], wo[2][2];                            // [half of the chunk][block of 32]; DQ: wo[0][block], the chunk flips bits 4 and 5
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         const int row = DQ ? 8 * h + (tr_r >> 2) + 4 * half : 4 * h + (tr_r >> 2) + 8 * half;
@@ -275,7 +300,7 @@ __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const u
             xo[half][u] = row * 128 + 8 * ((4 * (2 * wd + u) + 2 * tr_g16 + ((tr_r & 3) >> 1)) ^ swz<128>(row)) + 4 * (tr_r & 1);
             if (DQ) {
                 const int wr = 64 * wm + 32 * u + n;
-                wo[half][u] = wr * kWideStep + 8 * ((2 * half + h) ^ swz_row32(wr));
+                wo[half][u] = wr * kWideStep + 8 * (h ^ swz<64>(wr));
             } else {
                 wo[half][u] = row * 128 + 8 * ((4 * (2 * wm + u) + 2 * tr_g16 + ((tr_r & 3) >> 1)) ^ swz<128>(row)) + 4 * (tr_r & 1);
             }
@@ -294,35 +319,32 @@ __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const u
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[u][m][r] = 0.f;
 
+    WideRing ring;
     if (con_lo < con_hi) {
-        issue(con_lo, 0);
-        wait_vm0();
-        __syncthreads();
+        issue_x(con_lo, 0);
+        issue_w(con_lo, 1);
+        if (con_lo + kWideStep < con_hi) issue_x(con_lo + kWideStep, 2);
     }
-    int stage = 0;
-    for (int c0 = con_lo; c0 < con_hi; c0 += kWideStep, stage ^= 1) {
-        if (c0 + kWideStep < con_hi) issue(c0 + kWideStep, stage ^ 1);
-        const uint16_t* xt = lds + stage * T::STAGE_ELEMS;
-        const uint16_t* wt = xt + T::TILE_ELEMS;
+    for (int c0 = con_lo; c0 < con_hi; c0 += kWideStep, ring.next()) {
+        WideRing::landed(c0 + kWideStep >= con_hi);
+        if (c0 + kWideStep < con_hi) issue_w(c0 + kWideStep, ring.slot(3));
+        if (c0 + 2 * kWideStep < con_hi) issue_x(c0 + 2 * kWideStep, ring.slot(4));
+        const uint16_t* xt = lds + ring.slot(0) * WideRing::UNIT_ELEMS;
+        const uint16_t* wt = lds + ring.slot(1) * WideRing::UNIT_ELEMS;
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int c = 0; c < kWideStep / 16; ++c) {
             bf16x8 xf[2], wf[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 xf[u] = tr_frag(xt + 16 * c * 128, xo[0][u], xo[1][u]);
-                if constexpr (DQ) {
-                    wf[u] = *reinterpret_cast<const bf16x8*>(wt + wo[c][u]);
-                } else {
-                    wf[u] = tr_frag(wt + 16 * c * 128, wo[0][u], wo[1][u]);
-                }
+                if constexpr (DQ) wf[u] = *reinterpret_cast<const bf16x8*>(wt + (wo[0][u] ^ (16 * c)));
+                else wf[u] = tr_frag(wt + 16 * c * 128, wo[0][u], wo[1][u]);
             }
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int m = 0; m < 2; ++m) acc[u][m] = mfma32(xf[u], wf[m], acc[u][m]);
         }
-        wait_vm0();
-        __syncthreads();
     }
 #pragma unroll
     for (int m = 0; m < 2; ++m) {

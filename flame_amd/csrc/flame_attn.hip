@@ -1929,8 +1929,9 @@ size_t wide_workspace_bytes(int B, int H, int N_q, int N_kv) {
 }
 
 int launch_bwd_wide(BwdWideParams p, void* workspace, size_t bytes, hipStream_t s) {
-    static std::atomic<bool> lds_set{false};
-    if (const int rc = set_lds(reinterpret_cast<const void*>(bwd_wide_scores_kernel), BwdWideScoresTile::LDS_BYTES, lds_set)) return rc;
+    static std::atomic<bool> scores_set{false}, products_set{false};
+    if (const int rc = set_lds(reinterpret_cast<const void*>(bwd_wide_scores_kernel), WideRing::LDS_BYTES, scores_set)) return rc;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(bwd_wide_products_kernel), WideRing::LDS_BYTES, products_set)) return rc;
     const int bh = p.B * p.H;
     char* ws = static_cast<char*>(workspace);
     p.ndelta = reinterpret_cast<float*>(ws);
@@ -1948,9 +1949,9 @@ int launch_bwd_wide(BwdWideParams p, void* workspace, size_t bytes, hipStream_t 
     hipLaunchKernelGGL(bwd_wide_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, p);
     for (p.bh0 = 0; p.bh0 < bh; p.bh0 += group) {
         p.n_slices = std::min(group, bh - p.bh0);
-        hipLaunchKernelGGL(bwd_wide_scores_kernel, dim3((unsigned)(p.n_slices * n_kt * n_qt)), dim3(256), BwdWideScoresTile::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(bwd_wide_scores_kernel, dim3((unsigned)(p.n_slices * n_kt * n_qt)), dim3(256), WideRing::LDS_BYTES, s, p);
         hipLaunchKernelGGL(bwd_wide_products_kernel, dim3((unsigned)(p.n_slices * (2 * n_kt + n_qt) * n_dt)), dim3(256),
-                           BwdWideProductsTile::LDS_BYTES, s, p);
+                           WideRing::LDS_BYTES, s, p);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;

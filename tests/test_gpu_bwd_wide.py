@@ -1,5 +1,5 @@
 """The backward for head dims above 128 on kernels of its own, against the CPU oracle: head dims that end inside a contraction
-step (136, 264), inside a 128-column output tile (192) and on one (512), one row, one past the 128-row tiles, causal with more
+step (136, 152, 168, 264), inside a 128-column output tile (192) and on one (512), more key tiles than a band of eight, one row, one past the 128-row tiles, causal with more
 keys than queries and the reverse, key lengths (one of them 0), strided views, and a workspace that holds fewer (batch, head)
 slices than there are."""
 import numpy as np
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,H,Sq,Sk,D,causal,lens,small_ws,bnhd", [
     (1, 2, 1, 1, 136, False, None, False, False), (1, 2, 100, 77, 264, False, None, False, True), (1, 1, 129, 257, 512, False, None, False, False),
     (2, 2, 128, 128, 192, True, None, True, False), (1, 1, 300, 150, 136, True, None, False, True), (1, 2, 140, 290, 256, True, None, True, False),
-    (3, 1, 65, 200, 264, False, (200, 0, 129), True, False)])
+    (3, 1, 65, 200, 264, False, (200, 0, 129), True, False),
+    (1, 1, 200, 1300, 152, False, None, False, False), (1, 1, 1290, 260, 168, True, None, False, True)])
 def test_against_the_oracle(oracle, B, H, Sq, Sk, D, causal, lens, small_ws, bnhd):
     from flame_amd import capi
     print(f"[bwd wide] {B=} {H=} {Sq=} {Sk=} {D=} {causal=} {lens=} {small_ws=} {bnhd=}", flush=True)
