@@ -852,6 +852,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
     }
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len && p.dq_parts == 1) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
+    if ((KEYS || p.m.kv_len) && p.dq_parts == 1) bh = longest_batches_first<KEYS>(bh, p.B, p.H, p.Sk, p.m);
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 32;
