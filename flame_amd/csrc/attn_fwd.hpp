@@ -62,8 +62,13 @@ typedef uint16_t u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 
 // DROP (DropMode): the probabilities that multiply V are dropped element by element (drop_factor) and O is rescaled; the
 // row sums, and with them the log-sum-exp, stay those of the undropped softmax.
-template <int D, int EXCL, int NW, int DROP = kDropNone>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const FwdParams p) {
+// KG = 2: two groups of NW wavefronts share the workgroup's queries, each walks one half of the key tiles in LDS stages of its
+// own, and the second hands its running state to the first through LDS.  For grids that give a compute unit one workgroup at
+// most: its second wavefront per SIMD, which otherwise a second workgroup would be, and half the walk.  K and V are still
+// read once per workgroup.
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void fwd_kernel(const FwdParams p) {
+    static_assert(KG == 1 || (KG == 2 && EXCL == kExNone), "key groups: nothing excluded but by causal flag and key lengths");
     using T = FwdTile<D>;
     constexpr int BN = T::BN, RS = T::RS;
     constexpr int BM = 32 * NW;  // query rows per workgroup
@@ -79,12 +84,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     static_assert((2 * DC) % PD == 0 && (4 * DB) % PD == 0, "read-ahead depth must divide the fragment counts");
     static_assert(2 * DC == 16 || 2 * DC == 8, "softmax slicing assumes 16 or 8 logit MFMAs per tile");
 
-    extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
+    extern __shared__ __attribute__((aligned(1024))) uint16_t lds_all[];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KG == 1 ? wave_all : wave_all % NW, group = KG == 1 ? 0 : wave_all / NW;
     const int n = lane & 31, h = lane >> 5;
+    uint16_t* lds = lds_all + (KG == 1 ? 0 : group * (T::LDS_BYTES / 2));
 
     const int n_qt = (p.Sq + BM - 1) / BM;
     const int wg = p.m.kv_len || EXCL == kExKeys ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
@@ -105,6 +112,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     int kend = klimit;
     if (p.m.causal) kend = min(kend, q0 + BM);
     int n_tiles = (kend + BN - 1) / BN;
+    // The tiles of this wavefront's group become tiles 0 .. n_tiles - 1 of a walk that starts at key `key0`.
+    const int n_first = (n_tiles + 1) / 2;            // of group 0
+    const int key0 = KG == 1 ? 0 : group * n_first * BN;
+    if constexpr (KG == 2) {
+        n_tiles = group ? n_tiles - n_first : n_first;
+        klimit -= key0;
+        kbase += key0 * p.ks.n;
+        vbase += key0 * p.vs.n;
+    }
     const uint8_t* mbase = (EXCL != kExNone && p.m.mask) ? mask_head_base(p.m, b, hh) : nullptr;
     const char* bbase = (EXCL == kExGeneral && p.m.bias)
                             ? static_cast<const char*>(p.m.bias) + (b * p.m.bb + hh * p.m.bh) * (p.m.bias_f32 ? 4 : 2)
@@ -222,7 +238,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     constexpr int MPS = 32 / NP;   // logits handled per maximum-scan slice
 
     // DROP: flat index (mod 2^32) of this lane's first element of the row in the [B*H, Sq, Sk] probability tensor
-    const uint32_t drop_row = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qi) * (uint32_t)p.Sk + 4 * h;
+    const uint32_t drop_row = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qi) * (uint32_t)p.Sk + (uint32_t)key0 + 4 * h;
     (void)drop_row;
     // Exclusions of a tile.  The ragged tail / key length and the causal diagonal are one comparison per element with a
     // per-lane limit (excl_elem, threaded into the maximum scan); a keep-mask row is fetched when the step begins; the
@@ -236,7 +252,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             keep_bits[0] = (uint32_t)w >> (4 * h);
             keep_bits[1] = (uint32_t)(w >> 32) >> (4 * h);
         }
-        const int limit = (p.m.causal ? min(klimit, qi + 1) : klimit) - t * BN;
+        const int limit = (p.m.causal ? min(klimit, qi + 1 - key0) : klimit) - t * BN;
         lim = limit - 4 * h;
         if constexpr (EXCL == kExRows16) {
             // folded into the mask bytes where they cut the tile: the per-element test is then the mask byte alone
@@ -362,7 +378,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
                 else rsum0 += v;
                 const uint32_t off = 32 * kb + 8 * (r >> 2) + (r & 3);       // of the element, from drop_tile
                 if constexpr (DROP == kDropTiled) {
-                    cur[kb][r] = v * drop_factor_at(p.m, (uint32_t)bh, (uint32_t)qi, (uint32_t)(t * BN + 4 * h) + off, (uint32_t)p.Sq, (uint32_t)p.Sk);
+                    cur[kb][r] = v * drop_factor_at(p.m, (uint32_t)bh, (uint32_t)qi, (uint32_t)(key0 + t * BN + 4 * h) + off, (uint32_t)p.Sq, (uint32_t)p.Sk);
                 } else if constexpr (DROP != kDropNone) {
                     const uint32_t w = DROP == kDropRows64 ? drop_word ^ xorshift32(off) : xorshift32(p.m.drop_seed ^ (drop_tile + off));
                     cur[kb][r] = w >= p.m.drop_thr32 ? v : 0.f;
@@ -455,8 +471,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
     // Tiles below t_clean need no exclusions for any query of the workgroup; the rest (ragged tail, causal
     // diagonal, or everything under an explicit mask) carry per-element exclusions.
     int t_clean = KEYS ? kt.n_whole : (EXCL == kExNone || BIAS) ? klimit / BN : 0;
-    if (p.m.causal) t_clean = min(t_clean, (q0 + 1) / BN);
-    t_clean = min(t_clean, n_tiles);
+    if (p.m.causal) t_clean = min(t_clean, (q0 + 1 - key0) / BN);
+    t_clean = max(min(t_clean, n_tiles), 0);
 
     f32x16 sa[2], sb[2];
     if (n_tiles > 0) {
@@ -517,6 +533,37 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_kernel(const Fwd
             step(No{}, Last{}, sb, sa, t + 1);
         } else {
             step(No{}, Last{}, sa, sb, t);
+        }
+    }
+
+    // ---- the second group's state joins the first's
+    if constexpr (KG == 2) {
+        // a walk of n tiles passes n + 1 barriers; the second group's may be one tile shorter, or empty
+        const int mine = n_tiles > 0 ? n_tiles + 1 : 0, most = n_first > 0 ? n_first + 1 : 0;
+        for (int i = mine; i < most; ++i) __syncthreads();
+        __syncthreads();                               // nobody reads a tile any more
+        static_assert(NW * (4 * DB + 1) * 64 * 16 <= KG * T::LDS_BYTES, "the state of a group fits where the tiles were");
+        f32x4* slot = reinterpret_cast<f32x4*>(lds_all) + wave * (4 * DB + 1) * 64 + lane;
+        if (group == 1) {
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) {
+                const f32x16& a = oacc[i >> 2];
+                slot[64 * i] = f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]};
+            }
+            slot[64 * 4 * DB] = f32x4{m_run, l_run, 0.f, 0.f};
+        }
+        __syncthreads();
+        if (group == 1) return;
+        const f32x4 other = slot[64 * 4 * DB];
+        const float m_new = fmaxf(m_run, other[0]), m_to = (m_new == -INFINITY) ? 0.f : m_new;
+        const float w0 = exp2_fast((m_run - m_to) * c_log2), w1 = exp2_fast((other[0] - m_to) * c_log2);
+        l_run = l_run * w0 + other[1] * w1;
+        m_run = m_new;
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            const f32x4 v = slot[64 * i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oacc[i >> 2][4 * (i & 3) + e] = fmaf(oacc[i >> 2][4 * (i & 3) + e], w0, v[e] * w1);
         }
     }
 

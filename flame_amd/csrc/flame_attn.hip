@@ -138,21 +138,29 @@ void launch_fwd_merge(const FwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL(fwd_merge_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, p);
 }
 
+// Two groups of wavefronts per workgroup that share its keys (KG = 2 of the 128-query forward, dQ and Sage kernels): where every
+// compute unit gets one workgroup at most, so that a second wavefront per SIMD costs nothing, and the walk is long enough to
+// pay for joining the halves (about 1 us).  Forward, one group -> two: 192 workgroups, 256 keys, D = 128 10.7 -> 12.0 us, 577 keys
+// unchanged, 1024 keys 22.1 -> 21.5 us; 128 workgroups, 4096 keys 62.9 -> 52.8 us; 256 workgroups, causal, 2048 keys 36.5 -> 33.5 us.
+bool rule_key_groups(int64_t wgs, int Sk) { return wgs <= device_cu_count() && Sk >= 1024; }
+
 // wg_count workgroups from p.wg_base on (0: all of the problem's)
-template <int D, int EXCL, int NW, int DROP = kDropNone>
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
 int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     using T = FwdTile<D>;
     constexpr int BM = 32 * NW;
-    static std::atomic<bool> lds_set{false};
-    auto kern = fwd_kernel<D, EXCL, NW, DROP>;
-    constexpr bool KEYS = EXCL == kExKeys;
-    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
-    const int lds = T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
     const int64_t grid = wg_count ? wg_count : (int64_t)((p.Sq + BM - 1) / BM) * p.B * p.H;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    if constexpr (EXCL == kExNone && NW == 4 && KG == 1)
+        if (rule_key_groups(grid, p.Sk)) return launch_fwd<D, EXCL, NW, DROP, 2>(p, s, wg_count);
+    static std::atomic<bool> lds_set{false};
+    auto kern = fwd_kernel<D, EXCL, NW, DROP, KG>;
+    constexpr bool KEYS = EXCL == kExKeys;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), KG * T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
+    const int lds = KG * T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), lds, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW * KG), lds, s, p);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
