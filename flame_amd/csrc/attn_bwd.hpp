@@ -825,8 +825,11 @@ struct BwdDqTile {
 // NW wavefronts of 32 queries each per workgroup, two per SIMD (the library instantiates NW = 4; problems
 // that fill 256-query workgroups go to bwd_dq_wide_kernel below).
 // EXCL: see there.  Only the general form compiles per-element mask loads in; the others fit two workgroups per unit.
-template <int D, int EXCL, int NW, int DROP = kDropNone>
-__global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
+// KG = 2: two groups of NW wavefronts share the workgroup's queries, each walks one half of the key tiles in LDS stages of its
+// own, and the second adds its dQ to the first's through LDS: for grids that give a compute unit one workgroup at most.
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
+    static_assert(KG == 1 || (KG == 2 && EXCL == kExNone), "key groups: nothing excluded but by causal flag and key lengths");
     constexpr bool HASMASK = EXCL == kExRows16 || EXCL == kExGeneral, VECMASK = EXCL == kExRows16, KEYS = EXCL == kExKeys;
     using T = BwdDqTile<D>;
     constexpr int BM = 32 * NW, BN = T::BN, RS = T::RS;
@@ -834,11 +837,13 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
     constexpr int DB = D / 32;
     constexpr int GPR = D / 8;
 
-    extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
+    extern __shared__ __attribute__((aligned(1024))) uint16_t lds_all[];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KG == 1 ? wave_all : wave_all % NW, group = KG == 1 ? 0 : wave_all / NW;
+    uint16_t* lds = lds_all + (KG == 1 ? 0 : group * (T::LDS_BYTES / 2));
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
@@ -873,6 +878,11 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
         const int per = (n_tiles + p.dq_parts - 1) / p.dq_parts;
         t_lo = part * per;
         n_tiles = min(n_tiles, t_lo + per) - t_lo;      // not positive: nothing to do
+    }
+    const int n_first = (n_tiles + 1) / 2;              // KG: of group 0 (dq_parts is 1)
+    if constexpr (KG == 2) {
+        t_lo = group * n_first;
+        n_tiles = group ? n_tiles - n_first : n_first;
     }
     // step t of the walk takes tile tile_of(t)
     KeyTiles kt;
@@ -920,7 +930,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
             const float l = p.lse[(int64_t)bh * p.Sq + qrow];
             lse2 = (l == -INFINITY) ? INFINITY : l * kLog2e;
             delta = part;
-            if (h == 0) {
+            if (h == 0 && group == 0) {
                 p.ndelta[(int64_t)bh * p.Sq + qrow] = -delta;
                 p.lse2[(int64_t)bh * p.Sq + qrow] = lse2;
             }
@@ -1160,6 +1170,27 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) v
         }
         for (; t < n_full; ++t) tile_step(std::false_type{}, I2{}, IM{}, t);
         for (; t < n_tiles; ++t) tile_step(std::true_type{}, I2{}, IM{}, t);
+    }
+
+    if constexpr (KG == 2) {
+        for (int i = n_tiles; i < n_first; ++i) __syncthreads();        // one barrier per tile: the second group's walk may be one shorter
+        static_assert(NW * 4 * DB * 64 * 16 <= T::LDS_BYTES, "the sums of a group fit in its own stages");
+        f32x4* slot = reinterpret_cast<f32x4*>(lds_all + T::LDS_BYTES / 2) + wave * 4 * DB * 64 + lane;
+        if (group == 1) {
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) {
+                const f32x16& a = dqacc[i >> 2];
+                slot[64 * i] = f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]};
+            }
+        }
+        __syncthreads();
+        if (group == 1) return;
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            const f32x4 v = slot[64 * i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dqacc[i >> 2][4 * (i & 3) + e] += v[e];
+        }
     }
 
     // ---- epilogue: fp32 partial sums for bwd_dq_merge_kernel, in accumulator order: [db][group of four][thread] ...

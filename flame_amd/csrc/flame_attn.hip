@@ -142,7 +142,10 @@ void launch_fwd_merge(const FwdParams& p, hipStream_t s) {
 // compute unit gets one workgroup at most, so that a second wavefront per SIMD costs nothing, and the walk is long enough to
 // pay for joining the halves (about 1 us).  Forward, one group -> two: 192 workgroups, 256 keys, D = 128 10.7 -> 12.0 us, 577 keys
 // unchanged, 1024 keys 22.1 -> 21.5 us; 128 workgroups, 4096 keys 62.9 -> 52.8 us; 256 workgroups, causal, 2048 keys 36.5 -> 33.5 us.
-bool rule_key_groups(int64_t wgs, int Sk) { return wgs <= device_cu_count() && Sk >= 1024; }
+bool rule_key_groups(int64_t wgs, int Sk, int least_keys = 1024) { return wgs <= device_cu_count() && Sk >= least_keys; }
+// dQ, whose joining weighs more: B=1 H=16 S=2048 causal, backward, D = 64 62.8 -> 60.1 us, D = 128 96.9 -> 95.8 us; unchanged or
+// up to 2 % slower with 1024 keys.
+constexpr int kDqGroupKeys = 2048;
 
 // wg_count workgroups from p.wg_base on (0: all of the problem's)
 template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
@@ -245,6 +248,9 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     static bool attr_done = false;
     auto kern = bwd_dkdv_kernel<D, HASMASK, TIMING>;
     auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4>;
+    // the same with two key groups per workgroup (the rule never asks for it with an explicit mask)
+    constexpr int KG = HASMASK ? 1 : 2;
+    auto kern_dqg = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, kDropNone, KG>;
     auto kern_dqk = bwd_dq_kernel<D, kExKeys, 4>;                    // keep-mask of keys
     auto kern_dqv = bwd_dq_kernel<D, kExRows16, 4>;                  // keep-mask with vector-loadable rows over whole tiles
     auto kern_kvv = bwd_dkdv_kernel<D, true, false, true>;           // ... whose tiles travel through LDS
@@ -256,6 +262,9 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         if (e != hipSuccess) return (int)e;
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dq),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
+        if (e != hipSuccess) return (int)e;
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqg),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, KG * TQ::LDS_BYTES);
         if (e != hipSuccess) return (int)e;
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqw),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, TW::LDS_BYTES);
@@ -351,7 +360,8 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
             if (cut) {
                 BwdParams pt = p;
                 pt.dq_base = (int)(2 * (grid_dq - rest));
-                hipLaunchKernelGGL(kern_dq, dim3((unsigned)(2 * rest)), dim3(256), TQ::LDS_BYTES, s, pt);
+                if (!HASMASK && rule_key_groups(2 * rest, p.Sk, kDqGroupKeys)) hipLaunchKernelGGL(kern_dqg, dim3((unsigned)(2 * rest)), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pt);
+                else hipLaunchKernelGGL(kern_dq, dim3((unsigned)(2 * rest)), dim3(256), TQ::LDS_BYTES, s, pt);
             }
         }
         else if (!HASMASK && p.key_mask)
@@ -367,7 +377,10 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
                 while (parts > 1 && (size_t)(grid_dq * parts) * (TQ::BM * D * sizeof(float)) > p.split_ws_bytes) --parts;
                 if (parts > 1 && tiles - (tiles + parts - 1) / parts >= 12) pq.dq_parts = (int)parts;
             }
-            hipLaunchKernelGGL(kern_dq, dim3((unsigned)(grid_dq * pq.dq_parts)), dim3(256), TQ::LDS_BYTES, s, pq);
+            if (!HASMASK && pq.dq_parts == 1 && rule_key_groups(grid_dq, p.Sk, kDqGroupKeys))
+                hipLaunchKernelGGL(kern_dqg, dim3((unsigned)grid_dq), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pq);
+            else
+                hipLaunchKernelGGL(kern_dq, dim3((unsigned)(grid_dq * pq.dq_parts)), dim3(256), TQ::LDS_BYTES, s, pq);
             if (pq.dq_parts > 1) hipLaunchKernelGGL(bwd_dq_merge_kernel<D>, dim3((unsigned)(grid_dq * (D / 32))), dim3(256), 0, s, pq);
         }
     }
@@ -519,17 +532,21 @@ template <int D, bool HASMASK, int DROP>
 int launch_bwd_drop(const BwdParams& p, hipStream_t s) {
     using T = BwdTile<D>;
     using TQ = BwdDqTile<D>;
-    static std::atomic<bool> lds_set{false}, lds_set_dq{false};
+    static std::atomic<bool> lds_set{false}, lds_set_dq{false}, lds_set_dqg{false};
     auto kern = bwd_dkdv_kernel<D, HASMASK, false, false, DROP>;
     auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, DROP>;
+    constexpr int KG = HASMASK ? 1 : 2;
+    auto kern_dqg = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, DROP, KG>;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES_DROP, lds_set)) return rc;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern_dq), TQ::LDS_BYTES, lds_set_dq)) return rc;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_dqg), KG * TQ::LDS_BYTES, lds_set_dqg)) return rc;
     const int64_t grid = (int64_t)((p.Sk + T::BN - 1) / T::BN) * p.B * p.H;
     const int64_t grid_dq = (int64_t)((p.Sq + TQ::BM - 1) / TQ::BM) * p.B * p.H;
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);        // first: it leaves -delta and the rescaled LSE rows
-        hipLaunchKernelGGL(kern_dq, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
+        if (!HASMASK && p.dq_parts == 1 && rule_key_groups(grid_dq, p.Sk, kDqGroupKeys)) hipLaunchKernelGGL(kern_dqg, dim3((unsigned)grid_dq), dim3(256 * KG), KG * TQ::LDS_BYTES, s, p);
+        else hipLaunchKernelGGL(kern_dq, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
     }
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DKDV, s);

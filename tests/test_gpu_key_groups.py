@@ -1,5 +1,5 @@
 """The 128-query forward and dQ kernels whose workgroups hold two groups of wavefronts with half of the key tiles each (one
-workgroup per compute unit at most, 1024 keys or more): odd and even numbers of tiles, a ragged last tile, the second group
+workgroup per compute unit at most, 1024 keys or more, for dQ 2048): odd and even numbers of tiles, a ragged last tile, the second group
 empty or without an attended key for some queries (causal, key lengths, an empty sequence), dropout by rows and by elements,
 the largest grid that takes them and the next one, against the CPU oracle."""
 import numpy as np
@@ -13,10 +13,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,H,Sq,Sk,D,causal,lens,p", [
-    (1, 130, 40, 1024, 64, False, None, 0.0), (1, 130, 40, 1030, 128, False, None, 0.0), (1, 131, 33, 1090, 72, False, None, 0.0),
-    (1, 17, 1024, 1024, 128, True, None, 0.0), (2, 22, 300, 1100, 64, True, None, 0.0), (3, 44, 65, 1100, 64, False, (1100, 40, 0), 0.0),
-    (1, 256, 20, 1025, 64, False, None, 0.0), (1, 257, 20, 1025, 64, False, None, 0.0), (1, 130, 40, 1024, 64, False, None, 0.2),
-    (1, 130, 40, 1030, 128, False, None, 0.1), (1, 17, 1024, 1100, 64, True, None, 0.1)])
+    (1, 130, 40, 1024, 64, False, None, 0.0), (1, 130, 40, 2050, 128, False, None, 0.0), (1, 131, 33, 2048, 72, False, None, 0.0),
+    (1, 9, 2048, 2048, 128, True, None, 0.0), (2, 22, 300, 2100, 64, True, None, 0.0), (3, 44, 65, 2100, 64, False, (2100, 40, 0), 0.0),
+    (1, 256, 20, 2049, 64, False, None, 0.0), (1, 257, 20, 2049, 64, False, None, 0.0), (1, 130, 40, 2048, 64, False, None, 0.2),
+    (1, 130, 40, 2050, 128, False, None, 0.1), (1, 17, 1024, 1100, 64, True, None, 0.1)])
 def test_forward_and_backward_against_the_oracle(oracle, B, H, Sq, Sk, D, causal, lens, p):
     from flame_amd import capi
     print(f"[key groups] {B=} {H=} {Sq=} {Sk=} {D=} {causal=} {lens=} {p=}", flush=True)
