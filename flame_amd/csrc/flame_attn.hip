@@ -817,21 +817,23 @@ int flame_sage_quant_qk_int8_ks(const void* Q, const void* K, int B, int H, int 
 }  // extern "C"
 
 // wg_count workgroups starting at workgroup p.wg_base of the problem (0: all of them)
-template <int D, int NW>
+template <int D, int NW, int KG = 1>
 static int launch_sage_fwd(const SageFwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     using T = SageTile<D>;
-    static bool attr_done = false;
-    auto kern = sage_fwd_kernel<D, NW>;
-    if (!attr_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        attr_done = true;
-    }
     constexpr int BM = 32 * NW;
     const int64_t grid = wg_count ? wg_count : (int64_t)((p.Sq + BM - 1) / BM) * p.B * p.H;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), T::LDS_BYTES, s, p);
+    if constexpr (KG == 1)
+        if (rule_key_groups(grid, p.Sk) && !p.bias) return launch_sage_fwd<D, NW, 2>(p, s, wg_count);
+    static bool attr_done = false;
+    auto kern = sage_fwd_kernel<D, NW, KG>;
+    if (!attr_done) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, KG * T::LDS_BYTES);
+        if (e != hipSuccess) return (int)e;
+        attr_done = true;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW * KG), KG * T::LDS_BYTES, s, p);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
 }

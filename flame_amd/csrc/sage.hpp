@@ -284,9 +284,10 @@ __device__ __forceinline__ constexpr int swz_i8(int row) {
     return D == 128 ? swz<64>(row) : ((row >> 2) & 3);
 }
 
-// NW wavefronts (4 or 8) of 32 queries each per workgroup, as in the bf16 forward kernel.
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_kernel(const SageFwdParams p) {
+// NW wavefronts (4 or 8) of 32 queries each per workgroup, and KG = 2 groups of them with half of the key tiles each (no bias
+// then), as in the bf16 forward kernel.
+template <int D, int NW, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel(const SageFwdParams p) {
     using T = SageTile<D>;
     constexpr int BM = 32 * NW, BN = T::BN;
     constexpr int KC = D / 32;   // int8 contraction chunks (32 per MFMA)
@@ -304,12 +305,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_kernel(cons
     constexpr int MPS = 32 / NP; // logits per maximum-scan slice
     static_assert(MPS % 2 == 0, "maximum scan takes logits in pairs");
 
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds8[];
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds8_all[];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KG == 1 ? wave_all : wave_all % NW, group = KG == 1 ? 0 : wave_all / NW;
     const int n = lane & 31, h = lane >> 5;
+    uint8_t* lds8 = lds8_all + (KG == 1 ? 0 : group * T::LDS_BYTES);
 
     const int n_qt = (p.Sq + BM - 1) / BM;
     const int wg = p.kv_len ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
@@ -330,7 +333,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_kernel(cons
     if (p.kv_len) klimit = min(klimit, max(p.kv_len[b], 0));
     int kend = klimit;
     if (p.causal) kend = min(kend, q0 + BM);
-    const int n_tiles = (kend + BN - 1) / BN;
+    int n_tiles = (kend + BN - 1) / BN;
+    // The tiles of this wavefront's group become tiles 0 .. n_tiles - 1 of a walk that starts at key `key0`.
+    const int n_first = (n_tiles + 1) / 2;                   // of group 0
+    const int key0 = KG == 1 ? 0 : group * n_first * BN;
+    if constexpr (KG == 2) {
+        n_tiles = group ? n_tiles - n_first : n_first;
+        klimit -= key0;
+        kbase += (int64_t)key0 * D;
+        vbase += key0 * p.vs.n;
+        skb += group * n_first;
+    }
 
     // Q^ fragments: column = query, 16 consecutive int8 of the contraction per lane
     i32x4 qf[KC];
@@ -454,7 +467,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_kernel(cons
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = t * BN + 32 * kb + acc_row(r, h);
-                const bool drop = (key >= klimit) | ((p.causal != 0) & (key > qi));
+                const bool drop = (key >= klimit) | ((p.causal != 0) & (key0 + key > qi));
                 float v = (float)s[kb][r] * f;
                 if (bbase && !drop && qi < p.Sq) {      // the logits are in log2 units here
                     const int64_t e = (int64_t)qi * p.bq + (int64_t)key * p.bk;
@@ -602,7 +615,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_kernel(cons
 
     // tiles [0, n_full) need no exclusions for any query of the workgroup
     int n_full = p.bias ? 0 : klimit / BN;       // a bias touches every logit
-    if (p.causal) n_full = min(n_full, (q0 + 1) / BN);
+    if (p.causal) n_full = min(n_full, (q0 + 1 - key0) / BN);
     n_full = min(n_full, n_tiles);
 
     i32x16 sa[2], sb[2];
@@ -629,6 +642,37 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_kernel(cons
         for (; t < n_tiles; t += 2) {
             step(std::false_type{}, sa, sb, t);
             if (t + 1 < n_tiles) step(std::false_type{}, sb, sa, t + 1);
+        }
+    }
+
+    // ---- the second group's state joins the first's
+    if constexpr (KG == 2) {
+        // a walk of n tiles passes n + 2 barriers; the second group's may be one tile shorter, or empty
+        const int mine = n_tiles > 0 ? n_tiles + 2 : 0, most = n_first > 0 ? n_first + 2 : 0;
+        for (int i = mine; i < most; ++i) __syncthreads();
+        __syncthreads();                               // nobody reads a tile any more
+        static_assert(NW * (4 * DB + 1) * 64 * 16 <= KG * T::LDS_BYTES, "the state of a group fits where the tiles were");
+        f32x4* slot = reinterpret_cast<f32x4*>(lds8_all) + wave * (4 * DB + 1) * 64 + lane;
+        if (group == 1) {
+#pragma unroll
+            for (int i = 0; i < 4 * DB; ++i) {
+                const f32x16& a = oacc[i >> 2];
+                slot[64 * i] = f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]};
+            }
+            slot[64 * 4 * DB] = f32x4{m_run, l_run, 0.f, 0.f};
+        }
+        __syncthreads();
+        if (group == 1) return;
+        const f32x4 other = slot[64 * 4 * DB];
+        const float m_new = fmaxf(m_run, other[0]), m_to = (m_new == -INFINITY) ? 0.f : m_new;
+        const float w0 = exp2_fast(m_run - m_to), w1 = exp2_fast(other[0] - m_to);
+        l_run = l_run * w0 + other[1] * w1;
+        m_run = m_new;
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            const f32x4 v = slot[64 * i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oacc[i >> 2][4 * (i & 3) + e] = fmaf(oacc[i >> 2][4 * (i & 3) + e], w0, v[e] * w1);
         }
     }
 
