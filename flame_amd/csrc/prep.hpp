@@ -10,7 +10,7 @@
 //   y[2p+1] = bf16( v[2p] * sin[n,p] + v[2p+1] * cos[n,p] )
 //
 // One row (D elements) is served by D/8 adjacent lanes, 8 elements = 4 rotation pairs per lane, so
-// loads and stores are 16 bytes per lane and the mean of squares is a butterfly over D/8 lanes; the same
+// loads and stores are 16 bytes per lane and the mean of squares is a sum over D/8 lanes; the same
 // lanes serve that position in several heads, which share its table entries.
 #pragma once
 #include "attn_common.hpp"
@@ -31,8 +31,30 @@ struct PrepParams {
 };
 
 // Heads served by one thread: the rotation tables depend on the position only, so a thread loads its
-// four (cos, sin) pairs once and applies them to the same 8 elements of kPrepHeadsPerThread heads.
-constexpr int kPrepHeadsPerThread = 4;
+// four (cos, sin) pairs once and applies them to the same 8 elements of kPrepHeadsPerThread heads.  Few, because small and
+// ordinary inputs are bound by the length of a thread's own chain (loads, sum, square root, division, stores): 2 x 1536
+// positions x 24 heads of 128 8.6 us with two heads, 8.9 with four, 9.2 with six (9.7 with four and the sum through LDS);
+// 3 x 5000 x 1 4.6 / 6.2 / 7.8 us; 4 x 9216 x 30, at the rate of memory, 107 / 109 / 111 us.
+constexpr int kPrepHeadsPerThread = 2;
+
+// The value of another lane of the row: CTRL is a DPP pattern (no trip through LDS, as a shuffle takes).
+template <int CTRL>
+__device__ __forceinline__ double dpp_lane(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// Sum over the 8 or 16 adjacent lanes of a row of the head dim, in every one of them: pairs, pairs of pairs, mirrored halves.
+template <int LPR>
+__device__ __forceinline__ double row_sum(double v) {
+    static_assert(LPR == 8 || LPR == 16, "the lanes of a row are half a DPP row or a whole one");
+    v += dpp_lane<0xB1>(v);          // quad_perm(1, 0, 3, 2)
+    v += dpp_lane<0x4E>(v);          // quad_perm(2, 3, 0, 1)
+    v += dpp_lane<0x141>(v);         // row_half_mirror
+    if (LPR == 16) v += dpp_lane<0x140>(v);      // row_mirror
+    return v;
+}
 
 template <int D>
 __global__ __launch_bounds__(256) void prep_qk_kernel(const PrepParams p) {
@@ -100,8 +122,7 @@ __global__ __launch_bounds__(256) void prep_qk_kernel(const PrepParams p) {
             double ss = 0.0;
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += (double)v[i] * (double)v[i];
-#pragma unroll
-            for (int off = LPR / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+            ss = row_sum<LPR>(ss);
             const float ms = (float)(ss / (double)D);
             // __builtin_sqrtf and the division operator are the correctly rounded ones under hipcc's default
             // -fhip-fp32-correctly-rounded-divide-sqrt (the __fsqrt_rn intrinsic is the approximate native one here)
