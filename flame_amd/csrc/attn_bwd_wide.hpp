@@ -13,7 +13,7 @@
 // (WideRing): rows of a tile are whole 128-byte cache lines, and while one pair of tiles is multiplied the next pair and half
 // of the one after are on their way.  Two workgroups per compute unit.  Bound by LDS traffic: a wavefront's 64 x 64 tile reads
 // 8 KiB and its share of the copies writes 4 KiB per 8 MFMAs.
-// B=1 H=1 S=4096 D=512: scores 54 us (0.64 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
+// B=1 H=1 S=4096 D=512: scores 47 us (0.73 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
 // stages, whose 64-byte rows fetched every line twice, and stores straight from the accumulators; 246 us for the whole
 // backward by library GEMMs and separate passes.  B=3 H=2 S=640 D=512, where the library's 15 calls kept the host busy,
 // forward and backward: 615 -> 80 us.
@@ -174,24 +174,26 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
     issue(kbase, p.ks.n, k_rows, 0, 0);
     issue(qbase, p.qs.n, q_rows, 0, 1);
     issue(vbase, p.vs.n, k_rows, 0, 2);
-    for (int t = 0; t < n_steps; ++t) {
+    auto step = [&](auto tail_tag, int t) {
         const bool more = t + 1 < n_steps;
-        const int rest = p.d - kWideStep * t;
         WideRing::landed(false);                           // K and Q
         issue(gbase, p.dos.n, q_rows, t, ring.slot(3));
         if (more) issue(kbase, p.ks.n, k_rows, t + 1, ring.slot(4));
-        if (rest >= kWideStep) multiply(No{}, s, ring.slot(0), ring.slot(1), rest);
-        else multiply(Yes{}, s, ring.slot(0), ring.slot(1), rest);
+        multiply(tail_tag, s, ring.slot(0), ring.slot(1), p.d - kWideStep * t);
         ring.next();
         WideRing::landed(!more);                           // V and dO
         if (more) {
             issue(qbase, p.qs.n, q_rows, t + 1, ring.slot(3));
             issue(vbase, p.vs.n, k_rows, t + 1, ring.slot(4));
         }
-        if (rest >= kWideStep) multiply(No{}, dp, ring.slot(0), ring.slot(1), rest);
-        else multiply(Yes{}, dp, ring.slot(0), ring.slot(1), rest);
+        multiply(tail_tag, dp, ring.slot(0), ring.slot(1), p.d - kWideStep * t);
         ring.next();
-    }
+    };
+    // the step that ends inside 64 behind the loop: as a choice within it, it made the compiler move both accumulators
+    // (384 registers) around every step
+    const int n_whole = p.d / kWideStep;
+    for (int t = 0; t < n_whole; ++t) step(No{}, t);
+    if (n_whole < n_steps) step(Yes{}, n_whole);
     __syncthreads();                                       // the tiles are no longer needed: P and dS take their place
 
     // ---- P and dS: a lane owns one query per block and four consecutive keys per register group.  Through LDS (rows of 128
