@@ -11,9 +11,9 @@
 // formed nor read.
 // Tiles of 128 rows x 64 (or 64 x 128) elements, 16 KiB each, are copied global -> LDS by LDS-DMA through a ring of five
 // (WideRing): rows of a tile are whole 128-byte cache lines, and while one pair of tiles is multiplied the next pair and half
-// of the one after are on their way.  Two workgroups per compute unit.  Bound by LDS traffic: a wavefront's 64 x 64 tile reads
-// 8 KiB and its share of the copies writes 4 KiB per 8 MFMAs.
-// B=1 H=1 S=4096 D=512: scores 47 us (0.73 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
+// of the one after are on their way.  Two workgroups per compute unit.  Bound by what the L2s deliver: at S = 4096
+// the scores ask 650 MB of them and the products 900 MB, 13 to 14 TB/s; the matrix cores are busy a third of the time.
+// B=1 H=1 S=4096 D=512: scores 45 us (0.76 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
 // stages, whose 64-byte rows fetched every line twice, and stores straight from the accumulators; 246 us for the whole
 // backward by library GEMMs and separate passes.  B=3 H=2 S=640 D=512, where the library's 15 calls kept the host busy,
 // forward and backward: 615 -> 80 us.
@@ -138,6 +138,14 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
         fq[u] = rq * kWideStep + 8 * (h ^ swz<64>(rq));
     }
 
+    float rows_nd[2], rows_l2[2];                          // requested before the walk, so that its end does not wait for them
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+        const int qi = q0 + 64 * wq + 32 * qb + n;
+        rows_nd[qb] = qi < p.Sq ? p.ndelta[(int64_t)bh * p.Sq + qi] : 0.f;
+        rows_l2[qb] = qi < p.Sq ? p.lse2[(int64_t)bh * p.Sq + qi] : INFINITY;
+    }
+
     f32x16 s[2][2], dp[2][2];                              // [key block][query block]
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -207,7 +215,7 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
     for (int qb = 0; qb < 2; ++qb) {
         const int rq = 64 * wq + 32 * qb + n, qi = q0 + rq;
         const bool ok = qi < p.Sq;
-        const float nd = ok ? p.ndelta[(int64_t)bh * p.Sq + qi] : 0.f, l2 = ok ? p.lse2[(int64_t)bh * p.Sq + qi] : INFINITY;
+        const float nd = rows_nd[qb], l2 = rows_l2[qb];
         const int lim = ok ? (p.causal ? min(klimit, qi + 1) : klimit) : 0;     // keys below it are attended
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
