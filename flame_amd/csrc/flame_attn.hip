@@ -24,6 +24,7 @@
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
 #include "attn_fwd_keyshare.hpp"
+#include "last_round.hpp"
 #include "prep.hpp"
 #include "sage.hpp"
 #include "plan_cache.hpp"
@@ -193,23 +194,19 @@ int launch_fwd_wide(FwdParams p, hipStream_t s) {
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_wide_kernel<D>;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
-    const int64_t n_qt = (p.Sq + T::BM - 1) / T::BM;
-    const int64_t total = n_qt * p.B * p.H, cus = device_cu_count();
-    if (8 * total > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    if ((int64_t)((p.Sq + 255) / 256) * p.B * p.H * 8 > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     // A last round that would leave at least half of the compute units idle goes to smaller workgroups in a launch of its own:
     // 32-query ones that share the keys while these fit one per unit, else 128-query ones.  (B=2 H=24 S=1536 D=128: 288
     // units of 256 queries, 92 us as two rounds, 79 us as one round and 256 small workgroups.)
-    const int64_t rest = total % cus;
-    const bool cut = total > cus && rest > 0 && 2 * rest <= cus;
-    const int64_t count = cut ? total - rest : total;
+    static_assert(T::BM == 256, "cut_last_round counts in 256-query workgroups");
+    const LastRound r = cut_last_round(p.Sq, (int64_t)p.B * p.H, device_cu_count(), true);
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)count), dim3(256), T::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)r.wide), dim3(256), T::LDS_BYTES, s, p);
     }
-    if (cut) {
-        const bool share = 8 * rest <= cus && (p.Sq + 31) / 32 == 8 * n_qt;
-        p.wg_base = (int)(count * (share ? 8 : 2));
-        return share ? launch_fwd_keyshare<D, false>(p, s, 8 * rest) : launch_fwd<D, kExNone, 4>(p, s, 2 * rest);
+    if (r.count) {
+        p.wg_base = (int)r.base;
+        return r.rows == 32 ? launch_fwd_keyshare<D, false>(p, s, r.count) : launch_fwd<D, kExNone, 4>(p, s, r.count);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -354,14 +351,14 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         if (wide) {
             // a last round on at most half of the compute units: 128-query workgroups in a launch of their own (problems
             // whose walks are all equally long)
-            const int64_t cus = device_cu_count(), rest = grid_dq % cus;
-            const bool cut = grid_dq > cus && rest > 0 && 2 * rest <= cus && !p.m.causal && !p.m.kv_len && 2 * grid_dq <= 0x7fffffff;
-            hipLaunchKernelGGL(kern_dqw, dim3((unsigned)(cut ? grid_dq - rest : grid_dq)), dim3(256), TW::LDS_BYTES, s, p);
-            if (cut) {
+            const bool even = !p.m.causal && !p.m.kv_len && 2 * grid_dq <= 0x7fffffff;
+            const LastRound r = even ? cut_last_round(p.Sq, (int64_t)p.B * p.H, device_cu_count(), false) : LastRound{grid_dq};
+            hipLaunchKernelGGL(kern_dqw, dim3((unsigned)r.wide), dim3(256), TW::LDS_BYTES, s, p);
+            if (r.count) {
                 BwdParams pt = p;
-                pt.dq_base = (int)(2 * (grid_dq - rest));
-                if (!HASMASK && rule_key_groups(2 * rest, p.Sk, kDqGroupKeys)) hipLaunchKernelGGL(kern_dqg, dim3((unsigned)(2 * rest)), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pt);
-                else hipLaunchKernelGGL(kern_dq, dim3((unsigned)(2 * rest)), dim3(256), TQ::LDS_BYTES, s, pt);
+                pt.dq_base = (int)r.base;
+                if (!HASMASK && rule_key_groups(r.count, p.Sk, kDqGroupKeys)) hipLaunchKernelGGL(kern_dqg, dim3((unsigned)r.count), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pt);
+                else hipLaunchKernelGGL(kern_dq, dim3((unsigned)r.count), dim3(256), TQ::LDS_BYTES, s, pt);
             }
         }
         else if (!HASMASK && p.key_mask)
@@ -914,13 +911,12 @@ int flame_sage_attn_fwd_bias_int8(const void* Qi8, const void* Ki8, const void* 
     const bool wide = n256 * 256 <= ((N_q + 127) / 128) * 128 && total256 >= cus && !causal && !kv_len && !bias &&
                       N_kv % 64 == 0 && wg_waves_override() != 4;
     if (wide) {
-        const int64_t rest = total256 % cus;
-        const int64_t wide_count = rest <= cus / 2 ? total256 - rest : total256;
         if (2 * total256 > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
-        rc = Dp == 128 ? launch_sage_fwd_wide<128>(p, s, wide_count) : launch_sage_fwd_wide<64>(p, s, wide_count);
-        if (rc != FLAME_ATTN_OK || wide_count == total256) return rc;
-        p.wg_base = (int)(2 * wide_count);
-        return Dp == 128 ? launch_sage_fwd<128, 4>(p, s, 2 * rest) : launch_sage_fwd<64, 4>(p, s, 2 * rest);
+        const LastRound r = cut_last_round(N_q, (int64_t)B * H, cus, false);
+        rc = Dp == 128 ? launch_sage_fwd_wide<128>(p, s, r.wide) : launch_sage_fwd_wide<64>(p, s, r.wide);
+        if (rc != FLAME_ATTN_OK || r.count == 0) return rc;
+        p.wg_base = (int)r.base;
+        return Dp == 128 ? launch_sage_fwd<128, 4>(p, s, r.count) : launch_sage_fwd<64, 4>(p, s, r.count);
     }
     if (Dp == 128) return launch_sage_fwd<128, 4>(p, s);
     return launch_sage_fwd<64, 4>(p, s);

@@ -110,10 +110,10 @@ print(json.dumps(_stats(lib)))
 """ % ROOT
 
 
-def _child(env_extra):
+def _child(env_extra, code=CHILD):
     env = {k: v for k, v in os.environ.items() if not k.startswith("FLAME_SDPA_")}
     env.update(env_extra)
-    out = subprocess.run([sys.executable, "-c", CHILD], env=env, capture_output=True, text=True, timeout=300, cwd=ROOT)
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300, cwd=ROOT)
     assert out.returncode == 0, out.stdout + out.stderr
     return json.loads(out.stdout.strip().splitlines()[-1])
 
@@ -146,3 +146,23 @@ def test_cache_file_carries_a_plan_to_the_next_process(tmp_path):
     s2 = _child(env)
     assert s2["cache_loads"] == 1 and s2["cache_hits"] == 1 and s2["tuned"] == 0 and s2["last_plan_source"] == 1
     assert s2["last_q_chunk"] == s1["last_q_chunk"] and s2["cache_saved"] == 0      # nothing new to write
+
+
+# O lies between two margins in a buffer of its own: nothing outside it may be written, and every row of it is
+CHILD_MARGINS = CHILD.replace("B, H, Q, K, D = 1, 4, 384, 256, 128", "B, H, Q, K, D = %d, %d, %d, %d, %d").replace(
+    "out = torch.empty_like(q)",
+    "m = 256 * D; buf = torch.full((q.numel() + 2 * m,), 77.0, dtype=q.dtype, device=q.device); out = buf[m:-m].view(q.shape)").replace(
+    "assert lib.flame_sdpa_autotune_flush_cache() == 0", "assert (buf[:m] == 77).all() and (buf[-m:] == 77).all()")
+
+
+@pytest.mark.parametrize("forced", ["", "256"])
+@pytest.mark.parametrize("B,H,Q,K,D", [(1, 16, 4224, 64, 64),       # 272 units of 256 queries, 33 tiles of 128 per head
+                                       (1, 24, 2944, 128, 128),     # 288 units, 23 tiles of 128
+                                       (1, 17, 4096, 64, 64)])      # 272 units, whole: the last 16 run as 32-query ones
+def test_256_row_plan_past_one_round(forced, B, H, Q, K, D):
+    """A plan of 256 rows where the rule would not take them (an odd count of 128-query tiles), on more workgroups than
+    compute units: measured on a miss, and forced."""
+    print(f"[plan] {B}x{H} Q={Q} K={K} D={D} forced={forced!r}", flush=True)
+    s = _child({"FLAME_SDPA_QCHUNK": forced} if forced else {}, CHILD_MARGINS % (B, H, Q, K, D))
+    assert s["errors"] == 0 and s["last_q_chunk"] in ((256,) if forced else (128, 256))
+    assert s["tuned"] == (0 if forced else 1)
