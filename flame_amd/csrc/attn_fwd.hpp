@@ -42,7 +42,7 @@ struct FwdParams {
     // normalised fp32 partial output with its log-sum-exp; fwd_merge_kernel combines them.
     int key_splits = 1;          // 1: O and LSE are written directly
     float* part_o = nullptr;     // [key_splits][B*H*Sq][dv]
-    float* part_lse = nullptr;   // [key_splits][B*H*Sq], natural log, -inf for a slice without an attended key
+    float* part_lse = nullptr;   // [key_splits][B*H*Sq], natural log, -inf for a slice without an attended key, NaN for one with a NaN
 };
 
 template <int D>
@@ -586,8 +586,8 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     }
 }
 
-// Combines the partial outputs of a key split: LSE = log sum_s exp(LSE_s), O = sum_s exp(LSE_s - LSE) O_s.  One lane
-// per query row and 4 output columns.
+// Combines the partial outputs of a key split: LSE = log sum_s exp(LSE_s), O = sum_s exp(LSE_s - LSE) O_s.  A slice whose sum
+// was NaN makes O NaN (and LSE -inf, as in a walk over all keys by one workgroup).  One lane per query row and 4 output columns.
 static __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p) {
     const int groups = p.dv >> 2;
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
@@ -596,10 +596,15 @@ static __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p
     const int64_t row = idx / groups;
     const int g = (int)(idx % groups);
     float m = -INFINITY;
-    for (int s = 0; s < p.key_splits; ++s) m = fmaxf(m, p.part_lse[s * rows + row]);
+    bool nan = false;                  // fmaxf passes over a NaN
+    for (int s = 0; s < p.key_splits; ++s) {
+        const float l = p.part_lse[s * rows + row];
+        m = fmaxf(m, l);
+        nan |= l != l;
+    }
     float sum = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (m != -INFINITY) {
+    if (m != -INFINITY || nan) {
         for (int s = 0; s < p.key_splits; ++s) {
             const float w = expf(p.part_lse[s * rows + row] - m);
             const f32x4 v = *reinterpret_cast<const f32x4*>(p.part_o + (s * rows + row) * p.dv + 4 * g);

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(64 * NW) void fwd_bigd_kernel(const FwdParams p) {
                             *reinterpret_cast<f32x4*>(prow + d0) = w;
                         }
                     }
-            if (h == 0 && db0 == 0) p.part_lse[prow_i] = lse_val;
+            if (h == 0 && db0 == 0) p.part_lse[prow_i] = l != l ? l : lse_val;         // a NaN is not an empty slice
         }
         return;
     }

@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void fwd_keyshare_kernel(const FwdParams p) {
         const int64_t r = (int64_t)bh * p.Sq + q0 + row;
         if (p.key_splits > 1) {
             *reinterpret_cast<f32x4*>(p.part_o + ((int64_t)slice * rows + r) * p.dv + 4 * g) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-            if (g == 0) p.part_lse[(int64_t)slice * rows + r] = lse;
+            if (g == 0) p.part_lse[(int64_t)slice * rows + r] = l != l ? l : lse;      // a NaN is not an empty slice
         } else {
             uint16_t* orow = p.o + b * p.os.b + hh * p.os.h + (int64_t)(q0 + row) * p.os.n;
             *reinterpret_cast<u32x2*>(orow + 4 * g) = u32x2{pack_bf16(acc[0] * inv, acc[1] * inv), pack_bf16(acc[2] * inv, acc[3] * inv)};
