@@ -330,6 +330,9 @@ PyObject* py_sdpa(PyObject*, PyObject* const* a, Py_ssize_t n) {
         need_args(n, 6);
         const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v");
         if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) fail(PyExc_ValueError, "SDPA expects 4-D input [B, H, S, D]");
+        // whether or not a graph is recorded: without one the autograd node, which has no jvp either, is passed by
+        for (const Tensor* t : {&q, &k, &v})
+            TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(0).defined(), "SDPA has no forward-mode derivative: an input carries a tangent");
         const bool causal = bool_arg(a[4]);
         const double scale = a[5] == Py_None ? 1.0 / std::sqrt((double)q.size(3)) : float_arg(a[5]);
         Tensor mask;

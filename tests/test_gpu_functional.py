@@ -71,3 +71,17 @@ def test_rank_check():
     from flame_amd import functional as F
     with pytest.raises(ValueError):
         F.sdpa(torch.zeros(2, 3, 4, device="cuda"), torch.zeros(2, 3, 4, device="cuda"), torch.zeros(2, 3, 4, device="cuda"))
+
+
+def test_forward_mode_is_refused():
+    """No input requires a gradient and one carries a tangent: refused, not answered without a tangent."""
+    from flame_amd import functional as F
+    import torch.autograd.forward_ad as fwad
+    q, k, v = (torch.randn(1, 2, 64, 64, device="cuda").to(torch.bfloat16) for _ in range(3))
+    with fwad.dual_level():
+        for i in range(3):
+            args = [q, k, v]
+            args[i] = fwad.make_dual(args[i], torch.ones_like(args[i]))
+            with pytest.raises(NotImplementedError, match="forward-mode"):
+                F.sdpa(*args)
+        assert F.sdpa(q, k, v).shape == q.shape          # inputs without a tangent are served inside a dual level, too
