@@ -255,6 +255,18 @@ Tensor as_bf16_view(const Tensor& x) {
     return t;
 }
 
+// The copy of a keep-mask that a recorded graph holds, so that the caller may refill the buffer before the backward.  Axes
+// along which the tensor repeats itself are kept once, and rows start on 16 bytes (where the kernels load them as vectors).
+Tensor own_mask(const Tensor& m) {
+    Tensor src = m;
+    for (int ax = 0; ax < 4; ++ax)
+        if (src.stride(ax) == 0 && src.size(ax) > 1) src = src.narrow(ax, 0, 1);
+    const int64_t n = src.size(3);
+    Tensor own = empty({src.size(0), src.size(1), src.size(2), (n + 15) / 16 * 16}, at::kBool, m).narrow(3, 0, n);
+    at::ne_out(own, src, 0);
+    return own.view(at::kByte);
+}
+
 // forward of one call; true: served by the materialised path
 bool sdpa_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, bool causal, double scale, bool want_lse, Tensor& o, Tensor& lse) {
     const Sizes z{(int)q.size(0), (int)q.size(1), (int)q.size(2), (int)k.size(2), (int)q.size(3)};
@@ -336,11 +348,13 @@ PyObject* py_sdpa(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const bool causal = bool_arg(a[4]);
         const double scale = a[5] == Py_None ? 1.0 / std::sqrt((double)q.size(3)) : float_arg(a[5]);
         Tensor mask;
+        bool converted = false;      // the mask is a tensor of its own already
         if (!causal && a[3] != Py_None) {
             const Tensor& m = tensor_arg(a[3], "attn_mask");
             if (m.dim() != 4) fail(PyExc_ValueError, "mask must be 4D [B,H,Q,K]");
             // a boolean tensor holds one byte of 0 or 1 per element already
-            mask = m.scalar_type() == at::kByte ? m : (m.scalar_type() == at::kBool ? m : m.to(at::kFloat).ge(0.5)).view(at::kByte);
+            converted = m.scalar_type() != at::kByte && m.scalar_type() != at::kBool;
+            mask = m.scalar_type() == at::kByte ? m : (converted ? m.to(at::kFloat).ge(0.5) : m).view(at::kByte);
             int64_t st[4];
             const Sizes z{(int)q.size(0), (int)q.size(1), (int)q.size(2), (int)k.size(2), (int)q.size(3)};
             check_that(broadcast_strides(mask, z, st), "mask is not broadcastable to [B,H,Sq,Sk]");
@@ -352,7 +366,7 @@ PyObject* py_sdpa(PyObject*, PyObject* const* a, Py_ssize_t n) {
             const at::ScalarType orig = q.scalar_type();
             const Tensor qb = as_bf16_view(q), kb = as_bf16_view(k), vb = as_bf16_view(v);
             if (at::GradMode::is_enabled() && (qb.requires_grad() || kb.requires_grad() || vb.requires_grad())) {
-                out = Sdpa::apply(qb, kb, vb, mask.defined() ? std::optional<Tensor>(mask) : std::nullopt, causal, scale);
+                out = Sdpa::apply(qb, kb, vb, mask.defined() ? std::optional<Tensor>(converted ? mask : own_mask(mask)) : std::nullopt, causal, scale);
             } else {
                 Tensor lse;
                 sdpa_forward(qb, kb, vb, mask, causal, scale, false, out, lse);

@@ -16,8 +16,9 @@ def sdpa(q, k, v, attn_mask=None, is_causal=None, scale=None):
     """Scaled dot-product attention on [B,H,S,D] tensors.
 
     attn_mask: optional binary keep-mask broadcastable as [B|1, H|1, Sq, Sk] (values >= 0.5 attend; the
-    reference's public mask convention, src/sdpa.rs:458-470).  With is_causal=True the mask argument is
-    ignored, as in the reference, and the causal structure is applied natively (no mask tensor is built).
+    reference's public mask convention, src/sdpa.rs:458-470).  Its buffer may be refilled before the backward: the
+    recorded graph holds a copy.  With is_causal=True the mask argument is ignored, as in the reference, and the
+    causal structure is applied natively (no mask tensor is built).
     Inputs of another dtype are promoted to bf16 and the result is cast back."""
     return capi.host().sdpa(q, k, v, attn_mask, is_causal is not None and bool(is_causal), scale)
 

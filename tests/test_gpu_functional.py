@@ -85,3 +85,31 @@ def test_forward_mode_is_refused():
             with pytest.raises(NotImplementedError, match="forward-mode"):
                 F.sdpa(*args)
         assert F.sdpa(q, k, v).shape == q.shape          # inputs without a tangent are served inside a dual level, too
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8])
+@pytest.mark.parametrize("shape", ["keys", "expanded keys", "rows", "cut out of a larger mask"])
+def test_mask_buffer_may_be_refilled_before_the_backward(shape, dtype):
+    """The graph holds the mask as it was when the forward ran (also where the caller's tensor repeats along an axis or is
+    part of a larger one)."""
+    from flame_amd import functional as F
+    torch.manual_seed(5)
+    B, H, Sq, Sk, D = 2, 3, 130, 200, 64
+    q, k, v = (torch.randn(B, H, n, D, device="cuda").to(torch.bfloat16).requires_grad_(True) for n in (Sq, Sk, Sk))
+    g = torch.randn(B, H, Sq, D, device="cuda").to(torch.bfloat16)
+    buf = torch.rand(B, 1, 160 if shape.startswith("cut") else Sq if shape == "rows" else 1, 256 if shape.startswith("cut") else Sk, device="cuda") < 0.6
+    buf[..., 0] = True
+    buf = buf.to(dtype)
+    mask = buf.expand(B, H, Sq, Sk) if shape == "expanded keys" else buf[:, :, :Sq, 3:3 + Sk] if shape.startswith("cut") else buf
+    if shape.startswith("cut"):
+        mask[..., 0] = 1
+    frozen = mask.clone()
+    o = F.sdpa(q, k, v, attn_mask=mask)
+    buf.fill_(0)                         # the next batch's mask goes into the same buffer
+    got = torch.autograd.grad(o, (q, k, v), g)
+    ro, rin = _ref(q, k, v, mask=frozen)
+    want = torch.autograd.grad(ro, rin, g.float())
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        assert ((a.float() - b).pow(2).sum().sqrt() / b.pow(2).sum().sqrt()).item() <= 1e-2, name
+
+
