@@ -22,6 +22,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/flame_attn.h"
 
@@ -71,6 +72,8 @@ void check_rc(int rc, const char* fn) {
 template <class F>
 PyObject* guarded(F&& f) {
     HANDLE_TH_ERRORS
+    // torch.jit.trace records torch's operators only: the results of these calls would become constants of the trace
+    TORCH_CHECK(!torch::jit::tracer::isTracing(), "the attention calls cannot be recorded by torch.jit.trace");
     try {
         return f();
     } catch (const CallError& e) {

@@ -18,3 +18,13 @@ def test_forward_mode(which, recorded):
                 call()
             with torch.no_grad(), pytest.raises(NotImplementedError, match="forward-mode"):
                 call()
+
+
+@pytest.mark.parametrize("recorded", [False, True])
+def test_jit_trace(recorded):
+    """The trace would hold the result for its example inputs as a constant."""
+    from flame_amd import capi, functional as F
+    args = [torch.randn(1, 2, 8, 64).to(torch.bfloat16).requires_grad_(recorded) for _ in range(3)]
+    for call in (lambda q, k, v: F.sdpa(q, k, v) * 2, lambda q, k, v: capi.attn_fwd(q, k, v, 0.125)[0] * 2):
+        with pytest.raises(RuntimeError, match="cannot be recorded"):
+            torch.jit.trace(call, args)
