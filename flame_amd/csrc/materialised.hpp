@@ -37,7 +37,7 @@ __device__ __forceinline__ float mat_logit(const MatRowsParams& p, const uint8_t
 
 // One workgroup per query row of the band.  Forward: exclusions and bias, row maximum and sum (two passes over the
 // row, which sits in L2), LSE = max + ln(sum), P = exp(s - LSE) as bf16; a row without an attended key gets
-// LSE = -inf and P = 0; with dropout P is stored as P * f, f = 0 or 1 / (1 - p) per element (drop_factor_at), the
+// LSE = -inf and P = 0, a row with a NaN among its scores LSE and P NaN; with dropout P is stored as P * f, f = 0 or 1 / (1 - p) per element (drop_factor_at), the
 // LSE being that of the undropped row.  Backward: P = exp(s - LSE) from the saved LSE, undropped.
 __global__ __launch_bounds__(256) void mat_rows_kernel(const MatRowsParams p) {
     const int row = blockIdx.x;                      // over [BH, tq]
@@ -58,12 +58,19 @@ __global__ __launch_bounds__(256) void mat_rows_kernel(const MatRowsParams p) {
         lse = p.lse[(size_t)bh * p.Sq + qi];
     } else {
         float m = -INFINITY;
-        for (int j = tid; j < p.Sk; j += 256) m = fmaxf(m, mat_logit(p, mbase, bias_base, b, qi, j, klimit, s[j]));
+        bool nan = false;                            // fmaxf passes over a NaN
+        for (int j = tid; j < p.Sk; j += 256) {
+            const float v = mat_logit(p, mbase, bias_base, b, qi, j, klimit, s[j]);
+            m = fmaxf(m, v);
+            nan |= v != v;
+        }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-        if (lane == 0) red[wave] = m;
+        nan = __any(nan);
+        if (lane == 0) red[wave] = nan ? NAN : m;
         __syncthreads();
         m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+        for (int w = 0; w < 4; ++w) m = red[w] != red[w] ? red[w] : m;
         __syncthreads();
         float l = 0.f;
         if (m != -INFINITY)

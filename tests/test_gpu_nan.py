@@ -49,3 +49,17 @@ def test_nan_stays_nan(what, H, Sq, Sk, D):
     rows = room[1].cpu(), none[1].cpu()
     assert torch.equal(torch.isfinite(rows[0]), torch.isfinite(rows[1]))
     assert torch.equal(torch.isfinite(rows[0]), torch.ones_like(rows[0], dtype=torch.bool) if what == "value" else ~bad.any(-1).view(rows[0].shape))
+
+
+@pytest.mark.parametrize("what", ["query", "keys", "one key", "value"])
+def test_nan_stays_nan_materialised(what):
+    from flame_amd import capi
+    print(f"[nan] materialised, {what}", flush=True)
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn((1, 2, n, 20), generator=g).to(torch.bfloat16) for n in (70, 300, 300))
+    bad = _plant(what, q, k, v)
+    o, lse = (t.cpu() for t in capi.attn_fwd_materialised(q.cuda(), k.cuda(), v.cuda(), 0.2))
+    assert torch.equal(torch.isnan(o), bad)
+    want = torch.softmax(q.double() @ k.double().transpose(-1, -2) * 0.2, dim=-1) @ v.double()
+    assert torch.allclose(o.double()[~bad], want[~bad], atol=2e-2, rtol=1e-2)
+    assert torch.equal(torch.isfinite(lse), torch.ones_like(lse, dtype=torch.bool) if what == "value" else ~bad.any(-1).view(lse.shape))
