@@ -1036,7 +1036,8 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     if (dropout_p != 0.f) {
         if (!set_dropout(p.m, dropout_p, dropout_seed, draw_cq, draw_ck, N_q, N_kv)) return FLAME_ATTN_ERR_INVALID;
         const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
-        // the kernel of the undropped call, so that the log-sum-exp is the same to the bit
+        // the undropped call's choice between the kernels, without its split of the keys (this entry point has no workspace):
+        // the log-sum-exp is that of the undropped softmax, its sum joined in another order where that call splits
         if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q))
             return DP == 128 ? launch_fwd_keyshare<128, true>(p, s) : launch_fwd_keyshare<64, true>(p, s);
         return DP == 128 ? launch_fwd_dropout<128>(p, hm, s) : launch_fwd_dropout<64>(p, hm, s);
@@ -1943,7 +1944,8 @@ size_t mat_accum_bytes(int B, int H, int N_kv, int D, int Dv) { return align_up(
 int pad128(int n) { return (n + 127) / 128 * 128; }
 size_t wide_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
 size_t wide_slice_bytes(int N_q, int N_kv) { return (size_t)pad128(N_q) * pad128(N_kv) * 4; }         // P and dS, bf16
-// as many slices at a time as 512 MiB hold (a slice above 2 GiB: not served)
+// as many slices at a time as 512 MiB hold, and one of up to 2 GiB where none does (16384 x 16384: 1 GiB, twice what the
+// banded path takes); a larger one is not served
 size_t wide_workspace_bytes(int B, int H, int N_q, int N_kv) {
     const size_t slice = wide_slice_bytes(N_q, N_kv);
     if (slice > ((size_t)2 << 30)) return 0;

@@ -233,7 +233,10 @@ int flame_attn_bwd_bf16_noalloc(const void* Q, const void* K, const void* V, con
  * caller's workspace (8 bytes per score element of the band in the backward, 6 in the forward); what is kept
  * between forward and backward is O and LSE, as everywhere else.  flame_attn_materialised_workspace_bytes returns
  * the size with which the whole problem is one band or, for large problems, bands of about 512 MiB; any workspace
- * that holds 16 query rows is accepted (more bands).  The first call creates a rocBLAS handle per device, which
+ * that holds 16 query rows is accepted (more bands).  For a backward with D = Dv a multiple of 8 it is at least the size
+ * of the kernels for head dims above 128 (no keep-mask, no dropout): P and dS of as many (batch, head) slices as 512 MiB
+ * hold, 4 bytes per score element, or of one slice of up to 2 GiB (N_q = N_kv = 16384: 1 GiB); with less room than one
+ * slice those problems are computed in bands, too.  The first call creates a rocBLAS handle per device, which
  * allocates: these entry points are not meant for graph capture.  Several times slower than the fused kernels
  * where both apply.  dropout_p, dropout_seed, draw_chunk_q, draw_chunk_kv: dropout of the probabilities as in
  * flame_attn_fwd_dropout_bf16 / flame_attn_fwd_dropout_tiled_bf16 (dropout_p = 0: none; draw_chunk_* = 0: one draw
