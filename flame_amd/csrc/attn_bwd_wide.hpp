@@ -12,8 +12,8 @@
 // Tiles of 128 rows x 64 (or 64 x 128) elements, 16 KiB each, are copied global -> LDS by LDS-DMA through a ring of five
 // (WideRing): rows of a tile are whole 128-byte cache lines, and while one pair of tiles is multiplied the next pair and half
 // of the one after are on their way.  Two workgroups per compute unit.  Bound by what the L2s deliver: at S = 4096
-// the scores ask 650 MB of them and the products 900 MB, 13 to 14 TB/s; the matrix cores are busy a third of the time.
-// B=1 H=1 S=4096 D=512: scores 45 us (0.76 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
+// the scores ask 650 MB of them and the products 900 MB, 14 TB/s; the matrix cores are busy a third of the time.
+// B=1 H=1 S=4096 D=512: scores 47 us (0.74 PFLOP/s), products 63 us (0.82 PFLOP/s); 66 and 82 us with tiles 32 deep in two
 // stages, whose 64-byte rows fetched every line twice, and stores straight from the accumulators; 246 us for the whole
 // backward by library GEMMs and separate passes.  B=3 H=2 S=640 D=512, where the library's 15 calls kept the host busy,
 // forward and backward: 615 -> 80 us.

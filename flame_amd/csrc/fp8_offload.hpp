@@ -4,8 +4,9 @@
 // Byte work bound by HBM: 3 bytes move per element in either direction.  8 elements per lane and step (a 16-byte load and an
 // 8-byte store, or the reverse, neighbouring lanes on neighbouring addresses), two steps in flight, grid-stride over the
 // tensor, scalar code for the last n % 8 elements and for pointers that are not 16-byte aligned.  56.6 M elements (170 MB
-// move): encode 33.3 -> 25.9 us, decode 26.7 -> 25.3 us against 16 elements per lane, where each of the two wide accesses of
-// a step touched every line of both; a copy of as many bytes takes 25.6 us.
+// move; medians of 100 launches) against 16 elements per lane, where each of the two wide accesses of a step touched every
+// line of both: one kernel repeated, so that part of its data stays in the cache, encode 34.0 -> 26.8 us, decode
+// 26.4 -> 25.5 us (a copy of as many bytes: 25.6 us); encode and decode in turn 41 -> 31 to 35 and 30 -> 26 us.
 //
 // The codes are the reference's, bit for bit, including where they differ from OCP E4M3:
 //   * encode(x) = code of |x * inv_scale| after clamping to 448, sign bit from `product < 0`;
