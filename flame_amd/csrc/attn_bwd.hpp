@@ -84,8 +84,8 @@ struct BwdTile {
 };
 
 template <int D>
-__device__ __forceinline__ void dkdv_store(const BwdParams& p, const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32],
-                                           int b, int hh, int krow, int h, float dv_scale = 1.0f);
+__device__ __forceinline__ void dkdv_store(const BwdParams& p, uint16_t* own, const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32],
+                                           int b, int hh, int kw0, float dv_scale = 1.0f);
 
 // VECMASK (with HASMASK): the keep-mask rows are contiguous and 16-byte aligned, Sq is a multiple of 64, Sk
 // of 128, and there is no causal flag.  The 64 x 128 mask bytes of a step then travel to LDS with the step's other copies (two more
@@ -173,7 +173,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         for (int db = 0; db < D / 32; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) zero[db][r] = 0.f;
-        dkdv_store<D>(p, zero, zero, b, hh, kw0 + n, h);
+        dkdv_store<D>(p, lds + wave * 32 * D, zero, zero, b, hh, kw0);
         return;
     }
     const int n_it = n_qt - qt_begin;
@@ -729,7 +729,8 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
                 dvacc[db][r] = 0.f;
             }
     }
-    dkdv_store<D>(p, dkacc, dvacc, b, hh, kw0 + n, h, DROP == kDropFlat || DROP == kDropRows64 ? p.m.drop_scale : 1.0f);
+    __syncthreads();              // nobody reads a tile any more
+    dkdv_store<D>(p, lds + wave * 32 * D, dkacc, dvacc, b, hh, kw0, DROP == kDropFlat || DROP == kDropRows64 ? p.m.drop_scale : 1.0f);
 }
 
 template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone>
@@ -737,27 +738,18 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
     bwd_dkdv_body<D, HASMASK, TIMING, VECMASK, DROP>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
-// dK^T / dV^T accumulators (rows = d, column = this lane's key) -> bf16 rows of dK (scaled) and dV
+// dK^T / dV^T accumulators (rows = d, column = a lane's key) of the 32 keys from kw0 on -> bf16 rows of dK (scaled) and dV
 template <int D>
-__device__ __forceinline__ void dkdv_store(const BwdParams& p, const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32],
-                                           int b, int hh, int krow, int h, float dv_scale) {
-    constexpr int DB = D / 32;
-    if (krow < p.Sk) {
-        uint16_t* dkrow = p.dk + b * p.dks.b + hh * p.dks.h + (int64_t)krow * p.dks.n;
-        uint16_t* dvrow = p.dv + b * p.dvs.b + hh * p.dvs.h + (int64_t)krow * p.dvs.n;
-        const float s = p.scale;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x16& a = dkacc[db];
-                const f32x16& c = dvacc[db];
-                u32x2 wk = {pack_bf16(a[4 * g] * s, a[4 * g + 1] * s), pack_bf16(a[4 * g + 2] * s, a[4 * g + 3] * s)};
-                u32x2 wv = {pack_bf16(c[4 * g] * dv_scale, c[4 * g + 1] * dv_scale), pack_bf16(c[4 * g + 2] * dv_scale, c[4 * g + 3] * dv_scale)};
-                if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dkrow + 32 * db + 8 * g + 4 * h) = wk;
-                if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dvrow + 32 * db + 8 * g + 4 * h) = wv;
-            }
-    }
+__device__ __forceinline__ void dkdv_store(const BwdParams& p, uint16_t* own, const f32x16 (&dkacc)[D / 32], const f32x16 (&dvacc)[D / 32],
+                                           int b, int hh, int kw0, float dv_scale) {
+    const auto rows_of = [&](const f32x16 (&acc)[D / 32], float s) {
+        return [&acc, s](int db, int g) {
+            const f32x16& a = acc[db];
+            return u32x2{pack_bf16(a[4 * g] * s, a[4 * g + 1] * s), pack_bf16(a[4 * g + 2] * s, a[4 * g + 3] * s)};
+        };
+    };
+    store_rows32<D>(own, p.dk + b * p.dks.b + hh * p.dks.h + (int64_t)kw0 * p.dks.n, p.dks.n, p.Sk - kw0, p.d, rows_of(dkacc, p.scale));
+    store_rows32<D>(own, p.dv + b * p.dvs.b + hh * p.dvs.h + (int64_t)kw0 * p.dvs.n, p.dvs.n, p.Sk - kw0, p.d, rows_of(dvacc, dv_scale));
 }
 
 // Sums the fp32 partials that the split workgroups of one key block left behind and writes dK, dV; keys that nothing attends
@@ -1205,19 +1197,11 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
             }
         return;
     }
-    // ... or dQ = scale * dQ^T, bf16
-    if (qok) {
-        uint16_t* dqrow = p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)qrow * p.dqs.n;
-        const float s = p.scale;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x16& a = dqacc[db];
-                u32x2 w = {pack_bf16(a[4 * g] * s, a[4 * g + 1] * s), pack_bf16(a[4 * g + 2] * s, a[4 * g + 3] * s)};
-                if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dqrow + 32 * db + 8 * g + 4 * h) = w;
-            }
-    }
+    // ... or dQ = scale * dQ^T, bf16 (every walk ended with a barrier: the tiles are free)
+    store_rows32<D>(lds_all + wave * 32 * D, p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)qw0 * p.dqs.n, p.dqs.n, p.Sq - qw0, p.d, [&](int db, int g) {
+        const f32x16& a = dqacc[db];
+        return u32x2{pack_bf16(a[4 * g] * p.scale, a[4 * g + 1] * p.scale), pack_bf16(a[4 * g + 2] * p.scale, a[4 * g + 3] * p.scale)};
+    });
 }
 
 // Sums the fp32 partials of the workgroups that shared a 128-query tile and writes dQ.  One workgroup per (tile, 32-wide block
@@ -1606,20 +1590,15 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     }
 
     // ---- epilogue: dQ = scale * dQ^T, bf16
+    __syncthreads();              // nobody reads a tile any more
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
-        if (qrow[qb] < p.Sq) {
-            uint16_t* dqrow = p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)qrow[qb] * p.dqs.n;
-            const float s = p.scale;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const f32x16& a = dqacc[qb][db];
-                    u32x2 w = {pack_bf16(a[4 * g] * s, a[4 * g + 1] * s), pack_bf16(a[4 * g + 2] * s, a[4 * g + 3] * s)};
-                    if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dqrow + 32 * db + 8 * g + 4 * h) = w;
-                }
-        }
+    for (int qb = 0; qb < 2; ++qb) {
+        const int row0 = qw0 + 32 * qb;
+        store_rows32<D>(lds + wave * 32 * D, p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)row0 * p.dqs.n, p.dqs.n, p.Sq - row0, p.d, [&](int db, int g) {
+            const f32x16& a = dqacc[qb][db];
+            return u32x2{pack_bf16(a[4 * g] * p.scale, a[4 * g + 1] * p.scale), pack_bf16(a[4 * g + 2] * p.scale, a[4 * g + 3] * p.scale)};
+        });
+    }
 }
 
 template <int D>

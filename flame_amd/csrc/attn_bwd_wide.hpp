@@ -356,20 +356,14 @@ __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const u
                 for (int m = 0; m < 2; ++m) acc[u][m] = mfma32(xf[u], wf[m], acc[u][m]);
         }
     }
+    __syncthreads();                                   // the tiles are no longer needed: the output passes through their place
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-        const int row = m0 + 64 * wm + 32 * m + n;
-        if (row >= n_out) continue;
-        uint16_t* orow = out + b * outs.b + hh * outs.h + (int64_t)row * outs.n;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int col = d0 + 64 * wd + 32 * u + 8 * g + 4 * h;
-                const f32x16& a = acc[u][m];
-                if (col < p.d)
-                    *reinterpret_cast<u32x2*>(orow + col) = u32x2{pack_bf16(a[4 * g] * mul, a[4 * g + 1] * mul), pack_bf16(a[4 * g + 2] * mul, a[4 * g + 3] * mul)};
-            }
+        const int row0 = m0 + 64 * wm + 32 * m, col0 = d0 + 64 * wd;
+        store_rows32<64>(lds + wave * 32 * 64, out + b * outs.b + hh * outs.h + (int64_t)row0 * outs.n + col0, outs.n, n_out - row0, p.d - col0, [&](int u, int g) {
+            const f32x16& a = acc[u][m];
+            return u32x2{pack_bf16(a[4 * g] * mul, a[4 * g + 1] * mul), pack_bf16(a[4 * g + 2] * mul, a[4 * g + 3] * mul)};
+        });
     }
 }
 

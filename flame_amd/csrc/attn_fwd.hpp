@@ -567,23 +567,17 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         }
     }
 
-    // ---- epilogue
-    if (qi < p.Sq) {
-        const float l = l_run + xhalf(l_run);
-        float inv = l > 0.f ? 1.0f / l : 0.f;
-        if constexpr (DROP == kDropFlat || DROP == kDropRows64) inv *= p.m.drop_scale;
-        uint16_t* orow = p.o + b * p.os.b + hh * p.os.h + (int64_t)qi * p.os.n;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x16& a = oacc[db];
-                u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv),
-                           pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
-                if (32 * db + 8 * g + 4 * h < p.dv) *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * g + 4 * h) = w;
-            }
-        if (p.lse && h == 0) p.lse[(int64_t)bh * p.Sq + qi] = l > 0.f ? (m_run * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
-    }
+    // ---- epilogue: O through LDS where nobody reads any more (KG: the state of the second group this wavefront has joined)
+    if constexpr (KG == 1) __syncthreads();
+    uint16_t* own = KG == 1 ? lds + wave * 32 * D : lds_all + wave * (4 * DB + 1) * 64 * 8;
+    const float l = l_run + xhalf(l_run);
+    float inv = l > 0.f ? 1.0f / l : 0.f;
+    if constexpr (DROP == kDropFlat || DROP == kDropRows64) inv *= p.m.drop_scale;
+    store_rows32<D>(own, p.o + b * p.os.b + hh * p.os.h + (int64_t)qw0 * p.os.n, p.os.n, p.Sq - qw0, p.dv, [&](int db, int g) {
+        const f32x16& a = oacc[db];
+        return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
+    });
+    if (p.lse && h == 0 && qi < p.Sq) p.lse[(int64_t)bh * p.Sq + qi] = l > 0.f ? (m_run * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
 }
 
 // Combines the partial outputs of a key split: LSE = log sum_s exp(LSE_s), O = sum_s exp(LSE_s - LSE) O_s.  A slice whose sum
@@ -1004,31 +998,21 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
             step(I3{}, sb, sa, k3, v2);
             advance(t + 3);
         }
-        wait_vm0();          // no copy may land after the workgroup has gone
+        wait_vm0();          // no copy may land where O passes through LDS
     }
 
     // ---- epilogue
+    __syncthreads();
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-        const int row = qrow[qb];
+        const int row = qrow[qb], row0 = qw0 + 32 * qb;
         const float l = l_run[qb] + xhalf(l_run[qb]);
         const float inv = l > 0.f ? 1.0f / l : 0.f;
-        if (row < p.Sq) {
-            uint16_t* orow = obase + (int64_t)row * p.os.n;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const f32x16& a = oacc[qb][db];
-                    u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv),
-                               pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
-                    if (32 * db + 8 * g + 4 * h < p.dv) *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * g + 4 * h) = w;
-                }
-            if (p.lse && h == 0) {
-                const float v = l > 0.f ? (m_run[qb] * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
-                p.lse[(int64_t)bh * p.Sq + row] = v;
-            }
-        }
+        store_rows32<D>(lds + wave * 32 * D, obase + (int64_t)row0 * p.os.n, p.os.n, p.Sq - row0, p.dv, [&](int db, int g) {
+            const f32x16& a = oacc[qb][db];
+            return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
+        });
+        if (p.lse && h == 0 && row < p.Sq) p.lse[(int64_t)bh * p.Sq + row] = l > 0.f ? (m_run[qb] * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
     }
 }
 

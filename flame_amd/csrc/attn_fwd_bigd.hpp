@@ -359,43 +359,29 @@ __global__ __launch_bounds__(64 * NW) void fwd_bigd_kernel(const FwdParams p) {
     const float l = l_run + xhalf(l_run);
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     const float lse_val = l > 0.f ? (m_run * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
-    if (p.key_splits > 1) {
-        if (qi < p.Sq) {
-            const int64_t prow_i = ((int64_t)slice * n_bh + bh) * p.Sq + qi;
-            float* prow = p.part_o + prow_i * p.dv;
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-#pragma unroll
-                for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const int d0 = 128 * c + 32 * (db0 + db) + 8 * g + 4 * h;
-                        if (d0 < p.dv) {
-                            const f32x16& a = oacc[c][db];
-                            const f32x4 w = {a[4 * g] * inv, a[4 * g + 1] * inv, a[4 * g + 2] * inv, a[4 * g + 3] * inv};
-                            *reinterpret_cast<f32x4*>(prow + d0) = w;
-                        }
-                    }
-            if (h == 0 && db0 == 0) p.part_lse[prow_i] = l != l ? l : lse_val;         // a NaN is not an empty slice
+    wait_vm0();
+    __syncthreads();              // no copy may land, and nobody reads, where the rows pass through LDS
+    constexpr int CW = 32 * NDB;  // this wavefront's columns of a chunk
+    const int64_t prow0 = ((int64_t)slice * n_bh + bh) * p.Sq + qw0;
+    static_for<NC>([&](auto c_tag) {
+        constexpr int c = decltype(c_tag)::value;
+        const int d0 = 128 * c + 32 * db0;
+        if (p.key_splits > 1) {
+            static_assert(NW * 32 * CW * 4 <= T::LDS_BYTES, "the rows fit where the tiles were");
+            store_rows32_f32<CW>(reinterpret_cast<float*>(lds) + wave * 32 * CW, p.part_o + prow0 * p.dv + d0, p.dv, p.Sq - qw0, p.dv - d0, [&](int db, int g) {
+                const f32x16& a = oacc[c][db];
+                return f32x4{a[4 * g] * inv, a[4 * g + 1] * inv, a[4 * g + 2] * inv, a[4 * g + 3] * inv};
+            });
+        } else {
+            store_rows32<CW>(lds + wave * 32 * CW, obase + (int64_t)qw0 * p.os.n + d0, p.os.n, p.Sq - qw0, p.dv - d0, [&](int db, int g) {
+                const f32x16& a = oacc[c][db];
+                return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
+            });
         }
-        return;
-    }
-    if (qi < p.Sq) {
-        uint16_t* orow = obase + (int64_t)qi * p.os.n;
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-            for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int d0 = 128 * c + 32 * (db0 + db) + 8 * g + 4 * h;
-                    if (d0 < p.dv) {
-                        const f32x16& a = oacc[c][db];
-                        u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
-                        *reinterpret_cast<u32x2*>(orow + d0) = w;
-                    }
-                }
-        if (p.lse && h == 0 && db0 == 0) p.lse[(int64_t)bh * p.Sq + qi] = lse_val;
+    });
+    if (qi < p.Sq && h == 0 && db0 == 0) {
+        if (p.key_splits > 1) p.part_lse[prow0 + n] = l != l ? l : lse_val;         // a NaN is not an empty slice
+        else if (p.lse) p.lse[(int64_t)bh * p.Sq + qi] = lse_val;
     }
 }
 

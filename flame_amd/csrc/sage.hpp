@@ -679,21 +679,18 @@ __global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel
         }
     }
 
+    // O through LDS where nobody reads any more (KG: the state of the second group this wavefront has joined)
+    if constexpr (KG == 1) __syncthreads();
+    uint16_t* own = reinterpret_cast<uint16_t*>(KG == 1 ? lds8 : lds8_all) + wave * (KG == 1 ? 32 * D : (4 * DB + 1) * 64 * 8);
+    static_assert(NW * 32 * D * 2 <= T::LDS_BYTES, "the rows of O fit where the tiles were");
     const int row = qw0 + n;
     const float l = l_run + xhalf(l_run);
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    if (row < p.Sq) {
-        uint16_t* orow = obase + (int64_t)row * p.os.n;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x16& a = oacc[db];
-                u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
-                if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * g + 4 * h) = w;
-            }
-        if (p.lse && h == 0) p.lse[(int64_t)bh * p.Sq + row] = l > 0.f ? (m_run + log2_fast(l)) * kLn2 : -INFINITY;
-    }
+    store_rows32<D>(own, obase + (int64_t)qw0 * p.os.n, p.os.n, p.Sq - qw0, p.d, [&](int db, int g) {
+        const f32x16& a = oacc[db];
+        return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
+    });
+    if (p.lse && h == 0 && row < p.Sq) p.lse[(int64_t)bh * p.Sq + row] = l > 0.f ? (m_run + log2_fast(l)) * kLn2 : -INFINITY;
 }
 
 
@@ -1087,28 +1084,21 @@ __global__ __launch_bounds__(256) void sage_fwd_wide_kernel(const SageFwdParams 
             step(I3{}, sb, sa, k3, v2, fnext(t + 3));
             advance(t + 3);
         }
-        wait_vm0();          // no copy may land after the workgroup has gone
+        wait_vm0();          // no copy may land where O passes through LDS
     }
 
     // ---- epilogue
+    __syncthreads();
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-        const int row = qrow[qb];
+        const int row = qrow[qb], row0 = qw0 + 32 * qb;
         const float l = l_run[qb] + xhalf(l_run[qb]);
         const float inv = l > 0.f ? 1.0f / l : 0.f;
-        if (row < p.Sq) {
-            uint16_t* orow = obase + (int64_t)row * p.os.n;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const f32x16& a = oacc[qb][db];
-                    u32x2 w = {pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv),
-                               pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
-                    if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(orow + 32 * db + 8 * g + 4 * h) = w;
-                }
-            if (p.lse && h == 0) p.lse[(int64_t)bh * p.Sq + row] = l > 0.f ? (m_run[qb] + log2_fast(l)) * kLn2 : -INFINITY;
-        }
+        store_rows32<D>(reinterpret_cast<uint16_t*>(lds8) + wave * 32 * D, obase + (int64_t)row0 * p.os.n, p.os.n, p.Sq - row0, p.d, [&](int db, int g) {
+            const f32x16& a = oacc[qb][db];
+            return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
+        });
+        if (p.lse && h == 0 && row < p.Sq) p.lse[(int64_t)bh * p.Sq + row] = l > 0.f ? (m_run[qb] + log2_fast(l)) * kLn2 : -INFINITY;
     }
 }
 
