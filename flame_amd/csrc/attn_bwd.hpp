@@ -889,46 +889,6 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         else return t_lo + t;
     };
 
-    // ---- Q and dO fragments (B operands: column = query, 8 consecutive d), per-query scalars
-    const int qrow = qw0 + n;
-    const bool qok = qrow < p.Sq;
-    bf16x8 qf[DC], dof[DC];
-    {
-        const uint16_t* rq = qbase + (int64_t)qrow * p.qs.n + 8 * h;
-        const uint16_t* rd = dobase + (int64_t)qrow * p.dos.n + 8 * h;
-#pragma unroll
-        for (int dc = 0; dc < DC; ++dc) {
-            const bool in_d = qok && 16 * dc + 8 * h < p.d;
-            qf[dc] = __builtin_bit_cast(bf16x8, ldg16(rq + 16 * dc, in_d));
-            dof[dc] = __builtin_bit_cast(bf16x8, ldg16(rd + 16 * dc, in_d));
-        }
-    }
-    // Per-query scalars, formed here and also left in the workspace for the dK/dV kernel that runs next:
-    //   delta = rowsum(dO * O)   (the bf16 O that the forward saved)
-    //   lse2  = LSE * log2(e), +inf for fully excluded rows and rows past the end (P = exp2(s - inf) = 0)
-    float lse2 = INFINITY, delta = 0.f;
-    {
-        const uint16_t* ro = p.o + b * p.os.b + hh * p.os.h + (int64_t)qrow * p.os.n + 8 * h;
-        float part = 0.f;
-#pragma unroll
-        for (int dc = 0; dc < DC; ++dc) {
-            const u32x4 ov = ldg16(ro + 16 * dc, qok && 16 * dc + 8 * h < p.d);
-            const u32x4 dv = __builtin_bit_cast(u32x4, dof[dc]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) part += bf16_lo(dv[i]) * bf16_lo(ov[i]) + bf16_hi(dv[i]) * bf16_hi(ov[i]);
-        }
-        part += xhalf(part);
-        if (qok) {
-            const float l = p.lse[(int64_t)bh * p.Sq + qrow];
-            lse2 = (l == -INFINITY) ? INFINITY : l * kLog2e;
-            delta = part;
-            if (h == 0 && group == 0) {
-                p.ndelta[(int64_t)bh * p.Sq + qrow] = -delta;
-                p.lse2[(int64_t)bh * p.Sq + qrow] = lse2;
-            }
-        }
-    }
-
     const int dma_row_in = lane / GPR, dma_gran = lane % GPR;
     constexpr int NDMA = T::DMA_PER_WAVE * 4 / NW;
     const uint32_t lds0 = lds_addr(lds);
@@ -965,6 +925,43 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         }
     };
 
+    // on its way before anything else is loaded: on short walks a second round trip to memory is a good part of the run time
+    if (n_tiles > 0) issue_tile(0, 0);
+
+    // ---- Q and dO fragments (B operands: column = query, 8 consecutive d), per-query scalars; through stage 1
+    const int qrow = qw0 + n;
+    const bool qok = qrow < p.Sq;
+    bf16x8 qf[DC], dof[DC];
+    // Per-query scalars, formed here and also left in the workspace for the dK/dV kernel that runs next:
+    //   delta = rowsum(dO * O)   (the bf16 O that the forward saved)
+    //   lse2  = LSE * log2(e), +inf for fully excluded rows and rows past the end (P = exp2(s - inf) = 0)
+    float lse2 = INFINITY, delta = 0.f;
+    {
+        uint16_t* const pass = lds + T::STAGE_ELEMS + wave * 1024;
+        u32x4 wq[DC], wd[DC], wo[DC];
+        load_rows32<D>(wq, qbase + (int64_t)qw0 * p.qs.n, p.qs.n, p.Sq - qw0, p.d);
+        load_rows32<D>(wd, dobase + (int64_t)qw0 * p.dos.n, p.dos.n, p.Sq - qw0, p.d);
+        load_rows32<D>(wo, p.o + b * p.os.b + hh * p.os.h + (int64_t)qw0 * p.os.n, p.os.n, p.Sq - qw0, p.d);
+        const float l = qok ? p.lse[(int64_t)bh * p.Sq + qrow] : 0.f;
+        fragments_of_rows32<D>(pass, wq, [&](auto dc, u32x4 f) { qf[decltype(dc)::value] = __builtin_bit_cast(bf16x8, f); });
+        fragments_of_rows32<D>(pass, wd, [&](auto dc, u32x4 f) { dof[decltype(dc)::value] = __builtin_bit_cast(bf16x8, f); });
+        float part = 0.f;
+        fragments_of_rows32<D>(pass, wo, [&](auto dc, u32x4 ov) {
+            const u32x4 dv = __builtin_bit_cast(u32x4, dof[decltype(dc)::value]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part += bf16_lo(dv[i]) * bf16_lo(ov[i]) + bf16_hi(dv[i]) * bf16_hi(ov[i]);
+        });
+        part += xhalf(part);
+        if (qok) {
+            lse2 = (l == -INFINITY) ? INFINITY : l * kLog2e;
+            delta = part;
+            if (h == 0 && group == 0) {
+                p.ndelta[(int64_t)bh * p.Sq + qrow] = -delta;
+                p.lse2[(int64_t)bh * p.Sq + qrow] = lse2;
+            }
+        }
+    }
+
     int koff[DC];          // 16-byte row reads of K / V: row 32*kb + n, logical granule 2*dc + h
 #pragma unroll
     for (int dc = 0; dc < DC; ++dc) koff[dc] = n * RS + (((2 * dc + h) ^ swz<D>(n)) << 3);
@@ -985,7 +982,6 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
 #pragma unroll
         for (int r = 0; r < 16; ++r) dqacc[db][r] = 0.f;
 
-    if (n_tiles > 0) issue_tile(0, 0);
     MaskRow64 mnext;          // keep-mask bytes of this lane's query row for the next tile (vector-load layouts only)
 #pragma unroll
     for (int j = 0; j < 4; ++j) mnext.w[j] = u32x4{0u, 0u, 0u, 0u};
@@ -1290,55 +1286,6 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     if (p.m.causal) kend = min(kend, q0 + BM);
     const int n_tiles = (kend + BN - 1) / BN;
 
-    // ---- Q and dO fragments (B operands: column = query, 8 consecutive d) and the per-query scalars of
-    //      both query blocks; -delta and lse2 are also left in the workspace for the dK/dV kernel
-    bf16x8 qf[2][DC], dof[2][DC];          // pinned to accumulation registers: slots qb*DC + dc and 16 + qb*DC + dc
-    float lse2[2];
-    f32x16 ndelta16[2];
-    int qrow[2];
-    static_for<2>([&](auto qb_tag) {
-        constexpr int qb = decltype(qb_tag)::value;
-        qrow[qb] = qw0 + 32 * qb + n;
-        const bool qok = qrow[qb] < p.Sq;
-        const uint16_t* rq = qbase + (int64_t)qrow[qb] * p.qs.n + 8 * h;
-        const uint16_t* rd = dobase + (int64_t)qrow[qb] * p.dos.n + 8 * h;
-        const uint16_t* ro = p.o + b * p.os.b + hh * p.os.h + (int64_t)qrow[qb] * p.os.n + 8 * h;
-        float part = 0.f;
-        static_for<DC>([&](auto dc_tag) {
-            constexpr int dc = decltype(dc_tag)::value;
-            const bool in_d = qok && 16 * dc + 8 * h < p.d;
-            qf[qb][dc] = pin_b_fragment<qb * DC + dc>(ldg16(rq + 16 * dc, in_d));
-            const u32x4 dv = ldg16(rd + 16 * dc, in_d);
-            dof[qb][dc] = pin_b_fragment<16 + qb * DC + dc>(dv);
-            if (!p.rows_ready) {
-                const u32x4 ov = ldg16(ro + 16 * dc, in_d);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) part += bf16_lo(dv[i]) * bf16_lo(ov[i]) + bf16_hi(dv[i]) * bf16_hi(ov[i]);
-            }
-        });
-        lse2[qb] = INFINITY;
-        float nd = 0.f;
-        if (p.rows_ready) {       // bwd_rows_kernel has left both rows in the workspace
-            if (qok) {
-                nd = p.ndelta[(int64_t)bh * p.Sq + qrow[qb]];
-                lse2[qb] = p.lse2[(int64_t)bh * p.Sq + qrow[qb]];
-            }
-        } else {
-            part += xhalf(part);
-            if (qok) {
-                const float l = p.lse[(int64_t)bh * p.Sq + qrow[qb]];
-                lse2[qb] = (l == -INFINITY) ? INFINITY : l * kLog2e;
-                nd = -part;
-                if (h == 0) {
-                    p.ndelta[(int64_t)bh * p.Sq + qrow[qb]] = nd;
-                    p.lse2[(int64_t)bh * p.Sq + qrow[qb]] = lse2[qb];
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) ndelta16[qb][r] = nd;
-    });
-
     // ---- asynchronous staging of the K / V tiles
     const int dma_row_in = lane / GPR, dma_gran = lane % GPR;
     const uint32_t lds0 = lds_addr(lds);
@@ -1363,6 +1310,63 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
             dma16(vbase + (int64_t)key * p.vs.n + c * 8, dst_of(stg, 1, i));
         }
     };
+
+    if (n_tiles > 0) issue_tile(0, 0);
+
+    // ---- Q and dO fragments (B operands: column = query, 8 consecutive d) and the per-query scalars of
+    //      both query blocks, through stage 2; -delta and lse2 are also left in the workspace for the dK/dV kernel
+    bf16x8 qf[2][DC], dof[2][DC];          // pinned to accumulation registers: slots qb*DC + dc and 16 + qb*DC + dc
+    float lse2[2];
+    f32x16 ndelta16[2];
+    int qrow[2];
+    static_for<2>([&](auto qb_tag) {
+        constexpr int qb = decltype(qb_tag)::value;
+        const int row0 = qw0 + 32 * qb;
+        qrow[qb] = row0 + n;
+        const bool qok = qrow[qb] < p.Sq;
+        uint16_t* const pass = lds + 2 * T::STAGE_ELEMS + wave * 1024;
+        u32x4 wq[DC], wd[DC], wo[DC];
+        load_rows32<D>(wq, qbase + (int64_t)row0 * p.qs.n, p.qs.n, p.Sq - row0, p.d);
+        load_rows32<D>(wd, dobase + (int64_t)row0 * p.dos.n, p.dos.n, p.Sq - row0, p.d);
+        if (!p.rows_ready) load_rows32<D>(wo, p.o + b * p.os.b + hh * p.os.h + (int64_t)row0 * p.os.n, p.os.n, p.Sq - row0, p.d);
+        fragments_of_rows32<D>(pass, wq, [&](auto dc_tag, u32x4 f) {
+            constexpr int dc = decltype(dc_tag)::value;
+            qf[qb][dc] = pin_b_fragment<qb * DC + dc>(f);
+        });
+        u32x4 dvf[DC];
+        fragments_of_rows32<D>(pass, wd, [&](auto dc_tag, u32x4 f) {
+            constexpr int dc = decltype(dc_tag)::value;
+            dvf[dc] = f;
+            dof[qb][dc] = pin_b_fragment<16 + qb * DC + dc>(f);
+        });
+        lse2[qb] = INFINITY;
+        float nd = 0.f;
+        if (p.rows_ready) {       // bwd_rows_kernel has left both rows in the workspace
+            if (qok) {
+                nd = p.ndelta[(int64_t)bh * p.Sq + qrow[qb]];
+                lse2[qb] = p.lse2[(int64_t)bh * p.Sq + qrow[qb]];
+            }
+        } else {
+            float part = 0.f;
+            fragments_of_rows32<D>(pass, wo, [&](auto dc_tag, u32x4 ov) {
+                const u32x4 dv = dvf[decltype(dc_tag)::value];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) part += bf16_lo(dv[i]) * bf16_lo(ov[i]) + bf16_hi(dv[i]) * bf16_hi(ov[i]);
+            });
+            part += xhalf(part);
+            if (qok) {
+                const float l = p.lse[(int64_t)bh * p.Sq + qrow[qb]];
+                lse2[qb] = (l == -INFINITY) ? INFINITY : l * kLog2e;
+                nd = -part;
+                if (h == 0) {
+                    p.ndelta[(int64_t)bh * p.Sq + qrow[qb]] = nd;
+                    p.lse2[(int64_t)bh * p.Sq + qrow[qb]] = lse2[qb];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ndelta16[qb][r] = nd;
+    });
 
     int koff[DC];          // 16-byte row reads of K / V: row 32*kb + n, logical granule 2*dc + h
 #pragma unroll
@@ -1406,7 +1410,6 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     };
     bf16x8 fb[PD];
     if (n_tiles > 0) {
-        issue_tile(0, 0);
         wait_vm0();
         __syncthreads();
 #pragma unroll

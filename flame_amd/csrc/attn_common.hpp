@@ -430,6 +430,38 @@ __device__ __forceinline__ void store_rows32_f32(float* own, float* out, int64_t
     }
 }
 
+// The way in: 32 rows of a wavefront as MFMA fragments (lane: row n, 8 consecutive columns from 16 dc + 8 h on).  Loaded by the
+// lanes that hold them, an instruction touches 32 rows, 32 bytes of each, at 64 clocks of the address unit; here four
+// neighbouring lanes load 64 bytes of a row (16 clocks), and the rows pass through LDS, 32 columns at a time, two granules
+// swizzled so that neither side has bank conflicts.  All loads first (load_rows32), then the way through LDS
+// (fragments_of_rows32), so that several tensors can be in flight together.
+// Rows at and past `rows` and columns at and past `d` (a multiple of 8) are zero.
+template <int D>
+__device__ __forceinline__ void load_rows32(u32x4 (&w)[D / 16], const uint16_t* base, int64_t row_stride, int rows, int d) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) {
+        const int row = 16 * (i & 1) + (lane >> 2), col = 32 * (i >> 1) + 8 * (lane & 3);
+        w[i] = ldg16(base + row * row_stride + col, row < rows && col < d);
+    }
+}
+// own: 2 KiB of LDS that only this wavefront touches; take(dc, 16 bytes) for every dc < D / 16, given as a constant
+template <int D, class F>
+__device__ __forceinline__ void fragments_of_rows32(uint16_t* own, const u32x4 (&w)[D / 16], F&& take) {
+    const int lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5, row = lane >> 2;
+    uint16_t* const to = own + row * 32 + (((lane & 3) ^ ((row >> 2) & 3)) << 3);        // row + 16 has the same swizzle
+    const uint16_t* const from = own + n * 32;
+    static_for<D / 32>([&](auto c_tag) {
+        constexpr int c = decltype(c_tag)::value;
+        *reinterpret_cast<u32x4*>(to) = w[2 * c];
+        *reinterpret_cast<u32x4*>(to + 16 * 32) = w[2 * c + 1];
+        static_for<2>([&](auto u_tag) {
+            constexpr int u = decltype(u_tag)::value;
+            take(std::integral_constant<int, 2 * c + u>{}, *reinterpret_cast<const u32x4*>(from + (((2 * u + h) ^ ((n >> 2) & 3)) << 3)));
+        });
+    });
+}
+
 // Head dims below the compiled one (any multiple of 8, e.g. 96 on the 128-wide kernels) run zero-padded:
 // fragments loaded straight from global memory are zero past the real head dim, tile copies re-read
 // granule 0 of their row there (finite values that only ever meet those zero operands, or land in

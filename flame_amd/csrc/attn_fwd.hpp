@@ -181,19 +181,25 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         }
     };
     // the first tiles are on their way before anything else is loaded: on short walks their round trip is the run time
+    // (a K tile whose place Q passes through follows when it has)
+    constexpr bool K1_LATE = NW * 2048 > T::TILE_ELEMS * 2;
 #pragma unroll
     for (int i = 0; i < KD; ++i) {
-        if (i < n_tiles) issue_k(i);
+        if (i < n_tiles && !(K1_LATE && i == 1)) issue_k(i);
         if (i < VD && i < n_tiles) issue_v(i);
     }
 
-    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d
+    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d; through the place of V(1)
     bf16x8 qf[DC];
     {
-        const bool ok = qi < p.Sq;
-        const uint16_t* rp = qbase + (int64_t)qi * p.qs.n + 8 * h;
-#pragma unroll
-        for (int dc = 0; dc < DC; ++dc) qf[dc] = __builtin_bit_cast(bf16x8, ldg16(rp + 16 * dc, ok && 16 * dc + 8 * h < p.d));
+        u32x4 w[DC];
+        load_rows32<D>(w, qbase + (int64_t)qw0 * p.qs.n, p.qs.n, p.Sq - qw0, p.d);
+        fragments_of_rows32<D>(lds + T::STAGE_ELEMS + (K1_LATE ? 0 : T::TILE_ELEMS) + wave * 1024, w,
+                               [&](auto dc, u32x4 f) { qf[decltype(dc)::value] = __builtin_bit_cast(bf16x8, f); });
+    }
+    if constexpr (K1_LATE) {
+        __syncthreads();
+        if (1 < n_tiles) issue_k(1);
     }
 
     // ---- per-lane LDS read offsets (elements), constant over the key loop
@@ -678,20 +684,6 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
 
     const int n_tiles = p.Sk / BN;          // the launcher guarantees Sk % BN == 0 and no exclusions
 
-    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d; pinned slots qb*DC + dc
-    bf16x8 qf[2][DC];
-    int qrow[2];
-    static_for<2>([&](auto qb_tag) {
-        constexpr int qb = decltype(qb_tag)::value;
-        qrow[qb] = qw0 + 32 * qb + n;
-        const bool ok = qrow[qb] < p.Sq;
-        const uint16_t* rp = qbase + (int64_t)qrow[qb] * p.qs.n + 8 * h;
-        static_for<DC>([&](auto dc_tag) {
-            constexpr int dc = decltype(dc_tag)::value;
-            qf[qb][dc] = pin_b_fragment<qb * DC + dc>(ldg16(rp + 16 * dc, ok && 16 * dc + 8 * h < p.d));
-        });
-    });
-
     // ---- asynchronous tile copies: tile t (K and V) lives in stage t % 4
     const uint32_t lds0 = lds_addr(lds);
     const int dma_row_in = lane / GPR, dma_gran = lane % GPR;
@@ -712,6 +704,27 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) dma16u(tb, lane_off[i], dst_of(t & 3, which, i));
     };
+    // K(0) and Q first: the logits of the first tile need no more
+    if (n_tiles > 0) issue_whole(kbase, p.ks.n, k_lane_off, 0, 0);
+
+    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d; pinned slots qb*DC + dc; through stage 3
+    bf16x8 qf[2][DC];
+    int qrow[2];
+    {
+        u32x4 w[2][DC];
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            qrow[qb] = qw0 + 32 * qb + n;
+            load_rows32<D>(w[qb], qbase + (int64_t)(qw0 + 32 * qb) * p.qs.n, p.qs.n, p.Sq - qw0 - 32 * qb, p.d);
+        }
+        static_for<2>([&](auto qb_tag) {
+            constexpr int qb = decltype(qb_tag)::value;
+            fragments_of_rows32<D>(lds + 3 * T::STAGE_ELEMS + wave * 1024, w[qb], [&](auto dc_tag, u32x4 f) {
+                constexpr int dc = decltype(dc_tag)::value;
+                qf[qb][dc] = pin_b_fragment<qb * DC + dc>(f);
+            });
+        });
+    }
 
     // ---- per-lane LDS read offsets (elements), constant over the key loop
     int koff[DC];
@@ -958,17 +971,18 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
 
     f32x16 sa[2][2], sb[2][2];
     if (n_tiles > 0) {
-        // prologue: K(0..2) and V(0..1) land; logits and maximum of tile 0; the ring starts on K(1)
-        issue_whole(kbase, p.ks.n, k_lane_off, 0, 0);
-        issue_whole(kbase, p.ks.n, k_lane_off, 1, 0);
-        issue_whole(kbase, p.ks.n, k_lane_off, 2, 0);
-        issue_whole(vbase, p.vs.n, v_lane_off, 0, 1);
-        issue_whole(vbase, p.vs.n, v_lane_off, 1, 1);
+        // prologue: logits and maximum of tile 0 while K(1..2) and V(0..1) are on their way; the ring starts on K(1)
         wait_vm0();
-        __syncthreads();
+        issue_whole(kbase, p.ks.n, k_lane_off, 1, 0);
+        issue_whole(vbase, p.vs.n, v_lane_off, 0, 1);
+        issue_whole(kbase, p.ks.n, k_lane_off, 2, 0);
+        issue_whole(vbase, p.vs.n, v_lane_off, 1, 1);
+        asm volatile("s_barrier" ::: "memory");        // K(0) has landed for every wave
         logits_plain(sa, lds);
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) first_max(qb, tile_max(sa[qb]));
+        wait_vm0();
+        __syncthreads();
 #pragma unroll
         for (int i = 0; i < PD; ++i) fb[i] = k_frag(lds + T::STAGE_ELEMS, i);
 

@@ -88,9 +88,9 @@ __global__ __launch_bounds__(256) void fwd_keyshare_kernel(const FwdParams p) {
     // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d
     bf16x8 qf[DC];
     {
-        const uint16_t* rp = qbase + (int64_t)qi * p.qs.n + 8 * h;
-#pragma unroll
-        for (int dc = 0; dc < DC; ++dc) qf[dc] = __builtin_bit_cast(bf16x8, ldg16(rp + 16 * dc, qi < p.Sq && 16 * dc + 8 * h < p.d));
+        u32x4 w[DC];
+        load_rows32<D>(w, qbase + (int64_t)q0 * p.qs.n, p.qs.n, p.Sq - q0, p.d);
+        fragments_of_rows32<D>(own, w, [&](auto dc, u32x4 f) { qf[decltype(dc)::value] = __builtin_bit_cast(bf16x8, f); });
     }
     // before the first copies: the compiler's wait for these loads must not become one for the copies behind them
 #pragma unroll
