@@ -52,13 +52,14 @@ struct FwdTile {
     static constexpr int TILE_ELEMS = BN * D;       // one K or V tile
     static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;
     static constexpr int LDS_BYTES = 2 * STAGE_ELEMS * 2;
+    static constexpr int BIAS_PASS_BYTES = 4 * 2048;             // behind the stages: 2 KiB per wavefront that bias rows pass through
     static constexpr int ROWS_PER_DMA = 1024 / (D * 2);          // rows covered by one 64-lane x 16-byte copy
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;   // copies per wave and tensor
 };
 
-// four consecutive bias values, at any element's address
+// 16 bytes of a bias row, at any element's address
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint16_t u16x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint16_t u16x8_any __attribute__((ext_vector_type(8), aligned(2)));
 
 // DROP (DropMode): the probabilities that multiply V are dropped element by element (drop_factor) and O is rescaled; the
 // row sums, and with them the log-sum-exp, stay those of the undropped softmax.
@@ -98,6 +99,12 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
     if (EXCL == kExKeys || p.m.kv_len) bh = longest_batches_first<EXCL == kExKeys>(bh, p.B, p.H, p.Sk, p.m);
+    // a bias that all batches share: its rows are read by the batches' workgroups one after the other on one XCD, from its L2
+    if ((EXCL == kExBiasF32 || EXCL == kExBiasBf16) && p.m.bb == 0) {
+        const int rest = wg / p.B;
+        qt = rest % n_qt;
+        bh = (wg % p.B) * p.H + rest / n_qt;
+    }
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 32;
@@ -266,28 +273,56 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             if (__any(limit < BN)) mrow.restrict_to(limit);
         }
     };
-    // Bias: every lane needs 64 (of its half: 32) consecutive values of its query's row, four at a time, so a group of four
-    // is one 16-byte (bf16: 8-byte) load; group j of the next tile is requested at the j-th eighth of the logit phase, when
-    // the exponentials have freed the registers it takes, and added in the j-th eighth of the PV phase.
-    // (B=1 H=64 S=512 D=64, fp32: one load per element 62 us, this 24 us; 84 MB move, 18 us at the rate of a copy.)
-    using BiasGroup = typename std::conditional<EXCL == kExBiasF32, f32x4_any, u16x4_any>::type;
+    // Bias: every lane needs 64 (of its half: 32) consecutive values of its query's row.  Four neighbouring lanes load 64 bytes
+    // of a row (a "piece" is 16 rows of that, one instruction), and two pieces, 32 rows, at a time pass through 2 KiB of LDS
+    // to the lanes that own the rows, granules swizzled as in fragments_of_rows32: an instruction whose lanes each load from
+    // a row of their own keeps the address unit busy for 64 clocks instead of 16.  The pieces of the next tile are requested
+    // across the logit phase, when the exponentials have freed the registers they take; a pair of them goes through LDS in
+    // the PV phase, one ahead of the slices that add it.
+    // (B=1 H=64 S=512 D=64, fp32: 84 MB move, 16 us at the rate of a copy; four values per lane and load 23.5 us, this 19.4.
+    // B=3 H=16 S=1664 fp32: D = 64 123 -> 82 us, D = 128 166 -> 150 us; its two wavefronts per SIMD wait for the bias then.)
+    using BiasPiece = typename std::conditional<EXCL == kExBiasF32, f32x4_any, u16x8_any>::type;
     using BiasElem = typename std::conditional<EXCL == kExBiasF32, float, uint16_t>::type;
-    BiasGroup bg[BIAS ? 8 : 1];
-    const BiasElem* brow = nullptr;
-    if constexpr (BIAS)
-        brow = static_cast<const BiasElem*>(p.m.bias) + b * p.m.bb + hh * p.m.bh + (int64_t)min(qi, p.Sq - 1) * p.m.bq + 4 * h;
-    auto bias_request = [&](auto ragged_tag, int t, int j) {
-        if constexpr (BIAS) {
-            const int key = t * BN + 8 * j;          // of half 0
-            if constexpr (!decltype(ragged_tag)::value) {
-                bg[j] = *reinterpret_cast<const BiasGroup*>(brow + key);
-            } else {                                 // ragged tail: nothing past the row is read, keys past the end get -inf
-                const int last = p.Sk - 1 - 4 * h;
+    constexpr int BEL = EXCL == kExBiasF32 ? 4 : 8;           // values per piece and lane
+    constexpr int NPIECE = BIAS ? 32 / BEL : 1, NPASS = NPIECE / 2;
+    BiasPiece bw[NPIECE];
+    f32x4 bg[EXCL == kExBiasF32 ? 8 : 1];                     // keys 8 j + 4 h .. + 3 of this lane's row
+    u32x2 bgh[EXCL == kExBiasBf16 ? 8 : 1];
+    // the wavefront's first row, and this lane's place (bytes) in rows lane / 4 and lane / 4 + 16 (row pitches below 2^24 elements)
+    const BiasElem* const brow0 = BIAS ? static_cast<const BiasElem*>(p.m.bias) + b * p.m.bb + hh * p.m.bh + (int64_t)min(qw0, p.Sq - 1) * p.m.bq : nullptr;
+    uint32_t boff[2];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const BiasElem v = brow[min(key + e, last)];
-                    bg[j][e] = key + e > last ? (EXCL == kExBiasF32 ? (BiasElem)-INFINITY : (BiasElem)0xff80u) : v;
+    for (int u = 0; u < 2; ++u)
+        boff[u] = (uint32_t)sizeof(BiasElem) * (uint32_t)(min(16 * u + (lane >> 2), max(p.Sq - 1 - qw0, 0)) * (int)p.m.bq + BEL * (lane & 3));
+    uint16_t* const bpass = lds + T::LDS_BYTES / 2 + wave * 1024;
+    const int bto = (lane >> 2) * 32 + (((lane & 3) ^ ((lane >> 4) & 3)) << 3);
+    const int bfrom = n * 32 + (EXCL == kExBiasF32 ? (h ^ ((n >> 2) & 3)) << 3 : (((n >> 2) & 3) << 3) + 4 * h);
+    auto bias_request = [&](auto ragged_tag, int t, int i) {
+        if constexpr (BIAS) {
+            const int key = t * BN + 4 * BEL * (i >> 1);             // of lanes with lane % 4 == 0
+            if constexpr (!decltype(ragged_tag)::value) {
+                bw[i] = *reinterpret_cast<const BiasPiece*>(reinterpret_cast<const char*>(brow0 + key) + boff[i & 1]);
+            } else {                                 // ragged tail: nothing past the row is read, keys past the end get -inf
+                const BiasElem* row = reinterpret_cast<const BiasElem*>(reinterpret_cast<const char*>(brow0) + boff[i & 1]);
+                const int last = p.Sk - 1 - BEL * (lane & 3);
+#pragma unroll
+                for (int e = 0; e < BEL; ++e) {
+                    const BiasElem v = row[min(key + e, last)];
+                    bw[i][e] = key + e > last ? (EXCL == kExBiasF32 ? (BiasElem)-INFINITY : (BiasElem)0xff80u) : v;
                 }
+            }
+        }
+    };
+    auto bias_pass = [&](int c) {                    // pieces 2 c and 2 c + 1 to the rows' lanes
+        if constexpr (BIAS) {
+            *reinterpret_cast<u32x4*>(bpass + bto) = __builtin_bit_cast(u32x4, bw[2 * c]);
+            *reinterpret_cast<u32x4*>(bpass + bto + 16 * 32) = __builtin_bit_cast(u32x4, bw[2 * c + 1]);
+            if constexpr (EXCL == kExBiasF32) {      // granule 2 u + h
+#pragma unroll
+                for (int u = 0; u < 2; ++u) bg[2 * c + u] = *reinterpret_cast<const f32x4*>(bpass + (bfrom ^ (16 * u)));
+            } else {                                 // half h of granule u
+#pragma unroll
+                for (int u = 0; u < 4; ++u) bgh[4 * c + u] = *reinterpret_cast<const u32x2*>(bpass + (bfrom ^ (8 * u)));
             }
         }
     };
@@ -296,7 +331,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         if constexpr (BIAS) {     // scale * (s + bias / scale) = scale * s + bias
             float v;
             if constexpr (EXCL == kExBiasF32) v = bg[idx >> 2][idx & 3];
-            else v = __uint_as_float((uint32_t)bg[idx >> 2][idx & 3] << 16);
+            else v = idx & 1 ? bf16_hi(bgh[idx >> 2][(idx >> 1) & 1]) : bf16_lo(bgh[idx >> 2][(idx >> 1) & 1]);
             s[kb][r] = fmaf(v, p.m.inv_scale, s[kb][r]);
         }
         if constexpr (KEYS) s[kb][r] = keep_bits[kb] & (1u << (8 * (r >> 2) + (r & 3))) ? s[kb][r] : -INFINITY;
@@ -431,11 +466,11 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             for (int i = 0; i < NS; i += 2) {
                 nxt[1] = mfma32(fb[(i + 1) % PD], qf[i >> 1], nxt[1]);
                 exp_slice(i);
-                if (BIAS && i % (NS / 8) == 0) bias_request(ragged_tag, t + 1, i / (NS / 8));
+                if (BIAS && i % (NS / NPIECE) == 0) bias_request(ragged_tag, t + 1, i / (NS / NPIECE));
                 __builtin_amdgcn_sched_barrier(0);
                 nxt[0] = mfma32(fb[i % PD], qf[i >> 1], nxt[0]);
                 exp_slice(i + 1);
-                if (BIAS && (i + 1) % (NS / 8) == 0) bias_request(ragged_tag, t + 1, (i + 1) / (NS / 8));
+                if (BIAS && (i + 1) % (NS / NPIECE) == 0) bias_request(ragged_tag, t + 1, (i + 1) / (NS / NPIECE));
                 fb[i % PD] = frag_of(i + PD);
                 fb[(i + 1) % PD] = frag_of(i + 1 + PD);
                 __builtin_amdgcn_sched_barrier(0);
@@ -444,7 +479,9 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             if (NEXT == 1 && EXCL == kExGeneral) excl_general(nxt, t + 1);
             // ---- O^T += V(t)^T P(t)^T between the row-maximum scan of tile t+1
             float tmax = -INFINITY;
+            if constexpr (BIAS) bias_pass(0);
             auto max_slice = [&](int i) {
+                if (BIAS && i % (NP / NPASS) == 0 && i / (NP / NPASS) + 1 < NPASS) bias_pass(i / (NP / NPASS) + 1);
 #pragma unroll
                 for (int e = 0; e < MPS; e += 2) {
                     const int idx = MPS * i + e;
@@ -485,14 +522,24 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         wait_vm0();
         __syncthreads();
         if (t_clean == 0) excl_begin(0);
-        if constexpr (BIAS)
+        if constexpr (BIAS) {
+            if (t_clean > 0) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bias_request(std::true_type{}, 0, j);
+                for (int i = 0; i < NPIECE; ++i) bias_request(std::false_type{}, 0, i);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NPIECE; ++i) bias_request(std::true_type{}, 0, i);
+            }
+        }
         zero_tile(sa);
 #pragma unroll
         for (int i = 0; i < NS; ++i) sa[i & 1] = mfma32(k_frag(0, i), qf[i >> 1], sa[i & 1]);
         if (t_clean == 0 || BIAS) {
             if (EXCL == kExGeneral) excl_general(sa, 0);
+            if constexpr (BIAS) {
+#pragma unroll
+                for (int c = 0; c < NPASS; ++c) bias_pass(c);
+            }
 #pragma unroll
             for (int idx = 0; idx < 32; ++idx) excl_elem(sa, idx);
         }

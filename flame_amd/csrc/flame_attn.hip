@@ -160,8 +160,9 @@ int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_kernel<D, EXCL, NW, DROP, KG>;
     constexpr bool KEYS = EXCL == kExKeys;
-    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), KG * T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
-    const int lds = KG * T::LDS_BYTES + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
+    constexpr int tiles = KG * T::LDS_BYTES + (EXCL == kExBiasF32 || EXCL == kExBiasBf16 ? T::BIAS_PASS_BYTES : 0);
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern), tiles + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
+    const int lds = tiles + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW * KG), lds, s, p);
@@ -1057,8 +1058,8 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel
     if (keep_mask != nullptr && bias == nullptr && p.m.rows16 && N_kv % 64 == 0)
         return DP == 128 ? launch_fwd<128, kExRows16, 4>(p, s) : launch_fwd<64, kExRows16, 4>(p, s);
-    // a bias alone, its rows contiguous: loaded in fours
-    if (bias != nullptr && keep_mask == nullptr && !causal && kv_len == nullptr && p.m.bk == 1) {
+    // a bias alone, its rows contiguous (and a wavefront's 32 rows within 32-bit byte offsets): loaded in pieces of 16 bytes
+    if (bias != nullptr && keep_mask == nullptr && !causal && kv_len == nullptr && p.m.bk == 1 && p.m.bq >= 0 && p.m.bq < (1 << 24)) {
         if (p.m.bias_f32) return DP == 128 ? launch_fwd<128, kExBiasF32, 4>(p, s) : launch_fwd<64, kExBiasF32, 4>(p, s);
         return DP == 128 ? launch_fwd<128, kExBiasBf16, 4>(p, s) : launch_fwd<64, kExBiasBf16, 4>(p, s);
     }
