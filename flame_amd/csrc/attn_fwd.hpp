@@ -188,11 +188,10 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         }
     };
     // the first tiles are on their way before anything else is loaded: on short walks their round trip is the run time
-    // (a K tile whose place Q passes through follows when it has)
-    constexpr bool K1_LATE = NW * 2048 > T::TILE_ELEMS * 2;
+    static_assert(NW * 2048 <= T::TILE_ELEMS * 2, "Q passes through the place of a V tile");
 #pragma unroll
     for (int i = 0; i < KD; ++i) {
-        if (i < n_tiles && !(K1_LATE && i == 1)) issue_k(i);
+        if (i < n_tiles) issue_k(i);
         if (i < VD && i < n_tiles) issue_v(i);
     }
 
@@ -201,12 +200,8 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     {
         u32x4 w[DC];
         load_rows32<D>(w, qbase + (int64_t)qw0 * p.qs.n, p.qs.n, p.Sq - qw0, p.d);
-        fragments_of_rows32<D>(lds + T::STAGE_ELEMS + (K1_LATE ? 0 : T::TILE_ELEMS) + wave * 1024, w,
+        fragments_of_rows32<D>(lds + T::STAGE_ELEMS + T::TILE_ELEMS + wave * 1024, w,
                                [&](auto dc, u32x4 f) { qf[decltype(dc)::value] = __builtin_bit_cast(bf16x8, f); });
-    }
-    if constexpr (K1_LATE) {
-        __syncthreads();
-        if (1 < n_tiles) issue_k(1);
     }
 
     // ---- per-lane LDS read offsets (elements), constant over the key loop
@@ -284,7 +279,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     using BiasPiece = typename std::conditional<EXCL == kExBiasF32, f32x4_any, u16x8_any>::type;
     using BiasElem = typename std::conditional<EXCL == kExBiasF32, float, uint16_t>::type;
     constexpr int BEL = EXCL == kExBiasF32 ? 4 : 8;           // values per piece and lane
-    constexpr int NPIECE = BIAS ? 32 / BEL : 1, NPASS = NPIECE / 2;
+    constexpr int NPIECE = BIAS ? 32 / BEL : 1, NPASS = BIAS ? NPIECE / 2 : 1;
     BiasPiece bw[NPIECE];
     f32x4 bg[EXCL == kExBiasF32 ? 8 : 1];                     // keys 8 j + 4 h .. + 3 of this lane's row
     u32x2 bgh[EXCL == kExBiasBf16 ? 8 : 1];

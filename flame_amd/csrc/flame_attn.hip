@@ -287,9 +287,15 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     // 256-query workgroups (4 wavefronts of 64 queries) when they neither add padding rows nor leave compute units idle
     const int64_t n256 = (p.Sq + 255) / 256;
     // (with key lengths the walks differ in length and the longest ones set the time: unless the units fill two
-    // rounds, twice as many workgroups of half the size finish sooner)
-    const bool wide = !HASMASK && !p.key_mask && n256 * 256 <= ((int64_t)(p.Sq + 127) / 128) * 128 && n256 * p.B * p.H >= device_cu_count() &&
-                      !(p.m.kv_len && n256 * p.B * p.H < 2 * device_cu_count()) && wg_waves_override() != 4;
+    // rounds, twice as many workgroups of half the size finish sooner; so they do where the last round of the large ones is
+    // thin and cannot be cut, and on short walks unless every round is full: thin_last_round)
+    const int64_t total256 = n256 * p.B * p.H;
+    const bool even = !p.m.causal && !p.m.kv_len;           // all walks equally long
+    const bool wide_fits = !HASMASK && !p.key_mask && n256 * 256 <= ((int64_t)(p.Sq + 127) / 128) * 128 && total256 >= device_cu_count() &&
+                           !(p.m.kv_len && total256 < 2 * device_cu_count()) && wg_waves_override() != 4;
+    const bool wide = wide_fits && (bwd_schedule_override() != 0 ||      // (a schedule asked for by name has 256-query workgroups)
+                                    (!(thin_last_round(total256, device_cu_count(), 2) && (!even || total256 < 2 * device_cu_count())) &&
+                                     !(p.Sk <= 1024 && total256 % device_cu_count() != 0)));
     const int64_t n_qt = wide ? n256 : (p.Sq + TQ::BM - 1) / TQ::BM;
     const int64_t grid_dq = n_qt * p.B * p.H;
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
@@ -352,8 +358,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         if (wide) {
             // a last round on at most half of the compute units: 128-query workgroups in a launch of their own (problems
             // whose walks are all equally long)
-            const bool even = !p.m.causal && !p.m.kv_len && 2 * grid_dq <= 0x7fffffff;
-            const LastRound r = even ? cut_last_round(p.Sq, (int64_t)p.B * p.H, device_cu_count(), false) : LastRound{grid_dq};
+            const LastRound r = even && 2 * grid_dq <= 0x7fffffff ? cut_last_round(p.Sq, (int64_t)p.B * p.H, device_cu_count(), false) : LastRound{grid_dq};
             hipLaunchKernelGGL(kern_dqw, dim3((unsigned)r.wide), dim3(256), TW::LDS_BYTES, s, p);
             if (r.count) {
                 BwdParams pt = p;
@@ -1049,9 +1054,15 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     // a plan (128 or 256 query rows per workgroup) overrides the rule where the kernels leave the choice open
     if (q_tile_plan == 128) wide = false;
     else if (q_tile_plan == 256 && !hm) wide = true;
-    // ... as 4 wavefronts of 64 queries when nothing is excluded at all, else as 8 wavefronts of 32
+    // ... as 4 wavefronts of 64 queries when nothing is excluded at all, else as 8 wavefronts of 32 (D = 128 only)
     const bool plain = !causal && kv_len == nullptr && N_kv % 64 == 0;
     const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
+    if (wide && !plain && DP == 64) wide = false;
+    if (wide && q_tile_plan == 0) {
+        const int64_t total256 = (int64_t)((N_q + 255) / 256) * B * H, cus = device_cu_count();
+        // (without exclusions a last round on an eighth of the units is cut into 32-query workgroups, launch_fwd_wide)
+        wide = !thin_last_round(total256, cus, 3) || (plain && (total256 >= 2 * cus || thin_last_round(total256, cus, 8)));
+    }
     // a keep-mask of keys: the walk takes the attended tiles only (up to what their list holds)
     if (keep_mask != nullptr && bias == nullptr && keys_only(p.m, N_q, N_kv))
         return DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
@@ -1066,7 +1077,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     if (hm) return DP == 128 ? launch_fwd<128, kExGeneral, 4>(p, s) : launch_fwd<64, kExGeneral, 4>(p, s);
     if (wide) {
         if (plain) return DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
-        return DP == 128 ? launch_fwd<128, kExNone, 8>(p, s) : launch_fwd<64, kExNone, 8>(p, s);
+        return launch_fwd<128, kExNone, 8>(p, s);
     }
     if (q_tile_plan == 0 && fwd_rule_keyshare((int64_t)B * H, N_q)) {
         const int64_t rows = (int64_t)B * H * N_q;
