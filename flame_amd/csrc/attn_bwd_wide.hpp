@@ -81,6 +81,78 @@ struct WideRing {
     }
 };
 
+// Copies of a unit of 128 rows x 64 elements of the head dim: 16 of 8 rows x 128 bytes, four per wavefront; copy i: rows
+// 8 (4 wave + i) + lane / 8.  The swizzle of copies 0 and 2, and of 1 and 3, is the same, so two lane offsets per tensor do
+// where all 128 rows exist.
+struct WideRows {
+    int row0, gran0, gran1;
+    uint32_t lds0;
+    __device__ __forceinline__ explicit WideRows(const uint16_t* lds) {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+        row0 = 32 * wave + (lane >> 3);
+        gran0 = (lane & 7) ^ swz<64>(row0);
+        gran1 = (lane & 7) ^ swz<64>(row0 + 8);
+        lds0 = lds_addr(lds) + 4096u * (uint32_t)wave;
+    }
+    static_assert(swz<64>(0) == swz<64>(16) && swz<64>(8) == swz<64>(24) && swz<64>(7) == swz<64>(23), "the swizzle repeats every 16 rows");
+    // copy i (0 .. 3) of elements [64 t, 64 t + 64) of the rows from base on, `rows` of which exist, d the head dim
+    __device__ __forceinline__ void issue(const uint16_t* base, int64_t stride, int rows, int d, int t, int slot, int i) const {
+        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS) + 1024u * (uint32_t)i;
+        const uint16_t* src = base + kWideStep * t;
+        const int g = i & 1 ? gran1 : gran0;
+        if (kWideStep * (t + 1) <= d && rows >= kWideTile)
+            dma16u(src + 8 * i * stride, 2u * (uint32_t)(row0 * (int)stride + 8 * g), dst);
+        else                                               // rows past the end re-read the last one; granules past the head dim:
+            dma16u(src, 2u * (uint32_t)(min(row0 + 8 * i, max(rows - 1, 0)) * (int)stride + (kWideStep * t + 8 * g < d ? 8 * g : 0)), dst);     // filler, zeroed in the fragments
+    }
+    __device__ __forceinline__ void issue(const uint16_t* base, int64_t stride, int rows, int d, int t, int slot) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) issue(base, stride, rows, d, t, slot, i);
+    }
+};
+
+// One phase: the eight copies it requests, copy(i), then acc += A B^T over its unit pair, four chunks of 16 contraction elements;
+// a(c, u) and b(c, u) read the fragments of chunk c.  (Copies spread out between the MFMAs, and fragments read a chunk ahead
+// in an order fixed by hand, were slower, 80 -> 91 us for a forward: the requests have to leave early.)
+template <class A, class B, class Copy>
+__device__ __forceinline__ void wide_phase(f32x16 (&acc)[2][2], A&& a, B&& b, Copy&& copy) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) copy(i);
+#pragma unroll
+    for (int c = 0; c < kWideStep / 16; ++c) {
+        bf16x8 af[2], bf[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            af[u] = a(c, u);
+            bf[u] = b(c, u);
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[x][y] = mfma32(af[x], bf[y], acc[x][y]);
+    }
+}
+// The last step of a contraction over the head dim where `rest` < 64 elements are left, from tiles of rows: fragments at row
+// offsets fa / fb (row, granule 2 c + h: the chunk only flips bits 4 and 5 of the offset).
+__device__ __forceinline__ void wide_multiply_tail(f32x16 (&acc)[2][2], const uint16_t* a, const uint16_t* b, const int (&fa)[2], const int (&fb)[2], int rest) {
+    const int h = (threadIdx.x & 63) >> 5;
+#pragma unroll
+    for (int c = 0; c < kWideStep / 16; ++c) {
+        if (16 * c >= rest) break;
+        bf16x8 af[2], bf[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            af[u] = *reinterpret_cast<const bf16x8*>(a + (fa[u] ^ (16 * c)));
+            bf[u] = *reinterpret_cast<const bf16x8*>(b + (fb[u] ^ (16 * c)));
+            if (16 * c + 8 * h >= rest) af[u] = bf[u] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});   // both: a filler must not meet a zero as an infinity
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[x][y] = mfma32(af[x], bf[y], acc[x][y]);
+    }
+}
+
 // ---- P and dS.  Units of contraction step t: 4 t = K, + 1 = Q, + 2 = V, + 3 = dO (rows of 64 elements).
 static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const BwdWideParams p) {
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
@@ -101,35 +173,12 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
     int klimit = p.Sk;
     if (p.kv_len) klimit = min(klimit, max(p.kv_len[b], 0));
 
-    // ---- copies: 16 of 8 rows x 128 bytes per unit; rows past the end re-read the last one
     const int k_last = p.Sk - 1, q_last = p.Sq - 1, k_rows = p.Sk - k0, q_rows = p.Sq - q0;
     const uint16_t* kbase = p.k + b * p.ks.b + hh * p.ks.h + (int64_t)min(k0, k_last) * p.ks.n;
     const uint16_t* vbase = p.v + b * p.vs.b + hh * p.vs.h + (int64_t)min(k0, k_last) * p.vs.n;
     const uint16_t* qbase = p.q + b * p.qs.b + hh * p.qs.h + (int64_t)min(q0, q_last) * p.qs.n;
     const uint16_t* gbase = p.dout + b * p.dos.b + hh * p.dos.h + (int64_t)min(q0, q_last) * p.dos.n;
-    // Copy i of a unit: rows 8 (4 wave + i) + lane / 8.  The swizzle of copies 0 and 2, and of 1 and 3, is the same, so two
-    // lane offsets per tensor do where all 128 rows exist.
-    const int row0 = 32 * wave + (lane >> 3), gran0 = (lane & 7) ^ swz<64>(row0), gran1 = (lane & 7) ^ swz<64>(row0 + 8);
-    static_assert(swz<64>(0) == swz<64>(16) && swz<64>(8) == swz<64>(24) && swz<64>(7) == swz<64>(23), "the swizzle repeats every 16 rows");
-    const uint32_t lds0 = lds_addr(lds) + 4096u * (uint32_t)wave;
-    auto issue = [&](const uint16_t* base, int64_t stride, int rows, int t, int slot) {      // elements [64 t, 64 t + 64)
-        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS);
-        const uint16_t* src = base + kWideStep * t;
-        if (kWideStep * (t + 1) <= p.d && rows >= kWideTile) {
-            const uint32_t at = 2u * (uint32_t)(row0 * (int)stride + 8 * gran0), at1 = at + 16u * (uint32_t)(stride + gran1 - gran0);
-            dma16u(src, at, dst);
-            dma16u(src, at1, dst + 1024u);
-            dma16u(src + 16 * stride, at, dst + 2048u);
-            dma16u(src + 16 * stride, at1, dst + 3072u);
-        } else {                                           // rows past the end re-read the last one; granules past the head dim:
-#pragma unroll                                             // filler, zeroed in the fragments
-            for (int i = 0; i < 4; ++i) {
-                const int g = i & 1 ? gran1 : gran0;
-                dma16u(src, 2u * (uint32_t)(min(row0 + 8 * i, max(rows - 1, 0)) * (int)stride + (kWideStep * t + 8 * g < p.d ? 8 * g : 0)), dst + 1024u * i);
-            }
-        }
-    };
-    // fragment of 16 contraction elements c: row, granule 2 c + h; the chunk only flips bits 4 and 5 of the offset
+    const WideRows copies(lds);
     int fk[2], fq[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -154,48 +203,40 @@ static __global__ __launch_bounds__(256, 2) void bwd_wide_scores_kernel(const Bw
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[kb][qb][r] = dp[kb][qb][r] = 0.f;
 
-    auto multiply = [&](auto tail_tag, f32x16 (&acc)[2][2], int slot_k, int slot_q, int rest) {
-        constexpr bool TAIL = decltype(tail_tag)::value;
-        const uint16_t* kt_ = lds + slot_k * WideRing::UNIT_ELEMS;
-        const uint16_t* qt_ = lds + slot_q * WideRing::UNIT_ELEMS;
-#pragma unroll
-        for (int c = 0; c < kWideStep / 16; ++c) {
-            if (TAIL && 16 * c >= rest) break;
-            bf16x8 kf[2], qf[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                kf[u] = *reinterpret_cast<const bf16x8*>(kt_ + (fk[u] ^ (16 * c)));
-                qf[u] = *reinterpret_cast<const bf16x8*>(qt_ + (fq[u] ^ (16 * c)));
-                if (TAIL && 16 * c + 8 * h >= rest) kf[u] = qf[u] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});   // both: a filler must not meet a zero as an infinity
-            }
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int qb = 0; qb < 2; ++qb) acc[kb][qb] = mfma32(kf[kb], qf[qb], acc[kb][qb]);
-        }
-    };
     using Yes = std::integral_constant<bool, true>;
     using No = std::integral_constant<bool, false>;
 
     const int n_steps = (p.d + kWideStep - 1) / kWideStep;
     WideRing ring;
-    issue(kbase, p.ks.n, k_rows, 0, 0);
-    issue(qbase, p.qs.n, q_rows, 0, 1);
-    issue(vbase, p.vs.n, k_rows, 0, 2);
+    copies.issue(kbase, p.ks.n, k_rows, p.d, 0, 0);
+    copies.issue(qbase, p.qs.n, q_rows, p.d, 0, 1);
+    copies.issue(vbase, p.vs.n, k_rows, p.d, 0, 2);
+    auto multiply = [&](auto tail_tag, f32x16 (&acc)[2][2], int t, auto&& copy) {
+        const uint16_t* kt_ = lds + ring.slot(0) * WideRing::UNIT_ELEMS;
+        const uint16_t* qt_ = lds + ring.slot(1) * WideRing::UNIT_ELEMS;
+        if constexpr (decltype(tail_tag)::value) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) copy(i);
+            wide_multiply_tail(acc, kt_, qt_, fk, fq, p.d - kWideStep * t);
+        } else {
+            wide_phase(acc, [&](int c, int u) { return *reinterpret_cast<const bf16x8*>(kt_ + (fk[u] ^ (16 * c))); },
+                       [&](int c, int u) { return *reinterpret_cast<const bf16x8*>(qt_ + (fq[u] ^ (16 * c))); }, copy);
+        }
+        ring.next();
+    };
     auto step = [&](auto tail_tag, int t) {
         const bool more = t + 1 < n_steps;
         WideRing::landed(false);                           // K and Q
-        issue(gbase, p.dos.n, q_rows, t, ring.slot(3));
-        if (more) issue(kbase, p.ks.n, k_rows, t + 1, ring.slot(4));
-        multiply(tail_tag, s, ring.slot(0), ring.slot(1), p.d - kWideStep * t);
-        ring.next();
+        multiply(tail_tag, s, t, [&](int i) {
+            if (i < 4) copies.issue(gbase, p.dos.n, q_rows, p.d, t, ring.slot(3), i);
+            else if (more) copies.issue(kbase, p.ks.n, k_rows, p.d, t + 1, ring.slot(4), i - 4);
+        });
         WideRing::landed(!more);                           // V and dO
-        if (more) {
-            issue(qbase, p.qs.n, q_rows, t + 1, ring.slot(3));
-            issue(vbase, p.vs.n, k_rows, t + 1, ring.slot(4));
-        }
-        multiply(tail_tag, dp, ring.slot(0), ring.slot(1), p.d - kWideStep * t);
-        ring.next();
+        multiply(tail_tag, dp, t, [&](int i) {
+            if (!more) return;
+            if (i < 4) copies.issue(qbase, p.qs.n, q_rows, p.d, t + 1, ring.slot(3), i);
+            else copies.issue(vbase, p.vs.n, k_rows, p.d, t + 1, ring.slot(4), i - 4);
+        });
     };
     // the step that ends inside 64 behind the loop: as a choice within it, it made the compiler move both accumulators
     // (384 registers) around every step
@@ -285,18 +326,12 @@ __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const u
         }
     }
     const uint32_t lds0 = lds_addr(lds) + 4096u * (uint32_t)wave;
-    auto issue_x = [&](int c0, int slot) {             // contraction rows [c0, c0 + 64); past the end the last row, against zeros of W
-        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS);
+    auto issue_x = [&](int c0, int slot, int i) {      // copy i of contraction rows [c0, c0 + 64); past the end the last row, against zeros of W
         const int first = min(c0, n_con - 1), over = n_con - 1 - first;
-        const uint16_t* xsrc = xbase + (int64_t)first * xs.n;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dma16u(xsrc, xoff[i] + 2u * (uint32_t)(min(xrow[i], over) * (int)xs.n), dst + 1024u * i);
+        dma16u(xbase + (int64_t)first * xs.n, xoff[i] + 2u * (uint32_t)(min(xrow[i], over) * (int)xs.n), lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS) + 1024u * i);
     };
-    auto issue_w = [&](int c0, int slot) {
-        const uint32_t dst = lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS);
-        const uint16_t* wsrc = wbase + (DQ ? (int64_t)c0 : (int64_t)c0 * p.sk_pad);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dma16u(wsrc, woff[i], dst + 1024u * i);
+    auto issue_w = [&](int c0, int slot, int i) {
+        dma16u(wbase + (DQ ? (int64_t)c0 : (int64_t)c0 * p.sk_pad), woff[i], lds0 + 2u * (uint32_t)(slot * WideRing::UNIT_ELEMS) + 1024u * i);
     };
     // fragment addresses: transposing reads of a 64 x 128 tile, 16 contraction rows per chunk
     const int tr_r = lane & 15, tr_g16 = (lane >> 4) & 1;
@@ -331,30 +366,27 @@ __device__ __forceinline__ void bwd_wide_product(const BwdWideParams& p, const u
 
     WideRing ring;
     if (con_lo < con_hi) {
-        issue_x(con_lo, 0);
-        issue_w(con_lo, 1);
-        if (con_lo + kWideStep < con_hi) issue_x(con_lo + kWideStep, 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) issue_x(con_lo, 0, i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) issue_w(con_lo, 1, i);
+        if (con_lo + kWideStep < con_hi)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) issue_x(con_lo + kWideStep, 2, i);
     }
     for (int c0 = con_lo; c0 < con_hi; c0 += kWideStep, ring.next()) {
         WideRing::landed(c0 + kWideStep >= con_hi);
-        if (c0 + kWideStep < con_hi) issue_w(c0 + kWideStep, ring.slot(3));
-        if (c0 + 2 * kWideStep < con_hi) issue_x(c0 + 2 * kWideStep, ring.slot(4));
         const uint16_t* xt = lds + ring.slot(0) * WideRing::UNIT_ELEMS;
         const uint16_t* wt = lds + ring.slot(1) * WideRing::UNIT_ELEMS;
-#pragma unroll
-        for (int c = 0; c < kWideStep / 16; ++c) {
-            bf16x8 xf[2], wf[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                xf[u] = tr_frag(xt + 16 * c * 128, xo[0][u], xo[1][u]);
-                if constexpr (DQ) wf[u] = *reinterpret_cast<const bf16x8*>(wt + (wo[0][u] ^ (16 * c)));
-                else wf[u] = tr_frag(wt + 16 * c * 128, wo[0][u], wo[1][u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int m = 0; m < 2; ++m) acc[u][m] = mfma32(xf[u], wf[m], acc[u][m]);
-        }
+        wide_phase(acc, [&](int c, int u) { return tr_frag(xt + 16 * c * 128, xo[0][u], xo[1][u]); },
+                   [&](int c, int u) {
+                       if constexpr (DQ) return *reinterpret_cast<const bf16x8*>(wt + (wo[0][u] ^ (16 * c)));
+                       else return tr_frag(wt + 16 * c * 128, wo[0][u], wo[1][u]);
+                   },
+                   [&](int i) {
+                       if (i < 4 && c0 + kWideStep < con_hi) issue_w(c0 + kWideStep, ring.slot(3), i);
+                       if (i >= 4 && c0 + 2 * kWideStep < con_hi) issue_x(c0 + 2 * kWideStep, ring.slot(4), i - 4);
+                   });
     }
     __syncthreads();                                   // the tiles are no longer needed: the output passes through their place
 #pragma unroll

@@ -21,6 +21,7 @@
 
 #include "attn_bwd.hpp"
 #include "attn_bwd_wide.hpp"
+#include "attn_fwd_probs.hpp"
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
 #include "attn_fwd_keyshare.hpp"
@@ -464,6 +465,17 @@ inline int bigd_key_splits(int64_t query_tile_wgs, int Sk) {
 inline int bigd_query_tile(int D) { return D <= 256 ? 128 : 64; }
 inline size_t partials_bytes(int key_splits, int64_t rows, int dv) { return (size_t)key_splits * rows * (dv + 1) * sizeof(float); }
 
+// Head dims above 256: the forward in two matrix products (attn_fwd_probs.hpp) instead of the one-pass kernel below.  Not for a
+// few queries, whose tiles would be padding, and up to D = 384 not where the one-pass kernel's 64-query workgroups fill two or
+// more rounds of the chip and walk more than 1024 keys.  (One pass -> two products: B=1 H=8 S=2304 D=320, 288 workgroups,
+// 168 -> 92 us, B=4 H=1 S=2112 D=320 76 -> 60 us, B=1 H=1 S=4096 D=512 70 -> 60 us, B=4 H=8 S=1024 D=512 112 -> 91 us, B=2 H=8
+// S=2048 D=512 203 -> 179 us; not taken: B=4 H=8 S=2048 D=384 317 -> 339 us, one query and 4096 keys, 64 heads, D=320 68 -> 116.)
+bool fwd_rule_probs(int B, int H, int N_q, int N_kv, int D) {
+    const int64_t bh = (int64_t)B * H, wgs = (int64_t)((N_q + 63) / 64) * bh, rounds = (wgs + 255) / 256;
+    if (D <= 256 || N_q < 96 || bh * ((N_q + 127) / 128) * ((N_kv + 127) / 128) < 64) return false;
+    return !(D <= 384 && rounds >= 2 && 10 * wgs >= 8 * 256 * rounds && N_kv > 1024);
+}
+
 template <int NC, int NW>
 int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc) {
     constexpr bool SPLIT = NC > 2;
@@ -513,8 +525,77 @@ int launch_fwd_bigd_nw(const FwdParams& fp, hipStream_t s, const FwdScratch& sc)
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
 }
+// The forward in two matrix products (attn_fwd_probs.hpp).  Its workspace: P, maxima and sums of as many (batch, head) slices at
+// a time as 128 MiB hold (P then stays in the 256 MB cache between the two), and of one of up to 512 MiB where none does;
+// behind them the partial outputs, where output tiles on fewer than two workgroups per compute unit are shared by several.
+int pad128(int n) { return (n + 127) / 128 * 128; }
+size_t probs_slice_bytes(int N_q, int N_kv) {
+    return (size_t)pad128(N_q) * pad128(N_kv) * 2 + 2 * (size_t)(pad128(N_kv) / 128) * pad128(N_q) * sizeof(float);
+}
+int probs_group(int B, int H, int N_q, int N_kv) {                   // launches of about as many slices each
+    const int64_t bh = (int64_t)B * H, most = std::max<int64_t>(1, ((int64_t)128 << 20) / (int64_t)probs_slice_bytes(N_q, N_kv));
+    const int64_t launches = (bh + most - 1) / most;
+    return (int)((bh + launches - 1) / launches);
+}
+int probs_key_splits(int B, int H, int N_q, int N_kv, int D) {
+    if (probs_group(B, H, N_q, N_kv) < B * H) return 1;              // (one launch covers everything where the keys are split)
+    const int64_t tiles = (int64_t)B * H * (pad128(N_q) / 128) * ((D + 127) / 128), key_tiles = pad128(N_kv) / 128;
+    // (D = 512, one head: 4096 positions 81 / 66 / 64 us with 1 / 2 / 4 ranges of the keys, 1024 positions 24.3 / 25.0 / 25.7)
+    return tiles * 2 > 256 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(4, key_tiles / 8));
+}
+size_t probs_workspace_bytes(int B, int H, int N_q, int N_kv, int D) {            // 0: not for this problem
+    if (!fwd_rule_probs(B, H, N_q, N_kv, D)) return 0;
+    const size_t slice = probs_slice_bytes(N_q, N_kv);
+    if (slice > ((size_t)512 << 20)) return 0;
+    const int ks = probs_key_splits(B, H, N_q, N_kv, D);
+    return probs_group(B, H, N_q, N_kv) * slice + (ks > 1 ? partials_bytes(ks, (int64_t)B * H * N_q, D) : 0);
+}
+
+int launch_fwd_probs(const FwdParams& fp, hipStream_t s, void* workspace) {
+    static std::atomic<bool> probs_set{false}, pv_set{false};
+    if (const int rc = set_lds(reinterpret_cast<const void*>(fwd_probs_kernel), WideRing::LDS_BYTES, probs_set)) return rc;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(fwd_probs_pv_kernel), WideRing::LDS_BYTES, pv_set)) return rc;
+    FwdProbsParams p;
+    p.q = fp.q; p.k = fp.k; p.v = fp.v; p.o = fp.o; p.lse = fp.lse;
+    p.qs = fp.qs; p.ks = fp.ks; p.vs = fp.vs; p.os = fp.os;
+    p.B = fp.B; p.H = fp.H; p.Sq = fp.Sq; p.Sk = fp.Sk; p.d = fp.d;
+    p.sq_pad = pad128(fp.Sq);
+    p.sk_pad = pad128(fp.Sk);
+    p.scale = fp.scale;
+    p.kv_len = fp.m.kv_len;
+    p.causal = fp.m.causal;
+    const int bh = p.B * p.H, group = probs_group(p.B, p.H, p.Sq, p.Sk);
+    const int64_t n_kt = p.sk_pad / 128, n_qt = p.sq_pad / 128, n_dt = (p.d + 127) / 128;
+    p.key_splits = probs_key_splits(p.B, p.H, p.Sq, p.Sk, p.d);
+    if (group * n_kt * n_qt > 0x7fffffff || group * n_qt * n_dt * p.key_splits > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    p.probs = static_cast<uint16_t*>(workspace);
+    p.tile_max = reinterpret_cast<float*>(p.probs + (size_t)group * p.sq_pad * p.sk_pad);
+    p.tile_sum = p.tile_max + (size_t)group * n_kt * p.sq_pad;
+    p.part_o = p.tile_sum + (size_t)group * n_kt * p.sq_pad;
+    p.part_lse = p.part_o + (size_t)p.key_splits * bh * p.Sq * p.d;
+    ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
+    for (p.bh0 = 0; p.bh0 < bh; p.bh0 += group) {
+        const int64_t n = std::min(group, bh - p.bh0);
+        hipLaunchKernelGGL(fwd_probs_kernel, dim3((unsigned)(n * n_kt * n_qt)), dim3(256), WideRing::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(fwd_probs_pv_kernel, dim3((unsigned)(n * n_qt * n_dt * p.key_splits)), dim3(256), WideRing::LDS_BYTES, s, p);
+    }
+    if (p.key_splits > 1) {
+        FwdParams m = fp;
+        m.key_splits = p.key_splits;
+        m.part_o = p.part_o;
+        m.part_lse = p.part_lse;
+        launch_fwd_merge(m, s);
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
 template <int NC>
-int launch_fwd_bigd(const FwdParams& p, hipStream_t s, const FwdScratch& sc) { return launch_fwd_bigd_nw<NC, 4>(p, s, sc); }
+int launch_fwd_bigd(const FwdParams& p, hipStream_t s, const FwdScratch& sc) {
+    const size_t need = probs_workspace_bytes(p.B, p.H, p.Sq, p.Sk, p.d);
+    if (need && sc.ws && aligned16(sc.ws) && sc.bytes >= need) return launch_fwd_probs(p, s, sc.ws);
+    return launch_fwd_bigd_nw<NC, 4>(p, s, sc);
+}
 
 // how the kernels draw (after set_dropout)
 int drop_mode(const MaskArgs& m, int Sk) { return m.drop_cq != 0 ? kDropTiled : Sk % 64 == 0 ? kDropRows64 : kDropFlat; }
@@ -1117,7 +1198,7 @@ size_t flame_attn_fwd_workspace_bytes(int B, int H, int N_q, int N_kv, int D) {
 
 size_t flame_attn_fwd_scratch_bytes(int B, int H, int N_q, int N_kv, int D) {
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0) return 0;
-    if (!head_dim_ok(D)) return flame_attn_fwd_workspace_bytes(B, H, N_q, N_kv, D);
+    if (!head_dim_ok(D)) return std::max(flame_attn_fwd_workspace_bytes(B, H, N_q, N_kv, D), big_head_dim_ok(D) ? probs_workspace_bytes(B, H, N_q, N_kv, D) : 0);
     const int ks = fwd_key_splits((int64_t)B * H, N_q, N_kv, padded_head_dim(D));
     return ks > 1 ? partials_bytes(ks, (int64_t)B * H * N_q, D) : 0;
 }
@@ -1953,7 +2034,6 @@ size_t mat_fixed_bytes(int B, int H, int N_q, bool backward) { return backward ?
 size_t mat_accum_bytes(int B, int H, int N_kv, int D, int Dv) { return align_up((size_t)B * H * N_kv * (size_t)(D + Dv) * sizeof(float), 256); }
 
 // The backward for head dims above 128 on kernels of its own (attn_bwd_wide.hpp): what it needs per (batch, head) slice.
-int pad128(int n) { return (n + 127) / 128 * 128; }
 size_t wide_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
 size_t wide_slice_bytes(int N_q, int N_kv) { return (size_t)pad128(N_q) * pad128(N_kv) * 4; }         // P and dS, bf16
 // as many slices at a time as 512 MiB hold, and one of up to 2 GiB where none does (16384 x 16384: 1 GiB, twice what the

@@ -86,9 +86,11 @@ int flame_attn_fwd_bf16(const void* Q, const void* K, const void* V, void* O, vo
 
 /* The same forward with a caller workspace (16-byte aligned device memory, used only during the call; null or too
  * small is accepted).  A grid that leaves compute units idle uses it, for the fp32 partial outputs of workgroups that
- * share a query tile and walk slices of the keys; with less room than flame_attn_fwd_scratch_bytes returns (for head
- * dims above 128 the same as flame_attn_fwd_workspace_bytes, which is 0 below) it uses fewer slices, with none it runs
- * unsplit.  Never allocates, so a first
+ * share a query tile and walk slices of the keys; with less room than flame_attn_fwd_scratch_bytes returns (head dims
+ * up to 128) or flame_attn_fwd_workspace_bytes (above, 0 below) it uses fewer slices, with none it runs unsplit.  For head
+ * dims above 256 flame_attn_fwd_scratch_bytes may ask for more, room for the bf16 probabilities of one (batch, head) slice
+ * or several (128 MiB, or one slice of up to 512 MiB): with that much the forward runs as two matrix products, which is
+ * faster.  Never allocates, so a first
  * call can be captured into a HIP graph (the reference's contract for code on the backward path:
  * src/cuda_graph.rs:11-18).  No counterpart in the reference's FFI. */
 size_t flame_attn_fwd_workspace_bytes(int B, int H, int N_q, int N_kv, int D);
