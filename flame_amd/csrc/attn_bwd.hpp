@@ -94,11 +94,14 @@ __device__ __forceinline__ void dkdv_store(const BwdParams& p, uint16_t* own, co
 // registers back, the walk runs the same straight-line steps as the unmasked one.
 // DROP (DropMode): dV takes the dropped and rescaled probabilities, dP = f (dO V^T) with the same factor f (drop_factor), and
 // -delta is added per element instead of seeding the dP accumulators.
+// BITS: a keep-mask as bits (mask_bits.hpp): the walk takes the query tiles of which anything attends to one of the 128 keys, the
+// cut ones first, and a lane has one word of its key for every cut one.
 // block / nblocks: this workgroup's index in the dK/dV grid and the size of that grid (the kernel's own launch, or
 // the dK/dV part of bwd_joint_kernel's).
-template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone>
+template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone, bool BITS = false>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int block, const int nblocks) {
     static_assert(!VECMASK || HASMASK, "VECMASK is a special case of HASMASK");
+    static_assert(!BITS || (!HASMASK && DROP == kDropNone), "bits stand for the mask");
     constexpr bool DROPOUT = DROP != kDropNone;
     using T = BwdTile<D>;
     constexpr int BM = T::BM, BN = T::BN, RS = T::RS;
@@ -163,8 +166,20 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         dead = ((((wave & 2) ? b1 : b0) >> (32 * (wave & 1) + n)) & 1ull) == 0;
     }
     const int n_qt = (p.Sq + BM - 1) / BM;
-    int qt_begin = p.m.causal ? (k0 / BM) : 0;
-    if (k0 >= klimit || any_alive == 0 || (p.m.causal && k0 >= p.Sq)) {
+    int qt_begin = p.m.causal && !BITS ? (k0 / BM) : 0;
+    KeyTiles qtiles;                       // BITS: of queries
+    const uint64_t* bcols = nullptr;       // this lane's key's word of query tile 0; tiles lie 64 bit_nkt words apart
+    if constexpr (BITS) {
+        const int plane = b * p.m.plane_b + hh * p.m.plane_h;
+        const uint8_t* flags = p.m.tile_flags + (int64_t)plane * p.m.bit_nqt * p.m.bit_nkt + k0 / 64;
+        qtiles.build_of_tiles(reinterpret_cast<char*>(lds) + T::LDS_BYTES, n_qt, [&](int u) {
+            const int f0 = flags[(int64_t)u * p.m.bit_nkt], f1 = flags[(int64_t)u * p.m.bit_nkt + 1];
+            return f0 & f1 & kTileAllRows ? 2 : (f0 | f1) & kTileAny ? 1 : 0;
+        });
+        bcols = p.m.bit_cols + (int64_t)plane * p.m.bit_nqt * (64 * p.m.bit_nkt) + kw0 + n;
+        if (qtiles.n_tiles == 0) any_alive = 0;
+    }
+    if (k0 >= klimit || any_alive == 0 || (!BITS && p.m.causal && k0 >= p.Sq)) {
         // Nothing attends to these keys (past the key length, masked, or past the last query under the causal flag):
         // dK = dV = 0, written at once.  Padded batches launch many such workgroups; they must not cost a
         // prologue each.
@@ -176,7 +191,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         dkdv_store<D>(p, lds + wave * 32 * D, zero, zero, b, hh, kw0);
         return;
     }
-    const int n_it = n_qt - qt_begin;
+    const int n_it = BITS ? qtiles.n_tiles : n_qt - qt_begin;
     // The walk visits the query tiles that need per-element exclusions first (all of them when an explicit
     // mask is given, else the causal diagonal tiles and a partial last tile) and the fully attended ones afterwards, so that each of the two loops runs one
     // specialised, branch-free body.  The order of the tiles does not matter to the sums.
@@ -185,13 +200,15 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     const bool all_masked = HASMASK;
     int lead_end = qt_begin;
     if (n_it > 0) {
-        if (all_masked) lead_end = n_qt;
+        if (BITS) lead_end = n_it - qtiles.n_whole;
+        else if (all_masked) lead_end = n_qt;
         else if (p.m.causal) lead_end = max(qt_begin, min(n_qt, (k0 + BN - 2) / BM + 1));
     }
     const int n_lead = lead_end - qt_begin;
-    const int tail_extra = (n_it > 0 && !all_masked && (p.Sq % BM) != 0 && lead_end < n_qt) ? 1 : 0;
+    const int tail_extra = (n_it > 0 && !BITS && !all_masked && (p.Sq % BM) != 0 && lead_end < n_qt) ? 1 : 0;
     const int n_masked = n_lead + tail_extra;
     auto tile_of = [&](int it) {
+        if constexpr (BITS) return qtiles.tile(it < n_masked ? qtiles.n_whole + it : it - n_masked);
         if (it < n_lead) return qt_begin + it;
         if (it < n_masked) return n_qt - 1;
         return lead_end + (it - n_masked);
@@ -402,6 +419,10 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         for (int g4 = 0; g4 < 4; ++g4) ndelta_rows(rows0 + st * T::ROW_FLOATS, 0, g4);
     }
 
+    uint64_t word_ahead = 0;               // BITS: of the next cut tile
+    if constexpr (BITS) {
+        if (n_masked > 0) word_ahead = bcols[(int64_t)tile_of(0) * (64 * p.m.bit_nkt)];
+    }
     // COPY: 0 = this is the last step, 1 = the next tile is a full one (straight-line copies),
     //       2 = decide at run time (used by the few steps that need exclusions)
     // STAGE: LDS stage that holds this step's tile (0 / 1 / 2), or -1 to take it from `st`.
@@ -423,6 +444,12 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         f32x16 sacc[2];
         bf16x8 pf[2][2], dsf[2][2];
         f32x4 l4, l4n;
+        uint32_t keep_bits[2] = {0u, 0u};       // BITS: of this lane's half, query block by query block
+        if constexpr (BITS && MASKED) {
+            keep_bits[0] = (uint32_t)word_ahead >> (4 * h);
+            keep_bits[1] = (uint32_t)(word_ahead >> 32) >> (4 * h);
+            if (it + 1 < n_masked) word_ahead = bcols[(int64_t)qt_next * (64 * p.m.bit_nkt)];
+        }
         // keep-mask bytes of this lane's key for the 64 queries of the tile, fetched up front in one batch
         // (a load per element inside the pipelined slices would wait out a memory round trip each time)
         uint32_t mk[2][16];
@@ -494,6 +521,8 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
                 bool drop;
                 if constexpr (VECMASK) {
                     drop = m4[t] <= dead_thr;       // whole tiles, no causal flag: the mask byte decides, one compare
+                } else if constexpr (BITS) {
+                    drop = (keep_bits[qb] & (1u << (8 * g + t))) == 0;
                 } else {
                     // bitwise, not short-circuit: one select per element instead of a chain of branches
                     drop = (key >= klimit) | (qi >= p.Sq) | ((p.m.causal != 0) & (key > qi));
@@ -661,6 +690,41 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
             nq += q_tile_stride, ndo += do_tile_stride, nrow += BM;
         }
     }
+    if constexpr (BITS) {
+        // Cut tiles in straight-line steps of three as well, once the stage counter is 0: every next tile of theirs is a cut one
+        // that is not the last, which alone can be a partial one.
+        int it = 0;
+        auto one = [&]() {
+            const int qn = it + 1 < it_hi ? tile_of(it + 1) : 0;
+            step(std::true_type{}, I2{}, IM{}, st, it, 0, qn, qbase + qn * q_tile_stride, dobase + qn * do_tile_stride, rowbase + qn * BM);
+            st = st == 2 ? 0 : st + 1;
+            ++it;
+        };
+        while (it < n_masked && st != 0) one();
+        if (it + 3 < n_masked - 1) {
+            int at_tile = tile_of(it + 1);
+            const uint16_t* nq = qbase + at_tile * q_tile_stride;
+            const uint16_t* ndo = dobase + at_tile * do_tile_stride;
+            const float* nrow = rowbase + at_tile * BM;
+            auto advance = [&](int next) {
+                const int d = tile_of(next) - at_tile;
+                at_tile += d;
+                nq += d * q_tile_stride;
+                ndo += d * do_tile_stride;
+                nrow += d * BM;
+            };
+            for (; it + 3 < n_masked - 1; it += 3) {
+                step(std::true_type{}, I1{}, I0{}, 0, it, 0, at_tile, nq, ndo, nrow);
+                advance(it + 2);
+                step(std::true_type{}, I1{}, I1{}, 1, it + 1, 0, at_tile, nq, ndo, nrow);
+                advance(it + 3);
+                step(std::true_type{}, I1{}, I2{}, 2, it + 2, 0, at_tile, nq, ndo, nrow);
+                advance(it + 4);
+            }
+        }
+        while (it < n_masked) one();
+        it_m = n_masked;
+    }
     for (int it = it_m; it < n_masked_here + it_lo; ++it) {
         const int qn = it + 1 < it_hi ? tile_of(it + 1) : 0;
         step(std::true_type{}, I2{}, IM{}, st, it, tile_of(it), qn, qbase + qn * q_tile_stride, dobase + qn * do_tile_stride,
@@ -671,11 +735,29 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     // the stage counter is 0 here
     {
         int it = max(n_masked, it_lo);
-        int qt = lead_end + (it - n_masked);
+        int qt = lead_end + (it - n_masked);                       // (BITS: the list says which tile, and no step asks for its number)
         const uint16_t* nq = qbase + (qt + 1) * q_tile_stride;     // the tile after the current one
         const uint16_t* ndo = dobase + (qt + 1) * do_tile_stride;
         const float* nrow = rowbase + (qt + 1) * BM;
+        // BITS: the list says how many tiles to go on (from the one the pointers are at; kept as steps, not as places: pointers
+        // formed anew from the bases took so many scalar registers that 560 bytes per lane went to scratch)
+        int listed = it + 1, at_tile = qt + 1;
+        auto on_by_list = [&]() {
+            if (listed < it_hi) {
+                const int d = tile_of(listed) - at_tile;
+                at_tile += d;
+                ++listed;
+                nq += d * q_tile_stride;
+                ndo += d * do_tile_stride;
+                nrow += d * BM;
+            }
+        };
+        if constexpr (BITS) on_by_list();
         auto advance = [&]() {
+            if constexpr (BITS) {
+                on_by_list();
+                return;
+            }
             nq += q_tile_stride;
             ndo += do_tile_stride;
             nrow += BM;
@@ -733,9 +815,9 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     dkdv_store<D>(p, lds + wave * 32 * D, dkacc, dvacc, b, hh, kw0, DROP == kDropFlat || DROP == kDropRows64 ? p.m.drop_scale : 1.0f);
 }
 
-template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone>
+template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone, bool BITS = false>
 __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
-    bwd_dkdv_body<D, HASMASK, TIMING, VECMASK, DROP>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_dkdv_body<D, HASMASK, TIMING, VECMASK, DROP, BITS>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // dK^T / dV^T accumulators (rows = d, column = a lane's key) of the 32 keys from kw0 on -> bf16 rows of dK (scaled) and dV
@@ -822,7 +904,7 @@ struct BwdDqTile {
 template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
 __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
     static_assert(KG == 1 || (KG == 2 && EXCL == kExNone), "key groups: nothing excluded but by causal flag and key lengths");
-    constexpr bool HASMASK = EXCL == kExRows16 || EXCL == kExGeneral, VECMASK = EXCL == kExRows16, KEYS = EXCL == kExKeys;
+    constexpr bool HASMASK = EXCL == kExRows16 || EXCL == kExGeneral, VECMASK = EXCL == kExRows16, BITS = EXCL == kExBits, KEYS = EXCL == kExKeys || BITS;
     using T = BwdDqTile<D>;
     constexpr int BM = 32 * NW, BN = T::BN, RS = T::RS;
     constexpr int DC = D / 16;
@@ -849,7 +931,7 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     }
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len && p.dq_parts == 1) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
-    if ((KEYS || p.m.kv_len) && p.dq_parts == 1) bh = longest_batches_first<KEYS>(bh, p.B, p.H, p.Sk, p.m);
+    if (!BITS && (KEYS || p.m.kv_len) && p.dq_parts == 1) bh = longest_batches_first<KEYS>(bh, p.B, p.H, p.Sk, p.m);
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 32;
@@ -864,7 +946,7 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     int kend = klimit;
     if (p.m.causal) kend = min(kend, q0 + BM);
     int n_tiles = (kend + BN - 1) / BN;
-    const uint8_t* mbase = HASMASK || KEYS ? mask_head_base(p.m, b, hh) : nullptr;
+    const uint8_t* mbase = HASMASK || EXCL == kExKeys ? mask_head_base(p.m, b, hh) : nullptr;
     int t_lo = 0;             // first tile of this workgroup's share of the walk
     if (p.dq_parts > 1) {
         const int per = (n_tiles + p.dq_parts - 1) / p.dq_parts;
@@ -878,7 +960,17 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     }
     // step t of the walk takes tile tile_of(t)
     KeyTiles kt;
-    if constexpr (KEYS) {
+    const uint64_t* brows = nullptr;       // BITS: this lane's query's word of key tile 0; tiles lie 64 bit_nqt words apart
+    if constexpr (BITS) {
+        const int plane = b * p.m.plane_b + hh * p.m.plane_h;
+        const uint8_t* flags = p.m.tile_flags + ((int64_t)plane * p.m.bit_nqt + q0 / 64) * p.m.bit_nkt;       // of the first 64 queries, then of the others
+        kt.build_of_tiles(reinterpret_cast<char*>(lds) + T::LDS_BYTES, (klimit + 63) / 64, [&](int t) {
+            const int f0 = flags[t], f1 = flags[p.m.bit_nkt + t];
+            return f0 & f1 & kTileAllKeys ? 2 : (f0 | f1) & kTileAny ? 1 : 0;
+        });
+        n_tiles = kt.n_tiles;
+        brows = p.m.bit_rows + (int64_t)plane * p.m.bit_nkt * (64 * p.m.bit_nqt) + qw0 + n;
+    } else if constexpr (KEYS) {
         kt.build(reinterpret_cast<char*>(lds) + T::LDS_BYTES, klimit, NW, [&](int key) {
             return key < klimit && mask_attends(p.m, mbase, (int64_t)min(key, p.Sk - 1) * p.m.sk);
         });
@@ -989,6 +1081,10 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     wait_vm0();
     __syncthreads();
 
+    uint64_t word_ahead = 0;               // BITS: of the next cut tile
+    if constexpr (BITS) {
+        if (kt.n_whole < n_tiles) word_ahead = brows[(int64_t)kt.tile(kt.n_whole) * (64 * p.m.bit_nqt)];
+    }
     // One tile of 64 keys = two blocks of 32.  The phases of the two blocks are staggered so that the
     // element-wise work of one phase is threaded between the MFMAs of the next, two logits per MFMA:
     //   S(0) | dP(0) + P(0) | S(1) + dS(0) | dP(1) + P(1) | dQ(0) + dS(1) | dQ(1)
@@ -1012,7 +1108,8 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         (void)drop_word;
         uint32_t keep_bits[2] = {0u, 0u};
         if constexpr (KEYS && MASKED) {
-            const uint64_t w = kt.bits[kt.tile(t)];
+            const uint64_t w = BITS ? word_ahead : kt.bits[kt.tile(t)];
+            if (BITS && t + 1 < n_tiles) word_ahead = brows[(int64_t)kt.tile(t + 1) * (64 * p.m.bit_nqt)];
             keep_bits[0] = (uint32_t)w >> (4 * h);
             keep_bits[1] = (uint32_t)(w >> 32) >> (4 * h);
         }

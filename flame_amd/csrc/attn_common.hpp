@@ -500,6 +500,9 @@ enum MaskMode : int {
     kMaskBf16Drop = 2,       // bf16, a value above 0.5 excludes (the convention of the reference's streaming entry point)
 };
 
+// flags of a 64 x 64 tile of (query, key), see mask_bits.hpp
+constexpr uint8_t kTileAny = 1, kTileAllKeys = 2, kTileAllRows = 4;
+
 struct MaskArgs {
     const int32_t* kv_len;   // [B] or null
     const uint8_t* mask;     // explicit mask or null; element type and meaning per mask_mode
@@ -507,6 +510,12 @@ struct MaskArgs {
     int causal;              // key j > query i is excluded
     int rows16 = 0;          // uint8 keep-mask rows are contiguous along keys and 16-byte aligned (vector loads allowed)
     int mask_mode = kMaskU8;
+    // the mask as bits (kernels instantiated for them only): words and flags of the planes, see mask_bits.hpp
+    const uint64_t* bit_rows = nullptr;   // [plane][key tile][64 n_qt queries]
+    const uint64_t* bit_cols = nullptr;   // [plane][query tile][64 n_kt keys]
+    const uint8_t* tile_flags = nullptr;  // [plane][query tile][key tile]
+    int bit_nqt = 0, bit_nkt = 0;         // tiles, padded to even numbers
+    int plane_b = 0, plane_h = 0;         // plane of (b, h): b * plane_b + h * plane_h
     // additive bias on the scaled logits (forward only), fp32 or bf16, or null
     const void* bias = nullptr;
     int64_t bb = 0, bh = 0, bq = 0, bk = 0;   // element strides over (b,h,q,k); 0 broadcasts
@@ -576,6 +585,7 @@ enum Excl : int {
     kExBiasF32 = 3,      // (forward) an additive fp32 bias, contiguous along the keys, and no keep-mask, causal flag or key lengths
     kExBiasBf16 = 4,     // (forward) the same in bf16
     kExKeys = 5,         // a keep-mask that is the same for every query (a padded batch), no causal flag
+    kExBits = 6,         // a keep-mask as bits, with the key lengths and the causal flag folded in
 };
 
 // The 64-key tiles that a keep-mask of keys leaves anything of, in LDS: the tiles attended whole first, then the others
@@ -603,11 +613,25 @@ struct KeyTiles {
             if (lane == 0) bits[t] = b;
         }
         __syncthreads();
+        sort_out([&](int t) { return bits[t] == ~0ull ? 2 : bits[t] != 0ull ? 1 : 0; });
+    }
+    // The same from what is known of the tiles: attended(t) says whether nothing (0), something (1) or all (2) of tile t is.
+    template <class F>
+    __device__ __forceinline__ void build_of_tiles(void* lds, int n_tiles_all, F&& attended) {
+        n_all = n_tiles_all;
+        bits = static_cast<uint64_t*>(lds);           // unused
+        counts = reinterpret_cast<uint32_t*>(bits);
+        list = reinterpret_cast<uint16_t*>(counts + 2);
+        sort_out(attended);
+    }
+    template <class F>
+    __device__ __forceinline__ void sort_out(F&& attended) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         if (wave == 0) {
             int whole = 0, cut = 0;
             for (int t0 = 0; t0 < n_all; t0 += 64) {
-                const uint64_t b = t0 + lane < n_all ? bits[t0 + lane] : 0ull;
-                const bool is_whole = b == ~0ull, is_cut = b != 0ull && !is_whole;
+                const int a = t0 + lane < n_all ? attended(t0 + lane) : 0;
+                const bool is_whole = a == 2, is_cut = a == 1;
                 const uint64_t mw = __ballot(is_whole), mc = __ballot(is_cut), below = (1ull << lane) - 1ull;
                 if (is_whole) list[whole + __popcll(mw & below)] = (uint16_t)(t0 + lane);
                 if (is_cut) list[n_all - 1 - (cut + __popcll(mc & below))] = (uint16_t)(t0 + lane);

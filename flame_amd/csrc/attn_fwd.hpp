@@ -95,10 +95,10 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     uint16_t* lds = lds_all + (KG == 1 ? 0 : group * (T::LDS_BYTES / 2));
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len || EXCL == kExKeys ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.m.kv_len || EXCL == kExKeys || EXCL == kExBits ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
-    if (EXCL == kExKeys || p.m.kv_len) bh = longest_batches_first<EXCL == kExKeys>(bh, p.B, p.H, p.Sk, p.m);
+    if (EXCL == kExKeys || (p.m.kv_len && EXCL != kExBits)) bh = longest_batches_first<EXCL == kExKeys>(bh, p.B, p.H, p.Sk, p.m);
     // a bias that all batches share: its rows are read by the batches' workgroups one after the other on one XCD, from its L2
     if ((EXCL == kExBiasF32 || EXCL == kExBiasBf16) && p.m.bb == 0) {
         const int rest = wg / p.B;
@@ -134,9 +134,19 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
                             : nullptr;
 
     // KEYS: step t of the walk takes tile tile_of(t) (elsewhere the two are the same number); stages go by the step
-    constexpr bool KEYS = EXCL == kExKeys;
+    constexpr bool BITS = EXCL == kExBits, KEYS = EXCL == kExKeys || BITS;
     KeyTiles kt;
-    if constexpr (KEYS) {
+    const uint64_t* brows = nullptr;               // BITS: this lane's query's word of key tile 0; tiles lie 64 bit_nqt words apart
+    if constexpr (BITS) {
+        const int plane = b * p.m.plane_b + hh * p.m.plane_h;
+        const uint8_t* flags = p.m.tile_flags + ((int64_t)plane * p.m.bit_nqt + q0 / 64) * p.m.bit_nkt;       // of the first 64 queries, then of the others
+        kt.build_of_tiles(reinterpret_cast<char*>(lds) + T::LDS_BYTES, (klimit + 63) / 64, [&](int t) {
+            const int f0 = flags[t], f1 = flags[p.m.bit_nkt + t];
+            return f0 & f1 & kTileAllKeys ? 2 : (f0 | f1) & kTileAny ? 1 : 0;
+        });
+        n_tiles = kt.n_tiles;
+        brows = p.m.bit_rows + (int64_t)plane * p.m.bit_nkt * (64 * p.m.bit_nqt) + qi;
+    } else if constexpr (KEYS) {
         kt.build(reinterpret_cast<char*>(lds) + T::LDS_BYTES, klimit, NW, [&](int key) {
             return key < klimit && mask_attends(p.m, mbase, (int64_t)min(key, p.Sk - 1) * p.m.sk);
         });
@@ -256,7 +266,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     uint32_t keep_bits[2];         // KEYS: of this lane's half, key block by key block
     auto excl_begin = [&](int t) {
         if constexpr (KEYS) {
-            const uint64_t w = kt.bits[kt.tile(t)];
+            const uint64_t w = BITS ? brows[(int64_t)kt.tile(t) * (64 * p.m.bit_nqt)] : kt.bits[kt.tile(t)];
             keep_bits[0] = (uint32_t)w >> (4 * h);
             keep_bits[1] = (uint32_t)(w >> 32) >> (4 * h);
         }

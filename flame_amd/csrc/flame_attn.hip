@@ -22,6 +22,7 @@
 #include "attn_bwd.hpp"
 #include "attn_bwd_wide.hpp"
 #include "attn_fwd_probs.hpp"
+#include "mask_bits.hpp"
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
 #include "attn_fwd_keyshare.hpp"
@@ -160,7 +161,7 @@ int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
         if (rule_key_groups(grid, p.Sk)) return launch_fwd<D, EXCL, NW, DROP, 2>(p, s, wg_count);
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_kernel<D, EXCL, NW, DROP, KG>;
-    constexpr bool KEYS = EXCL == kExKeys;
+    constexpr bool KEYS = EXCL == kExKeys || EXCL == kExBits;
     constexpr int tiles = KG * T::LDS_BYTES + (EXCL == kExBiasF32 || EXCL == kExBiasBf16 ? T::BIAS_PASS_BYTES : 0);
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), tiles + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
     const int lds = tiles + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
@@ -240,10 +241,90 @@ int padded_head_dim(int D) { return D <= 64 ? 64 : 128; }
 size_t bwd_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
 size_t bwd_split_slot_bytes(int D) { return (size_t)2 * 128 * D * sizeof(float); }   // dK^T and dV^T of one 128-key block
 
+// The keep-mask as bits (mask_bits.hpp).  Planes: one per batch where the mask or, with key lengths, what they leave of it
+// differs by batch, one per head where it differs by head.  0 bytes: not for this call (a mask that is the same for every query has
+// kernels of its own, and a list of tiles holds 1024).
+struct MaskPlanes {
+    int64_t planes;
+    int plane_b, plane_h, n_qt, n_kt;
+};
+MaskPlanes mask_planes(const MaskArgs& m, int B, int H, int N_q, int N_kv) {
+    const bool per_b = m.sb != 0 || m.kv_len, per_h = m.sh != 0;
+    return {(int64_t)(per_b ? B : 1) * (per_h ? H : 1), per_b ? (per_h ? H : 1) : 0, per_h ? 1 : 0, (N_q + 127) / 128 * 2, (N_kv + 127) / 128 * 2};
+}
+size_t mask_bits_bytes(const MaskArgs& m, int B, int H, int N_q, int N_kv) {
+    const MaskPlanes z = mask_planes(m, B, H, N_q, N_kv);
+    if (keys_only(m, N_q, N_kv) || z.n_qt > KeyTiles::kMaxTiles || z.n_kt > KeyTiles::kMaxTiles) return 0;
+    if ((int64_t)z.n_qt * z.n_kt < 36) return 0;            // (256 x 256, 4 heads: a training step of 35 us; the pass over the mask costs 2 launches)
+    const int64_t tiles = z.planes * z.n_qt * z.n_kt;
+    return tiles > (int64_t)1 << 20 ? 0 : align_up((size_t)tiles * (2 * 512 + 1), 256);       // 1 GiB
+}
+// (a workspace that nothing was kept in before may have any alignment)
+bool mask_bits_fit(const MaskArgs& m, int B, int H, int N_q, int N_kv, const void* ws, size_t bytes) {
+    const size_t need = mask_bits_bytes(m, B, H, N_q, N_kv);
+    return need && ws && need <= bytes && reinterpret_cast<uintptr_t>(ws) % 16 == 0;
+}
+// writes the words and flags to `ws` (mask_bits_bytes) and points `m` to them; the causal flag is in them then
+int launch_mask_bits(MaskArgs& m, int B, int H, int N_q, int N_kv, void* ws, hipStream_t s) {
+    const MaskPlanes z = mask_planes(m, B, H, N_q, N_kv);
+    const int64_t tiles = z.planes * z.n_qt * z.n_kt, grid = z.planes * z.n_qt * ((z.n_kt + 3) / 4);
+    if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    MaskBitsParams p;
+    p.m = m;
+    p.Sq = N_q;
+    p.Sk = N_kv;
+    p.H = z.plane_h ? H : 1;
+    p.n_qt = z.n_qt;
+    p.n_kt = z.n_kt;
+    p.rows = static_cast<uint64_t*>(ws);
+    p.cols = p.rows + 64 * tiles;
+    p.flags = reinterpret_cast<uint8_t*>(p.cols + 64 * tiles);
+    hipLaunchKernelGGL(m.mask_mode == kMaskU8 && m.sk == 1 && N_kv >= 16 ? mask_bits_kernel<true> : mask_bits_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, p);
+    m.bit_rows = p.rows;
+    m.bit_cols = p.cols;
+    m.tile_flags = p.flags;
+    m.bit_nqt = z.n_qt;
+    m.bit_nkt = z.n_kt;
+    m.plane_b = z.plane_b;
+    m.plane_h = z.plane_h;
+    m.causal = 0;
+    return FLAME_ATTN_OK;
+}
+
+// the backward with a keep-mask as bits, which the part of the workspace behind the rows holds
+template <int D>
+int launch_bwd_bits(BwdParams p, hipStream_t s) {
+    using T = BwdTile<D>;
+    using TQ = BwdDqTile<D>;
+    static std::atomic<bool> dq_set{false}, kv_set{false};
+    auto kern_dq = bwd_dq_kernel<D, kExBits, 4>;
+    auto kern_kv = bwd_dkdv_kernel<D, false, false, false, kDropNone, true>;
+    const int most = KeyTiles::lds_bytes(KeyTiles::kMaxTiles);
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_dq), TQ::LDS_BYTES + most, dq_set)) return rc;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_kv), T::LDS_BYTES + most, kv_set)) return rc;
+    const int64_t grid = (int64_t)((p.Sk + T::BN - 1) / T::BN) * p.B * p.H, grid_dq = (int64_t)((p.Sq + TQ::BM - 1) / TQ::BM) * p.B * p.H;
+    if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    if (const int rc = launch_mask_bits(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, s)) return rc;
+    p.split_ws = nullptr;
+    {
+        ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);
+        hipLaunchKernelGGL(kern_dq, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
+    }
+    {
+        ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DKDV, s);
+        hipLaunchKernelGGL(kern_kv, dim3((unsigned)grid), dim3(256), T::LDS_BYTES + KeyTiles::lds_bytes((p.Sq + 63) / 64), s, p);
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
 template <int D, bool HASMASK, bool TIMING = false>
 int launch_bwd(const BwdParams& p, hipStream_t s) {
     using T = BwdTile<D>;
     using TQ = BwdDqTile<D>;
+    if constexpr (HASMASK && !TIMING) {
+        if (mask_bits_fit(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, p.split_ws_bytes)) return launch_bwd_bits<D>(p, s);
+    }
     static bool attr_done = false;
     auto kern = bwd_dkdv_kernel<D, HASMASK, TIMING>;
     auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4>;
@@ -1147,6 +1228,11 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     // a keep-mask of keys: the walk takes the attended tiles only (up to what their list holds)
     if (keep_mask != nullptr && bias == nullptr && keys_only(p.m, N_q, N_kv))
         return DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
+    // any other keep-mask, with room for it as bits
+    if (keep_mask != nullptr && bias == nullptr && mask_bits_fit(p.m, B, H, N_q, N_kv, scratch.ws, scratch.bytes)) {
+        if ((rc = launch_mask_bits(p.m, B, H, N_q, N_kv, scratch.ws, s))) return rc;
+        return DP == 128 ? launch_fwd<128, kExBits, 4>(p, s) : launch_fwd<64, kExBits, 4>(p, s);
+    }
     // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel
     if (keep_mask != nullptr && bias == nullptr && p.m.rows16 && N_kv % 64 == 0)
         return DP == 128 ? launch_fwd<128, kExRows16, 4>(p, s) : launch_fwd<64, kExRows16, 4>(p, s);
@@ -1201,6 +1287,18 @@ size_t flame_attn_fwd_scratch_bytes(int B, int H, int N_q, int N_kv, int D) {
     if (!head_dim_ok(D)) return std::max(flame_attn_fwd_workspace_bytes(B, H, N_q, N_kv, D), big_head_dim_ok(D) ? probs_workspace_bytes(B, H, N_q, N_kv, D) : 0);
     const int ks = fwd_key_splits((int64_t)B * H, N_q, N_kv, padded_head_dim(D));
     return ks > 1 ? partials_bytes(ks, (int64_t)B * H * N_q, D) : 0;
+}
+
+size_t flame_attn_mask_workspace_bytes(int B, int H, int N_q, int N_kv, const int64_t* mask_strides, int has_kv_len, int causal) {
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !mask_strides) return 0;
+    static const uint8_t mask = 0;
+    static const int32_t len = 0;
+    MaskArgs m{};
+    m.mask = &mask;
+    m.kv_len = has_kv_len ? &len : nullptr;
+    m.sb = mask_strides[0]; m.sh = mask_strides[1]; m.sq = mask_strides[2]; m.sk = mask_strides[3];
+    m.causal = causal ? 1 : 0;
+    return mask_bits_bytes(m, B, H, N_q, N_kv);
 }
 
 int flame_attn_fwd_ws_bf16(const void* Q, const void* K, const void* V, void* O, void* LSE,

@@ -31,7 +31,7 @@ namespace {
 using at::Tensor;
 
 #define FLAME_HOST_ENTRY_POINTS(X)                                                                                      \
-    X(flame_attn_fwd_bf16) X(flame_attn_fwd_ws_bf16) X(flame_attn_fwd_scratch_bytes) X(flame_attn_fwd_bias_bf16)      \
+    X(flame_attn_fwd_bf16) X(flame_attn_fwd_ws_bf16) X(flame_attn_fwd_scratch_bytes) X(flame_attn_mask_workspace_bytes) X(flame_attn_fwd_bias_bf16) \
     X(flame_attn_bwd_bf16) X(flame_attn_bwd_workspace_bytes) X(flame_attn_fwd_dropout_tiled_bf16)                       \
     X(flame_attn_bwd_dropout_tiled_bf16) X(flame_attn_materialised_workspace_bytes) X(flame_attn_fwd_materialised_bf16) \
     X(flame_attn_bwd_materialised_bf16) X(flame_sage_quant_qk_int8_ks) X(flame_sage_attn_fwd_bias_int8)                 \
@@ -192,8 +192,9 @@ int call_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Sizes& z, 
     if (!o.defined()) o = empty({z.B, z.H, z.Sq, z.D}, at::kBFloat16, q);
     if (!lse.defined() && f.want_lse) lse = empty({(int64_t)z.B * z.H, z.Sq}, at::kFloat, q);
     Tensor ws = f.workspace;
-    if (!ws.defined() && !f.mask.data) {       // room for the slices of a key split, where the grid would leave compute units idle
-        const size_t need = g_api.flame_attn_fwd_scratch_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
+    if (!ws.defined()) {       // room for the slices of a key split, where the grid would leave compute units idle, or for the mask as bits
+        const size_t need = f.mask.data ? g_api.flame_attn_mask_workspace_bytes(z.B, z.H, z.Sq, z.Sk, f.mask.strides(), f.kv_len.defined(), f.causal)
+                                        : g_api.flame_attn_fwd_scratch_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
         if (need) ws = bytes_like(need, q);
     }
     if (ws.defined())
@@ -215,7 +216,11 @@ void alloc_grads(const Tensor& q, const Sizes& z, Grads& g) {
 }
 int call_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& d_o, const Tensor& lse, const Sizes& z, float scale,
              bool causal, const Tensor& kv_len, const MaskView& mask, Tensor workspace, Grads& g) {
-    if (!workspace.defined()) workspace = bytes_like(g_api.flame_attn_bwd_workspace_bytes(z.B, z.H, z.Sq, z.D), q);
+    if (!workspace.defined()) {
+        size_t need = g_api.flame_attn_bwd_workspace_bytes(z.B, z.H, z.Sq, z.D);
+        if (mask.data) need += g_api.flame_attn_mask_workspace_bytes(z.B, z.H, z.Sq, z.Sk, mask.strides(), kv_len.defined(), causal);
+        workspace = bytes_like(need, q);
+    }
     if (!g.dq.defined()) alloc_grads(q, z, g);
     return g_api.flame_attn_bwd_bf16(ptr(q), ptr(k), ptr(v), ptr(o), ptr(d_o), ptr(lse), ptr(g.dq), ptr(g.dk), ptr(g.dv), z.B, z.H, z.Sq, z.Sk, z.D,
                                      scale, strides4(q), strides4(k), strides4(v), strides4(o), strides4(d_o), strides4(g.dq), strides4(g.dk),

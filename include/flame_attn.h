@@ -95,6 +95,11 @@ int flame_attn_fwd_bf16(const void* Q, const void* K, const void* V, void* O, vo
  * src/cuda_graph.rs:11-18).  No counterpart in the reference's FFI. */
 size_t flame_attn_fwd_workspace_bytes(int B, int H, int N_q, int N_kv, int D);
 size_t flame_attn_fwd_scratch_bytes(int B, int H, int N_q, int N_kv, int D);
+/* Room that a keep-mask which differs by query is worth (0 for other masks): with that much workspace in
+ * flame_attn_fwd_ws_bf16, and that much beyond flame_attn_bwd_workspace_bytes (or within its optional part) in
+ * flame_attn_bwd_bf16, one pass turns the mask into bits and the kernels walk only the 64-key tiles it leaves something of,
+ * without a test per element where it leaves all of one.  Mask strides as in the calls (0 broadcasts). */
+size_t flame_attn_mask_workspace_bytes(int B, int H, int N_q, int N_kv, const int64_t* mask_strides, int has_kv_len, int causal);
 int flame_attn_fwd_ws_bf16(const void* Q, const void* K, const void* V, void* O, void* LSE,
                            int B, int H, int N_q, int N_kv, int D, float scale,
                            const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,

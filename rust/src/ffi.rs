@@ -94,6 +94,9 @@ extern "C" {
     pub fn flame_attn_fwd_scratch_bytes(
         b: c_int, h: c_int, n_q: c_int, n_kv: c_int, d: c_int
     ) -> usize;
+    pub fn flame_attn_mask_workspace_bytes(
+        b: c_int, h: c_int, n_q: c_int, n_kv: c_int, mask_strides: *const i64, has_kv_len: c_int, causal: c_int
+    ) -> usize;
     pub fn flame_attn_fwd_ws_bf16(
         q: *const c_void, k: *const c_void, v: *const c_void, o: *mut c_void, lse: *mut c_void, b: c_int,
         h: c_int, n_q: c_int, n_kv: c_int, d: c_int, scale: f32, q_strides: *const i64, k_strides: *const i64,
