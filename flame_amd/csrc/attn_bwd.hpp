@@ -42,6 +42,7 @@ struct BwdParams {
     int joint_n_dq = 0;            // bwd_joint_kernel: the first joint_n_dq workgroups are dQ workgroups
     float* split_ws = nullptr;
     size_t split_ws_bytes = 0;     // host side only
+    float dv_scale = 1.f;          // merge kernel: what the sums of dV are multiplied by (dropout: 1 / (1 - p))
     const uint16_t* q;
     const uint16_t* k;
     const uint16_t* v;
@@ -875,7 +876,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_merge_kernel(const BwdParams p) 
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             u32x2 wk = {pack_bf16(ak[g][0] * s, ak[g][1] * s), pack_bf16(ak[g][2] * s, ak[g][3] * s)};
-            u32x2 wv = {pack_bf16(av[g][0], av[g][1]), pack_bf16(av[g][2], av[g][3])};
+            u32x2 wv = {pack_bf16(av[g][0] * p.dv_scale, av[g][1] * p.dv_scale), pack_bf16(av[g][2] * p.dv_scale, av[g][3] * p.dv_scale)};
             if (dead) wk = wv = u32x2{0u, 0u};
             if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dkrow + 32 * db + 8 * g + 4 * h) = wk;
             if (32 * db + 8 * g + 4 * h < p.d) *reinterpret_cast<u32x2*>(dvrow + 32 * db + 8 * g + 4 * h) = wv;

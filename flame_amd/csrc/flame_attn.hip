@@ -241,6 +241,56 @@ int padded_head_dim(int D) { return D <= 64 ? 64 : 128; }
 size_t bwd_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
 size_t bwd_split_slot_bytes(int D) { return (size_t)2 * 128 * D * sizeof(float); }   // dK^T and dV^T of one 128-key block
 
+// Query tiles on at most half of the compute units: how many workgroups share the key walk of one of them, where the steps saved
+// outweigh the merge (about 5 us, a step being about 1 us).
+template <int D>
+int dq_walk_parts(const BwdParams& p, int64_t grid_dq) {
+    using TQ = BwdDqTile<D>;
+    const int cus = device_cu_count(), tiles = (p.Sk + TQ::BN - 1) / TQ::BN;
+    if (2 * grid_dq > cus || !p.split_ws) return 1;
+    int64_t parts = std::min<int64_t>(std::min<int64_t>(cus / grid_dq, 16), tiles / 4);
+    while (parts > 1 && (size_t)(grid_dq * parts) * (TQ::BM * D * sizeof(float)) > p.split_ws_bytes) --parts;
+    return parts > 1 && tiles - (tiles + parts - 1) / parts >= 12 ? (int)parts : 1;
+}
+
+// The dK/dV kernel keeps one workgroup per compute unit.  When the key blocks do not fill the last round of that schedule, the
+// blocks of the last round are split over the idle units along the query walk (fp32 partial sums, merged by a small second
+// kernel).  Needs equally long walks (no causal, key-length or explicit mask) and room in the workspace.  Sets n_whole and
+// split_parts; returns the number of workgroups, and that of the split key blocks in n_split.
+template <int D>
+int64_t dkdv_walk_parts(BwdParams& p, int64_t grid, bool uniform, int& n_split) {
+    using T = BwdTile<D>;
+    const int cus = device_cu_count();
+    const int64_t rem = grid % cus, n_qtiles = (p.Sq + T::BM - 1) / T::BM;
+    const size_t slot = bwd_split_slot_bytes(D);
+    n_split = 0;
+    if (!p.split_ws) return grid;
+    if (uniform && grid > cus && rem > 0 && 2 * rem <= cus && n_qtiles >= 16) {
+        int parts = (int)std::min<int64_t>(cus / rem, 4);
+        while (parts > 1 && (size_t)(rem * parts) * slot > p.split_ws_bytes) --parts;
+        if (parts > 1) {
+            p.n_whole = (int)(grid - rem);
+            p.split_parts = parts;
+            n_split = (int)rem;
+            return p.n_whole + rem * parts;
+        }
+    }
+    // Key blocks on at most half of the compute units (few keys or few heads): every one is split along its query walk,
+    // where the steps saved outweigh the merge (about 5 us, or 8 steps).  (B=8 H=1, 1993 queries, 64 keys, D = 64:
+    // 8 workgroups, dK/dV 30 us; 14 us with the split, backward 36.6 -> 25 us.)
+    if (2 * grid <= cus) {
+        int64_t parts = std::min<int64_t>(std::min<int64_t>(cus / grid, 16), n_qtiles / 4);
+        while (parts > 1 && (size_t)(grid * parts) * slot > p.split_ws_bytes) --parts;
+        if (parts > 1 && n_qtiles - (n_qtiles + parts - 1) / parts >= 12) {
+            p.n_whole = 0;
+            p.split_parts = (int)parts;
+            n_split = (int)grid;
+            return grid * parts;
+        }
+    }
+    return grid;
+}
+
 // The keep-mask as bits (mask_bits.hpp).  Planes: one per batch where the mask or, with key lengths, what they leave of it
 // differs by batch, one per head where it differs by head.  0 bytes: not for this call (a mask that is the same for every query has
 // kernels of its own, and a list of tiles holds 1024).
@@ -375,7 +425,8 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     const bool even = !p.m.causal && !p.m.kv_len;           // all walks equally long
     const bool wide_fits = !HASMASK && !p.key_mask && n256 * 256 <= ((int64_t)(p.Sq + 127) / 128) * 128 && total256 >= device_cu_count() &&
                            !(p.m.kv_len && total256 < 2 * device_cu_count()) && wg_waves_override() != 4;
-    const bool wide = wide_fits && (bwd_schedule_override() != 0 ||      // (a schedule asked for by name has 256-query workgroups)
+    const int joint_mode = wide_fits ? bwd_schedule_override() : 0;
+    const bool wide = wide_fits && (joint_mode != 0 ||      // (a schedule asked for by name has 256-query workgroups)
                                     (!(thin_last_round(total256, device_cu_count(), 2) && (!even || total256 < 2 * device_cu_count())) &&
                                      !(p.Sk <= 1024 && total256 % device_cu_count() != 0)));
     const int64_t n_qt = wide ? n256 : (p.Sq + TQ::BM - 1) / TQ::BM;
@@ -383,7 +434,6 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     // Equally long walks everywhere and 256-query workgroups: a pass over O and dO leaves the per-query rows in the
     // workspace, then dQ and dK/dV workgroups share one grid (bwd_joint_kernel).
-    const int joint_mode = bwd_schedule_override();
     if (joint_mode != 0 && wide && !HASMASK && !TIMING && !p.m.causal && !p.m.kv_len && p.split_ws) {
         static bool joint_attr_done = false;
         auto kern_joint = bwd_joint_kernel<D>;
@@ -453,15 +503,8 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
             hipLaunchKernelGGL(kern_dqk, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
         else if (HASMASK && p.m.rows16 && p.Sk % TQ::BN == 0) hipLaunchKernelGGL(kern_dqv, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
         else {
-            // query tiles on at most half of the compute units: their key walks are shared, where the steps saved outweigh the
-            // merge (about 5 us, a step being about 1 us)
             BwdParams pq = p;
-            const int tiles = (p.Sk + TQ::BN - 1) / TQ::BN;
-            if (!HASMASK && 2 * grid_dq <= device_cu_count() && p.split_ws) {
-                int64_t parts = std::min<int64_t>(std::min<int64_t>(device_cu_count() / grid_dq, 16), tiles / 4);
-                while (parts > 1 && (size_t)(grid_dq * parts) * (TQ::BM * D * sizeof(float)) > p.split_ws_bytes) --parts;
-                if (parts > 1 && tiles - (tiles + parts - 1) / parts >= 12) pq.dq_parts = (int)parts;
-            }
+            if (!HASMASK) pq.dq_parts = dq_walk_parts<D>(p, grid_dq);
             if (!HASMASK && pq.dq_parts == 1 && rule_key_groups(grid_dq, p.Sk, kDqGroupKeys))
                 hipLaunchKernelGGL(kern_dqg, dim3((unsigned)grid_dq), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pq);
             else
@@ -469,43 +512,9 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
             if (pq.dq_parts > 1) hipLaunchKernelGGL(bwd_dq_merge_kernel<D>, dim3((unsigned)(grid_dq * (D / 32))), dim3(256), 0, s, pq);
         }
     }
-    // The dK/dV kernel keeps one workgroup per compute unit.  When the key blocks do not fill the last
-    // round of that schedule, the blocks of the last round are split over the idle units along the query
-    // walk (fp32 partial sums, merged by a small second kernel).  Needs equally long walks (no causal,
-    // key-length or explicit mask) and room in the workspace.
     BwdParams pk = p;
-    int64_t grid_kv = grid;
     int n_split = 0;
-    {
-        const int cus = device_cu_count();
-        const int64_t rem = grid % cus;
-        const int64_t n_qtiles = (p.Sq + T::BM - 1) / T::BM;
-        const bool uniform = !HASMASK && !p.key_mask && !p.m.causal && !p.m.kv_len;
-        if (uniform && grid > cus && rem > 0 && 2 * rem <= cus && n_qtiles >= 16 && p.split_ws) {
-            int parts = (int)std::min<int64_t>(cus / rem, 4);
-            const size_t room = p.split_ws_bytes / bwd_split_slot_bytes(D);
-            while (parts > 1 && (size_t)(rem * parts) > room) --parts;
-            if (parts > 1) {
-                pk.n_whole = (int)(grid - rem);
-                pk.split_parts = parts;
-                n_split = (int)rem;
-                grid_kv = pk.n_whole + rem * parts;
-            }
-        }
-        // Key blocks on at most half of the compute units (few keys or few heads): every one is split along its query walk,
-        // where the steps saved outweigh the merge (about 5 us, or 8 steps).  (B=8 H=1, 1993 queries, 64 keys, D = 64:
-        // 8 workgroups, dK/dV 30 us; 14 us with the split, backward 36.6 -> 25 us.)
-        if (!HASMASK && 2 * grid <= cus && p.split_ws) {
-            int64_t parts = std::min<int64_t>(std::min<int64_t>(cus / grid, 16), n_qtiles / 4);
-            while (parts > 1 && (size_t)(grid * parts) * bwd_split_slot_bytes(D) > p.split_ws_bytes) --parts;
-            if (parts > 1 && n_qtiles - (n_qtiles + parts - 1) / parts >= 12) {
-                pk.n_whole = 0;
-                pk.split_parts = (int)parts;
-                n_split = (int)grid;
-                grid_kv = grid * parts;
-            }
-        }
-    }
+    const int64_t grid_kv = HASMASK ? grid : dkdv_walk_parts<D>(pk, grid, !p.key_mask && !p.m.causal && !p.m.kv_len, n_split);
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DKDV, s);
         if (HASMASK && !TIMING && p.m.rows16 && !p.m.causal && p.Sk % T::BN == 0 && p.Sq % T::BM == 0 &&
@@ -681,8 +690,10 @@ int launch_fwd_bigd(const FwdParams& p, hipStream_t s, const FwdScratch& sc) {
 // how the kernels draw (after set_dropout)
 int drop_mode(const MaskArgs& m, int Sk) { return m.drop_cq != 0 ? kDropTiled : Sk % 64 == 0 ? kDropRows64 : kDropFlat; }
 
-// Dropout of the probabilities: the 128-query forward and dQ kernels and the dK/dV kernel in their DROP
-// instantiations, without the split of the last round; HASMASK: the general kernels for an explicit mask or bias.
+// Dropout of the probabilities: the 128-query forward and dQ kernels and the dK/dV kernel in their DROP instantiations, walks
+// shared and last rounds split as without it; HASMASK: the general kernels for an explicit mask or bias.
+// (p = 0.1, forward and backward: B=1 H=1 S=4000 D=64 228 -> 110 us, B=1 H=2 S=1000 D=64 73 -> 50 us with the walks shared;
+// B=1 H=12 S=3000, the last round split, D=64 356 -> 307 us, D=128 457 -> 400 us.)
 template <int D>
 int launch_fwd_dropout(const FwdParams& p, bool has_mask, hipStream_t s) {
     if (has_mask) return launch_fwd<D, kExGeneral, 4, kDropTiled>(p, s);
@@ -710,12 +721,23 @@ int launch_bwd_drop(const BwdParams& p, hipStream_t s) {
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);        // first: it leaves -delta and the rescaled LSE rows
-        if (!HASMASK && p.dq_parts == 1 && rule_key_groups(grid_dq, p.Sk, kDqGroupKeys)) hipLaunchKernelGGL(kern_dqg, dim3((unsigned)grid_dq), dim3(256 * KG), KG * TQ::LDS_BYTES, s, p);
-        else hipLaunchKernelGGL(kern_dq, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
+        BwdParams pq = p;
+        if (!HASMASK) pq.dq_parts = dq_walk_parts<D>(p, grid_dq);
+        if (!HASMASK && pq.dq_parts == 1 && rule_key_groups(grid_dq, p.Sk, kDqGroupKeys)) hipLaunchKernelGGL(kern_dqg, dim3((unsigned)grid_dq), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pq);
+        else hipLaunchKernelGGL(kern_dq, dim3((unsigned)(grid_dq * pq.dq_parts)), dim3(256), TQ::LDS_BYTES, s, pq);
+        if (pq.dq_parts > 1) hipLaunchKernelGGL(bwd_dq_merge_kernel<D>, dim3((unsigned)(grid_dq * (D / 32))), dim3(256), 0, s, pq);
     }
+    BwdParams pk = p;
+    int n_split = 0;
+    const int64_t grid_kv = HASMASK ? grid : dkdv_walk_parts<D>(pk, grid, !p.m.causal && !p.m.kv_len, n_split);
+    if (DROP == kDropFlat || DROP == kDropRows64) pk.dv_scale = p.m.drop_scale;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DKDV, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES_DROP, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid_kv), dim3(256), T::LDS_BYTES_DROP, s, pk);
+    }
+    if (n_split > 0) {
+        ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_MERGE, s);
+        hipLaunchKernelGGL(bwd_dkdv_merge_kernel<D>, dim3((unsigned)(n_split * (D / 32))), dim3(256), 0, s, pk);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
