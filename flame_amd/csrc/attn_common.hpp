@@ -289,13 +289,18 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* p) {
     return __builtin_bit_cast(u32x2, v);
 }
 
-// 16-byte-granule XOR swizzle of a row-major bf16 tile whose rows are D*2 bytes (no padding).
+// Elements between the rows of a tile in LDS.  The tiles of the kernels compiled for head dim 96 keep the layout of 128: six of
+// eight steps of every contraction and three of four column blocks are computed, the last 32 columns of a row are never read.
+template <int D>
+constexpr int kRowPitch = D == 96 ? 128 : D;
+
+// 16-byte-granule XOR swizzle of a row-major bf16 tile whose rows are kRowPitch<D> * 2 bytes (no padding).
 // 16 consecutive rows get distinct bank groups for the same logical granule, and 4 consecutive rows
 // land in 4 disjoint 64-byte bank groups: both access patterns used by the kernels (16-byte row
 // reads, transposing 8-byte reads of a 4-row x 64-byte block) are conflict-free on the 64-bank LDS.
 template <int D>
 __device__ __forceinline__ constexpr int swz(int row) {
-    return D == 128 ? (((row & 3) << 2) | ((row >> 2) & 3)) : ((((row >> 1) & 1) << 2) | ((row >> 2) & 3));
+    return kRowPitch<D> == 128 ? (((row & 3) << 2) | ((row >> 2) & 3)) : ((((row >> 1) & 1) << 2) | ((row >> 2) & 3));
 }
 
 // One wave-wide asynchronous copy global -> LDS: lane l delivers 16 (or 4) bytes to lds_dst + 16*l (4*l).
@@ -394,20 +399,20 @@ struct Strides {
 // neither side has bank conflicts) and an instruction writes whole lines.  dK/dV of 256 key blocks, D = 128: 4.1 -> 1.9 us
 // from the last step to the last store, D = 64 1.9 -> 1.1 us; forward and backward of B=3 H=16 128 x 138 D=128 31.4 -> 28.6 us,
 // of B=4 H=16 1101 x 1101 D=128 with a key-padding mask 162 -> 155 us, of B=1 H=24 4608 x 4608 D=128 995 -> 985 us.
-// own: 32 x D elements of LDS that only this wavefront touches; quad(db, g): columns 32 db + 8 g + 4 h .. + 3 of row n;
+// own: 32 x kRowPitch<D> elements of LDS that only this wavefront touches; quad(db, g): columns 32 db + 8 g + 4 h .. + 3 of row n;
 // rows: how many of the 32 exist; d: real head dim, a multiple of 8.  out and row_stride keep rows on 16 bytes.
 template <int D, class F>
 __device__ __forceinline__ void store_rows32(uint16_t* own, uint16_t* out, int64_t row_stride, int rows, int d, F&& quad) {
-    constexpr int GPR = D / 8;
+    constexpr int RS = kRowPitch<D>, GPR = RS / 8;
     const int lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) *reinterpret_cast<u32x2*>(own + n * D + (((4 * db + g) ^ swz<D>(n)) << 3) + 4 * h) = quad(db, g);
+        for (int g = 0; g < 4; ++g) *reinterpret_cast<u32x2*>(own + n * RS + (((4 * db + g) ^ swz<D>(n)) << 3) + 4 * h) = quad(db, g);
 #pragma unroll
     for (int i = 0; i < GPR / 2; ++i) {
         const int row = (i * 64 + lane) / GPR, g = (i * 64 + lane) % GPR;
-        const u32x4 w = *reinterpret_cast<const u32x4*>(own + row * D + ((g ^ swz<D>(row)) << 3));
+        const u32x4 w = *reinterpret_cast<const u32x4*>(own + row * RS + ((g ^ swz<D>(row)) << 3));
         if (row < rows && 8 * g < d) *reinterpret_cast<u32x4*>(out + row * row_stride + 8 * g) = w;
     }
 }
@@ -462,7 +467,7 @@ __device__ __forceinline__ void fragments_of_rows32(uint16_t* own, const u32x4 (
     });
 }
 
-// Head dims below the compiled one (any multiple of 8, e.g. 96 on the 128-wide kernels) run zero-padded:
+// Head dims below the compiled one (any multiple of 8, e.g. 80 on the 96-wide kernels) run zero-padded:
 // fragments loaded straight from global memory are zero past the real head dim, tile copies re-read
 // granule 0 of their row there (finite values that only ever meet those zero operands, or land in
 // output rows past the real head dim, which are not stored), and stores skip those rows.

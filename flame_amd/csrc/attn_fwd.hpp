@@ -48,12 +48,12 @@ struct FwdParams {
 template <int D>
 struct FwdTile {
     static constexpr int BN = 64;                   // keys per tile
-    static constexpr int RS = D;                    // LDS row stride, elements
-    static constexpr int TILE_ELEMS = BN * D;       // one K or V tile
+    static constexpr int RS = kRowPitch<D>;         // LDS row stride, elements
+    static constexpr int TILE_ELEMS = BN * RS;      // one K or V tile
     static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;
     static constexpr int LDS_BYTES = 2 * STAGE_ELEMS * 2;
     static constexpr int BIAS_PASS_BYTES = 4 * 2048;             // behind the stages: 2 KiB per wavefront that bias rows pass through
-    static constexpr int ROWS_PER_DMA = 1024 / (D * 2);          // rows covered by one 64-lane x 16-byte copy
+    static constexpr int ROWS_PER_DMA = 1024 / (RS * 2);         // rows covered by one 64-lane x 16-byte copy
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;   // copies per wave and tensor
 };
 
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     constexpr int BM = 32 * NW;  // query rows per workgroup
     constexpr int DC = D / 16;   // contraction chunks of QK^T
     constexpr int DB = D / 32;   // 32-row blocks of O^T
-    constexpr int GPR = D / 8;   // 16-byte granules per row
+    constexpr int GPR = RS / 8;  // 16-byte granules per row in LDS
     constexpr int NDMA = T::DMA_PER_WAVE * 4 / NW;
     constexpr int PD = 4;        // LDS read-ahead depth, in fragments
     // Tile t lives in stage t % 2; K runs 2 tiles and V 1 tile ahead of use, one barrier per step.
@@ -83,7 +83,6 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     // workgroup that has its compute unit to itself: the step is bound by instruction issue, not by the copies.)
     constexpr int KD = 2, VD = 1;
     static_assert((2 * DC) % PD == 0 && (4 * DB) % PD == 0, "read-ahead depth must divide the fragment counts");
-    static_assert(2 * DC == 16 || 2 * DC == 8, "softmax slicing assumes 16 or 8 logit MFMAs per tile");
 
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds_all[];
 
@@ -252,8 +251,8 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
 
     constexpr int NS = 2 * DC;     // logit MFMAs per tile
     constexpr int NP = 4 * DB;     // PV MFMAs per tile
-    constexpr int EPS = 32 / NS;   // logits handled per softmax slice
-    constexpr int MPS = 32 / NP;   // logits handled per maximum-scan slice
+    // logits 32 j / NS to 32 (j + 1) / NS belong to softmax slice j, pairs 16 i / NP to 16 (i + 1) / NP to maximum-scan slice i
+    constexpr int EPS = (32 + NS - 1) / NS, PPS = (16 + NP - 1) / NP;
 
     // DROP: flat index (mod 2^32) of this lane's first element of the row in the [B*H, Sq, Sk] probability tensor
     const uint32_t drop_row = ((uint32_t)bh * (uint32_t)p.Sq + (uint32_t)qi) * (uint32_t)p.Sk + (uint32_t)key0 + 4 * h;
@@ -414,13 +413,14 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         const uint32_t drop_tile = drop_row + (uint32_t)(t * BN), drop_word = DROP == kDropRows64 ? xorshift32(p.m.drop_seed ^ drop_tile) : 0u;
         (void)drop_tile;
         (void)drop_word;
-        // P(t): slice j covers logits [EPS*j, EPS*j + EPS) of the tile in (kb, r) order
+        // P(t): the logits of the tile in (kb, r) order
         auto exp_slice = [&](int j) {
 #pragma unroll
             for (int e = 0; e < EPS; ++e) {
-                const int idx = EPS * j + e, kb = idx >> 4, r = idx & 15;
+                const int idx = 32 * j / NS + e, kb = idx >> 4, r = idx & 15;
+                if (idx >= 32 * (j + 1) / NS) continue;
                 const float v = exp2_fast(fmaf(cur[kb][r], c_log2, -msc));
-                if (e & 1) rsum1 += v;
+                if (idx & 1) rsum1 += v;
                 else rsum0 += v;
                 const uint32_t off = 32 * kb + 8 * (r >> 2) + (r & 3);       // of the element, from drop_tile
                 if constexpr (DROP == kDropTiled) {
@@ -488,8 +488,9 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             auto max_slice = [&](int i) {
                 if (BIAS && i % (NP / NPASS) == 0 && i / (NP / NPASS) + 1 < NPASS) bias_pass(i / (NP / NPASS) + 1);
 #pragma unroll
-                for (int e = 0; e < MPS; e += 2) {
-                    const int idx = MPS * i + e;
+                for (int e = 0; e < PPS; ++e) {
+                    const int idx = 2 * (16 * i / NP + e);
+                    if (idx >= 2 * (16 * (i + 1) / NP)) continue;
                     if (NEXT == 1 || BIAS) {
                         excl_elem(nxt, idx);
                         excl_elem(nxt, idx + 1);
@@ -627,7 +628,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
 
     // ---- epilogue: O through LDS where nobody reads any more (KG: the state of the second group this wavefront has joined)
     if constexpr (KG == 1) __syncthreads();
-    uint16_t* own = KG == 1 ? lds + wave * 32 * D : lds_all + wave * (4 * DB + 1) * 64 * 8;
+    uint16_t* own = KG == 1 ? lds + wave * 32 * RS : lds_all + wave * (4 * DB + 1) * 64 * 8;
     const float l = l_run + xhalf(l_run);
     float inv = l > 0.f ? 1.0f / l : 0.f;
     if constexpr (DROP == kDropFlat || DROP == kDropRows64) inv *= p.m.drop_scale;
@@ -692,12 +693,12 @@ template <int D>
 struct FwdWideTile {
     static constexpr int BM = 256;
     static constexpr int BN = 64;
-    static constexpr int RS = D;
-    static constexpr int TILE_ELEMS = BN * D;
+    static constexpr int RS = kRowPitch<D>;
+    static constexpr int TILE_ELEMS = BN * RS;
     static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;
     static constexpr int NSTAGE = 4;
     static constexpr int LDS_BYTES = NSTAGE * STAGE_ELEMS * 2;
-    static constexpr int ROWS_PER_DMA = 1024 / (D * 2);
+    static constexpr int ROWS_PER_DMA = 1024 / (RS * 2);
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;
 };
 
@@ -705,13 +706,12 @@ template <int D>
 __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
     using T = FwdWideTile<D>;
     constexpr int BN = T::BN, RS = T::RS, BM = T::BM;
-    constexpr int DC = D / 16, DB = D / 32, GPR = D / 8;
+    constexpr int DC = D / 16, DB = D / 32, GPR = RS / 8;
     constexpr int NDMA = T::DMA_PER_WAVE;
     constexpr int PD = 4;
     constexpr int NKF = 2 * DC;          // K fragments per tile (dc, kb); two logit MFMAs each
     constexpr int NVF = 4 * DB;          // V^T fragments per tile (16-key chunk, db); two PV MFMAs each
     static_assert(NKF % PD == 0 && NVF % PD == 0, "read-ahead depth must divide the fragment counts");
-    static_assert(NKF == 16 || NKF == 8, "softmax slicing assumes 16 or 8 K fragments per tile");
     static_assert(DB <= 4, "O^T tuples are pinned four to a query block");
 
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
@@ -897,13 +897,14 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
 
         {
             constexpr int NSL = 2 * NKF;             // MFMA slots of the logit phase
-            static_assert(NSL == 32 || NSL == 16, "slicing");
             // copies of K(t+3) and V(t+2); copy j goes with slot CS*j + 1
             constexpr int NCOPY = 2 * NDMA, CS = (NSL - 2) / NCOPY;
             // exponentials per slot and query block: the first key block's in the logit phase, the second's
             // in the first half of the other phase, whose slots have the vector unit to spare
-            constexpr int E1 = 16 / NKF, E2 = 32 / NVF;
-            static_assert(E1 >= 1 && E2 >= 2 && E2 % 2 == 0, "slicing");
+            constexpr int HV = NVF / 2;
+            constexpr auto e1 = [](int i) { return 16 * i / NKF; };        // the first of slot i
+            constexpr auto e2 = [](int i) { return 16 * i / HV; };
+            constexpr auto scan = [](int k) { return 32 * k / HV; };       // of the row maximum, in the second half
             static_assert(CS >= 2, "copies do not fit the logit phase");
             auto copy_dst = [&](int g) {
                 const int j = (g - 1) / CS;
@@ -931,13 +932,13 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
                     mfma32_vgpr_bpinned<qb * DC + (i >> 1), (i >> 1) == 0 ? 0 : 1>(nxt[qb][i & 1], fb[i % PD], qf[qb][i >> 1], nxt[qb][i & 1]);
                     __builtin_amdgcn_sched_barrier(0);
                     copy_issue(g);
-                    // slot g: exponentials of E1 logits of the first key block of query block qb, packing of
-                    // the pairs that were complete a slot ago
+                    // slot g: exponentials of logits of the first key block of query block qb, packing of the pairs that
+                    // were complete a slot ago
 #pragma unroll
-                    for (int e = 0; e < E1; ++e) exp_elem(qb, E1 * i + e);
+                    for (int e = e1(i); e < e1(i + 1); ++e) exp_elem(qb, e);
                     if (i > 0) {
 #pragma unroll
-                        for (int j = E1 * (i - 1) / 2; j < E1 * i / 2; ++j) pack_pair(qb, j);
+                        for (int j = e1(i - 1) / 2; j < e1(i) / 2; ++j) pack_pair(qb, j);
                     }
                     // the ring is refilled two fragments at a time, so that one wait covers both
                     if (qb == 1 && (i & 1)) {
@@ -953,7 +954,7 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb) {
 #pragma unroll
-                for (int j = E1 * (NKF - 1) / 2; j < 8; ++j) pack_pair(qb, j);
+                for (int j = e1(NKF - 1) / 2; j < 8; ++j) pack_pair(qb, j);
             }
             // ---- O^T += V(t)^T P(t)^T, with the rest of the exponentials and the row-maximum scan of tile t+1
             float tmax[2];
@@ -969,25 +970,21 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
                     }
                     oacc[qb][db] = mfma32(fb[i % PD], __builtin_bit_cast(bf16x8, pw[qb][cc]), oacc[qb][db]);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (i < NVF / 2) {
-                        // first half: the exponentials of the second key block, due at slot NVF / 2
+                    if (i < HV) {
+                        // first half: the exponentials of the second key block, due at slot HV
 #pragma unroll
-                        for (int e = 0; e < E2; ++e) exp_elem(qb, 16 + E2 * i + e);
+                        for (int e = e2(i); e < e2(i + 1); ++e) exp_elem(qb, 16 + e);
                     }
-                    if (i >= 1 && i <= NVF / 2) {
+                    if (i >= 1 && i <= HV) {
 #pragma unroll
-                        for (int j = 8 + E2 * (i - 1) / 2; j < 8 + E2 * i / 2; ++j) pack_pair(qb, j);
+                        for (int j = 8 + e2(i - 1) / 2; j < 8 + e2(i) / 2; ++j) pack_pair(qb, j);
                     }
-                    if (i >= NVF / 2) {
+                    if (i >= HV) {
                         // second half: row maximum of tile t+1 (its logits may be touched from slot 2 on)
-                        constexpr int MPS = 64 / NVF;     // logits per slot and block
-                        constexpr int k = i - NVF / 2;
+                        constexpr int k = i - HV;
                         if (k == 0) tmax[qb] = nxt[qb][0][0];
 #pragma unroll
-                        for (int e = 0; e < MPS; ++e) {
-                            const int idx = MPS * k + e;
-                            tmax[qb] = fmaxf(tmax[qb], nxt[qb][idx >> 4][idx & 15]);
-                        }
+                        for (int idx = scan(k); idx < scan(k + 1); ++idx) tmax[qb] = fmaxf(tmax[qb], nxt[qb][idx >> 4][idx & 15]);
                         // the scan feeds nothing before the end of the step: keep this slot's part in this slot
                         asm volatile("" : "+v"(tmax[qb]));
                     }
@@ -1074,7 +1071,7 @@ __global__ __launch_bounds__(256) void fwd_wide_kernel(const FwdParams p) {
         const int row = qrow[qb], row0 = qw0 + 32 * qb;
         const float l = l_run[qb] + xhalf(l_run[qb]);
         const float inv = l > 0.f ? 1.0f / l : 0.f;
-        store_rows32<D>(lds + wave * 32 * D, obase + (int64_t)row0 * p.os.n, p.os.n, p.Sq - row0, p.dv, [&](int db, int g) {
+        store_rows32<D>(lds + wave * 32 * RS, obase + (int64_t)row0 * p.os.n, p.os.n, p.Sq - row0, p.dv, [&](int db, int g) {
             const f32x16& a = oacc[qb][db];
             return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
         });

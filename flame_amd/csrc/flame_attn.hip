@@ -209,7 +209,7 @@ int launch_fwd_wide(FwdParams p, hipStream_t s) {
     }
     if (r.count) {
         p.wg_base = (int)r.base;
-        return r.rows == 32 ? launch_fwd_keyshare<D, false>(p, s, r.count) : launch_fwd<D, kExNone, 4>(p, s, r.count);
+        return r.rows == 32 ? launch_fwd_keyshare<kRowPitch<D>, false>(p, s, r.count) : launch_fwd<D, kExNone, 4>(p, s, r.count);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -230,12 +230,16 @@ int bwd_schedule_override() {
     return strcmp(v, "joint") == 0 ? 1 : strcmp(v, "rows") == 0 ? 2 : 0;
 }
 
-// Head dims: the kernels are compiled for 64 and 128; any other multiple of 8 up to 128 (96 among them) runs
-// zero-padded on the next compiled size.
+// Head dims: the kernels are compiled for 64 and 128, those of the main paths for 96 as well (narrow); any other multiple of 8
+// up to 128 runs zero-padded on the next compiled size.
 bool head_dim_ok(int D) { return D > 0 && D <= 128 && D % 8 == 0; }
 // head dims served by the forward alone, in chunks of 128 (attn_fwd_bigd.hpp)
 bool big_head_dim_ok(int D) { return D > 128 && D <= 512 && D % 8 == 0; }
 int padded_head_dim(int D) { return D <= 64 ? 64 : 128; }
+// Head dims above 64 and up to 96 (72, 80 and 96 among them): a quarter of the matrix work of 128 is padding.
+// (Forward, us: B=1 H=24 S=4608 D=96 215 -> 189, B=1 H=16 S=8192 D=96 causal 238 -> 201, B=2 H=16 S=1500 D=80 with a key mask
+// 45 -> 39.5, B=4 H=8 S=300 D=72 9.9 -> 8.8.)
+bool narrow(int D) { return D > 64 && D <= 96; }
 
 // backward workspace: [-delta rows][lse2 rows][fp32 partials of the split dK/dV workgroups]
 size_t bwd_rows_bytes(int B, int H, int N_q) { return 2 * align_up((size_t)B * H * N_q * sizeof(float), 256); }
@@ -696,7 +700,8 @@ int drop_mode(const MaskArgs& m, int Sk) { return m.drop_cq != 0 ? kDropTiled : 
 // B=1 H=12 S=3000, the last round split, D=64 356 -> 307 us, D=128 457 -> 400 us.)
 template <int D>
 int launch_fwd_dropout(const FwdParams& p, bool has_mask, hipStream_t s) {
-    if (has_mask) return launch_fwd<D, kExGeneral, 4, kDropTiled>(p, s);
+    if constexpr (D != 96)       // (a mask or bias with dropout keeps the kernels of 128)
+        if (has_mask) return launch_fwd<D, kExGeneral, 4, kDropTiled>(p, s);
     switch (drop_mode(p.m, p.Sk)) {
         case kDropRows64: return launch_fwd<D, kExNone, 4, kDropRows64>(p, s);
         case kDropFlat: return launch_fwd<D, kExNone, 4, kDropFlat>(p, s);
@@ -1230,6 +1235,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         // the log-sum-exp is that of the undropped softmax, its sum joined in another order where that call splits
         if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q))
             return DP == 128 ? launch_fwd_keyshare<128, true>(p, s) : launch_fwd_keyshare<64, true>(p, s);
+        if (DP == 128 && narrow(std::max(D, Dv)) && !hm) return launch_fwd_dropout<96>(p, hm, s);
         return DP == 128 ? launch_fwd_dropout<128>(p, hm, s) : launch_fwd_dropout<64>(p, hm, s);
     }
     // 256-query workgroups when they neither add padding rows nor leave compute units
@@ -1241,6 +1247,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     // ... as 4 wavefronts of 64 queries when nothing is excluded at all, else as 8 wavefronts of 32 (D = 128 only)
     const bool plain = !causal && kv_len == nullptr && N_kv % 64 == 0;
     const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
+    const bool d96 = narrow(std::max(D, Dv));
     if (wide && !plain && DP == 64) wide = false;
     if (wide && q_tile_plan == 0) {
         const int64_t total256 = (int64_t)((N_q + 255) / 256) * B * H, cus = device_cu_count();
@@ -1249,11 +1256,11 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     }
     // a keep-mask of keys: the walk takes the attended tiles only (up to what their list holds)
     if (keep_mask != nullptr && bias == nullptr && keys_only(p.m, N_q, N_kv))
-        return DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
+        return d96 ? launch_fwd<96, kExKeys, 4>(p, s) : DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
     // any other keep-mask, with room for it as bits
     if (keep_mask != nullptr && bias == nullptr && mask_bits_fit(p.m, B, H, N_q, N_kv, scratch.ws, scratch.bytes)) {
         if ((rc = launch_mask_bits(p.m, B, H, N_q, N_kv, scratch.ws, s))) return rc;
-        return DP == 128 ? launch_fwd<128, kExBits, 4>(p, s) : launch_fwd<64, kExBits, 4>(p, s);
+        return d96 ? launch_fwd<96, kExBits, 4>(p, s) : DP == 128 ? launch_fwd<128, kExBits, 4>(p, s) : launch_fwd<64, kExBits, 4>(p, s);
     }
     // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel
     if (keep_mask != nullptr && bias == nullptr && p.m.rows16 && N_kv % 64 == 0)
@@ -1265,8 +1272,8 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     }
     if (hm) return DP == 128 ? launch_fwd<128, kExGeneral, 4>(p, s) : launch_fwd<64, kExGeneral, 4>(p, s);
     if (wide) {
-        if (plain) return DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
-        return launch_fwd<128, kExNone, 8>(p, s);
+        if (plain) return d96 ? launch_fwd_wide<96>(p, s) : DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
+        return d96 ? launch_fwd<96, kExNone, 8>(p, s) : launch_fwd<128, kExNone, 8>(p, s);
     }
     if (q_tile_plan == 0 && fwd_rule_keyshare((int64_t)B * H, N_q)) {
         const int64_t rows = (int64_t)B * H * N_q;
@@ -1278,7 +1285,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         }
         return DP == 128 ? launch_fwd_keyshare<128, false>(p, s) : launch_fwd_keyshare<64, false>(p, s);
     }
-    return DP == 128 ? launch_fwd<128, kExNone, 4>(p, s) : launch_fwd<64, kExNone, 4>(p, s);
+    return d96 ? launch_fwd<96, kExNone, 4>(p, s) : DP == 128 ? launch_fwd<128, kExNone, 4>(p, s) : launch_fwd<64, kExNone, 4>(p, s);
 }
 
 
