@@ -68,7 +68,7 @@ template <int D>
 struct BwdTile {
     static constexpr int BM = 64;                   // query rows per step
     static constexpr int BN = 128;                  // keys per workgroup
-    static constexpr int RS = D;                    // LDS row stride of the Q / dO / K / V tiles (swizzled, unpadded)
+    static constexpr int RS = kRowPitch<D>;         // LDS row stride of the Q / dO / K / V tiles (swizzled)
     static constexpr int Q_ELEMS = BM * RS;
     static constexpr int STAGE_ELEMS = 2 * Q_ELEMS;               // Q tile + dO tile (also one 128-row tile)
     static constexpr int ROW_FLOATS = 2 * BM;                     // lse2 and -delta of one step
@@ -80,7 +80,7 @@ struct BwdTile {
     static constexpr int LDS_BYTES_VECMASK = LDS_BYTES + NSTAGE * MASK_STAGE_BYTES;
     // kDropRows64: the generator's word of every query row at each wavefront's first key, behind the rest
     static constexpr int LDS_BYTES_DROP = LDS_BYTES + 4 * BM * 4;
-    static constexpr int ROWS_PER_DMA = 1024 / (D * 2);
+    static constexpr int ROWS_PER_DMA = 1024 / (RS * 2);
     static constexpr int DMA_PER_WAVE = BM / ROWS_PER_DMA / 4;    // 1 KiB copies per wave and tensor
 };
 
@@ -108,7 +108,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     constexpr int BM = T::BM, BN = T::BN, RS = T::RS;
     constexpr int DC = D / 16;     // contraction chunks over the head dim
     constexpr int DB = D / 32;     // 32-row blocks of dK^T / dV^T
-    constexpr int GPR = D / 8;     // 16-byte granules per row
+    constexpr int GPR = RS / 8;    // 16-byte granules per row in LDS
     constexpr int RPD = T::ROWS_PER_DMA, NDQ = T::DMA_PER_WAVE;
 
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
@@ -189,7 +189,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         for (int db = 0; db < D / 32; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) zero[db][r] = 0.f;
-        dkdv_store<D>(p, lds + wave * 32 * D, zero, zero, b, hh, kw0);
+        dkdv_store<D>(p, lds + wave * 32 * RS, zero, zero, b, hh, kw0);
         return;
     }
     const int n_it = BITS ? qtiles.n_tiles : n_qt - qt_begin;
@@ -556,12 +556,16 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
                 pf[qb][c] = pack8(s[o8], s[o8 + 1], s[o8 + 2], s[o8 + 3], s[o8 + 4], s[o8 + 5], s[o8 + 6], s[o8 + 7]);
             }
         };
-        // slice s (of NS per block) of the element-wise work: one logit register for D = 128, two for D = 64;
-        // slice NS is the last product
+        // slice s (of NS per block) of the element-wise work: logit registers 16 s / NS to 16 (s + 1) / NS; slice NS is the
+        // last product
         auto elem_slot = [&](int qb, int s) {
-            if (s == NS) ds_mul(qb, 15);
-            else if (NS == 16) elem(qb, s);
-            else { elem(qb, 2 * s); elem(qb, 2 * s + 1); }
+            if (s == NS) {
+                ds_mul(qb, 15);
+                return;
+            }
+#pragma unroll
+            for (int e = 0; e < (16 + NS - 1) / NS; ++e)
+                if (16 * s / NS + e < 16 * (s + 1) / NS) elem(qb, 16 * s / NS + e);
         };
 
         // copies of the next tile, one instruction at a time (full tiles: uniform base + lane offset), each
@@ -813,7 +817,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
             }
     }
     __syncthreads();              // nobody reads a tile any more
-    dkdv_store<D>(p, lds + wave * 32 * D, dkacc, dvacc, b, hh, kw0, DROP == kDropFlat || DROP == kDropRows64 ? p.m.drop_scale : 1.0f);
+    dkdv_store<D>(p, lds + wave * 32 * RS, dkacc, dvacc, b, hh, kw0, DROP == kDropFlat || DROP == kDropRows64 ? p.m.drop_scale : 1.0f);
 }
 
 template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone, bool BITS = false>
@@ -889,11 +893,11 @@ template <int D>
 struct BwdDqTile {
     static constexpr int BM = 128;                  // query rows per workgroup (32 per wavefront)
     static constexpr int BN = 64;                   // keys per tile
-    static constexpr int RS = D;
-    static constexpr int TILE_ELEMS = BN * D;
+    static constexpr int RS = kRowPitch<D>;
+    static constexpr int TILE_ELEMS = BN * RS;
     static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;            // K tile + V tile
     static constexpr int LDS_BYTES = 2 * STAGE_ELEMS * 2;
-    static constexpr int ROWS_PER_DMA = 1024 / (D * 2);
+    static constexpr int ROWS_PER_DMA = 1024 / (RS * 2);
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;
 };
 
@@ -910,7 +914,7 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     constexpr int BM = 32 * NW, BN = T::BN, RS = T::RS;
     constexpr int DC = D / 16;
     constexpr int DB = D / 32;
-    constexpr int GPR = D / 8;
+    constexpr int GPR = RS / 8;
 
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds_all[];
 
@@ -1096,7 +1100,6 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         constexpr int COPY = decltype(copy_tag)::value;
         constexpr int BUF = decltype(buf_tag)::value;
         constexpr int PD = 4;
-        static_assert(DC % PD == 0 && (2 * DB) % PD == 0, "read-ahead depth must divide the fragment counts");
         const int buf = BUF >= 0 ? BUF : (t & 1);
         if (COPY == 1) issue_full_tile(t + 1, buf ^ 1);
         else if (t + 1 < n_tiles) issue_tile(t + 1, buf ^ 1);
@@ -1188,8 +1191,9 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
                 dsf[kb][r >> 3] = pack8(d[o8], d[o8 + 1], d[o8 + 2], d[o8 + 3], d[o8 + 4], d[o8 + 5], d[o8 + 6], d[o8 + 7]);
             }
         };
-        constexpr int EPM = 16 / DC;                // logits per MFMA slot in the row phases
-        constexpr int EPQ = 16 / (2 * DB);          // ... and in the dQ phases
+        // logits per MFMA slot of a phase: slot s of n has 16 s / n to 16 (s + 1) / n
+        static_assert(DC == 2 * DB, "the phases have the same number of slots");
+        constexpr int EPM = (16 + DC - 1) / DC;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -1208,7 +1212,8 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
                 fb[f % PD] = fetch(f + PD);
 #pragma unroll
                 for (int e = 0; e < EPM; ++e) {
-                    const int r = EPM * dc + e;
+                    const int r = 16 * dc / DC + e;
+                    if (r >= 16 * (dc + 1) / DC) continue;
                     if (PH == 1) p_elem(0, r);
                     if (PH == 2) ds_elem(0, r);
                     if (PH == 3) p_elem(1, r);
@@ -1225,7 +1230,8 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
                 if (f + PD < NALL) fb[f % PD] = fetch(f + PD);
                 if (KB == 0) {
 #pragma unroll
-                    for (int e = 0; e < EPQ; ++e) ds_elem(1, EPQ * g + e);
+                    for (int e = 0; e < EPM; ++e)
+                        if (16 * g / DC + e < 16 * (g + 1) / DC) ds_elem(1, 16 * g / DC + e);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1292,7 +1298,7 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         return;
     }
     // ... or dQ = scale * dQ^T, bf16 (every walk ended with a barrier: the tiles are free)
-    store_rows32<D>(lds_all + wave * 32 * D, p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)qw0 * p.dqs.n, p.dqs.n, p.Sq - qw0, p.d, [&](int db, int g) {
+    store_rows32<D>(lds_all + wave * 32 * RS, p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)qw0 * p.dqs.n, p.dqs.n, p.Sq - qw0, p.d, [&](int db, int g) {
         const f32x16& a = dqacc[db];
         return u32x2{pack_bf16(a[4 * g] * p.scale, a[4 * g + 1] * p.scale), pack_bf16(a[4 * g + 2] * p.scale, a[4 * g + 3] * p.scale)};
     });
@@ -1340,12 +1346,12 @@ template <int D>
 struct BwdDqWideTile {
     static constexpr int BM = 256;                  // query rows per workgroup (64 per wavefront)
     static constexpr int BN = 64;                   // keys per tile
-    static constexpr int RS = D;
-    static constexpr int TILE_ELEMS = BN * D;
+    static constexpr int RS = kRowPitch<D>;
+    static constexpr int TILE_ELEMS = BN * RS;
     static constexpr int STAGE_ELEMS = 2 * TILE_ELEMS;            // K tile + V tile
     static constexpr int NSTAGE = 3;
     static constexpr int LDS_BYTES = NSTAGE * STAGE_ELEMS * 2;
-    static constexpr int ROWS_PER_DMA = 1024 / (D * 2);
+    static constexpr int ROWS_PER_DMA = 1024 / (RS * 2);
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;    // 1 KiB copies per wave and tensor
 };
 
@@ -1355,7 +1361,7 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     constexpr int BM = T::BM, BN = T::BN, RS = T::RS;
     constexpr int DC = D / 16;
     constexpr int DB = D / 32;
-    constexpr int GPR = D / 8;
+    constexpr int GPR = RS / 8;
     constexpr int NDMA = T::DMA_PER_WAVE;
 
     extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
@@ -1493,7 +1499,7 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     //   [4DC, 4DC + 2DB) K^T of key block 0 by (16-key chunk, db) (dQ), then of block 1
     constexpr int NROW = 4 * DC, NF = NROW + 4 * DB;
     constexpr int PD = 4;                            // read-ahead depth of the fragment ring
-    static_assert(DC % PD == 0 && (2 * DB) % PD == 0, "read-ahead depth must divide the fragment counts");
+    static_assert(NF % PD == 0, "read-ahead depth must divide the fragment count");
     auto fetch = [&](const uint16_t* ks, int f) {
         const uint16_t* vs = ks + T::TILE_ELEMS;
         if (f < NROW) {
@@ -1517,7 +1523,7 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     // One tile of 64 keys = two key blocks of 32, six phases of 2 DC MFMAs (MFMA slot = 2 * fragment +
     // query block).  The element-wise work of a phase is threaded between the MFMAs of the next one:
     //   S(0) | dP(0) + P(0) | S(1) + dS(0) | dP(1) + P(1) | dQ(0) + dS(1) | dQ(1)
-    // Element e of query block 0 goes with slot e of its phase, that of query block 1 with slot e + 1
+    // (16 slots:) element e of query block 0 goes with slot e of its phase, that of query block 1 with slot e + 1
     // (its S / dP are complete one MFMA later), the sixteenth spilling into the first slot of the
     // next phase: every hand-emitted MFMA result is first touched two MFMAs after it was issued.
     // COPY: 1 = the next tile is a full one (copies split around the MFMAs), 2 = decide at run time.
@@ -1554,22 +1560,17 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
         };
         // element-wise work that goes with MFMA slot i of phase ph
         constexpr int NSL = 2 * DC;                 // MFMA slots per phase
-        static_assert(NSL == 16 || NSL == 8, "element schedule written for 16 or 8 slots per phase");
+        constexpr int EL = (16 + NSL - 1) / NSL;
+        auto elems_at = [&](int qb, int i, auto fn) {      // elements 16 i / NSL to 16 (i + 1) / NSL
+#pragma unroll
+            for (int e = 0; e < EL; ++e)
+                if (16 * i / NSL + e < 16 * (i + 1) / NSL) fn(qb, 16 * i / NSL + e);
+        };
         auto elems_of = [&](int ph, int i, auto fn) {      // fn(qb, e) for the elements scheduled at (ph, i)
-            // query block 0: elements [EL*i, EL*(i+1)) at slot i; query block 1: one slot later
-            constexpr int EL = 16 / NSL;            // 1 or 2 elements per slot and block
-#pragma unroll
-            for (int e = 0; e < EL; ++e) fn(0, EL * i + e);
-            if (i > 0) {
-#pragma unroll
-                for (int e = 0; e < EL; ++e) fn(1, EL * (i - 1) + e);
-            }
+            elems_at(0, i, fn);
+            if (i > 0) elems_at(1, i - 1, fn);             // query block 1: one slot later
         };
-        auto spill_of = [&](auto fn) {               // the last elements of query block 1, in slot 0 of the next phase
-            constexpr int EL = 16 / NSL;
-#pragma unroll
-            for (int e = 0; e < EL; ++e) fn(1, EL * (NSL - 1) + e);
-        };
+        auto spill_of = [&](auto fn) { elems_at(1, NSL - 1, fn); };     // its last elements, in slot 0 of the next phase
         // copies of the next tile: copy j goes with MFMA slot CS * j + 1 of the S / dP phases
         constexpr int NCOPY = 2 * NDMA;
         constexpr int CS = (4 * NSL - 2) / NCOPY;
@@ -1695,7 +1696,7 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
         const int row0 = qw0 + 32 * qb;
-        store_rows32<D>(lds + wave * 32 * D, p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)row0 * p.dqs.n, p.dqs.n, p.Sq - row0, p.d, [&](int db, int g) {
+        store_rows32<D>(lds + wave * 32 * RS, p.dq + b * p.dqs.b + hh * p.dqs.h + (int64_t)row0 * p.dqs.n, p.dqs.n, p.Sq - row0, p.d, [&](int db, int g) {
             const f32x16& a = dqacc[qb][db];
             return u32x2{pack_bf16(a[4 * g] * p.scale, a[4 * g + 1] * p.scale), pack_bf16(a[4 * g + 2] * p.scale, a[4 * g + 3] * p.scale)};
         });

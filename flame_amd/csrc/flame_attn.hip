@@ -238,7 +238,8 @@ bool big_head_dim_ok(int D) { return D > 128 && D <= 512 && D % 8 == 0; }
 int padded_head_dim(int D) { return D <= 64 ? 64 : 128; }
 // Head dims above 64 and up to 96 (72, 80 and 96 among them): a quarter of the matrix work of 128 is padding.
 // (Forward, us: B=1 H=24 S=4608 D=96 215 -> 189, B=1 H=16 S=8192 D=96 causal 238 -> 201, B=2 H=16 S=1500 D=80 with a key mask
-// 45 -> 39.5, B=4 H=8 S=300 D=72 9.9 -> 8.8.)
+// 45 -> 39.5, B=4 H=8 S=300 D=72 9.9 -> 8.8.  Forward and backward: S=4608 930 -> 790, S=8192 causal 988 -> 826, B=2 H=16
+// S=1024 D=80 81 -> 72, the key mask 194 -> 170, B=2 H=16 S=1024 D=96 with dropout 97 -> 86.)
 bool narrow(int D) { return D > 64 && D <= 96; }
 
 // backward workspace: [-delta rows][lse2 rows][fp32 partials of the split dK/dV workgroups]
@@ -377,7 +378,8 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     using T = BwdTile<D>;
     using TQ = BwdDqTile<D>;
     if constexpr (HASMASK && !TIMING) {
-        if (mask_bits_fit(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, p.split_ws_bytes)) return launch_bwd_bits<D>(p, s);
+        if (mask_bits_fit(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, p.split_ws_bytes))
+            return D == 128 && narrow(p.d) ? launch_bwd_bits<96>(p, s) : launch_bwd_bits<D>(p, s);
     }
     static bool attr_done = false;
     auto kern = bwd_dkdv_kernel<D, HASMASK, TIMING>;
@@ -450,10 +452,10 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         BwdParams pj = p;
         pj.rows_ready = 1;
         const int64_t n_rows = (int64_t)p.B * p.H * p.Sq;
-        constexpr int rows_per_wg = 256 / (D / 8);
+        constexpr int DR = kRowPitch<D>, rows_per_wg = 256 / (DR / 8);
         {
             ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_ROWS, s);
-            hipLaunchKernelGGL(bwd_rows_kernel<D>, dim3((unsigned)((n_rows + rows_per_wg - 1) / rows_per_wg)), dim3(256), 0, s, pj);
+            hipLaunchKernelGGL(bwd_rows_kernel<DR>, dim3((unsigned)((n_rows + rows_per_wg - 1) / rows_per_wg)), dim3(256), 0, s, pj);
         }
         const int cus = device_cu_count();
         const size_t room = p.split_ws_bytes / bwd_split_slot_bytes(D);
@@ -749,7 +751,8 @@ int launch_bwd_drop(const BwdParams& p, hipStream_t s) {
 }
 template <int D>
 int launch_bwd_dropout(const BwdParams& p, bool has_mask, hipStream_t s) {
-    if (has_mask) return launch_bwd_drop<D, true, kDropTiled>(p, s);
+    if constexpr (D != 96)
+        if (has_mask) return launch_bwd_drop<D, true, kDropTiled>(p, s);
     switch (drop_mode(p.m, p.Sk)) {
         case kDropRows64: return launch_bwd_drop<D, false, kDropRows64>(p, s);
         case kDropFlat: return launch_bwd_drop<D, false, kDropFlat>(p, s);
@@ -883,10 +886,12 @@ static int attn_bwd_impl(const void* Q, const void* K, const void* V, const void
 #endif
     if (dropout_p != 0.f) {
         if (!set_dropout(p.m, dropout_p, dropout_seed, draw_cq, draw_ck, N_q, N_kv)) return FLAME_ATTN_ERR_INVALID;
+        if (narrow(D) && !keep_mask) return launch_bwd_dropout<96>(p, false, s);
         return padded_head_dim(D) == 128 ? launch_bwd_dropout<128>(p, keep_mask != nullptr, s) : launch_bwd_dropout<64>(p, keep_mask != nullptr, s);
     }
     p.key_mask = keys_only(p.m, N_q, N_kv) ? 1 : 0;
     if (p.key_mask) keep_mask = nullptr;           // served by the kernels without the general mask code
+    if (narrow(D) && !keep_mask) return launch_bwd<96, false>(p, s);
     if (padded_head_dim(D) == 128) return keep_mask ? launch_bwd<128, true>(p, s) : launch_bwd<128, false>(p, s);
     return keep_mask ? launch_bwd<64, true>(p, s) : launch_bwd<64, false>(p, s);
 }

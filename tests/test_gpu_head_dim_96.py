@@ -1,6 +1,7 @@
 """Head dims 72 to 96 on the kernels compiled for 96: bit for bit what the kernels of 128 give for the same tensors padded with
-zeros (the contraction gains zeros only, nothing changes its order), in each of the forms the forward takes: 256-query
-workgroups with and without the causal flag, 128-query ones, key groups, key masks, masks by query, key lengths, dropout."""
+zeros (the contraction gains zeros only, nothing changes its order), in each of the forms that forward and backward take:
+256-query workgroups with and without the causal flag, 128-query ones, key groups, shared walks, split last rounds, key masks,
+masks by query, key lengths, dropout."""
 import pytest
 import torch
 
@@ -51,3 +52,19 @@ def test_forward_as_padded_to_128(B, H, Sq, Sk, D, causal, kv_len, mask, p):
     o1, lse1 = forward(capi, pad(q), pad(k), pad(v), D ** -0.5, causal, dl, m, p)
     same("O", o, o1[..., :D])
     same("LSE", lse, lse1)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,D,causal,kv_len,mask,p", CASES + [
+    (1, 2, 1200, 1200, 80, False, None, None, 0.0),        # shared walks
+    (1, 30, 1100, 1100, 72, False, None, None, 0.0),       # the last round of the key blocks split
+    (1, 2, 1100, 1100, 96, False, None, None, 0.1)])
+def test_backward_as_padded_to_128(B, H, Sq, Sk, D, causal, kv_len, mask, p):
+    from flame_amd import capi
+    print(f"[head dim 96] backward {B=} {H=} {Sq=} {Sk=} {D=} {causal=} {kv_len=} {mask=} {p=}", flush=True)
+    q, k, v, do, dl, m = make(B, H, Sq, Sk, D, kv_len, mask)
+    sc = D ** -0.5
+    o, lse = forward(capi, q, k, v, sc, causal, dl, m, p)
+    f = (lambda *t: capi.attn_bwd_dropout(*t, sc, p, SEED, causal=causal, kv_len=dl, mask=m)) if p else \
+        (lambda *t: capi.attn_bwd(*t, sc, causal=causal, kv_len=dl, mask=m))
+    for name, a, b in zip(("dQ", "dK", "dV"), f(q, k, v, o, do, lse), f(*(pad(t) for t in (q, k, v, o, do)), lse)):
+        same(name, a, b[..., :D])
