@@ -932,10 +932,10 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         part = all % p.dq_parts;
         wg = all / p.dq_parts;
     } else {
-        wg = p.m.kv_len || KEYS ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
+        wg = p.m.kv_len || KEYS ? xcd_remap_heads<KG == 1 && !BITS>(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
     }
     int qt = wg % n_qt, bh = wg / n_qt;
-    if (p.m.causal && !p.m.kv_len && p.dq_parts == 1) causal_longest_first(wg, n_qt, gridDim.x, qt, bh);
+    if (p.m.causal && !p.m.kv_len && p.dq_parts == 1) causal_longest_first<KG == 1>(wg, n_qt, gridDim.x, qt, bh);
     if (!BITS && (KEYS || p.m.kv_len) && p.dq_parts == 1) bh = longest_batches_first<KEYS>(bh, p.B, p.H, p.Sk, p.m);
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
