@@ -23,6 +23,7 @@
 #include "attn_bwd_wide.hpp"
 #include "attn_fwd_probs.hpp"
 #include "mask_bits.hpp"
+#include "fast_div.hpp"
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
 #include "attn_fwd_keyshare.hpp"
@@ -1572,6 +1573,51 @@ __global__ void cast_f32_to_bf16_kernel(const float* src, uint16_t* dst, int64_t
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = (uint16_t)(pack_bf16(src[i], 0.f) & 0xffffu);
 }
+// Q, K and V from fp32 views to contiguous bf16 in one launch; a lane takes four consecutive elements of a row.  Bound by
+// memory: 6 bytes per element (25 million of them, 151 MB: 30 us).  It saves launches; see cast_qkv of the host module.
+struct CastQkvParams {
+    const float* src[3];
+    uint16_t* dst[3];
+    Strides st[3];
+    uint32_t first[3], end;        // units of four elements
+    FastDiv rows[2], heads, per_row;          // rows: of Q, of K and V
+};
+typedef float f32x4_word __attribute__((ext_vector_type(4), aligned(4)));      // 16 bytes at any element's address
+__global__ __launch_bounds__(256) void cast_qkv_kernel(const CastQkvParams p) {
+    f32x4_word x[4];
+    uint16_t* to[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t u = blockIdx.x * 1024u + 256u * i + threadIdx.x;
+        to[i] = nullptr;
+        if (u < p.end) {
+            const int t = (u >= p.first[1]) + (u >= p.first[2]);
+            const uint32_t at = u - p.first[t], row = p.per_row(at), c = at - row * p.per_row.d;
+            const FastDiv rows = t == 0 ? p.rows[0] : p.rows[1];
+            const uint32_t bh = rows(row), n = row - bh * rows.d, b = p.heads(bh), h = bh - b * p.heads.d;
+            x[i] = *reinterpret_cast<const f32x4_word*>(p.src[t] + b * p.st[t].b + h * p.st[t].h + n * p.st[t].n + 4 * c);
+            to[i] = p.dst[t] + 4 * (int64_t)at;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (to[i]) *reinterpret_cast<u32x2*>(to[i]) = u32x2{pack_bf16(x[i][0], x[i][1]), pack_bf16(x[i][2], x[i][3])};
+}
+// n contiguous elements, both sides on 16 bytes
+__global__ __launch_bounds__(256) void cast_bf16_to_f32_kernel(const uint16_t* src, float* dst, int64_t n) {
+    const int64_t i0 = (int64_t)blockIdx.x * 2048 + 4 * threadIdx.x;
+    u32x2 w[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (i0 + 1024 * u + 4 <= n) w[u] = *reinterpret_cast<const u32x2*>(src + i0 + 1024 * u);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int64_t i = i0 + 1024 * u;
+        if (i + 4 <= n) *reinterpret_cast<f32x4*>(dst + i) = f32x4{bf16_lo(w[u][0]), bf16_hi(w[u][0]), bf16_lo(w[u][1]), bf16_hi(w[u][1])};
+        else
+            for (int64_t j = i; j < n; ++j) dst[j] = __uint_as_float((uint32_t)src[j] << 16);
+    }
+}
 // gradient accumulation of the host layer: acc += float(g) with g bf16 or fp32; fill with a constant
 __global__ void accumulate_f32_kernel(float* acc, const void* g, int g_is_f32, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1862,6 +1908,40 @@ int flame_attn_cast_f32_to_bf16(const void* src_f32, void* dst_bf16, int64_t n, 
                        static_cast<hipStream_t>(stream), static_cast<const float*>(src_f32),
                        static_cast<uint16_t*>(dst_bf16), n);
     hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
+int flame_attn_cast_qkv_f32_to_bf16(const void* Q, const void* K, const void* V, void* Q16, void* K16, void* V16, int B, int H,
+                                    int N_q, int N_kv, int D, const int64_t* q_strides, const int64_t* k_strides,
+                                    const int64_t* v_strides, void* stream) {
+    if (!Q || !K || !V || !Q16 || !K16 || !V16 || !q_strides || !k_strides || !v_strides) return FLAME_ATTN_ERR_INVALID;
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || D <= 0) return FLAME_ATTN_ERR_INVALID;
+    if (D % 4 != 0 || q_strides[3] != 1 || k_strides[3] != 1 || v_strides[3] != 1) return FLAME_ATTN_ERR_UNSUPPORTED;
+    if ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V)) % 4 != 0 || !aligned16(Q16) ||
+        !aligned16(K16) || !aligned16(V16))
+        return FLAME_ATTN_ERR_UNSUPPORTED;
+    const double units = (double)B * H * ((double)N_q + 2.0 * N_kv) * (D / 4);
+    if (units > 2e9) return FLAME_ATTN_ERR_UNSUPPORTED;
+    const uint32_t nq = (uint32_t)B * H * N_q * (D / 4), nk = (uint32_t)B * H * N_kv * (D / 4);
+    const CastQkvParams p{{static_cast<const float*>(Q), static_cast<const float*>(K), static_cast<const float*>(V)},
+                          {static_cast<uint16_t*>(Q16), static_cast<uint16_t*>(K16), static_cast<uint16_t*>(V16)},
+                          {mk(q_strides), mk(k_strides), mk(v_strides)},
+                          {0u, nq, nq + nk},
+                          nq + 2 * nk,
+                          {FastDiv(N_q), FastDiv(N_kv)},
+                          FastDiv(H),
+                          FastDiv(D / 4)};
+    hipLaunchKernelGGL(cast_qkv_kernel, dim3((p.end + 1023) / 1024), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
+int flame_attn_cast_bf16_to_f32(const void* src_bf16, void* dst_f32, int64_t n, void* stream) {
+    if (!src_bf16 || !dst_f32 || n <= 0) return FLAME_ATTN_ERR_INVALID;
+    if (n > (int64_t)0x7fffffff * 2048 || !aligned16(src_bf16) || !aligned16(dst_f32)) return FLAME_ATTN_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(cast_bf16_to_f32_kernel, dim3((unsigned)((n + 2047) / 2048)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(src_bf16), static_cast<float*>(dst_f32), n);
+    const hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
 }
 

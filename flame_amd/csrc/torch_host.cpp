@@ -35,7 +35,7 @@ using at::Tensor;
     X(flame_attn_bwd_bf16) X(flame_attn_bwd_workspace_bytes) X(flame_attn_fwd_dropout_tiled_bf16)                       \
     X(flame_attn_bwd_dropout_tiled_bf16) X(flame_attn_materialised_workspace_bytes) X(flame_attn_fwd_materialised_bf16) \
     X(flame_attn_bwd_materialised_bf16) X(flame_sage_quant_qk_int8_ks) X(flame_sage_attn_fwd_bias_int8)                 \
-    X(flame_attn_prep_rmsnorm_rope_bf16) X(flame_bf16_to_fp8) X(flame_fp8_to_bf16)
+    X(flame_attn_prep_rmsnorm_rope_bf16) X(flame_bf16_to_fp8) X(flame_fp8_to_bf16) X(flame_attn_cast_qkv_f32_to_bf16) X(flame_attn_cast_bf16_to_f32)
 
 struct Api {
 #define FLAME_HOST_MEMBER(name) decltype(&::name) name = nullptr;
@@ -263,6 +263,41 @@ Tensor as_bf16_view(const Tensor& x) {
     return t;
 }
 
+// A tensor whose elements are what its address and strides say: no mode, transform or subclass has a part in what .to() does to it.
+bool plain_f32(const Tensor& t) {
+    static const c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::Functionalize,
+                                              c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Batched,
+                                              c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+    if (t.scalar_type() != at::kFloat || !t.is_cuda() || t.layout() != at::kStrided || t.key_set().has_any(special) || t.stride(3) != 1) return false;
+    for (int ax = 0; ax < 3; ++ax)          // .to() keeps such strides, and the kernels refuse them
+        if (t.size(ax) == 1 && t.stride(ax) % 8 != 0) return false;
+    return true;
+}
+// Where no graph is recorded, fp32 Q, K and V become bf16 in one launch instead of three, and the output fp32 in one: of a small
+// call's time most was the four conversions of the tensor library and the gaps between them.  false: not these tensors.
+// (Whole call, us: B=2 H=12 S=77 D=64 24 -> 13, B=1 H=16 S=257 D=80 24 -> 14.7, B=2 H=16 S=577 D=64 24 -> 21.7.  Large ones gain
+// nothing: 19 million elements in Q, K and V 86.7 -> 87.3, 25 million 178 -> 181.)
+constexpr int64_t kMostCast = (int64_t)12 << 20;
+bool cast_qkv(const Tensor& q, const Tensor& k, const Tensor& v, Tensor& qb, Tensor& kb, Tensor& vb) {
+    if (!plain_f32(q) || !plain_f32(k) || !plain_f32(v)) return false;
+    if (k.device() != q.device() || v.device() != q.device() || k.sizes() != v.sizes() || q.size(0) != k.size(0) || q.size(1) != k.size(1) ||
+        q.size(3) != k.size(3) || q.size(3) % 8 != 0 || q.numel() == 0 || k.numel() == 0 || q.numel() + 2 * k.numel() > kMostCast)
+        return false;
+    for (int64_t n : q.sizes())
+        if (n > INT32_MAX) return false;
+    if (k.size(2) > INT32_MAX) return false;
+    qb = empty(q.sizes(), at::kBFloat16, q);
+    kb = empty(k.sizes(), at::kBFloat16, q);
+    vb = empty(v.sizes(), at::kBFloat16, q);
+    return g_api.flame_attn_cast_qkv_f32_to_bf16(ptr(q), ptr(k), ptr(v), ptr(qb), ptr(kb), ptr(vb), (int)q.size(0), (int)q.size(1), (int)q.size(2),
+                                                 (int)k.size(2), (int)q.size(3), strides4(q), strides4(k), strides4(v), stream_of(q)) == FLAME_ATTN_OK;
+}
+Tensor f32_of(const Tensor& o) {       // contiguous bf16
+    Tensor out = empty(o.sizes(), at::kFloat, o);
+    check_rc(g_api.flame_attn_cast_bf16_to_f32(ptr(o), ptr(out), o.numel(), stream_of(o)), "flame_attn_cast_bf16_to_f32");
+    return out;
+}
+
 // The copy of a keep-mask that a recorded graph holds, so that the caller may refill the buffer before the backward.  Axes
 // along which the tensor repeats itself are kept once, and rows start on 16 bytes (where the kernels load them as vectors).
 // One launch: 3 us of a training step of 185 us (B=4 H=16 S=1101 D=128, a mask of keys).
@@ -373,11 +408,15 @@ PyObject* py_sdpa(PyObject*, PyObject* const* a, Py_ssize_t n) {
             WithoutGil nogil;
             c10::OptionalDeviceGuard device(q.device());
             const at::ScalarType orig = q.scalar_type();
-            const Tensor qb = as_bf16_view(q), kb = as_bf16_view(k), vb = as_bf16_view(v);
-            if (at::GradMode::is_enabled() && (qb.requires_grad() || kb.requires_grad() || vb.requires_grad())) {
+            Tensor qb, kb, vb, lse;
+            const bool graph = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+            if (!graph && cast_qkv(q, k, v, qb, kb, vb)) {
+                sdpa_forward(qb, kb, vb, mask, causal, scale, false, out, lse);
+                out = f32_of(out);
+            } else if (qb = as_bf16_view(q), kb = as_bf16_view(k), vb = as_bf16_view(v);
+                       at::GradMode::is_enabled() && (qb.requires_grad() || kb.requires_grad() || vb.requires_grad())) {
                 out = Sdpa::apply(qb, kb, vb, mask.defined() ? std::optional<Tensor>(converted ? mask : own_mask(mask)) : std::nullopt, causal, scale);
             } else {
-                Tensor lse;
                 sdpa_forward(qb, kb, vb, mask, causal, scale, false, out, lse);
             }
             if (orig != at::kBFloat16) out = out.to(orig);

@@ -487,6 +487,13 @@ int flame_attn_convert_keep_mask(const void* src, int src_dtype, void* dst_u8, i
  * upstream gradient to the bf16 backward instead of falling back to the materialising recompute as
  * the reference does (src/autograd.rs:702-705). */
 int flame_attn_cast_f32_to_bf16(const void* src_f32, void* dst_bf16, int64_t n, void* stream);
+/* Q [B,H,N_q,D], K and V [B,H,N_kv,D] from fp32 views (element strides over b, h, n, d; that of d is 1) to contiguous bf16
+ * buffers (16-byte aligned), round to nearest even, in one launch; D a multiple of 4.  And the way back for an output: n
+ * contiguous elements, both buffers 16-byte aligned. */
+int flame_attn_cast_qkv_f32_to_bf16(const void* Q, const void* K, const void* V, void* Q16, void* K16, void* V16, int B, int H,
+                                    int N_q, int N_kv, int D, const int64_t* q_strides, const int64_t* k_strides,
+                                    const int64_t* v_strides, void* stream);
+int flame_attn_cast_bf16_to_f32(const void* src_bf16, void* dst_f32, int64_t n, void* stream);
 /* acc_f32[i] += float(grad[i]), grad bf16 or fp32, n contiguous elements: what Gradients::accumulate
  * of the reference's v4 engine does with tensor ops (src/autograd_v4/gradients.rs:20-32, gradients are
  * kept in fp32). */

@@ -308,6 +308,14 @@ extern "C" {
     pub fn flame_attn_cast_f32_to_bf16(
         src_f32: *const c_void, dst_bf16: *mut c_void, n: i64, stream: *mut c_void
     ) -> c_int;
+    pub fn flame_attn_cast_qkv_f32_to_bf16(
+        q: *const c_void, k: *const c_void, v: *const c_void, q16: *mut c_void, k16: *mut c_void, v16: *mut c_void, b: c_int,
+        h: c_int, n_q: c_int, n_kv: c_int, d: c_int, q_strides: *const i64, k_strides: *const i64, v_strides: *const i64,
+        stream: *mut c_void
+    ) -> c_int;
+    pub fn flame_attn_cast_bf16_to_f32(
+        src_bf16: *const c_void, dst_f32: *mut c_void, n: i64, stream: *mut c_void
+    ) -> c_int;
     pub fn flame_attn_accumulate_f32(
         acc_f32: *mut c_void, grad: *const c_void, grad_dtype: c_int, n: i64, stream: *mut c_void
     ) -> c_int;
