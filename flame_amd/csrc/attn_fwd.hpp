@@ -67,7 +67,8 @@ typedef uint16_t u16x8_any __attribute__((ext_vector_type(8), aligned(2)));
 // own, and the second hands its running state to the first through LDS.  For grids that give a compute unit one workgroup at
 // most: its second wavefront per SIMD, which otherwise a second workgroup would be, and half the walk.  K and V are still
 // read once per workgroup.
-template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
+// AHEAD: a bias is requested a step earlier (see EARLY).
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1, bool AHEAD = false>
 __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void fwd_kernel(const FwdParams p) {
     static_assert(KG == 1 || (KG == 2 && EXCL == kExNone), "key groups: nothing excluded but by causal flag and key lengths");
     using T = FwdTile<D>;
@@ -277,6 +278,12 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             if (__any(limit < BN)) mrow.restrict_to(limit);
         }
     };
+    // Tiles below t_clean need no exclusions for any query of the workgroup; the rest (ragged tail, causal
+    // diagonal, or everything under an explicit mask) carry per-element exclusions.
+    int t_clean = KEYS ? kt.n_whole : (EXCL == kExNone || BIAS) ? klimit / BN : 0;
+    if (p.m.causal) t_clean = min(t_clean, (q0 + 1 - key0) / BN);
+    t_clean = max(min(t_clean, n_tiles), 0);
+
     // Bias: every lane needs 64 (of its half: 32) consecutive values of its query's row.  Four neighbouring lanes load 64 bytes
     // of a row (a "piece" is 16 rows of that, one instruction), and two pieces, 32 rows, at a time pass through 2 KiB of LDS
     // to the lanes that own the rows, granules swizzled as in fragments_of_rows32: an instruction whose lanes each load from
@@ -285,10 +292,16 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     // the PV phase, one ahead of the slices that add it.
     // (B=1 H=64 S=512 D=64, fp32: 84 MB move, 16 us at the rate of a copy; four values per lane and load 23.5 us, this 19.4.
     // B=3 H=16 S=1664 fp32: D = 64 123 -> 82 us, D = 128 166 -> 150 us; its two wavefronts per SIMD wait for the bias then.)
+    // EARLY (D = 64, which has the registers): a pair of pieces is requested for the tile after the next as soon as it has gone through
+    // LDS, so that it has a whole step to arrive instead of half of one, and the last wait of a step that
+    // copies two whole tiles counts these loads out; the other steps request it behind their barrier, all at once.  A ragged tile is
+    // requested across the logit phase as above.  B=1 H=64 S=512 19.7 -> 15.5 us, the rate of a copy; S=256 10.9 -> 8.0; B=1 H=12
+    // S=2048 42.3 -> 36.6, B=4 H=64 S=700 84.7 -> 77.4, B=3 H=16 S=1664 78.5 -> 70.2 us; B=4 H=16 S=1344 gains nothing (63.9 -> 65).
     using BiasPiece = typename std::conditional<EXCL == kExBiasF32, f32x4_any, u16x8_any>::type;
     using BiasElem = typename std::conditional<EXCL == kExBiasF32, float, uint16_t>::type;
     constexpr int BEL = EXCL == kExBiasF32 ? 4 : 8;           // values per piece and lane
     constexpr int NPIECE = BIAS ? 32 / BEL : 1, NPASS = BIAS ? NPIECE / 2 : 1;
+    constexpr bool EARLY = BIAS && AHEAD;
     BiasPiece bw[NPIECE];
     f32x4 bg[EXCL == kExBiasF32 ? 8 : 1];                     // keys 8 j + 4 h .. + 3 of this lane's row
     u32x2 bgh[EXCL == kExBiasBf16 ? 8 : 1];
@@ -328,6 +341,12 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
 #pragma unroll
                 for (int u = 0; u < 4; ++u) bgh[4 * c + u] = *reinterpret_cast<const u32x2*>(bpass + (bfrom ^ (8 * u)));
             }
+        }
+    };
+    auto bias_request_whole = [&](int t) {
+        if (t < t_clean) {
+#pragma unroll
+            for (int i = 0; i < NPIECE; ++i) bias_request(std::false_type{}, t, i);
         }
     };
     auto excl_elem = [&](f32x16 (&s)[2], int idx) {
@@ -471,11 +490,11 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             for (int i = 0; i < NS; i += 2) {
                 nxt[1] = mfma32(fb[(i + 1) % PD], qf[i >> 1], nxt[1]);
                 exp_slice(i);
-                if (BIAS && i % (NS / NPIECE) == 0) bias_request(ragged_tag, t + 1, i / (NS / NPIECE));
+                if (BIAS && (!EARLY || (NEXT == 1 && t + 1 >= t_clean)) && i % (NS / NPIECE) == 0) bias_request(ragged_tag, t + 1, i / (NS / NPIECE));
                 __builtin_amdgcn_sched_barrier(0);
                 nxt[0] = mfma32(fb[i % PD], qf[i >> 1], nxt[0]);
                 exp_slice(i + 1);
-                if (BIAS && (i + 1) % (NS / NPIECE) == 0) bias_request(ragged_tag, t + 1, (i + 1) / (NS / NPIECE));
+                if (BIAS && (!EARLY || (NEXT == 1 && t + 1 >= t_clean)) && (i + 1) % (NS / NPIECE) == 0) bias_request(ragged_tag, t + 1, (i + 1) / (NS / NPIECE));
                 fb[i % PD] = frag_of(i + PD);
                 fb[(i + 1) % PD] = frag_of(i + 1 + PD);
                 __builtin_amdgcn_sched_barrier(0);
@@ -484,9 +503,16 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             if (NEXT == 1 && EXCL == kExGeneral) excl_general(nxt, t + 1);
             // ---- O^T += V(t)^T P(t)^T between the row-maximum scan of tile t+1
             float tmax = -INFINITY;
-            if constexpr (BIAS) bias_pass(0);
+            auto bias_through = [&](int c) {
+                bias_pass(c);
+                if (EARLY && COPY) {       // tile t + 2 is a whole one
+                    bias_request(std::false_type{}, t + 2, 2 * c);
+                    bias_request(std::false_type{}, t + 2, 2 * c + 1);
+                }
+            };
+            if constexpr (BIAS) bias_through(0);
             auto max_slice = [&](int i) {
-                if (BIAS && i % (NP / NPASS) == 0 && i / (NP / NPASS) + 1 < NPASS) bias_pass(i / (NP / NPASS) + 1);
+                if (BIAS && i % (NP / NPASS) == 0 && i / (NP / NPASS) + 1 < NPASS) bias_through(i / (NP / NPASS) + 1);
 #pragma unroll
                 for (int e = 0; e < PPS; ++e) {
                     const int idx = 2 * (16 * i / NP + e);
@@ -512,16 +538,13 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
                 __builtin_amdgcn_sched_barrier(0);
             }
             fold_max(tmax);
-            wait_vm0();          // the copies issued by this step have landed
+            // the copies issued by this step have landed
+            if constexpr (EARLY && COPY) wait_vm<NPIECE>();          // (younger than they are: the bias of tile t + 2)
+            else wait_vm0();
             __syncthreads();     // ... for every wave, and everyone is done reading this step's tiles
+            if constexpr (EARLY && !COPY) bias_request_whole(t + 2);
         }
     };
-
-    // Tiles below t_clean need no exclusions for any query of the workgroup; the rest (ragged tail, causal
-    // diagonal, or everything under an explicit mask) carry per-element exclusions.
-    int t_clean = KEYS ? kt.n_whole : (EXCL == kExNone || BIAS) ? klimit / BN : 0;
-    if (p.m.causal) t_clean = min(t_clean, (q0 + 1 - key0) / BN);
-    t_clean = max(min(t_clean, n_tiles), 0);
 
     f32x16 sa[2], sb[2];
     if (n_tiles > 0) {
@@ -549,6 +572,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
 #pragma unroll
             for (int idx = 0; idx < 32; ++idx) excl_elem(sa, idx);
         }
+        if constexpr (EARLY) bias_request_whole(1);
         float tmax = sa[0][0];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
