@@ -55,6 +55,8 @@ struct FwdTile {
     static constexpr int BIAS_PASS_BYTES = 4 * 2048;             // behind the stages: 2 KiB per wavefront that bias rows pass through
     static constexpr int ROWS_PER_DMA = 1024 / (RS * 2);         // rows covered by one 64-lane x 16-byte copy
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;   // copies per wave and tensor
+    // Q passes through the place of a V tile, 2 KiB per wavefront; behind the stages where a tile is smaller than that
+    static constexpr int q_pass_bytes(int nw) { return nw * 2048 > TILE_ELEMS * 2 ? nw * 2048 : 0; }
 };
 
 // 16 bytes of a bias row, at any element's address
@@ -198,19 +200,19 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         }
     };
     // the first tiles are on their way before anything else is loaded: on short walks their round trip is the run time
-    static_assert(NW * 2048 <= T::TILE_ELEMS * 2, "Q passes through the place of a V tile");
 #pragma unroll
     for (int i = 0; i < KD; ++i) {
         if (i < n_tiles) issue_k(i);
         if (i < VD && i < n_tiles) issue_v(i);
     }
 
-    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d; through the place of V(1)
+    // ---- Q fragments (B operand of S^T = K Q^T): column = query, 8 consecutive d; through the place of V(1), or behind the stages
     bf16x8 qf[DC];
     {
+        static_assert(T::q_pass_bytes(NW) == 0 || (KG == 1 && !BIAS && !KEYS), "nothing else lies behind the stages");
         u32x4 w[DC];
         load_rows32<D>(w, qbase + (int64_t)qw0 * p.qs.n, p.qs.n, p.Sq - qw0, p.d);
-        fragments_of_rows32<D>(lds + T::STAGE_ELEMS + T::TILE_ELEMS + wave * 1024, w,
+        fragments_of_rows32<D>(lds + (T::q_pass_bytes(NW) ? 2 * T::STAGE_ELEMS : T::STAGE_ELEMS + T::TILE_ELEMS) + wave * 1024, w,
                                [&](auto dc, u32x4 f) { qf[decltype(dc)::value] = __builtin_bit_cast(bf16x8, f); });
     }
 

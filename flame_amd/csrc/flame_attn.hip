@@ -163,7 +163,7 @@ int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_kernel<D, EXCL, NW, DROP, KG, AHEAD>;
     constexpr bool KEYS = EXCL == kExKeys || EXCL == kExBits;
-    constexpr int tiles = KG * T::LDS_BYTES + (EXCL == kExBiasF32 || EXCL == kExBiasBf16 ? T::BIAS_PASS_BYTES : 0);
+    constexpr int tiles = KG * T::LDS_BYTES + (EXCL == kExBiasF32 || EXCL == kExBiasBf16 ? T::BIAS_PASS_BYTES : T::q_pass_bytes(NW));
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), tiles + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
     const int lds = tiles + (KEYS ? KeyTiles::lds_bytes((p.Sk + 63) / 64) : 0);
     {
@@ -1158,11 +1158,24 @@ static int fwd_key_splits(int64_t bh, int N_q, int N_kv, int DP) {
     return best_s;
 }
 
-// the rule for the forward's query tile: 256 rows per workgroup (true) or 128
-static bool fwd_rule_wide(int B, int H, int N_q, bool has_mask_or_bias, bool has_kv_len) {
+// Whether 256-query workgroups neither add padding rows nor leave compute units without a workgroup.
+static bool fwd_fits_256(int B, int H, int N_q, bool has_mask_or_bias, bool has_kv_len) {
     const int64_t n256 = (N_q + 255) / 256;
     return !has_mask_or_bias && n256 * 256 <= ((int64_t)(N_q + 127) / 128) * 128 && n256 * B * H >= device_cu_count() &&
            !(has_kv_len && n256 * B * H < 2 * device_cu_count()) && wg_waves_override() != 4;
+}
+// nothing is excluded at all: 4 wavefronts of 64 queries (launch_fwd_wide), else 8 of 32
+static bool fwd_plain(int N_kv, bool causal, bool has_kv_len) { return !causal && !has_kv_len && N_kv % 64 == 0; }
+
+// The rule for the forward's query tile, 256 rows per workgroup (true) or 128, of a call and of a launch plan; DP: padded head
+// dim.  Ragged or causal calls up to D = 64 take 128, and so do thin last rounds (last_round.hpp, with the figures); a plan
+// may still ask for 256 there.
+static bool fwd_rule_wide(int B, int H, int N_q, int N_kv, int DP, bool causal, bool has_mask_or_bias, bool has_kv_len) {
+    const bool plain = fwd_plain(N_kv, causal, has_kv_len);
+    if (!fwd_fits_256(B, H, N_q, has_mask_or_bias, has_kv_len) || (!plain && DP == 64)) return false;
+    const int64_t total256 = (int64_t)((N_q + 255) / 256) * B * H, cus = device_cu_count();
+    // (without exclusions a last round on an eighth of the units is cut into 32-query workgroups, launch_fwd_wide)
+    return !thin_last_round(total256, cus, 3) || (plain && (total256 >= 2 * cus || thin_last_round(total256, cus, 8)));
 }
 
 static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, void* LSE,
@@ -1244,22 +1257,11 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         if (DP == 128 && narrow(std::max(D, Dv)) && !hm) return launch_fwd_dropout<96>(p, hm, s);
         return DP == 128 ? launch_fwd_dropout<128>(p, hm, s) : launch_fwd_dropout<64>(p, hm, s);
     }
-    // 256-query workgroups when they neither add padding rows nor leave compute units
-    // without a workgroup
-    bool wide = fwd_rule_wide(B, H, N_q, hm, kv_len != nullptr);
-    // a plan (128 or 256 query rows per workgroup) overrides the rule where the kernels leave the choice open
-    if (q_tile_plan == 128) wide = false;
-    else if (q_tile_plan == 256 && !hm) wide = true;
-    // ... as 4 wavefronts of 64 queries when nothing is excluded at all, else as 8 wavefronts of 32 (D = 128 only)
-    const bool plain = !causal && kv_len == nullptr && N_kv % 64 == 0;
+    const bool plain = fwd_plain(N_kv, causal != 0, kv_len != nullptr);
     const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
     const bool d96 = narrow(std::max(D, Dv));
-    if (wide && !plain && DP == 64) wide = false;
-    if (wide && q_tile_plan == 0) {
-        const int64_t total256 = (int64_t)((N_q + 255) / 256) * B * H, cus = device_cu_count();
-        // (without exclusions a last round on an eighth of the units is cut into 32-query workgroups, launch_fwd_wide)
-        wide = !thin_last_round(total256, cus, 3) || (plain && (total256 >= 2 * cus || thin_last_round(total256, cus, 8)));
-    }
+    // a plan (128 or 256 query rows per workgroup) stands in for the rule where the kernels leave the choice open
+    const bool wide = q_tile_plan == 0 ? fwd_rule_wide(B, H, N_q, N_kv, DP, causal != 0, hm, kv_len != nullptr) : q_tile_plan == 256 && !hm;
     // a keep-mask of keys: the walk takes the attended tiles only (up to what their list holds)
     if (keep_mask != nullptr && bias == nullptr && keys_only(p.m, N_q, N_kv))
         return d96 ? launch_fwd<96, kExKeys, 4>(p, s) : DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
@@ -1282,7 +1284,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     if (hm) return DP == 128 ? launch_fwd<128, kExGeneral, 4>(p, s) : launch_fwd<64, kExGeneral, 4>(p, s);
     if (wide) {
         if (plain) return d96 ? launch_fwd_wide<96>(p, s) : DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
-        return d96 ? launch_fwd<96, kExNone, 8>(p, s) : launch_fwd<128, kExNone, 8>(p, s);
+        return d96 ? launch_fwd<96, kExNone, 8>(p, s) : DP == 128 ? launch_fwd<128, kExNone, 8>(p, s) : launch_fwd<64, kExNone, 8>(p, s);
     }
     if (q_tile_plan == 0 && fwd_rule_keyshare((int64_t)B * H, N_q)) {
         const int64_t rows = (int64_t)B * H * N_q;
@@ -1752,7 +1754,8 @@ FlameAttnStatus flame_sdpa_chunked_bf16(const void* q, const void* k, const void
     // the masked kernels come with 128-row workgroups only, and head dims other than the multiples of 8 up to 128 have
     // one kernel (or the materialised path): nothing to choose, so nothing is measured
     const bool one_tile = mask != nullptr || !head_dim_ok(Dh);
-    const int rule_q = (!one_tile && fwd_rule_wide(B, H, Q, false, false)) ? 256 : 128;
+    const int DP = std::max(padded_head_dim(Dh), padded_head_dim(Dv));
+    const int rule_q = (!one_tile && fwd_rule_wide(B, H, Q, K, DP, causal != 0, false, false)) ? 256 : 128;
     const PlanKey key{B, H, Q, K, Dh, Dv, mask ? mask_heads : 0, causal ? 1 : 0};
     int q_tile = rule_q;
     uint64_t source = kPlanRule, candidates = 1, best_ns = 0;

@@ -1,4 +1,6 @@
 """Helpers shared by the GPU parity tests: numpy bf16 bit patterns <-> torch device tensors."""
+import ctypes
+
 import numpy as np
 import torch
 
@@ -62,3 +64,37 @@ def assert_close_bf16(oracle, name, got_f32, ref_bits, ref_f32, max_abs=TOL_MAX_
     else:
         assert n_bad == 0, name
     return ma_f, rl_f
+
+
+class _Dim3(ctypes.Structure):
+    _fields_ = [(a, ctypes.c_uint) for a in "xyz"]
+
+
+class _KernelNodeParams(ctypes.Structure):
+    _fields_ = [("block", _Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", _Dim3), ("params", ctypes.c_void_p),
+                ("lds", ctypes.c_uint)]
+
+
+def recorded_launches(call):
+    """[(kernel's name, workgroups, lanes per workgroup)] of what `call` launches, in the order of the nodes of a HIP graph that
+    records it; the graph is not run.  The kernels' attributes are set by a call before that."""
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        kept = call()
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))      # the one in use
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    handle, n, kind = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0), ctypes.c_int(0)
+    assert hip.hipGraphGetNodes(handle, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(handle, nodes, ctypes.byref(n)) == 0
+    out = []
+    for node in nodes:
+        node, p = ctypes.c_void_p(node), _KernelNodeParams()
+        assert hip.hipGraphNodeGetType(node, ctypes.byref(kind)) == 0
+        if kind.value == 0:                     # a kernel
+            assert hip.hipGraphKernelNodeGetParams(node, ctypes.byref(p)) == 0
+            out.append((hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), None).decode(), p.grid.x, p.block.x))
+    del kept
+    return out

@@ -166,3 +166,45 @@ def test_256_row_plan_past_one_round(forced, B, H, Q, K, D):
     s = _child({"FLAME_SDPA_QCHUNK": forced} if forced else {}, CHILD_MARGINS % (B, H, Q, K, D))
     assert s["errors"] == 0 and s["last_q_chunk"] in ((256,) if forced else (128, 256))
     assert s["tuned"] == (0 if forced else 1)
+
+
+# what runs is what the plan says: a 256-row workgroup has 8 wavefronts where something is excluded, a 128-row one 4
+CHILD_RUNS = CHILD.replace("B, H, Q, K, D = 1, 4, 384, 256, 128", "B, H, Q, K, D, causal = %d, %d, %d, %d, %d, %d").replace(
+    "_chunked(lib, q, k, v, out, 0.09)", "_chunked(lib, q, k, v, out, 0.09, causal)").replace("0.09, want_f32", "0.09, causal=bool(causal), want_f32").replace(
+    "print(json.dumps(_stats(lib)))", r"""
+st = _stats(lib)
+from tests.gpu_util import recorded_launches
+def call():
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert lib.flame_sdpa_chunked_bf16(p(q), p(k), p(v), B, H, Q, K, D, D, ctypes.c_float(0.09), 64, causal, 1, None, p(out), None,
+                                       ctypes.c_uint64(0), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+st["launches"] = [x[1:] for x in recorded_launches(call)]
+print(json.dumps(st))""")
+
+
+@pytest.mark.parametrize("B,H,Q,K,D,causal", [(1, 4, 384, 256, 64, 1), (2, 3, 300, 200, 40, 0), (1, 4, 384, 200, 96, 1), (1, 3, 500, 320, 128, 1)])
+@pytest.mark.parametrize("forced,lanes", [("256", 512), ("128", 256)])
+def test_forced_tile_is_the_one_that_runs(B, H, Q, K, D, causal, forced, lanes):
+    print(f"[plan] {B}x{H} Q={Q} K={K} D={D} causal={causal} FLAME_SDPA_QCHUNK={forced}", flush=True)
+    s = _child({"FLAME_SDPA_QCHUNK": forced}, CHILD_RUNS % (B, H, Q, K, D, causal))
+    assert s["last_q_chunk"] == int(forced) and s["clamped"] == 0
+    assert s["launches"] == [[-(-Q // int(forced)) * B * H, lanes]]
+
+
+def test_a_stored_plan_of_256_rows_is_the_one_that_runs(tmp_path):
+    f = tmp_path / "plans.json"
+    f.write_text('{"meta":{"version":1}}\n{"key":{"B":1,"H":4,"Q":384,"K":256,"Dh":64,"Dv":64,"mask_heads":0,"causal":1},"plan":{"q":256,"k":64}}\n')
+    s = _child({"FLAME_SDPA_AUTOTUNE_CACHE": str(f)}, CHILD_RUNS % (1, 4, 384, 256, 64, 1))
+    assert s["last_plan_source"] == 1 and s["last_q_chunk"] == 256 and s["launches"] == [[8, 512]]
+
+
+@pytest.mark.parametrize("B,H,Q,K,D,causal,rows", [(1, 36, 2048, 256, 128, 1, 128),      # 288 units of 256 queries: a thin last round
+                                                   (1, 32, 2048, 256, 128, 1, 256),      # a whole one
+                                                   (1, 32, 2048, 256, 64, 1, 128), (1, 32, 2048, 200, 64, 0, 128)])
+def test_the_rule_is_that_of_a_call_without_a_plan(B, H, Q, K, D, causal, rows):
+    print(f"[plan] rule {B}x{H} Q={Q} K={K} D={D} causal={causal}", flush=True)
+    code = (CHILD_RUNS % (B, H, Q, K, D, causal)).replace("print(json.dumps(st))", r"""
+st["plain_call"] = [x[1:] for x in recorded_launches(lambda: capi.attn_fwd(q, k, v, 0.09, causal=bool(causal), out=out))]
+print(json.dumps(st))""")
+    s = _child({"FLAME_SDPA_AUTOTUNE": "0"}, code)
+    assert s["last_q_chunk"] == rows and s["launches"] == s["plain_call"] == [[-(-Q // rows) * B * H, 512 if rows == 256 else 256]]
