@@ -344,12 +344,17 @@ __device__ __forceinline__ void dma4(const void* gsrc, void* lds_dst) { dma4(gsr
 __device__ __forceinline__ void dma16u(const void* gbase_wave_uniform, uint32_t lane_byte_off, void* lds_dst) {
     dma16u(gbase_wave_uniform, lane_byte_off, lds_addr(lds_dst));
 }
-__device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0) only
-// at most N of this wavefront's vector memory operations are still outstanding (they complete in order)
+__device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0) only; a barrier follows
+// At most N of this wavefront's vector memory operations are still outstanding (they complete in order).  The builtin is no
+// access to memory for the compiler, which would move a plain load past it: the count would then stand for copies, and a read of
+// their tile could come too early.  The empty statements keep every access on its side; the wait itself stays the builtin, so
+// that the compiler knows what has landed.
 template <int N>
 __device__ __forceinline__ void wait_vm() {
     static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit field");
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+    asm volatile("" ::: "memory");
 }
 
 // Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by linear id.  Remap the id

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void fwd_keyshare_kernel(const FwdParams p) {
             issue_tile(t + NW, stage ^ 1);
             wait_vm<2 * NDMA>();                   // this tile has landed, the next one is in flight
         } else {
-            wait_vm0();
+            wait_vm<0>();                          // no barrier follows: the tile is this wavefront's own
         }
         __builtin_amdgcn_sched_barrier(0);
         const uint16_t* ks = own + stage * T::STAGE_ELEMS;

@@ -186,3 +186,62 @@ def test_every_lds_dma_finds_its_destination_in_m0(text):
                 raise AssertionError(f"{name}: `{l}` has no M0 write before it")
             assert between >= 1, f"{name}: `{l}` follows its M0 write without a wait state"
     assert checked >= 100
+
+
+WAIT_PROBE = r"""
+#include "attn_common.hpp"
+using namespace fattn;
+template <class W> __device__ void around(const float* x, float* out, const char* src, int n, W wait) {
+    extern __shared__ __attribute__((aligned(1024))) uint16_t lds[];
+    dma16u(src, threadIdx.x * 16, lds_addr(lds));
+    const float v = x[threadIdx.x];
+    wait();
+    if (n > 3) out[threadIdx.x] = v;           // the one use: the compiler would rather load there
+}
+extern "C" __global__ void counted(const float* x, float* out, const char* src, int n) { around(x, out, src, n, [] { wait_vm<1>(); }); }
+extern "C" __global__ void drained(const float* x, float* out, const char* src, int n) { around(x, out, src, n, [] { wait_vm<0>(); }); }
+"""
+
+
+def test_no_load_moves_past_a_wait(tmp_path):
+    """A counted wait says how many younger operations may still be on their way; a load that the compiler moved past it would
+    leave as many copies unfinished."""
+    if shutil.which(fb.HIPCC) is None and not os.path.exists(fb.HIPCC):
+        pytest.skip("hipcc not available")
+    src, out = tmp_path / "probe.hip", tmp_path / "probe.s"
+    src.write_text(WAIT_PROBE)
+    flags = [f for f in fb.FLAGS if f not in ("-shared", "-fPIC")]
+    subprocess.run([fb.HIPCC, *flags, "-I" + fb.CSRC, "-S", "--cuda-device-only", str(src), "-o", str(out)], check=True, stdout=subprocess.DEVNULL,
+                   stderr=subprocess.DEVNULL)
+    for name, count in (("counted", 1), ("drained", 0)):
+        body = re.search(r"^%s:.*?s_endpgm" % name, out.read_text(), re.S | re.M).group(0)
+        order = re.findall(r"^\s+(global_load_lds_dwordx4|global_load_dword\b|s_waitcnt vmcnt\(%d\))" % count, body, re.M)
+        assert order[:3] == ["global_load_lds_dwordx4", "global_load_dword", f"s_waitcnt vmcnt({count})"], (name, order)
+
+
+def test_the_bias_counted_out_of_a_wait_is_younger_than_the_copies(text):
+    """The forward that requests its bias a step ahead: between a step's last copy and the wait that leaves N operations on their
+    way, which the step's barrier follows, there are at least N loads of the bias."""
+    checked = 0
+    for excl, pieces in ((3, 8), (4, 4)):                # fp32, bf16: loads per lane and tile
+        name = "_ZN5fattn10fwd_kernelILi64ELi%dELi4ELi0ELi1ELb1EEEvNS_9FwdParamsE" % excl
+        body = re.search(r"^%s:.*?\.end_amdhsa_kernel" % name, text, re.S | re.M).group(0)
+        ins = [l.strip() for l in body.split("\n") if re.match(r"^\s+[a-z]", l) or re.match(r"^\.LBB\S+:", l)]
+        for i, l in enumerate(ins):
+            if not l.startswith(f"s_waitcnt vmcnt({pieces})") or not any(x.startswith("s_barrier") for x in ins[i + 1:i + 8]):
+                continue
+            loads, skipped = 0, None                     # skipped: the label that a branch over a few instructions goes to
+            for l2 in reversed(ins[:i]):
+                if l2.startswith(".LBB"):
+                    assert skipped is None, f"{name}: more than a branch over a few instructions between copies and wait"
+                    skipped = l2.split(":")[0]
+                elif l2.startswith("s_cbranch") and l2.endswith(skipped or "-"):
+                    skipped = None
+                elif l2.startswith("global_load_lds"):
+                    break
+                elif l2.startswith("global_load_dword"):
+                    assert skipped is None, f"{name}: `{l2}` is not always executed"
+                    loads += 1
+            assert skipped is None and loads >= pieces, (name, loads)
+            checked += 1
+    assert checked == 4                                  # two steps per trip of the loop in either kernel
