@@ -31,7 +31,8 @@ namespace {
 using at::Tensor;
 
 #define FLAME_HOST_ENTRY_POINTS(X)                                                                                      \
-    X(flame_attn_fwd_bf16) X(flame_attn_fwd_ws_bf16) X(flame_attn_fwd_scratch_bytes) X(flame_attn_mask_workspace_bytes) X(flame_attn_fwd_bias_bf16) \
+    X(flame_attn_fwd_bf16) X(flame_attn_fwd_ws_bf16) X(flame_attn_fwd_workspace_bytes) X(flame_attn_fwd_scratch_bytes) X(flame_attn_mask_workspace_bytes) \
+    X(flame_attn_fwd_bias_bf16)                                                                                         \
     X(flame_attn_bwd_bf16) X(flame_attn_bwd_workspace_bytes) X(flame_attn_fwd_dropout_tiled_bf16)                       \
     X(flame_attn_bwd_dropout_tiled_bf16) X(flame_attn_materialised_workspace_bytes) X(flame_attn_fwd_materialised_bf16) \
     X(flame_attn_bwd_materialised_bf16) X(flame_sage_quant_qk_int8_ks) X(flame_sage_attn_fwd_bias_int8)                 \
@@ -177,6 +178,16 @@ Tensor empty(at::IntArrayRef size, at::ScalarType dt, const Tensor& like) {
     return at::Tensor(at::detail::empty_cuda(size, dt, like.device(), std::nullopt));
 }
 Tensor bytes_like(size_t n, const Tensor& like) { return empty({(int64_t)n}, at::kByte, like); }
+// Room that a call is faster with but does not need (up to 1 GiB of mask words, one slice's probabilities): undefined where the
+// device has none left.
+Tensor optional_bytes_like(size_t n, const Tensor& like) {
+    if (n == 0) return Tensor();
+    try {
+        return bytes_like(n, like);
+    } catch (const c10::OutOfMemoryError&) {
+        return Tensor();
+    }
+}
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
 
 // ---------------------------------------------------------------- forward and backward
@@ -195,7 +206,11 @@ int call_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Sizes& z, 
     if (!ws.defined()) {       // room for the slices of a key split, where the grid would leave compute units idle, or for the mask as bits
         const size_t need = f.mask.data ? g_api.flame_attn_mask_workspace_bytes(z.B, z.H, z.Sq, z.Sk, f.mask.strides(), f.kv_len.defined(), f.causal)
                                         : g_api.flame_attn_fwd_scratch_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
-        if (need) ws = bytes_like(need, q);
+        ws = optional_bytes_like(need, q);
+        if (need && !ws.defined() && !f.mask.data) {       // the probabilities of wide heads do not fit: partial outputs may
+            const size_t less = g_api.flame_attn_fwd_workspace_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
+            if (less < need) ws = optional_bytes_like(less, q);
+        }
     }
     if (ws.defined())
         return g_api.flame_attn_fwd_ws_bf16(ptr(q), ptr(k), ptr(v), ptr(o), ptr(lse), z.B, z.H, z.Sq, z.Sk, z.D, scale, strides4(q), strides4(k),
@@ -217,9 +232,10 @@ void alloc_grads(const Tensor& q, const Sizes& z, Grads& g) {
 int call_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& d_o, const Tensor& lse, const Sizes& z, float scale,
              bool causal, const Tensor& kv_len, const MaskView& mask, Tensor workspace, Grads& g) {
     if (!workspace.defined()) {
-        size_t need = g_api.flame_attn_bwd_workspace_bytes(z.B, z.H, z.Sq, z.D);
-        if (mask.data) need += g_api.flame_attn_mask_workspace_bytes(z.B, z.H, z.Sq, z.Sk, mask.strides(), kv_len.defined(), causal);
-        workspace = bytes_like(need, q);
+        const size_t need = g_api.flame_attn_bwd_workspace_bytes(z.B, z.H, z.Sq, z.D);
+        const size_t words = mask.data ? g_api.flame_attn_mask_workspace_bytes(z.B, z.H, z.Sq, z.Sk, mask.strides(), kv_len.defined(), causal) : 0;
+        if (words) workspace = optional_bytes_like(need + words, q);
+        if (!workspace.defined()) workspace = bytes_like(need, q);
     }
     if (!g.dq.defined()) alloc_grads(q, z, g);
     return g_api.flame_attn_bwd_bf16(ptr(q), ptr(k), ptr(v), ptr(o), ptr(d_o), ptr(lse), ptr(g.dq), ptr(g.dk), ptr(g.dv), z.B, z.H, z.Sq, z.Sk, z.D,
