@@ -1,5 +1,6 @@
 """Room that a call is faster with but does not need: where the device has none left (here: past the limit set for the process) the
-kernels that do without serve the call, bit for bit as with a workspace too small."""
+kernels that do without serve the call, bit for bit as with a workspace too small; and none is asked for by a call that the
+fused kernels refuse."""
 import pytest
 import torch
 
@@ -64,3 +65,22 @@ def test_wide_heads(slack, split):
         capi.attn_fwd(q, k, v, D ** -0.5, out=o1, lse_out=lse1)
         torch.cuda.synchronize()
     assert torch.equal(o, o1) and torch.equal(lse, lse1)
+
+
+@pytest.mark.parametrize("D", [160, 36])
+def test_a_refused_call_asks_for_none(D):
+    from flame_amd import capi
+    B, H, S = 1, 4, 1024
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (_randn(g, B, H, S, D) for _ in range(3))
+    o, lse = torch.empty_like(q), torch.empty((B * H, S), device="cuda")
+    mask = torch.randint(0, 2, (B, H, S, S), device="cuda", generator=g, dtype=torch.uint8)
+    asked = lambda: torch.cuda.memory_stats()["requested_bytes.all.allocated"]                        # noqa: E731
+    grads = tuple(torch.empty_like(t) for t in (q, k, v))
+    before = asked()
+    with pytest.raises(capi.FlameAttnError):
+        capi.attn_fwd(q, k, v, D ** -0.5, mask=mask, out=o, lse_out=lse)
+    assert asked() == before
+    with pytest.raises(capi.FlameAttnError):
+        capi.attn_bwd(q, k, v, o, q, lse, D ** -0.5, mask=mask, grads=grads)
+    assert asked() - before <= capi.bwd_workspace_bytes(B, H, S, D)
