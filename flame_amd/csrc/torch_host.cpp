@@ -19,6 +19,7 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>      // this torch names its HIP devices "cuda"
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -283,12 +284,16 @@ Tensor as_bf16_view(const Tensor& x) {
     return t;
 }
 
-// A tensor whose elements are what its address and strides say: no mode, transform or subclass has a part in what .to() does to it.
+// A tensor whose elements are what its address and strides say, where no subclass, mode or transform, of the tensor's or of the
+// calling thread's, has a part in what .to() does to it.
 bool plain_f32(const Tensor& t) {
-    static const c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::Functionalize,
-                                              c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Batched,
-                                              c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
-    if (t.scalar_type() != at::kFloat || !t.is_cuda() || t.layout() != at::kStrided || t.key_set().has_any(special) || t.stride(3) != 1) return false;
+    static const c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::PythonDispatcher,
+                                              c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                              c10::DispatchKey::FuncTorchVmapMode, c10::DispatchKey::FuncTorchDynamicLayerFrontMode,
+                                              c10::DispatchKey::Batched, c10::DispatchKey::VmapMode, c10::DispatchKey::Conjugate,
+                                              c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+    if ((t.key_set() | c10::impl::tls_local_dispatch_key_set().included_).has_any(special)) return false;
+    if (t.scalar_type() != at::kFloat || !t.is_cuda() || t.layout() != at::kStrided || t.stride(3) != 1) return false;
     for (int ax = 0; ax < 3; ++ax)          // .to() keeps such strides, and the kernels refuse them
         if (t.size(ax) == 1 && t.stride(ax) % 8 != 0) return false;
     return true;

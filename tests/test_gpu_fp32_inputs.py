@@ -52,3 +52,28 @@ def test_special_values_and_graph():
     a = [t.detach().nan_to_num(0.0).requires_grad_(True) for t in (q, k, v)]        # a graph: recorded as before
     F.sdpa(*a).sum().backward()
     assert all(t.grad is not None and t.grad.dtype == torch.float32 and bool(t.grad.isfinite().all()) for t in a)
+
+
+def test_a_dispatch_mode_sees_the_conversions():
+    """... as they were before the one-launch conversion, which calls outside of such a mode take."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from flame_amd import functional as F
+    from tests.gpu_util import recorded_launches
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(func.name())
+            return func(*args, **(kwargs or {}))
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v = (torch.randn((1, 2, 100, 64), device="cuda", generator=g) for _ in range(3))
+    want = F.sdpa(q, k, v)
+    with Seen() as seen:
+        got = F.sdpa(q, k, v)
+    assert seen.names.count("aten::_to_copy") == 4          # Q, K, V and the output
+    assert torch.equal(got, want)
+    assert any("cast_qkv_kernel" in name for name, _, _ in recorded_launches(lambda: F.sdpa(q, k, v)))
