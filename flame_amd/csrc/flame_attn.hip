@@ -320,8 +320,9 @@ bool mask_bits_fit(const MaskArgs& m, int B, int H, int N_q, int N_kv, const voi
     const size_t need = mask_bits_bytes(m, B, H, N_q, N_kv);
     return need && ws && need <= bytes && reinterpret_cast<uintptr_t>(ws) % 16 == 0;
 }
-// writes the words and flags to `ws` (mask_bits_bytes) and points `m` to them; the causal flag is in them then
-int launch_mask_bits(MaskArgs& m, int B, int H, int N_q, int N_kv, void* ws, hipStream_t s) {
+// writes the words and flags to `ws` (mask_bits_bytes) and points `m` to them; the causal flag is in them then.
+// kind: of the kernel that walks by them first, whose time the pass counts to
+int launch_mask_bits(MaskArgs& m, int B, int H, int N_q, int N_kv, void* ws, int kind, hipStream_t s) {
     const MaskPlanes z = mask_planes(m, B, H, N_q, N_kv);
     const int64_t tiles = z.planes * z.n_qt * z.n_kt, grid = z.planes * z.n_qt * ((z.n_kt + 3) / 4);
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
@@ -335,7 +336,10 @@ int launch_mask_bits(MaskArgs& m, int B, int H, int N_q, int N_kv, void* ws, hip
     p.rows = static_cast<uint64_t*>(ws);
     p.cols = p.rows + 64 * tiles;
     p.flags = reinterpret_cast<uint8_t*>(p.cols + 64 * tiles);
-    hipLaunchKernelGGL(m.mask_mode == kMaskU8 && m.sk == 1 && N_kv >= 16 ? mask_bits_kernel<true> : mask_bits_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, p);
+    {
+        ScopedKernelTimer t(kind, s);
+        hipLaunchKernelGGL(m.mask_mode == kMaskU8 && m.sk == 1 && N_kv >= 16 ? mask_bits_kernel<true> : mask_bits_kernel<false>, dim3((unsigned)grid), dim3(256), 0, s, p);
+    }
     m.bit_rows = p.rows;
     m.bit_cols = p.cols;
     m.tile_flags = p.flags;
@@ -360,7 +364,7 @@ int launch_bwd_bits(BwdParams p, hipStream_t s) {
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern_kv), T::LDS_BYTES + most, kv_set)) return rc;
     const int64_t grid = (int64_t)((p.Sk + T::BN - 1) / T::BN) * p.B * p.H, grid_dq = (int64_t)((p.Sq + TQ::BM - 1) / TQ::BM) * p.B * p.H;
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
-    if (const int rc = launch_mask_bits(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, s)) return rc;
+    if (const int rc = launch_mask_bits(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, FLAME_ATTN_KERNEL_BWD_DQ, s)) return rc;
     p.split_ws = nullptr;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);
@@ -1267,7 +1271,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         return d96 ? launch_fwd<96, kExKeys, 4>(p, s) : DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
     // any other keep-mask, with room for it as bits
     if (keep_mask != nullptr && bias == nullptr && mask_bits_fit(p.m, B, H, N_q, N_kv, scratch.ws, scratch.bytes)) {
-        if ((rc = launch_mask_bits(p.m, B, H, N_q, N_kv, scratch.ws, s))) return rc;
+        if ((rc = launch_mask_bits(p.m, B, H, N_q, N_kv, scratch.ws, FLAME_ATTN_KERNEL_FWD, s))) return rc;
         return d96 ? launch_fwd<96, kExBits, 4>(p, s) : DP == 128 ? launch_fwd<128, kExBits, 4>(p, s) : launch_fwd<64, kExBits, 4>(p, s);
     }
     // a keep-mask with vector-loadable rows over whole tiles and no bias: the lean masked kernel

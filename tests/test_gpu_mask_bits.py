@@ -64,3 +64,17 @@ def test_against_the_oracle(oracle, kind, B, H, Sq, Sk, D, causal, kv_len):
     want = oracle.sdpa_bwd(t[0], t[1], t[2], ro, t[3], sc, causal=causal, kv_len=kv_len, mask=full, want_f32=True)
     for name, g, w, w32 in zip(("dQ", "dK", "dV"), got, want[:3], want[3:]):
         assert_close_bf16(oracle, name, to_f32(g), w, w32)
+
+
+def test_the_pass_over_the_mask_is_timed():
+    """The library's kernel times hold the pass that turns the mask into bits: with the forward, and with dQ."""
+    from flame_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(4)
+    q, k, v, do = (torch.randn((1, 2, 512, 64), device="cuda", generator=g).bfloat16() for _ in range(4))
+    mask = torch.randint(0, 2, (1, 1, 512, 512), device="cuda", generator=g, dtype=torch.uint8)
+    capi.profiling_enable(True)
+    o, lse = capi.attn_fwd(q, k, v, 0.125, mask=mask)
+    capi.attn_bwd(q, k, v, o, do, lse, 0.125, mask=mask)
+    launches = {kind: n for kind, (_, n) in capi.profiling_read().items() if n}
+    capi.profiling_enable(False)
+    assert launches == {"fwd": 2, "bwd_dq": 2, "bwd_dkdv": 1}
