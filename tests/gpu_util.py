@@ -1,5 +1,7 @@
 """Helpers shared by the GPU parity tests: numpy bf16 bit patterns <-> torch device tensors."""
 import ctypes
+import re
+import subprocess
 
 import numpy as np
 import torch
@@ -76,8 +78,8 @@ class _KernelNodeParams(ctypes.Structure):
 
 
 def recorded_launches(call):
-    """[(kernel's name, workgroups, lanes per workgroup)] of what `call` launches, in the order of the nodes of a HIP graph that
-    records it; the graph is not run.  The kernels' attributes are set by a call before that."""
+    """[(kernel's name with its template arguments, workgroups, lanes per workgroup)] of what `call` launches, in the order of the
+    nodes of a HIP graph that records it; the graph is not run.  The kernels' attributes are set by a call before that."""
     call()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph(keep_graph=True)
@@ -97,4 +99,5 @@ def recorded_launches(call):
             assert hip.hipGraphKernelNodeGetParams(node, ctypes.byref(p)) == 0
             out.append((hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), None).decode(), p.grid.x, p.block.x))
     del kept
-    return out
+    plain = subprocess.run(["c++filt"], input="\n".join(name for name, _, _ in out), capture_output=True, text=True, check=True).stdout.split("\n")
+    return [(re.sub(r"^void |fattn::|\(anonymous namespace\)::|\([^()]*\)$", "", name), *rest) for name, (_, *rest) in zip(plain, out)]
