@@ -9,7 +9,8 @@ MIB = 1 << 20
 
 
 class _Limit:
-    """At most `slack` bytes beyond what the process holds now."""
+    """No block above `slack` bytes, whatever room earlier tests left within the segments that the process holds, and at most
+    `slack` bytes beyond those."""
 
     def __init__(self, slack):
         self.slack = slack
@@ -19,9 +20,16 @@ class _Limit:
         torch.cuda.empty_cache()
         total = torch.cuda.get_device_properties(0).total_memory
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + self.slack) / total)
+        self.held = []
+        try:
+            while True:
+                self.held.append(torch.empty(self.slack + 1, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            pass
 
     def __exit__(self, *exc):
         torch.cuda.set_per_process_memory_fraction(1.0)
+        self.held = None
 
 
 def _randn(g, *shape):
