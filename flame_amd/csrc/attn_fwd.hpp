@@ -138,7 +138,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     // KEYS: step t of the walk takes tile tile_of(t) (elsewhere the two are the same number); stages go by the step
     constexpr bool BITS = EXCL == kExBits, KEYS = EXCL == kExKeys || BITS;
     KeyTiles kt;
-    const uint64_t* brows = nullptr;               // BITS: this lane's query's word of key tile 0; tiles lie 64 bit_nqt words apart
+    const uint64_t* brows = nullptr;               // BITS: words of key tile 0, one per query; tiles lie 64 bit_nqt words apart
     if constexpr (BITS) {
         const int plane = b * p.m.plane_b + hh * p.m.plane_h;
         const uint8_t* flags = p.m.tile_flags + ((int64_t)plane * p.m.bit_nqt + q0 / 64) * p.m.bit_nkt;       // of the first 64 queries, then of the others
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
             return f0 & f1 & kTileAllKeys ? 2 : (f0 | f1) & kTileAny ? 1 : 0;
         });
         n_tiles = kt.n_tiles;
-        brows = p.m.bit_rows + (int64_t)plane * p.m.bit_nkt * (64 * p.m.bit_nqt) + qi;
+        brows = p.m.bit_rows + (int64_t)plane * p.m.bit_nkt * (64 * p.m.bit_nqt);
     } else if constexpr (KEYS) {
         kt.build(reinterpret_cast<char*>(lds) + T::LDS_BYTES, klimit, NW, [&](int key) {
             return key < klimit && mask_attends(p.m, mbase, (int64_t)min(key, p.Sk - 1) * p.m.sk);
@@ -266,9 +266,16 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     int lim = 0;                   // keys of the tile below it attend, counted from 4h
     MaskRow64 mrow;
     uint32_t keep_bits[2];         // KEYS: of this lane's half, key block by key block
+    // BITS: the word of the next cut tile.  Requested a step ahead: loads return in order, so that one which a step itself waits
+    // for makes it wait for the copies that it has just issued as well.
+    uint64_t word_ahead = 0;
+    auto word_of = [&](int t) {
+        return *reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(brows + (int64_t)kt.tile(t) * (64 * p.m.bit_nqt)) + 8u * (uint32_t)qi);
+    };
     auto excl_begin = [&](int t) {
         if constexpr (KEYS) {
-            const uint64_t w = BITS ? brows[(int64_t)kt.tile(t) * (64 * p.m.bit_nqt)] : kt.bits[kt.tile(t)];
+            const uint64_t w = BITS ? word_ahead : kt.bits[kt.tile(t)];
+            if (BITS && t + 1 < n_tiles) word_ahead = word_of(t + 1);
             keep_bits[0] = (uint32_t)w >> (4 * h);
             keep_bits[1] = (uint32_t)(w >> 32) >> (4 * h);
         }
@@ -285,6 +292,10 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     int t_clean = KEYS ? kt.n_whole : (EXCL == kExNone || BIAS) ? klimit / BN : 0;
     if (p.m.causal) t_clean = min(t_clean, (q0 + 1 - key0) / BN);
     t_clean = max(min(t_clean, n_tiles), 0);
+    if constexpr (BITS) {
+        const int first = t_clean == 0 ? 0 : (t_clean - 1) | 1;      // that a step with exclusions takes: steps go in pairs, see below
+        if (first < n_tiles) word_ahead = word_of(first);
+    }
 
     // Bias: every lane needs 64 (of its half: 32) consecutive values of its query's row.  Four neighbouring lanes load 64 bytes
     // of a row (a "piece" is 16 rows of that, one instruction), and two pieces, 32 rows, at a time pass through 2 KiB of LDS

@@ -245,3 +245,19 @@ def test_the_bias_counted_out_of_a_wait_is_younger_than_the_copies(text):
             assert skipped is None and loads >= pieces, (name, loads)
             checked += 1
     assert checked == 4                                  # two steps per trip of the loop in either kernel
+
+
+def test_words_of_a_mask_are_not_waited_for_within_their_step(text):
+    """The forward that walks by a mask's bits: loads return in order, so a step that waits for a word which it has requested itself waits
+    for its tile copies as well.  The word is the next step's; the first wait behind it is the one in front of the barrier."""
+    for D, mfmas in ((64, 16), (96, 24), (128, 32)):          # half a step's or more are between
+        name = "_ZN5fattn10fwd_kernelILi%dELi6ELi4ELi0ELi1ELb0EEEvNS_9FwdParamsE" % D
+        body = re.search(r"^%s:.*?\.end_amdhsa_kernel" % name, text, re.S | re.M).group(0)
+        ins = [l.strip() for l in body.split("\n") if re.match(r"^\s+[a-z]", l)]
+        first = next(i for i, l in enumerate(ins) if l.startswith("v_mfma"))
+        words = [i for i, l in enumerate(ins) if i > first and l.startswith("global_load_dwordx2")]
+        assert len(words) == 2                                # two steps per trip of the loop
+        for i in words:
+            j = next(j for j in range(i, len(ins)) if ins[j].startswith("s_waitcnt") and "vmcnt" in ins[j])
+            assert any(l.startswith("s_barrier") for l in ins[j:j + 8]), (name, ins[i:j + 1])
+            assert sum(l.startswith("v_mfma") for l in ins[i:j]) >= mfmas, name
