@@ -33,7 +33,8 @@ def _bwd(schedule, *args, **kw):
 
 @pytest.mark.parametrize("B,H,S,D", [(1, 32, 2048, 128),      # 256 workgroups of 256 queries, 512 key blocks: whole rounds
                                      (1, 36, 2304, 128),      # 324 / 648: a partial last round, cut key blocks
-                                     (2, 20, 2048, 64)])      # head dim 64
+                                     (2, 20, 2048, 64),       # head dim 64
+                                     (1, 36, 2304, 96), (1, 32, 2048, 80)])       # on the kernels of head dim 96
 def test_joint_and_rows_schedules_against_default_and_oracle(oracle, B, H, S, D):
     from flame_amd import capi
     print(f"[bwd schedules] {B}x{H} S={S} D={D}", flush=True)

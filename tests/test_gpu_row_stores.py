@@ -5,6 +5,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 from flame_amd import capi  # noqa: E402
+from tests.gpu_util import recorded_launches  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 PATTERN = -7.5
@@ -22,9 +23,11 @@ def _check(buf, view, want):
 
 
 # sizes: a few rows (32 queries per workgroup), partial wavefronts of 128-query workgroups, with two key groups, and 256-query
-# workgroups past one round (129 or more rows of the last tile exist, so that they are used)
+# workgroups (129 or more rows of the last tile exist, so that they are used): of the forward past one round, of forward and dQ
+# in one whole round, also causal
 @pytest.mark.parametrize("D", [8, 40, 64, 72, 96, 128])
-@pytest.mark.parametrize("B,H,Sq,Sk,causal", [(1, 2, 5, 70, False), (2, 40, 129, 65, False), (1, 24, 1055, 1024, True), (2, 70, 481, 128, False)])
+@pytest.mark.parametrize("B,H,Sq,Sk,causal", [(1, 2, 5, 70, False), (2, 40, 129, 65, False), (1, 24, 1055, 1024, True), (2, 70, 481, 128, False),
+                                              (2, 64, 481, 1088, False), (2, 64, 481, 1088, True)])
 def test_rows_in_room(D, B, H, Sq, Sk, causal):
     g = torch.Generator(device="cuda").manual_seed(D + Sq)
     q, k, v, do = (torch.randn((B, H, n, D), device="cuda", generator=g).to(torch.bfloat16) for n in (Sq, Sk, Sk, Sq))
@@ -38,3 +41,9 @@ def test_rows_in_room(D, B, H, Sq, Sk, causal):
     capi.attn_bwd(q, k, v, o, do, lse, scale, causal=causal, grads=tuple(v for _, v in bufs))
     for (b, w), ref in zip(bufs, want):
         _check(b, w, ref)
+    if Sk == 1088:
+        names = [name for call in (lambda: capi.attn_fwd(q, k, v, scale, causal=causal), lambda: capi.attn_bwd(q, k, v, o, do, lse, scale, causal=causal))
+                 for name, _, _ in recorded_launches(call) if name.startswith(("fwd", "bwd_dq"))]
+        compiled = 64 if D <= 64 else 96 if D <= 96 else 128
+        fwd = f"fwd_wide_kernel<{compiled}>" if not causal else f"fwd_kernel<{compiled}, 0, {4 if D <= 64 else 8}, 0, 1, false>"
+        assert names == [fwd, f"bwd_dq_wide_kernel<{compiled}>"], names

@@ -15,7 +15,7 @@ def _reference(q, k, v, do, sc, keep):
     return (o, *torch.autograd.grad(o, (q, k, v), do.float()))
 
 
-@pytest.mark.parametrize("B,H,S,D,kind", [(1, 40, 640, 64, "causal"), (2, 32, 1024, 128, "causal"), (1, 80, 1000, 72, "causal"), (2, 80, 900, 64, "causal"),
+@pytest.mark.parametrize("B,H,S,D,kind", [(1, 40, 640, 64, "causal"), (2, 32, 1024, 128, "causal"), (1, 56, 1000, 64, "causal"), (1, 80, 1000, 72, "causal"), (2, 80, 900, 64, "causal"),
                                           (1, 41, 640, 64, "causal"), (8, 8, 700, 64, "kv_len"), (4, 16, 1101, 128, "keys"), (6, 16, 900, 96, "keys")])
 def test_every_unit_once(B, H, S, D, kind):
     from flame_amd import capi
