@@ -23,6 +23,7 @@
 #include "attn_bwd_wide.hpp"
 #include "attn_fwd_probs.hpp"
 #include "mask_bits.hpp"
+#include "mask_route.hpp"
 #include "fast_div.hpp"
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
@@ -311,12 +312,13 @@ MaskPlanes mask_planes(const MaskArgs& m, int B, int H, int N_q, int N_kv) {
 size_t mask_bits_bytes(const MaskArgs& m, int B, int H, int N_q, int N_kv) {
     const MaskPlanes z = mask_planes(m, B, H, N_q, N_kv);
     if (keys_only(m, N_q, N_kv) || z.n_qt > KeyTiles::kMaxTiles || z.n_kt > KeyTiles::kMaxTiles) return 0;
-    if ((int64_t)z.n_qt * z.n_kt < 36) return 0;            // (256 x 256, 4 heads: a training step of 35 us; the pass over the mask costs 2 launches)
+    if (!mask_bits_pay(true, false, false, 0, N_q, N_kv, false)) return 0;      // too few tiles whatever the mask's rows are
     const int64_t tiles = z.planes * z.n_qt * z.n_kt;
     return tiles > (int64_t)1 << 20 ? 0 : align_up((size_t)tiles * (2 * 512 + 1), 256);       // 1 GiB
 }
-// (a workspace that nothing was kept in before may have any alignment)
-bool mask_bits_fit(const MaskArgs& m, int B, int H, int N_q, int N_kv, const void* ws, size_t bytes) {
+// whether they are formed: they pay, and there is room (a workspace that nothing was kept in before may have any alignment)
+bool mask_bits_fit(const MaskArgs& m, bool backward, int B, int H, int N_q, int N_kv, const void* ws, size_t bytes) {
+    if (!mask_bits_pay(backward, m.rows16 != 0, m.sh != 0 && H > 1, m.sq, N_q, N_kv, m.causal != 0)) return false;
     const size_t need = mask_bits_bytes(m, B, H, N_q, N_kv);
     return need && ws && need <= bytes && reinterpret_cast<uintptr_t>(ws) % 16 == 0;
 }
@@ -383,7 +385,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     using T = BwdTile<D>;
     using TQ = BwdDqTile<D>;
     if constexpr (HASMASK && !TIMING) {
-        if (mask_bits_fit(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, p.split_ws_bytes))
+        if (mask_bits_fit(p.m, true, p.B, p.H, p.Sq, p.Sk, p.split_ws, p.split_ws_bytes))
             return D == 128 && narrow(p.d) ? launch_bwd_bits<96>(p, s) : launch_bwd_bits<D>(p, s);
     }
     static bool attr_done = false;
@@ -880,8 +882,7 @@ static int attn_bwd_impl(const void* Q, const void* K, const void* V, const void
     p.m.sh = keep_mask ? mask_strides[1] : 0;
     p.m.sq = keep_mask ? mask_strides[2] : 0;
     p.m.sk = keep_mask ? mask_strides[3] : 0;
-    p.m.rows16 = keep_mask && p.m.sk == 1 && (reinterpret_cast<uintptr_t>(keep_mask) | (uintptr_t)p.m.sb | (uintptr_t)p.m.sh |
-                                              (uintptr_t)p.m.sq) % 16 == 0;
+    p.m.rows16 = mask_rows16(keep_mask, p.m.sb, p.m.sh, p.m.sq, p.m.sk);
     p.m.causal = causal ? 1 : 0;
     p.phase_cycles = nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1238,8 +1239,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     p.m.sq = keep_mask ? mask_strides[2] : 0;
     p.m.sk = keep_mask ? mask_strides[3] : 0;
     p.m.mask_mode = mask_mode;
-    p.m.rows16 = keep_mask && mask_mode == kMaskU8 && p.m.sk == 1 &&
-                 (reinterpret_cast<uintptr_t>(keep_mask) | (uintptr_t)p.m.sb | (uintptr_t)p.m.sh | (uintptr_t)p.m.sq) % 16 == 0;
+    p.m.rows16 = mask_mode == kMaskU8 && mask_rows16(keep_mask, p.m.sb, p.m.sh, p.m.sq, p.m.sk);
     p.m.causal = causal ? 1 : 0;
     p.m.bias = bias;
     if (bias) {
@@ -1269,8 +1269,8 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     // a keep-mask of keys: the walk takes the attended tiles only (up to what their list holds)
     if (keep_mask != nullptr && bias == nullptr && keys_only(p.m, N_q, N_kv))
         return d96 ? launch_fwd<96, kExKeys, 4>(p, s) : DP == 128 ? launch_fwd<128, kExKeys, 4>(p, s) : launch_fwd<64, kExKeys, 4>(p, s);
-    // any other keep-mask, with room for it as bits
-    if (keep_mask != nullptr && bias == nullptr && mask_bits_fit(p.m, B, H, N_q, N_kv, scratch.ws, scratch.bytes)) {
+    // any other keep-mask, where it pays and there is room, as bits
+    if (keep_mask != nullptr && bias == nullptr && mask_bits_fit(p.m, false, B, H, N_q, N_kv, scratch.ws, scratch.bytes)) {
         if ((rc = launch_mask_bits(p.m, B, H, N_q, N_kv, scratch.ws, FLAME_ATTN_KERNEL_FWD, s))) return rc;
         return d96 ? launch_fwd<96, kExBits, 4>(p, s) : DP == 128 ? launch_fwd<128, kExBits, 4>(p, s) : launch_fwd<64, kExBits, 4>(p, s);
     }

@@ -26,6 +26,7 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/flame_attn.h"
+#include "mask_route.hpp"
 
 namespace {
 
@@ -192,9 +193,12 @@ Tensor optional_bytes_like(size_t n, const Tensor& like) {
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
 
 // ---------------------------------------------------------------- forward and backward
-// Room that a mask as bits takes; none for head dims that the fused kernels refuse with a mask, which go on to the materialised path.
-size_t mask_room(const Sizes& z, const MaskView& mask, const Tensor& kv_len, bool causal) {
+// Room that a mask as bits takes; none for calls that would not form them, nor for head dims that the fused kernels refuse with a
+// mask, which go on to the materialised path.
+size_t mask_room(const Sizes& z, const MaskView& mask, const Tensor& kv_len, bool causal, bool backward) {
     if (!mask.data || z.D > 128 || z.D % 8 != 0) return 0;
+    const bool rows16 = fattn::mask_rows16(mask.data, mask.st[0], mask.st[1], mask.st[2], mask.st[3]);
+    if (!fattn::mask_bits_pay(backward, rows16, mask.st[1] != 0 && z.H > 1, mask.st[2], z.Sq, z.Sk, causal)) return 0;
     return g_api.flame_attn_mask_workspace_bytes(z.B, z.H, z.Sq, z.Sk, mask.strides(), kv_len.defined(), causal);
 }
 struct FwdOpts {
@@ -210,7 +214,7 @@ int call_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Sizes& z, 
     if (!lse.defined() && f.want_lse) lse = empty({(int64_t)z.B * z.H, z.Sq}, at::kFloat, q);
     Tensor ws = f.workspace;
     if (!ws.defined()) {       // room for the slices of a key split, where the grid would leave compute units idle, or for the mask as bits
-        const size_t need = f.mask.data ? mask_room(z, f.mask, f.kv_len, f.causal) : g_api.flame_attn_fwd_scratch_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
+        const size_t need = f.mask.data ? mask_room(z, f.mask, f.kv_len, f.causal, false) : g_api.flame_attn_fwd_scratch_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
         ws = optional_bytes_like(need, q);
         if (need && !ws.defined() && !f.mask.data) {       // the probabilities of wide heads do not fit: partial outputs may
             const size_t less = g_api.flame_attn_fwd_workspace_bytes(z.B, z.H, z.Sq, z.Sk, z.D);
@@ -238,7 +242,7 @@ int call_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
              bool causal, const Tensor& kv_len, const MaskView& mask, Tensor workspace, Grads& g) {
     if (!workspace.defined()) {
         const size_t need = g_api.flame_attn_bwd_workspace_bytes(z.B, z.H, z.Sq, z.D);
-        const size_t words = mask_room(z, mask, kv_len, causal);
+        const size_t words = mask_room(z, mask, kv_len, causal, true);
         if (words) workspace = optional_bytes_like(need + words, q);
         if (!workspace.defined()) workspace = bytes_like(need, q);
     }

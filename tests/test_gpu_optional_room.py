@@ -36,12 +36,20 @@ def _randn(g, *shape):
     return torch.randn(shape, device="cuda", generator=g).bfloat16()
 
 
+def _mask(g, *shape):
+    """One byte off alignment: the kernels that read it do not load its rows as vectors, so that bits pay at any size."""
+    n = 1
+    for x in shape:
+        n *= x
+    return torch.randint(0, 2, (n + 1,), device="cuda", generator=g, dtype=torch.uint8)[1:].view(shape)
+
+
 def test_masks_by_query():
     from flame_amd import capi
     B, H, S, D = 2, 32, 2048, 64                       # 64 planes of a mask: 64 MiB of words
     g = torch.Generator(device="cuda").manual_seed(1)
     q, k, v, do = (_randn(g, B, H, S, D) for _ in range(4))
-    mask = torch.randint(0, 2, (B, H, S, S), device="cuda", generator=g, dtype=torch.uint8)
+    mask = _mask(g, B, H, S, S)
     none = torch.empty(16, dtype=torch.uint8, device="cuda")
     ws = torch.empty(capi.bwd_workspace_bytes(B, H, S, D), dtype=torch.uint8, device="cuda")
     o, lse = capi.attn_fwd(q, k, v, 0.125, mask=mask, workspace=none)
@@ -82,7 +90,7 @@ def test_a_refused_call_asks_for_none(D):
     g = torch.Generator(device="cuda").manual_seed(3)
     q, k, v = (_randn(g, B, H, S, D) for _ in range(3))
     o, lse = torch.empty_like(q), torch.empty((B * H, S), device="cuda")
-    mask = torch.randint(0, 2, (B, H, S, S), device="cuda", generator=g, dtype=torch.uint8)
+    mask = _mask(g, B, H, S, S)
     asked = lambda: torch.cuda.memory_stats()["requested_bytes.all.allocated"]                        # noqa: E731
     grads = tuple(torch.empty_like(t) for t in (q, k, v))
     before = asked()
