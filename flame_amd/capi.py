@@ -92,7 +92,9 @@ def fwd_workspace_bytes(B, H, Sq, Sk, D) -> int:
 
 def attn_fwd(q, k, v, scale, causal=False, kv_len=None, mask=None, want_lse=True, out=None, lse_out=None, workspace=None):
     """O, LSE = flame_attn_fwd_bf16(...).  q [B,H,Sq,D], k/v [B,H,Sk,D] bf16, D stride 1.
-    `workspace` (uint8 device tensor): flame_attn_fwd_ws_bf16 instead, which may use it."""
+    `workspace` (uint8 device tensor): flame_attn_fwd_ws_bf16 uses what it can of it.  Omitted, what the call is faster
+    with is allocated here (more than fwd_workspace_bytes for masks that differ by query and for head dims above 256:
+    flame_attn_mask_workspace_bytes and flame_attn_fwd_scratch_bytes of the C header)."""
     return host().attn_fwd(q, k, v, scale, causal, kv_len, mask, want_lse, out, lse_out, workspace)
 
 

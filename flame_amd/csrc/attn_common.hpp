@@ -371,7 +371,8 @@ __device__ __forceinline__ int xcd_remap(int linear, int total) {
 // (Forward and backward, us: B=4 H=16 S=1101 D=128 key mask 154.5 -> 150.7, B=4 H=16 1024 x 2049 D=64 key lengths 123.5 -> 121.5,
 // B=1 H=16 S=3000 D=128 causal 203 -> 198, its forward 55.3 -> 52.7; four deals turned in pairs: B=4 H=32 S=1024 D=64 causal,
 // forward 27.8 -> 29.2.)
-// j: place in the order of the `total` workgroups of an XCD with 32 compute units.
+// j: place in the order of the `total` workgroups of an XCD with 32 compute units (the whole card's; with another number the
+// order is another one, as complete).
 __device__ __forceinline__ int snake_order(int j, int total) {
     constexpr int kUnits = 32;
     const int end = min(2 * kUnits, total);

@@ -309,7 +309,8 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     // LDS, so that it has a whole step to arrive instead of half of one, and the last wait of a step that
     // copies two whole tiles counts these loads out; the other steps request it behind their barrier, all at once.  A ragged tile is
     // requested across the logit phase as above.  B=1 H=64 S=512 19.7 -> 15.5 us, the rate of a copy; S=256 10.9 -> 8.0; B=1 H=12
-    // S=2048 42.3 -> 36.6, B=4 H=64 S=700 84.7 -> 77.4, B=3 H=16 S=1664 78.5 -> 70.2 us; B=4 H=16 S=1344 gains nothing (63.9 -> 65).
+    // S=2048 42.3 -> 36.6, B=4 H=64 S=700 84.7 -> 77.4, B=3 H=16 S=1664 78.5 -> 70.2 us; B=4 H=16 S=1344 gains
+    // nothing (63.9 -> 65 us, and 59.8 to 60.8 over later runs).
     using BiasPiece = typename std::conditional<EXCL == kExBiasF32, f32x4_any, u16x8_any>::type;
     using BiasElem = typename std::conditional<EXCL == kExBiasF32, float, uint16_t>::type;
     constexpr int BEL = EXCL == kExBiasF32 ? 4 : 8;           // values per piece and lane

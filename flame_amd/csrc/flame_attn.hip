@@ -149,7 +149,7 @@ void launch_fwd_merge(const FwdParams& p, hipStream_t s) {
 // unchanged, 1024 keys 22.1 -> 21.5 us; 128 workgroups, 4096 keys 62.9 -> 52.8 us; 256 workgroups, causal, 2048 keys 36.5 -> 33.5 us.
 bool rule_key_groups(int64_t wgs, int Sk, int least_keys = 1024) { return wgs <= device_cu_count() && Sk >= least_keys; }
 // dQ, whose joining weighs more: B=1 H=16 S=2048 causal, backward, D = 64 62.8 -> 60.1 us, D = 128 96.9 -> 95.8 us; unchanged or
-// up to 2 % slower with 1024 keys.
+// up to 2 % slower with 1024 keys.  (Measured without dropout, which shares the line.)
 constexpr int kDqGroupKeys = 2048;
 
 // wg_count workgroups from p.wg_base on (0: all of the problem's)

@@ -3,11 +3,12 @@
 // whether all of it is.  The attention kernels then walk the attended tiles only, those attended whole without a test per
 // element, and a lane whose query (forward, dQ) or key (dK/dV) meets a cut tile loads one word for it, 8 bytes next to its
 // neighbours', instead of 64 bytes of a row of its own.  Key lengths and the causal flag are folded in.
-// Packed sequences, which attend to themselves, are the case it is made for: B=2 H=16 S=1500, four documents each, forward and
-// backward D = 64 718 -> 122 us, D = 128 1040 -> 183 us, of which the pass over the mask takes 4 us twice.  Where every tile is cut
-// (each element of a mask kept by chance) the words cost about what the rows did where those could be loaded in vectors: B=2 H=16
-// S=1536 D = 128 231 -> 240 us, with S=1500 1046 -> 242 us.
-// Without room for the words (capi: flame_attn_mask_workspace_bytes) the kernels that read the mask itself serve the call.
+// Packed sequences, which attend to themselves, are the case it is made for: B=2 H=16 S=1500, four documents each, D = 64 forward
+// 221 -> 34 us and backward 832 -> 78, D = 128 543 -> 51 and 967 -> 153 us, of which the pass over the mask takes 4 us twice.  Where
+// every tile is cut (each element of a mask kept by chance) the words cost about what the rows did where those could be loaded
+// in vectors: B=2 H=16 S=1536 D = 128 62 -> 64 and 174 -> 170 us, with S=1500 543 -> 57 and 968 -> 168 us.
+// The kernels that read the mask itself serve the call where the bits would not pay (mask_route.hpp) and where there is no room for
+// the words (flame_attn_mask_workspace_bytes).
 #pragma once
 #include "attn_common.hpp"
 

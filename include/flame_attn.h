@@ -98,7 +98,8 @@ size_t flame_attn_fwd_scratch_bytes(int B, int H, int N_q, int N_kv, int D);
 /* Room that a keep-mask which differs by query is worth (0 for other masks): with that much workspace in
  * flame_attn_fwd_ws_bf16, and that much beyond flame_attn_bwd_workspace_bytes (or within its optional part) in
  * flame_attn_bwd_bf16, one pass turns the mask into bits and the kernels walk only the 64-key tiles it leaves something of,
- * without a test per element where it leaves all of one.  Mask strides as in the calls (0 broadcasts). */
+ * without a test per element where it leaves all of one.  Calls to which that would be slower leave the room unused (masks whose
+ * rows load as vectors, on short sequences or, in the forward, one for every head).  Mask strides as in the calls (0 broadcasts). */
 size_t flame_attn_mask_workspace_bytes(int B, int H, int N_q, int N_kv, const int64_t* mask_strides, int has_kv_len, int causal);
 int flame_attn_fwd_ws_bf16(const void* Q, const void* K, const void* V, void* O, void* LSE,
                            int B, int H, int N_q, int N_kv, int D, float scale,
@@ -470,8 +471,9 @@ typedef struct {
     double total_ms[FLAME_ATTN_N_KERNEL_KINDS];
     int launches[FLAME_ATTN_N_KERNEL_KINDS];
 } FlameAttnKernelTimes;
-/* When on, every kernel launch is bracketed by HIP events on the launch stream (events are created
- * on demand: this mode allocates).  Turning it on or off clears the samples. */
+/* When on, every launch of these kinds (the pass that turns a mask into bits counts to the kernel it serves; conversions of
+ * element type are none of them) is bracketed by HIP events on the launch stream (events are created on demand: this mode
+ * allocates).  Turning it on or off clears the samples. */
 int flame_attn_profiling_enable(int on);
 /* Waits for the recorded events and returns per-kernel sums since the last read. */
 int flame_attn_profiling_read(FlameAttnKernelTimes* out);
