@@ -175,21 +175,35 @@ int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
 }
 
-template <int D, bool DROPOUT>
-int launch_fwd_keyshare(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
-    using T = FwdKeyShareTile<D>;
+// workgroups of NW wavefronts (fwd_keyshare_waves)
+template <int D, int NW, int DROP>
+int launch_fwd_keyshare_nw(const FwdParams& p, int64_t grid, hipStream_t s) {
+    using T = FwdKeyShareTile<D, NW>;
     static std::atomic<bool> lds_set{false};
-    auto kern = fwd_keyshare_kernel<D, DROPOUT>;
+    auto kern = fwd_keyshare_kernel<D, NW, DROP>;
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), T::LDS_BYTES, lds_set)) return rc;
-    const int64_t grid = (wg_count ? wg_count : (int64_t)((p.Sq + T::BQ - 1) / T::BQ) * p.B * p.H) * p.key_splits;
-    if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_FWD, s);
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), T::LDS_BYTES, s, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), T::LDS_BYTES, s, p);
         if (p.key_splits > 1) launch_fwd_merge(p, s);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
+}
+
+// Eight wavefronts, two per SIMD, while a compute unit gets one workgroup at most; where there are more, twice as many
+// workgroups of four fit (four times at D = 64), and the start of one runs under the walk of another.  (Four -> eight, us:
+// 160 workgroups, 2560 keys, D = 128 25.0 -> 20.4; 128, 1024 keys, D = 64 9.8 -> 8.2; 96, 785 keys, D = 72 9.8 -> 9.1;
+// above 256: 330, 433 keys, D = 80 12.3 -> 15.6; 512, 128 keys, D = 128 9.2 -> 11.2; 512, 300 keys, D = 64 9.7 -> 10.1.)
+int fwd_keyshare_waves(int64_t grid) { return grid <= device_cu_count() ? 8 : 4; }
+
+template <int D, int DROP>
+int launch_fwd_keyshare(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
+    const int64_t grid = (wg_count ? wg_count : (int64_t)((p.Sq + 31) / 32) * p.B * p.H) * p.key_splits;
+    if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    if constexpr (DROP == kDropNone)       // (dropout: a grid above one workgroup per unit has at most 32 queries per sequence)
+        if (fwd_keyshare_waves(grid) == 4) return launch_fwd_keyshare_nw<D, 4, DROP>(p, grid, s);
+    return launch_fwd_keyshare_nw<D, 8, DROP>(p, grid, s);
 }
 
 // 256-query workgroups, one wavefront per SIMD (builds without keep-mask / bias only)
@@ -211,7 +225,7 @@ int launch_fwd_wide(FwdParams p, hipStream_t s) {
     }
     if (r.count) {
         p.wg_base = (int)r.base;
-        return r.rows == 32 ? launch_fwd_keyshare<kRowPitch<D>, false>(p, s, r.count) : launch_fwd<D, kExNone, 4>(p, s, r.count);
+        return r.rows == 32 ? launch_fwd_keyshare<kRowPitch<D>, kDropNone>(p, s, r.count) : launch_fwd<D, kExNone, 4>(p, s, r.count);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
@@ -1132,29 +1146,33 @@ int flame_sage_attn_fwd_bias_int8(const void* Qi8, const void* Ki8, const void* 
 
 // fwd_keyshare_kernel instead of fwd_kernel (head dims up to 128, nothing excluded but by causal flag and key lengths): a
 // few query rows, or 128-query workgroups on at most a quarter of the compute units, so that four times as many still run
-// in one round.  Measured with 32 such workgroups, D = 128: 62 -> 31 us at 4096 keys, 20 -> 16 us at 1024; with 128 of
-// them 35 -> 51 us (each K / V tile is fetched four times as often, and a step then waits for it).
+// in one round.  Measured, us: with 40 such workgroups, D = 128, 2560 keys 35.1 -> 20.4; 64 of them, 1024 keys, 18.5 -> 13.8,
+// D = 64 12.9 -> 8.8; with 128 of them D = 128 1024 keys 19.5 -> 21.1, 4096 keys 52.9 -> 56.2, 256 keys 9.5 -> 11.5 (each K / V
+// tile is fetched four times as often), D = 64 13.6 -> 13.6, 36.5 -> 34.3, 6.9 -> 7.2.
 static bool fwd_rule_keyshare(int64_t bh, int N_q) {
     return N_q <= 32 || (int64_t)((N_q + 127) / 128) * bh * 4 <= device_cu_count();
 }
 
 // ... and the workgroups that share the keys of one of its query tiles: the least of an estimate in microseconds.  Every
-// round of the chip costs a start and its steps, all of K and V take at least the time of reading them, a split one merge
-// launch and the traffic of its fp32 partials.  (The constants were measured; one row against 4097 keys of 64 heads,
-// D = 128: 39 / 27 / 27 / 32 us with 1 / 2 / 4 / 8 slices.)
+// round of the chip costs a start and its steps, a split one merge launch and the traffic of its fp32 partials.  All of K and
+// V take at least the time of reading them, and where they are more than stays in the caches a workgroup asks for no more than
+// 37 GB/s.  (The constants were measured.  One row, us with 1 / 2 / 4 / 8 slices: D = 128, 4097 keys of 64 heads 45.7 / 32.5 /
+// 30.4 / -, 2000 keys of 8 heads 15.0 / 12.9 / 11.4 / 11.7, of 32 heads 15.8 / 14.0 / 14.0 / 16.0; D = 64, 2000 keys of 8 heads
+// 10.0 / 10.2 / 9.5 / 10.3, 4000 of 128 heads 28.0 / 29.0 / 30.2 / -; D = 72, 785 keys of 96 heads 9.1 / 11.5 / - / -.)
 static int fwd_key_splits(int64_t bh, int N_q, int N_kv, int DP) {
     if (!fwd_rule_keyshare(bh, N_q)) return 1;
-    const int64_t wgs = (int64_t)((N_q + 31) / 32) * bh;
-    const int64_t slots = device_cu_count() * (DP == 64 ? 2 : 1);             // LDS: two workgroups per compute unit at D = 64
-    const int steps = (N_kv + 127) / 128;
-    const double step_us = DP == 64 ? 0.8 : 1.1, start_us = 2.5;
-    const double read_us = 4.0 * bh * N_kv * DP / 5.2e6;
+    const int64_t wgs = (int64_t)((N_q + 31) / 32) * bh, cus = device_cu_count();
+    const double step_us = DP == 64 ? 0.75 : 1.45, start_us = 4.0;          // a step: one 32-key tile per wavefront
+    const double read_bytes = 4.0 * bh * N_kv * DP;
     double best = 1e30;
     int best_s = 1;
-    for (int s = 1; s <= 64 && s <= (steps + 1) / 2; ++s) {
+    for (int s = 1; s <= 64 && s <= ((N_kv + 127) / 128 + 1) / 2; ++s) {
+        const int waves = fwd_keyshare_waves(wgs * s), keys = 32 * waves * s;
+        const int64_t slots = waves == 8 ? cus : cus * (DP == 64 ? 4 : 2);        // LDS: the workgroups of four that fit a unit
         const int64_t rounds = (wgs * s + slots - 1) / slots;
+        const double tb_s = read_bytes < 64e6 ? 5.2 : std::min(5.2, 0.037 * (double)std::min(wgs * s, cus));
         const double merge_us = s == 1 ? 0.0 : 2.5 + 0.55 * s + 2.0 * s * (double)bh * N_q * DP * 4 / 8e6;
-        const double t = std::max((double)rounds * (start_us + step_us * ((steps + s - 1) / s)), read_us) + merge_us;
+        const double t = std::max((double)rounds * (start_us + step_us * ((N_kv + keys - 1) / keys)), read_bytes / (tb_s * 1e6)) + merge_us;
         if (t < best) {
             best = t;
             best_s = s;
@@ -1257,7 +1275,11 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         // the undropped call's choice between the kernels, without its split of the keys (this entry point has no workspace):
         // the log-sum-exp is that of the undropped softmax, its sum joined in another order where that call splits
         if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q))
-            return DP == 128 ? launch_fwd_keyshare<128, true>(p, s) : launch_fwd_keyshare<64, true>(p, s);
+            switch (drop_mode(p.m, N_kv)) {
+                case kDropRows64: return DP == 128 ? launch_fwd_keyshare<128, kDropRows64>(p, s) : launch_fwd_keyshare<64, kDropRows64>(p, s);
+                case kDropFlat: return DP == 128 ? launch_fwd_keyshare<128, kDropFlat>(p, s) : launch_fwd_keyshare<64, kDropFlat>(p, s);
+                default: return DP == 128 ? launch_fwd_keyshare<128, kDropTiled>(p, s) : launch_fwd_keyshare<64, kDropTiled>(p, s);
+            }
         if (DP == 128 && narrow(std::max(D, Dv)) && !hm) return launch_fwd_dropout<96>(p, hm, s);
         return DP == 128 ? launch_fwd_dropout<128>(p, hm, s) : launch_fwd_dropout<64>(p, hm, s);
     }
@@ -1298,7 +1320,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
             p.part_o = static_cast<float*>(scratch.ws);
             p.part_lse = p.part_o + (size_t)p.key_splits * rows * Dv;
         }
-        return DP == 128 ? launch_fwd_keyshare<128, false>(p, s) : launch_fwd_keyshare<64, false>(p, s);
+        return d96 ? launch_fwd_keyshare<96, kDropNone>(p, s) : DP == 128 ? launch_fwd_keyshare<128, kDropNone>(p, s) : launch_fwd_keyshare<64, kDropNone>(p, s);
     }
     return d96 ? launch_fwd<96, kExNone, 4>(p, s) : DP == 128 ? launch_fwd<128, kExNone, 4>(p, s) : launch_fwd<64, kExNone, 4>(p, s);
 }
