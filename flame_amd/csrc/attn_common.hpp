@@ -270,11 +270,14 @@ __device__ __forceinline__ float log2_fast(float x) { return __builtin_amdgcn_lo
 // exchange with the lane 32 positions away (the other half of the wave)
 __device__ __forceinline__ float xhalf(float x) { return __shfl_xor(x, 32, 64); }
 
-// max(x, xhalf(x)) without the way through the LDS crossbar (v_permlane32_swap_b32: the upper half of the first register
-// changes places with the lower half of the second)
+// max(x, xhalf(x)) without the way through the LDS crossbar: v_permlane32_swap_b32 makes the upper half of the first register
+// change places with the lower half of the second.  By hand: given the same value twice, the compiler takes the two results of
+// the builtin for one and folds the maximum away.  Two wait states in front, as it may read a register that the vector ALU has
+// just written no earlier.
 __device__ __forceinline__ float max_of_halves(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-    return fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+    float lo = x, hi = x;
+    asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(lo), "+v"(hi));
+    return fmaxf(lo, hi);
 }
 
 // 16-byte global load of 8 bf16, zero when the predicate is false

@@ -61,3 +61,16 @@ def test_dropout(oracle, B, H, Sq, Sk, D, causal, chunk):
     p = float(np.quantile(oracle.dropout_uniforms(B, H, Sq, Sk, seed, cq, ck), 0.25))
     o, lse = capi.attn_fwd_dropout(*(to_dev(t) for t in (q, k, v)), sc, p, seed, causal=causal, draw_chunk_q=cq, draw_chunk_kv=ck)
     check(oracle, o, lse, oracle.sdpa_fwd_dropout(q, k, v, sc, p, seed, causal=causal, want_f32=True, chunk_q=cq, chunk_kv=ck))
+
+
+# the largest logit among the keys of either half of a wavefront (keys 0 .. 3 of every eight, keys 4 .. 7), hundreds above all
+# others: the maximum in use has to be that of both
+@pytest.mark.parametrize("Sk,key", [(64, 6), (64, 33), (300, 299), (300, 260)])
+def test_one_key_dominates(oracle, Sk, key):
+    from flame_amd import capi
+    print(f"[keyshare waves] {Sk=} {key=}", flush=True)
+    q, k, v = make(1, 2, 5, Sk, 64)
+    q[..., 0], k[..., 0] = W.f32_to_bf16_bits(np.float32([40.0])), 0
+    k[:, :, key, 0] = W.f32_to_bf16_bits(np.float32([80.0]))
+    o, lse = capi.attn_fwd(*(to_dev(t) for t in (q, k, v)), 0.125)
+    check(oracle, o, lse, oracle.sdpa_fwd(q, k, v, 0.125, want_f32=True))
