@@ -403,10 +403,11 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     };
     // Fold the maximum of a freshly computed tile into the running state.  The reference maximum
     // moves (and the running sums are rescaled) only when some lane's tile maximum exceeds it by more
-    // than 2^8 in the exponent domain; the branch is wave-uniform.
+    // than 2^8 in the exponent domain; the branch is wave-uniform.  Both lanes of a query hold the same reference maximum, so
+    // each may test its own half of the keys: the exchange between the halves stays inside the branch.
     auto fold_max = [&](float tmax) {
-        tmax = fmaxf(tmax, xhalf(tmax));
         if (__any(tmax > m_run + stale_ok)) {
+            tmax = fmaxf(tmax, xhalf(tmax));
             const float m_old = m_run;
             const float m_new = fmaxf(m_old, tmax);
             const float m_to = (m_new == -INFINITY) ? 0.f : m_new;

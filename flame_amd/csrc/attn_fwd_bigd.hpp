@@ -220,10 +220,10 @@ __global__ __launch_bounds__(64 * NW) void fwd_bigd_kernel(const FwdParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
         asm volatile("" : "+v"(tmax));       // the scan stays in its slot
-        tmax = fmaxf(tmax, xhalf(tmax));
         float alpha = 1.0f;
-        rescale = __any(tmax > m_run + stale_ok);
+        rescale = __any(tmax > m_run + stale_ok);       // each half of a query's lanes tests its own keys
         if (rescale) {
+            tmax = fmaxf(tmax, xhalf(tmax));
             const float m_new = fmaxf(m_run, tmax);
             const float m_to = (m_new == -INFINITY) ? 0.f : m_new;
             alpha = exp2_fast((m_run - m_to) * c_log2);

@@ -155,8 +155,8 @@ __global__ __launch_bounds__(64 * NW_, D == 64 ? 4 : 2) void fwd_keyshare_kernel
         float tmax = s[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
-        tmax = max_of_halves(tmax);
-        if (__any(tmax > m_run)) {
+        if (__any(tmax > m_run)) {                     // each half tests its own keys
+            tmax = max_of_halves(tmax);
             const float m_new = fmaxf(m_run, tmax);
             const float m_to = (m_new == -INFINITY) ? 0.f : m_new;
             const float alpha = exp2_fast((m_run - m_to) * c_log2);

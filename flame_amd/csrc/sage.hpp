@@ -440,8 +440,8 @@ __global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel
         for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
 
     auto fold_max = [&](float tmax) {        // tmax in log2 units
-        tmax = fmaxf(tmax, xhalf(tmax));
-        if (__any(tmax > m_run + 8.0f)) {    // the reference maximum may lag the true one by 2^8
+        if (__any(tmax > m_run + 8.0f)) {    // the reference maximum may lag the true one by 2^8; each half tests its own keys
+            tmax = fmaxf(tmax, xhalf(tmax));
             const float m_old = m_run;
             const float m_new = fmaxf(m_old, tmax);
             const float m_to = (m_new == -INFINITY) ? 0.f : m_new;
@@ -843,8 +843,8 @@ __global__ __launch_bounds__(256) void sage_fwd_wide_kernel(const SageFwdParams 
 
     auto fold_max = [&](auto qb_tag, float tmax) {           // tmax in log2 units
         constexpr int qb = decltype(qb_tag)::value;
-        tmax = fmaxf(tmax, xhalf(tmax));
-        if (__any(tmax > m_run[qb] + 8.0f)) {                // the reference maximum may lag the true one by 2^8
+        if (__any(tmax > m_run[qb] + 8.0f)) {                // the reference maximum may lag the true one by 2^8; each half tests its own keys
+            tmax = fmaxf(tmax, xhalf(tmax));
             const float m_old = m_run[qb];
             const float m_new = fmaxf(m_old, tmax);
             const float m_to = (m_new == -INFINITY) ? 0.f : m_new;
