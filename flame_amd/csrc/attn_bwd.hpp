@@ -133,8 +133,12 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         wg = p.n_whole + e / nparts;
         part = e % nparts;
     }
-    const int kt = wg % n_kt;
-    const int bh = wg / n_kt;
+    int kt = wg % n_kt, bh = wg / n_kt;
+    // (under the causal flag the first key blocks have the longest walks)
+    if (int t, s; DROP == kDropNone && __builtin_expect(p.n_whole < 0 && dealt_unit(block, nblocks, n_kt, p.B, p.H, p.m.causal && !p.m.kv_len && !p.key_mask, p.m.kv_len || p.key_mask, 1, t, s), 0)) {
+        kt = __builtin_amdgcn_readfirstlane(t);
+        bh = __builtin_amdgcn_readfirstlane(s);
+    }
     const int b = bh / p.H, hh = bh % p.H;
     const int k0 = kt * BN;
     const int kw0 = k0 + 32 * wave;
@@ -935,7 +939,13 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
         wg = p.m.kv_len || KEYS ? xcd_remap_heads<KG == 1 && !BITS>(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
     }
     int qt = wg % n_qt, bh = wg / n_qt;
-    if (p.m.causal && !p.m.kv_len && p.dq_parts == 1) causal_longest_first<KG == 1>(wg, n_qt, gridDim.x, qt, bh);
+    const bool falling = !(EXCL == kExKeys) && p.m.causal && !p.m.kv_len;
+    if (int t, s; KG == 1 && DROP == kDropNone && __builtin_expect(p.dq_parts == 1 && dealt_unit<KG == 1 && !BITS>(blockIdx.x, gridDim.x, n_qt, p.B, p.H, falling, (p.m.kv_len || KEYS) && !falling, 1, t, s), 0)) {
+        qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
+        bh = __builtin_amdgcn_readfirstlane(s);
+    } else if (falling && p.dq_parts == 1) {
+        causal_longest_first<KG == 1>(blockIdx.x, wg, n_qt, gridDim.x, qt, bh);
+    }
     if (!BITS && (KEYS || p.m.kv_len) && p.dq_parts == 1) bh = longest_batches_first<KEYS>(bh, p.B, p.H, p.Sk, p.m);
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
@@ -1374,7 +1384,13 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     const int n_qt = (p.Sq + BM - 1) / BM;
     const int wg = p.m.kv_len ? xcd_remap_heads(block, nblocks, n_qt) : xcd_remap(block, nblocks);
     int qt = wg % n_qt, bh = wg / n_qt;
-    if (p.m.causal && !p.m.kv_len) causal_longest_first(wg, n_qt, nblocks, qt, bh);
+    const bool falling = p.m.causal && !p.m.kv_len;
+    if (int t, s; __builtin_expect(dealt_unit(block, nblocks, n_qt, p.B, p.H, falling, p.m.kv_len != nullptr, 1, t, s), 0)) {
+        qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
+        bh = __builtin_amdgcn_readfirstlane(s);
+    } else if (falling) {
+        causal_longest_first(block, wg, n_qt, nblocks, qt, bh);
+    }
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 64;

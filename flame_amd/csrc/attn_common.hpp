@@ -6,6 +6,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "causal_order.hpp"
+#include "xcd_order.hpp"
+
 namespace fattn {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -367,47 +370,13 @@ __device__ __forceinline__ void wait_vm() {
     asm volatile("" ::: "memory");
 }
 
-// Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by linear id.  Remap the id
-// so that XCD x works on the contiguous range [x*total/8, (x+1)*total/8) of tiles: all tiles of one
-// (batch, head) then share one L2 and its K/V (forward) or Q/dO (backward) stay resident there.
-__device__ __forceinline__ int xcd_remap(int linear, int total) {
-    constexpr int kXcd = 8;
-    return (total % kXcd == 0) ? (linear % kXcd) * (total / kXcd) + linear / kXcd : linear;
-}
-// Workgroups of which a compute unit holds two are dealt out one per unit, then a second one each.  Where (nearly) all fit at once
-// nothing is left to even out unequal walks: in the order of falling length the units with the longest walks would get the
-// longer ones of the second deal as well, so that one is turned round.  With more than three deals the order of falling length
-// is better: the units that finish first take what is left.
-// (Forward and backward, us: B=4 H=16 S=1101 D=128 key mask 154.5 -> 150.7, B=4 H=16 1024 x 2049 D=64 key lengths 123.5 -> 121.5,
-// B=1 H=16 S=3000 D=128 causal 203 -> 198, its forward 55.3 -> 52.7; four deals turned in pairs: B=4 H=32 S=1024 D=64 causal,
-// forward 27.8 -> 29.2.)
-// j: place in the order of the `total` workgroups of an XCD with 32 compute units (the whole card's; with another number the
-// order is another one, as complete).
-__device__ __forceinline__ int snake_order(int j, int total) {
-    constexpr int kUnits = 32;
-    const int end = min(2 * kUnits, total);
-    return total <= 3 * kUnits && j >= kUnits && j < end ? kUnits + end - 1 - j : j;
-}
-// The same for batches whose sequences differ in length (per-batch key lengths): contiguous ranges would hand
-// whole batches, the long ones and the short ones, to different XCDs.  Here XCD x takes the (batch, head)
-// slices x, x + 8, x + 16, ...: every slice still stays in one L2, and the heads of one batch are spread
-// over all XCDs.  `per_head`: tiles per (batch, head) slice; the id runs slice-major.
-// SNAKE: workgroups of which a compute unit holds two, the longest walks first: see snake_order.
-template <bool SNAKE = false>
-__device__ __forceinline__ int xcd_remap_heads(int linear, int total, int per_head) {
-    constexpr int kXcd = 8;
-    const int n_heads = total / per_head;
-    if (n_heads % kXcd != 0) return xcd_remap(linear, total);
-    const int x = linear % kXcd, j = SNAKE ? snake_order(linear / kXcd, total / kXcd) : linear / kXcd;
-    return ((j / per_head) * kXcd + x) * per_head + j % per_head;
-}
-
 // Causal problems: the key walk of query unit qt grows with qt, and workgroups start in id order, so the longest
 // walks must come first or they finish alone at the end.  Within the contiguous range of units that one XCD
 // works through (whole heads where the counts allow), the order becomes: last unit of every head, then the
-// units before them, and so on.  `wg`: unit id after xcd_remap, head-major; returns (qt, head) through refs.
+// units before them, and so on.  `wg`: unit id after xcd_remap, head-major, of workgroup `linear`; returns (qt, head) through refs.
 template <bool SNAKE = false>
-__device__ __forceinline__ void causal_longest_first(int wg, int n_qt, int total, int& qt, int& bh) {
+__device__ __forceinline__ void causal_longest_first(int linear, int wg, int n_qt, int total, int& qt, int& bh) {
+    if (total % 8 != 0) wg = linear;               // all of them in one order, dealt to the XCDs in turn
     const int per_xcd = (total % 8 == 0) ? total / 8 : total;
     if (per_xcd % n_qt == 0) {
         const int heads = per_xcd / n_qt;

@@ -97,9 +97,19 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     uint16_t* lds = lds_all + (KG == 1 ? 0 : group * (T::LDS_BYTES / 2));
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len || EXCL == kExKeys || EXCL == kExBits ? xcd_remap_heads<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
+    constexpr bool KNOWS_BIAS = EXCL == kExBiasF32 || EXCL == kExBiasBf16;       // no causal flag, no key lengths
+    const bool falling = !KNOWS_BIAS && EXCL != kExKeys && p.m.causal && !p.m.kv_len;
+    const bool by_batch = !KNOWS_BIAS && (p.m.kv_len || EXCL == kExKeys || EXCL == kExBits);
+    const int wg = by_batch ? xcd_remap_heads<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
-    if (p.m.causal && !p.m.kv_len) causal_longest_first<NW == 4 && KG == 1>(wg, n_qt, gridDim.x, qt, bh);
+    // (two groups: one workgroup per compute unit at most; dropout keeps the order it had)
+    constexpr bool DEALT = !KNOWS_BIAS && KG == 1 && DROP == kDropNone;
+    if (int t, s; DEALT && __builtin_expect(dealt_unit<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt, p.B, p.H, falling, by_batch && !falling, 8, t, s), 0)) {
+        qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);         // (the compiler divides in vector registers)
+        bh = __builtin_amdgcn_readfirstlane(s);
+    } else if (falling) {
+        causal_longest_first<NW == 4 && KG == 1>(blockIdx.x, wg, n_qt, gridDim.x, qt, bh);
+    }
     if (EXCL == kExKeys || (p.m.kv_len && EXCL != kExBits)) bh = longest_batches_first<EXCL == kExKeys>(bh, p.B, p.H, p.Sk, p.m);
     // a bias that all batches share: its rows are read by the batches' workgroups one after the other on one XCD, from its L2
     if ((EXCL == kExBiasF32 || EXCL == kExBiasBf16) && p.m.bb == 0) {

@@ -318,10 +318,16 @@ __global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel
     uint8_t* lds8 = lds8_all + (KG == 1 ? 0 : group * T::LDS_BYTES);
 
     const int n_qt = (p.Sq + BM - 1) / BM;
+    const bool falling = p.causal && !p.kv_len;
     const int wg = p.kv_len ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     // (shortest first before: B=2 H=24 S=4608 D=128 causal 307 -> 276 us, B=1 H=24 S=2048 D=128 75.1 -> 61.8)
-    if (p.causal && !p.kv_len) causal_longest_first<KG == 1>(wg, n_qt, gridDim.x, qt, bh);
+    if (int t, s; KG == 1 && __builtin_expect(dealt_unit<KG == 1>(blockIdx.x, gridDim.x, n_qt, p.B, p.H, falling, p.kv_len != nullptr, 8, t, s), 0)) {
+        qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
+        bh = __builtin_amdgcn_readfirstlane(s);
+    } else if (falling) {
+        causal_longest_first<KG == 1>(blockIdx.x, wg, n_qt, gridDim.x, qt, bh);
+    }
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;
     const int qw0 = q0 + wave * 32;

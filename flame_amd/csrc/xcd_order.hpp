@@ -1,0 +1,64 @@
+// Which unit of a problem a workgroup takes, so that the units that read the same keys and values share an XCD's L2: integer
+// arithmetic only, so that it can be checked without a GPU.
+#pragma once
+#include "causal_order.hpp"
+
+namespace fattn {
+
+// Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by linear id.  Remap the id
+// so that XCD x works on the contiguous range [x*total/8, (x+1)*total/8) of tiles: all tiles of one
+// (batch, head) then share one L2 and its K/V (forward) or Q/dO (backward) stay resident there.
+// Where the total does not divide, the first total % 8 ranges are one longer, as the shares of the XCDs are.
+FATTN_HOST_DEVICE int xcd_remap(int linear, int total) {
+    constexpr int kXcd = 8;
+    const int x = linear % kXcd;
+    return x * (total / kXcd) + (x < total % kXcd ? x : total % kXcd) + linear / kXcd;
+}
+// Workgroups of which a compute unit holds two are dealt out one per unit, then a second one each.  Where (nearly) all fit at once
+// nothing is left to even out unequal walks: in the order of falling length the units with the longest walks would get the
+// longer ones of the second deal as well, so that one is turned round.  With more than three deals the order of falling length
+// is better: the units that finish first take what is left.
+// (Forward and backward, us: B=4 H=16 S=1101 D=128 key mask 154.5 -> 150.7, B=4 H=16 1024 x 2049 D=64 key lengths 123.5 -> 121.5,
+// B=1 H=16 S=3000 D=128 causal 203 -> 198, its forward 55.3 -> 52.7; four deals turned in pairs: B=4 H=32 S=1024 D=64 causal,
+// forward 27.8 -> 29.2.)
+// j: place in the order of the `total` workgroups of an XCD with 32 compute units (the whole card's; with another number the
+// order is another one, as complete).
+FATTN_HOST_DEVICE int snake_order(int j, int total) {
+    constexpr int kUnits = 32;
+    const int end = total < 2 * kUnits ? total : 2 * kUnits;
+    return total <= 3 * kUnits && j >= kUnits && j < end ? kUnits + end - 1 - j : j;
+}
+// The same for batches whose sequences differ in length (per-batch key lengths): contiguous ranges would hand
+// whole batches, the long ones and the short ones, to different XCDs.  Here XCD x takes the (batch, head)
+// slices x, x + 8, x + 16, ...: every slice still stays in one L2, and the heads of one batch are spread
+// over all XCDs.  `per_head`: tiles per (batch, head) slice; the id runs slice-major.
+// SNAKE: workgroups of which a compute unit holds two, the longest walks first: see snake_order.
+template <bool SNAKE = false>
+FATTN_HOST_DEVICE int xcd_remap_heads(int linear, int total, int per_head) {
+    constexpr int kXcd = 8;
+    const int n_heads = total / per_head;
+    if (n_heads % kXcd != 0) return total % kXcd == 0 ? xcd_remap(linear, total) : linear;
+    const int x = linear % kXcd, j = SNAKE ? snake_order(linear / kXcd, total / kXcd) : linear / kXcd;
+    return ((j / per_head) * kXcd + x) * per_head + j % per_head;
+}
+
+// Problems whose walks differ in length and whose slices do not divide by the XCDs: true, with the unit of workgroup `linear`, where the
+// units left over are dealt one by one (causal_order.hpp).  Under the causal flag (falling): all B H slices, `tile` counted from the longest
+// walk.  Where the batches differ (by_batch): the H heads of every batch, batch after batch.  (Key lengths, forward and backward, us, contiguous ranges ->
+// this order: B=7 H=12 512 x 1500 D=128 43 -> 31 and 128 -> 90, B=3 H=12 S=4233 D=64 183 -> 125 and 522 -> 387, D=128 a key mask 317 -> 204 and 966 -> 611.)
+// least: the fewest tiles per slice under the causal flag.  (Forward with fewer than eight: 75 heads of 512 at D = 64 11.0 -> 12.1 us, 107 of 1024 with
+// 256-query workgroups 46.8 -> 53.4.)
+// The condition is marked as unlikely, so that the code is not in the way of every other workgroup's first instructions, and kernels that gain little or
+// never have more than one workgroup per unit leave it out: 400 instructions in line cost B=2 H=16 S=1024 D=64 with dropout 64.0 -> 65.3 us.
+template <bool SNAKE = false>
+FATTN_HOST_DEVICE bool dealt_unit(int linear, int total, int tiles, int B, int H, bool falling, bool by_batch, int least, int& tile, int& bh) {
+    const int slices = by_batch ? H : B * H;
+    if (__builtin_expect(!(by_batch || (falling && tiles >= least)) || !causal_order_pays(slices, total), 1)) return false;
+    int slice, level;
+    causal_order(linear, slices, by_batch ? B * tiles : tiles, slice, level, [](int j, int count) { return SNAKE ? snake_order(j, count) : j; });
+    tile = by_batch ? level % tiles : level;
+    bh = by_batch ? level / tiles * H + slice : slice;
+    return true;
+}
+
+}  // namespace fattn
