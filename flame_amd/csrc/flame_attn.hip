@@ -194,16 +194,18 @@ int launch_fwd_keyshare_nw(const FwdParams& p, int64_t grid, hipStream_t s) {
 // Eight wavefronts, two per SIMD, while a compute unit gets one workgroup at most; where there are more, twice as many
 // workgroups of four fit (four times at D = 64), and the start of one runs under the walk of another.  (Four -> eight, us:
 // 160 workgroups, 2560 keys, D = 128 25.0 -> 20.4; 128, 1024 keys, D = 64 9.8 -> 8.2; 96, 785 keys, D = 72 9.8 -> 9.1;
-// above 256: 330, 433 keys, D = 80 12.3 -> 15.6; 512, 128 keys, D = 128 9.2 -> 11.2; 512, 300 keys, D = 64 9.7 -> 10.1.)
-int fwd_keyshare_waves(int64_t grid) { return grid <= device_cu_count() ? 8 : 4; }
+// above 256: 330, 433 keys, D = 80 12.3 -> 15.6; 512, 128 keys, D = 128 9.2 -> 11.2.  At D = 64 two of eight fit as well and pay from 2048 keys
+// on: 384 workgroups, 512 keys 8.9 -> 9.6, 1024 keys 12.4 -> 12.8, 2048 keys 19.6 -> 19.1, 4096 keys 32.1 -> 30.3.)
+int fwd_keyshare_waves(int64_t grid, int DP, int Sk) {
+    const int64_t cus = device_cu_count();
+    return grid <= cus || (DP == 64 && Sk >= 2048 && grid <= 2 * cus) ? 8 : 4;
+}
 
 template <int D, int DROP>
 int launch_fwd_keyshare(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     const int64_t grid = (wg_count ? wg_count : (int64_t)((p.Sq + 31) / 32) * p.B * p.H) * p.key_splits;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
-    if constexpr (DROP == kDropNone)       // (dropout: a grid above one workgroup per unit has at most 32 queries per sequence)
-        if (fwd_keyshare_waves(grid) == 4) return launch_fwd_keyshare_nw<D, 4, DROP>(p, grid, s);
-    return launch_fwd_keyshare_nw<D, 8, DROP>(p, grid, s);
+    return fwd_keyshare_waves(grid, D, p.Sk) == 4 ? launch_fwd_keyshare_nw<D, 4, DROP>(p, grid, s) : launch_fwd_keyshare_nw<D, 8, DROP>(p, grid, s);
 }
 
 // 256-query workgroups, one wavefront per SIMD (builds without keep-mask / bias only)
@@ -1160,12 +1162,13 @@ int flame_sage_attn_fwd_bias_int8(const void* Qi8, const void* Ki8, const void* 
 }  // extern "C"
 
 // fwd_keyshare_kernel instead of fwd_kernel (head dims up to 128, nothing excluded but by causal flag and key lengths): a
-// few query rows, or 128-query workgroups on at most a quarter of the compute units, so that four times as many still run
-// in one round.  Measured, us: with 40 such workgroups, D = 128, 2560 keys 35.1 -> 20.4; 64 of them, 1024 keys, 18.5 -> 13.8,
+// few query rows, or 128-query workgroups on at most a quarter of the compute units (half of them at D = 64, two fitting a unit),
+// so that four times as many still run in one round.  Measured, us: with 40 such workgroups, D = 128, 2560 keys 35.1 -> 20.4; 64 of them, 1024 keys, 18.5 -> 13.8,
 // D = 64 12.9 -> 8.8; with 128 of them D = 128 1024 keys 19.5 -> 21.1, 4096 keys 52.9 -> 56.2, 256 keys 9.5 -> 11.5 (each K / V
-// tile is fetched four times as often), D = 64 13.6 -> 13.6, 36.5 -> 34.3, 6.9 -> 7.2.
-static bool fwd_rule_keyshare(int64_t bh, int N_q) {
-    return N_q <= 32 || (int64_t)((N_q + 127) / 128) * bh * 4 <= device_cu_count();
+// tile is fetched four times as often), D = 64 512 keys 9.4 -> 9.4, 1024 keys 13.5 -> 13.1, 2048 keys 20.7 -> 20.3, 4096 keys 35.7 -> 33.0; 80 of them,
+// D = 64 2048 keys 20.5 -> 18.2, 1024 keys 13.0 -> 12.2, D = 128 29.3 -> 28.8, 18.5 -> 19.1.
+static bool fwd_rule_keyshare(int64_t bh, int N_q, int DP) {
+    return N_q <= 32 || (int64_t)((N_q + 127) / 128) * bh * (DP == 64 ? 2 : 4) <= device_cu_count();
 }
 
 // ... and the workgroups that share the keys of one of its query tiles: the least of an estimate in microseconds.  Every
@@ -1175,15 +1178,15 @@ static bool fwd_rule_keyshare(int64_t bh, int N_q) {
 // 30.4 / -, 2000 keys of 8 heads 15.0 / 12.9 / 11.4 / 11.7, of 32 heads 15.8 / 14.0 / 14.0 / 16.0; D = 64, 2000 keys of 8 heads
 // 10.0 / 10.2 / 9.5 / 10.3, 4000 of 128 heads 28.0 / 29.0 / 30.2 / -; D = 72, 785 keys of 96 heads 9.1 / 11.5 / - / -.)
 static int fwd_key_splits(int64_t bh, int N_q, int N_kv, int DP) {
-    if (!fwd_rule_keyshare(bh, N_q)) return 1;
+    if (!fwd_rule_keyshare(bh, N_q, DP)) return 1;
     const int64_t wgs = (int64_t)((N_q + 31) / 32) * bh, cus = device_cu_count();
     const double step_us = DP == 64 ? 0.75 : 1.45, start_us = 4.0;          // a step: one 32-key tile per wavefront
     const double read_bytes = 4.0 * bh * N_kv * DP;
     double best = 1e30;
     int best_s = 1;
     for (int s = 1; s <= 64 && s <= ((N_kv + 127) / 128 + 1) / 2; ++s) {
-        const int waves = fwd_keyshare_waves(wgs * s), keys = 32 * waves * s;
-        const int64_t slots = waves == 8 ? cus : cus * (DP == 64 ? 4 : 2);        // LDS: the workgroups of four that fit a unit
+        const int waves = fwd_keyshare_waves(wgs * s, DP, N_kv), keys = 32 * waves * s;
+        const int64_t slots = cus * (DP == 64 ? 2 : 1) * (8 / waves);             // LDS: the workgroups that fit a unit
         const int64_t rounds = (wgs * s + slots - 1) / slots;
         const double tb_s = read_bytes < 64e6 ? 5.2 : std::min(5.2, 0.037 * (double)std::min(wgs * s, cus));
         const double merge_us = s == 1 ? 0.0 : 2.5 + 0.55 * s + 2.0 * s * (double)bh * N_q * DP * 4 / 8e6;
@@ -1311,7 +1314,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
         // the undropped call's choice between the kernels, without its split of the keys (this entry point has no workspace):
         // the log-sum-exp is that of the undropped softmax, its sum joined in another order where that call splits
-        if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q))
+        if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q, DP))
             switch (drop_mode(p.m, N_kv)) {
                 case kDropRows64: return DP == 128 ? launch_fwd_keyshare<128, kDropRows64>(p, s) : launch_fwd_keyshare<64, kDropRows64>(p, s);
                 case kDropFlat: return DP == 128 ? launch_fwd_keyshare<128, kDropFlat>(p, s) : launch_fwd_keyshare<64, kDropFlat>(p, s);
@@ -1349,7 +1352,7 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
         if (plain) return d96 ? launch_fwd_wide<96>(p, s) : DP == 128 ? launch_fwd_wide<128>(p, s) : launch_fwd_wide<64>(p, s);
         return d96 ? launch_fwd<96, kExNone, 8>(p, s) : DP == 128 ? launch_fwd<128, kExNone, 8>(p, s) : launch_fwd<64, kExNone, 8>(p, s);
     }
-    if (q_tile_plan == 0 && fwd_rule_keyshare((int64_t)B * H, N_q)) {
+    if (q_tile_plan == 0 && fwd_rule_keyshare((int64_t)B * H, N_q, DP)) {
         const int64_t rows = (int64_t)B * H * N_q;
         if (scratch.ws) {
             p.key_splits = fwd_key_splits((int64_t)B * H, N_q, N_kv, DP);
