@@ -97,9 +97,10 @@ __device__ __forceinline__ void dkdv_store(const BwdParams& p, uint16_t* own, co
 // -delta is added per element instead of seeding the dP accumulators.
 // BITS: a keep-mask as bits (mask_bits.hpp): the walk takes the query tiles of which anything attends to one of the 128 keys, the
 // cut ones first, and a lane has one word of its key for every cut one.
+// DEALT: the units come in the order of causal_order.hpp (deals_units, which the host asks).
 // block / nblocks: this workgroup's index in the dK/dV grid and the size of that grid (the kernel's own launch, or
 // the dK/dV part of bwd_joint_kernel's).
-template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone, bool BITS = false>
+template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDropNone, bool BITS = false, bool DEALT = false>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int block, const int nblocks) {
     static_assert(!VECMASK || HASMASK, "VECMASK is a special case of HASMASK");
     static_assert(!BITS || (!HASMASK && DROP == kDropNone), "bits stand for the mask");
@@ -134,8 +135,9 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
         part = e % nparts;
     }
     int kt = wg % n_kt, bh = wg / n_kt;
-    // (under the causal flag the first key blocks have the longest walks)
-    if (int t, s; DROP == kDropNone && __builtin_expect(p.n_whole < 0 && dealt_unit(block, nblocks, n_kt, p.B, p.H, p.m.causal && !p.m.kv_len && !p.key_mask, p.m.kv_len || p.key_mask, 1, t, s), 0)) {
+    if constexpr (DEALT) {       // under the causal flag the first key blocks have the longest walks
+        int t, s;
+        dealt_unit(block, n_kt, p.B, p.H, p.m.kv_len || p.key_mask, t, s);
         kt = __builtin_amdgcn_readfirstlane(t);
         bh = __builtin_amdgcn_readfirstlane(s);
     }
@@ -828,6 +830,10 @@ template <int D, bool HASMASK, bool TIMING, bool VECMASK = false, int DROP = kDr
 __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
     bwd_dkdv_body<D, HASMASK, TIMING, VECMASK, DROP, BITS>(p, (int)blockIdx.x, (int)gridDim.x);
 }
+template <int D, bool BITS>
+__global__ __launch_bounds__(256) void bwd_dkdv_dealt_kernel(const BwdParams p) {
+    bwd_dkdv_body<D, false, false, false, kDropNone, BITS, true>(p, (int)blockIdx.x, (int)gridDim.x);
+}
 
 // dK^T / dV^T accumulators (rows = d, column = a lane's key) of the 32 keys from kw0 on -> bf16 rows of dK (scaled) and dV
 template <int D>
@@ -907,11 +913,11 @@ struct BwdDqTile {
 
 // NW wavefronts of 32 queries each per workgroup, two per SIMD (the library instantiates NW = 4; problems
 // that fill 256-query workgroups go to bwd_dq_wide_kernel below).
-// EXCL: see there.  Only the general form compiles per-element mask loads in; the others fit two workgroups per unit.
+// EXCL, DEALT: see there.  Only the general form compiles per-element mask loads in; the others fit two workgroups per unit.
 // KG = 2: two groups of NW wavefronts share the workgroup's queries, each walks one half of the key tiles in LDS stages of its
 // own, and the second adds its dQ to the first's through LDS: for grids that give a compute unit one workgroup at most.
-template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
-__global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
+template <int D, int EXCL, int NW, int DROP, int KG, bool DEALT>
+__device__ __forceinline__ void bwd_dq_body(const BwdParams& p) {
     static_assert(KG == 1 || (KG == 2 && EXCL == kExNone), "key groups: nothing excluded but by causal flag and key lengths");
     constexpr bool HASMASK = EXCL == kExRows16 || EXCL == kExGeneral, VECMASK = EXCL == kExRows16, BITS = EXCL == kExBits, KEYS = EXCL == kExKeys || BITS;
     using T = BwdDqTile<D>;
@@ -940,7 +946,9 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     }
     int qt = wg % n_qt, bh = wg / n_qt;
     const bool falling = !(EXCL == kExKeys) && p.m.causal && !p.m.kv_len;
-    if (int t, s; KG == 1 && DROP == kDropNone && __builtin_expect(p.dq_parts == 1 && dealt_unit<KG == 1 && !BITS>(blockIdx.x, gridDim.x, n_qt, p.B, p.H, falling, (p.m.kv_len || KEYS) && !falling, 1, t, s), 0)) {
+    if constexpr (DEALT) {
+        int t, s;
+        dealt_unit<!BITS>(blockIdx.x, n_qt, p.B, p.H, !falling, t, s);
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling && p.dq_parts == 1) {
@@ -1314,6 +1322,15 @@ __global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 :
     });
 }
 
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_kernel(const BwdParams p) {
+    bwd_dq_body<D, EXCL, NW, DROP, KG, false>(p);
+}
+template <int D, int EXCL, int NW>
+__global__ __launch_bounds__(64 * NW, (NW == 4 && EXCL != kExGeneral) ? 2 : 1) void bwd_dq_dealt_kernel(const BwdParams p) {
+    bwd_dq_body<D, EXCL, NW, kDropNone, 1, true>(p);
+}
+
 // Sums the fp32 partials of the workgroups that shared a 128-query tile and writes dQ.  One workgroup per (tile, 32-wide block
 // of d); the thread layout mirrors the accumulators.
 template <int D>
@@ -1365,7 +1382,7 @@ struct BwdDqWideTile {
     static constexpr int DMA_PER_WAVE = BN / ROWS_PER_DMA / 4;    // 1 KiB copies per wave and tensor
 };
 
-template <int D>
+template <int D, bool DEALT = false>
 __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int block, const int nblocks) {
     using T = BwdDqWideTile<D>;
     constexpr int BM = T::BM, BN = T::BN, RS = T::RS;
@@ -1385,7 +1402,9 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     const int wg = p.m.kv_len ? xcd_remap_heads(block, nblocks, n_qt) : xcd_remap(block, nblocks);
     int qt = wg % n_qt, bh = wg / n_qt;
     const bool falling = p.m.causal && !p.m.kv_len;
-    if (int t, s; __builtin_expect(dealt_unit(block, nblocks, n_qt, p.B, p.H, falling, p.m.kv_len != nullptr, 1, t, s), 0)) {
+    if constexpr (DEALT) {
+        int t, s;
+        dealt_unit(block, n_qt, p.B, p.H, !falling, t, s);
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
@@ -1722,6 +1741,10 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
 template <int D>
 __global__ __launch_bounds__(256) void bwd_dq_wide_kernel(const BwdParams p) {
     bwd_dq_wide_body<D>(p, (int)blockIdx.x, (int)gridDim.x);
+}
+template <int D>
+__global__ __launch_bounds__(256) void bwd_dq_wide_dealt_kernel(const BwdParams p) {
+    bwd_dq_wide_body<D, true>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ------------------------------------------------------------------------------- per-query rows

@@ -70,9 +70,11 @@ typedef uint16_t u16x8_any __attribute__((ext_vector_type(8), aligned(2)));
 // most: its second wavefront per SIMD, which otherwise a second workgroup would be, and half the walk.  K and V are still
 // read once per workgroup.
 // AHEAD: a bias is requested a step earlier (see EARLY).
-template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1, bool AHEAD = false>
-__global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void fwd_kernel(const FwdParams p) {
+// DEALT: the units come in the order of causal_order.hpp (deals_units, which the host asks).
+template <int D, int EXCL, int NW, int DROP, int KG, bool AHEAD, bool DEALT>
+__device__ __forceinline__ void fwd_body(const FwdParams& p) {
     static_assert(KG == 1 || (KG == 2 && EXCL == kExNone), "key groups: nothing excluded but by causal flag and key lengths");
+    static_assert(!DEALT || (KG == 1 && DROP == kDropNone), "more than one workgroup per compute unit, no dropout");
     using T = FwdTile<D>;
     constexpr int BN = T::BN, RS = T::RS;
     constexpr int BM = 32 * NW;  // query rows per workgroup
@@ -102,9 +104,9 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
     const bool by_batch = !KNOWS_BIAS && (p.m.kv_len || EXCL == kExKeys || EXCL == kExBits);
     const int wg = by_batch ? xcd_remap_heads<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
-    // (two groups: one workgroup per compute unit at most; dropout keeps the order it had)
-    constexpr bool DEALT = !KNOWS_BIAS && KG == 1 && DROP == kDropNone;
-    if (int t, s; DEALT && __builtin_expect(dealt_unit<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt, p.B, p.H, falling, by_batch && !falling, 8, t, s), 0)) {
+    if constexpr (DEALT) {
+        int t, s;
+        dealt_unit<NW == 4 && EXCL != kExBits>(blockIdx.x, n_qt, p.B, p.H, !falling, t, s);
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);         // (the compiler divides in vector registers)
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
@@ -686,6 +688,15 @@ __global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void
         return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
     });
     if (p.lse && h == 0 && qi < p.Sq) p.lse[(int64_t)bh * p.Sq + qi] = l > 0.f ? (m_run * c_log2 + log2_fast(l)) * kLn2 : -INFINITY;
+}
+
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1, bool AHEAD = false>
+__global__ __launch_bounds__(64 * NW * KG, NW * KG == 4 || KG == 2 ? 2 : 1) void fwd_kernel(const FwdParams p) {
+    fwd_body<D, EXCL, NW, DROP, KG, AHEAD, false>(p);
+}
+template <int D, int EXCL, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void fwd_dealt_kernel(const FwdParams p) {
+    fwd_body<D, EXCL, NW, kDropNone, 1, false, true>(p);
 }
 
 // Combines the partial outputs of a key split: LSE = log sum_s exp(LSE_s), O = sum_s exp(LSE_s - LSE) O_s.  A slice whose sum

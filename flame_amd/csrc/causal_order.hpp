@@ -12,7 +12,7 @@
 namespace fattn {
 
 // Up to one workgroup per compute unit the order is nothing but its divisions' time (0.3 us); the products below stay under 2^31.
-FATTN_HOST_DEVICE bool causal_order_pays(int slices, int total) { return slices % 8 != 0 && total > 256 && total <= 1 << 18; }
+inline bool causal_order_pays(int64_t slices, int64_t total) { return slices % 8 != 0 && total > 256 && total <= 1 << 18; }
 
 // Workgroup `linear` of `slices` * `levels`, slices % 8 != 0: its slice and its level, 0 being the longest walk of a slice.
 // Workgroups go to the XCDs in turn by `linear`.  An XCD keeps floor(slices / 8) whole slices, whose K and V stay in its L2; the

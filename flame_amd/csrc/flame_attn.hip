@@ -153,7 +153,7 @@ bool rule_key_groups(int64_t wgs, int Sk, int least_keys = 1024) { return wgs <=
 constexpr int kDqGroupKeys = 2048;
 
 // wg_count workgroups from p.wg_base on (0: all of the problem's)
-template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1, bool AHEAD = false>
+template <int D, int EXCL, int NW, int DROP = kDropNone, int KG = 1, bool AHEAD = false, bool DEALT = false>
 int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     using T = FwdTile<D>;
     constexpr int BM = 32 * NW;
@@ -161,8 +161,14 @@ int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     if constexpr (EXCL == kExNone && NW == 4 && KG == 1)
         if (rule_key_groups(grid, p.Sk)) return launch_fwd<D, EXCL, NW, DROP, 2>(p, s, wg_count);
+    if constexpr ((EXCL == kExNone || EXCL == kExKeys || EXCL == kExBits) && DROP == kDropNone && KG == 1 && !DEALT) {
+        const bool falling = p.m.causal && !p.m.kv_len;
+        if (!wg_count && deals_units(grid, (p.Sq + BM - 1) / BM, p.B, p.H, falling, !falling && (p.m.kv_len || EXCL != kExNone), 8))
+            return launch_fwd<D, EXCL, NW, DROP, KG, AHEAD, true>(p, s);
+    }
     static std::atomic<bool> lds_set{false};
     auto kern = fwd_kernel<D, EXCL, NW, DROP, KG, AHEAD>;
+    if constexpr (DEALT) kern = fwd_dealt_kernel<D, EXCL, NW>;
     constexpr bool KEYS = EXCL == kExKeys || EXCL == kExBits;
     constexpr int tiles = KG * T::LDS_BYTES + (EXCL == kExBiasF32 || EXCL == kExBiasBf16 ? T::BIAS_PASS_BYTES : T::q_pass_bytes(NW));
     if (const int rc = set_lds(reinterpret_cast<const void*>(kern), tiles + (KEYS ? KeyTiles::lds_bytes(KeyTiles::kMaxTiles) : 0), lds_set)) return rc;
@@ -374,14 +380,17 @@ template <int D>
 int launch_bwd_bits(BwdParams p, hipStream_t s) {
     using T = BwdTile<D>;
     using TQ = BwdDqTile<D>;
-    static std::atomic<bool> dq_set{false}, kv_set{false};
-    auto kern_dq = bwd_dq_kernel<D, kExBits, 4>;
-    auto kern_kv = bwd_dkdv_kernel<D, false, false, false, kDropNone, true>;
-    const int most = KeyTiles::lds_bytes(KeyTiles::kMaxTiles);
-    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_dq), TQ::LDS_BYTES + most, dq_set)) return rc;
-    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_kv), T::LDS_BYTES + most, kv_set)) return rc;
-    const int64_t grid = (int64_t)((p.Sk + T::BN - 1) / T::BN) * p.B * p.H, grid_dq = (int64_t)((p.Sq + TQ::BM - 1) / TQ::BM) * p.B * p.H;
+    const int64_t n_kt = (p.Sk + T::BN - 1) / T::BN, n_qt = (p.Sq + TQ::BM - 1) / TQ::BM, grid = n_kt * p.B * p.H, grid_dq = n_qt * p.B * p.H;
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
+    // (the causal flag goes into the bits: the walks of dQ differ by batch, those of dK/dV by the key lengths)
+    const bool dealt_dq = deals_units(grid_dq, (int)n_qt, p.B, p.H, false, true, 1);
+    const bool dealt_kv = p.m.kv_len && deals_units(grid, (int)n_kt, p.B, p.H, false, true, 1);
+    static std::atomic<bool> dq_set[2], kv_set[2];
+    auto kern_dq = dealt_dq ? bwd_dq_dealt_kernel<D, kExBits, 4> : bwd_dq_kernel<D, kExBits, 4>;
+    auto kern_kv = dealt_kv ? bwd_dkdv_dealt_kernel<D, true> : bwd_dkdv_kernel<D, false, false, false, kDropNone, true>;
+    const int most = KeyTiles::lds_bytes(KeyTiles::kMaxTiles);
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_dq), TQ::LDS_BYTES + most, dq_set[dealt_dq])) return rc;
+    if (const int rc = set_lds(reinterpret_cast<const void*>(kern_kv), T::LDS_BYTES + most, kv_set[dealt_kv])) return rc;
     if (const int rc = launch_mask_bits(p.m, p.B, p.H, p.Sq, p.Sk, p.split_ws, FLAME_ATTN_KERNEL_BWD_DQ, s)) return rc;
     p.split_ws = nullptr;
     {
@@ -405,33 +414,45 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
             return D == 128 && narrow(p.d) ? launch_bwd_bits<96>(p, s) : launch_bwd_bits<D>(p, s);
     }
     static bool attr_done = false;
+    // the instances for units dealt one by one (deals_units): not with an explicit mask
+    constexpr bool DEAL = !HASMASK && !TIMING;
     auto kern = bwd_dkdv_kernel<D, HASMASK, TIMING>;
+    auto kern_deal = bwd_dkdv_dealt_kernel<D, false>;
     auto kern_dq = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4>;
+    auto kern_dq_deal = bwd_dq_dealt_kernel<D, kExNone, 4>;
     // the same with two key groups per workgroup (the rule never asks for it with an explicit mask)
     constexpr int KG = HASMASK ? 1 : 2;
     auto kern_dqg = bwd_dq_kernel<D, HASMASK ? kExGeneral : kExNone, 4, kDropNone, KG>;
     auto kern_dqk = bwd_dq_kernel<D, kExKeys, 4>;                    // keep-mask of keys
+    auto kern_dqk_deal = bwd_dq_dealt_kernel<D, kExKeys, 4>;
     auto kern_dqv = bwd_dq_kernel<D, kExRows16, 4>;                  // keep-mask with vector-loadable rows over whole tiles
     auto kern_kvv = bwd_dkdv_kernel<D, true, false, true>;           // ... whose tiles travel through LDS
     using TW = BwdDqWideTile<D>;
     auto kern_dqw = bwd_dq_wide_kernel<D>;                           // 256-query workgroups, builds without a keep-mask only
+    auto kern_dqw_deal = bwd_dq_wide_dealt_kernel<D>;
     if (!attr_done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dq),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
+        hipError_t e = hipSuccess;
+        for (auto k : {kern, kern_deal}) {
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
+            if (e != hipSuccess) return (int)e;
+        }
+        for (auto k : {kern_dq, kern_dq_deal}) {
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
+            if (e != hipSuccess) return (int)e;
+        }
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqg),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, KG * TQ::LDS_BYTES);
         if (e != hipSuccess) return (int)e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqw),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, TW::LDS_BYTES);
-        if (e != hipSuccess) return (int)e;
-        if (!HASMASK) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqk), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    TQ::LDS_BYTES + KeyTiles::lds_bytes(KeyTiles::kMaxTiles));
+        for (auto k : {kern_dqw, kern_dqw_deal}) {
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, TW::LDS_BYTES);
             if (e != hipSuccess) return (int)e;
+        }
+        if (!HASMASK) {
+            for (auto k : {kern_dqk, kern_dqk_deal}) {
+                e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        TQ::LDS_BYTES + KeyTiles::lds_bytes(KeyTiles::kMaxTiles));
+                if (e != hipSuccess) return (int)e;
+            }
         }
         if (HASMASK) {
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern_dqv),
@@ -524,15 +545,17 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
     }
+    const bool falling = p.m.causal && !p.m.kv_len && !p.key_mask, by_batch = p.m.kv_len || p.key_mask;
     // dQ first: besides dQ it leaves -delta = -rowsum(dO * O) and the rescaled LSE of every query row in the
     // workspace, which the dK/dV kernel stages per query tile.
     {
+        const bool dealt = DEAL && deals_units(grid_dq, (int)n_qt, p.B, p.H, falling, by_batch, 1);
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_DQ, s);
         if (wide) {
             // a last round on at most half of the compute units: 128-query workgroups in a launch of their own (problems
             // whose walks are all equally long)
             const LastRound r = even && 2 * grid_dq <= 0x7fffffff ? cut_last_round(p.Sq, (int64_t)p.B * p.H, device_cu_count(), false) : LastRound{grid_dq};
-            hipLaunchKernelGGL(kern_dqw, dim3((unsigned)r.wide), dim3(256), TW::LDS_BYTES, s, p);
+            hipLaunchKernelGGL(dealt ? kern_dqw_deal : kern_dqw, dim3((unsigned)r.wide), dim3(256), TW::LDS_BYTES, s, p);
             if (r.count) {
                 BwdParams pt = p;
                 pt.dq_base = (int)r.base;
@@ -541,7 +564,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
             }
         }
         else if (!HASMASK && p.key_mask)
-            hipLaunchKernelGGL(kern_dqk, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
+            hipLaunchKernelGGL(dealt ? kern_dqk_deal : kern_dqk, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES + KeyTiles::lds_bytes((p.Sk + 63) / 64), s, p);
         else if (HASMASK && p.m.rows16 && p.Sk % TQ::BN == 0) hipLaunchKernelGGL(kern_dqv, dim3((unsigned)grid_dq), dim3(256), TQ::LDS_BYTES, s, p);
         else {
             BwdParams pq = p;
@@ -549,7 +572,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
             if (!HASMASK && pq.dq_parts == 1 && rule_key_groups(grid_dq, p.Sk, kDqGroupKeys))
                 hipLaunchKernelGGL(kern_dqg, dim3((unsigned)grid_dq), dim3(256 * KG), KG * TQ::LDS_BYTES, s, pq);
             else
-                hipLaunchKernelGGL(kern_dq, dim3((unsigned)(grid_dq * pq.dq_parts)), dim3(256), TQ::LDS_BYTES, s, pq);
+                hipLaunchKernelGGL(dealt && pq.dq_parts == 1 ? kern_dq_deal : kern_dq, dim3((unsigned)(grid_dq * pq.dq_parts)), dim3(256), TQ::LDS_BYTES, s, pq);
             if (pq.dq_parts > 1) hipLaunchKernelGGL(bwd_dq_merge_kernel<D>, dim3((unsigned)(grid_dq * (D / 32))), dim3(256), 0, s, pq);
         }
     }
@@ -561,8 +584,11 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         if (HASMASK && !TIMING && p.m.rows16 && !p.m.causal && p.Sk % T::BN == 0 && p.Sq % T::BM == 0 &&
             (int64_t)T::BM * p.m.sq < (int64_t)1 << 31)
             hipLaunchKernelGGL(kern_kvv, dim3((unsigned)grid_kv), dim3(256), T::LDS_BYTES_VECMASK, s, pk);
-        else
-            hipLaunchKernelGGL(kern, dim3((unsigned)grid_kv), dim3(256), T::LDS_BYTES, s, pk);
+        else {
+            // (a block whose walk is shared keeps its place: such grids fit the chip)
+            const bool dealt = DEAL && n_split == 0 && deals_units(grid_kv, (int)n_kt, p.B, p.H, falling, by_batch, 1);
+            hipLaunchKernelGGL(dealt ? kern_deal : kern, dim3((unsigned)grid_kv), dim3(256), T::LDS_BYTES, s, pk);
+        }
     }
     if (n_split > 0) {
         ScopedKernelTimer t(FLAME_ATTN_KERNEL_BWD_MERGE, s);
@@ -1048,7 +1074,7 @@ int flame_sage_quant_qk_int8_ks(const void* Q, const void* K, int B, int H, int 
 }  // extern "C"
 
 // wg_count workgroups starting at workgroup p.wg_base of the problem (0: all of them)
-template <int D, int NW, int KG = 1>
+template <int D, int NW, int KG = 1, bool DEALT = false>
 static int launch_sage_fwd(const SageFwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     using T = SageTile<D>;
     constexpr int BM = 32 * NW;
@@ -1056,8 +1082,12 @@ static int launch_sage_fwd(const SageFwdParams& p, hipStream_t s, int64_t wg_cou
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     if constexpr (KG == 1)
         if (rule_key_groups(grid, p.Sk) && !p.bias) return launch_sage_fwd<D, NW, 2>(p, s, wg_count);
+    if constexpr (KG == 1 && !DEALT)
+        if (!wg_count && deals_units(grid, (p.Sq + BM - 1) / BM, p.B, p.H, p.causal && !p.kv_len, p.kv_len != nullptr, 8))
+            return launch_sage_fwd<D, NW, KG, true>(p, s);
     static bool attr_done = false;
     auto kern = sage_fwd_kernel<D, NW, KG>;
+    if constexpr (DEALT) kern = sage_fwd_dealt_kernel<D, NW>;
     if (!attr_done) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, KG * T::LDS_BYTES);

@@ -288,9 +288,9 @@ __device__ __forceinline__ constexpr int swz_i8(int row) {
 }
 
 // NW wavefronts (4 or 8) of 32 queries each per workgroup, and KG = 2 groups of them with half of the key tiles each (no bias
-// then), as in the bf16 forward kernel.
-template <int D, int NW, int KG = 1>
-__global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel(const SageFwdParams p) {
+// then), as in the bf16 forward kernel.  DEALT: the units come in the order of causal_order.hpp (deals_units, which the host asks).
+template <int D, int NW, int KG, bool DEALT>
+__device__ __forceinline__ void sage_fwd_body(const SageFwdParams& p) {
     using T = SageTile<D>;
     constexpr int BM = 32 * NW, BN = T::BN;
     constexpr int KC = D / 32;   // int8 contraction chunks (32 per MFMA)
@@ -322,7 +322,9 @@ __global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel
     const int wg = p.kv_len ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
     int qt = wg % n_qt, bh = wg / n_qt;
     // (shortest first before: B=2 H=24 S=4608 D=128 causal 307 -> 276 us, B=1 H=24 S=2048 D=128 75.1 -> 61.8)
-    if (int t, s; KG == 1 && __builtin_expect(dealt_unit<KG == 1>(blockIdx.x, gridDim.x, n_qt, p.B, p.H, falling, p.kv_len != nullptr, 8, t, s), 0)) {
+    if constexpr (DEALT) {
+        int t, s;
+        dealt_unit<true>(blockIdx.x, n_qt, p.B, p.H, !falling, t, s);
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
@@ -698,6 +700,15 @@ __global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel
         return u32x2{pack_bf16(a[4 * g] * inv, a[4 * g + 1] * inv), pack_bf16(a[4 * g + 2] * inv, a[4 * g + 3] * inv)};
     });
     if (p.lse && h == 0 && row < p.Sq) p.lse[(int64_t)bh * p.Sq + row] = l > 0.f ? (m_run + log2_fast(l)) * kLn2 : -INFINITY;
+}
+
+template <int D, int NW, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, NW == 4 ? 2 : 1) void sage_fwd_kernel(const SageFwdParams p) {
+    sage_fwd_body<D, NW, KG, false>(p);
+}
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void sage_fwd_dealt_kernel(const SageFwdParams p) {
+    sage_fwd_body<D, NW, 1, true>(p);
 }
 
 

@@ -42,23 +42,22 @@ FATTN_HOST_DEVICE int xcd_remap_heads(int linear, int total, int per_head) {
     return ((j / per_head) * kXcd + x) * per_head + j % per_head;
 }
 
-// Problems whose walks differ in length and whose slices do not divide by the XCDs: true, with the unit of workgroup `linear`, where the
-// units left over are dealt one by one (causal_order.hpp).  Under the causal flag (falling): all B H slices, `tile` counted from the longest
-// walk.  Where the batches differ (by_batch): the H heads of every batch, batch after batch.  (Key lengths, forward and backward, us, contiguous ranges ->
-// this order: B=7 H=12 512 x 1500 D=128 43 -> 31 and 128 -> 90, B=3 H=12 S=4233 D=64 183 -> 125 and 522 -> 387, D=128 a key mask 317 -> 204 and 966 -> 611.)
+// Problems whose walks differ in length and whose slices do not divide by the XCDs: the units left over are dealt one by one
+// (causal_order.hpp).  Under the causal flag (falling): all B H slices, `tile` counted from the longest walk.  Where the batches differ
+// (by_batch): the H heads of every batch, batch after batch.
+// deals_units: the host's choice between a kernel's two instances.  (As a condition within the kernels it was 200 to 270 instructions ahead of every
+// problem's first load: forward, us, B=4 H=16 S=1101 D=128 with a key mask 40.2 -> 40.6, B=4 H=16 S=1101 D=64 30.5 -> 30.8.)
 // least: the fewest tiles per slice under the causal flag.  (Forward with fewer than eight: 75 heads of 512 at D = 64 11.0 -> 12.1 us, 107 of 1024 with
 // 256-query workgroups 46.8 -> 53.4.)
-// The condition is marked as unlikely, so that the code is not in the way of every other workgroup's first instructions, and kernels that gain little or
-// never have more than one workgroup per unit leave it out: 400 instructions in line cost B=2 H=16 S=1024 D=64 with dropout 64.0 -> 65.3 us.
+inline bool deals_units(int64_t total, int tiles, int B, int H, bool falling, bool by_batch, int least) {
+    return (by_batch || (falling && tiles >= least)) && causal_order_pays(by_batch ? H : (int64_t)B * H, total);
+}
 template <bool SNAKE = false>
-FATTN_HOST_DEVICE bool dealt_unit(int linear, int total, int tiles, int B, int H, bool falling, bool by_batch, int least, int& tile, int& bh) {
-    const int slices = by_batch ? H : B * H;
-    if (__builtin_expect(!(by_batch || (falling && tiles >= least)) || !causal_order_pays(slices, total), 1)) return false;
+FATTN_HOST_DEVICE void dealt_unit(int linear, int tiles, int B, int H, bool by_batch, int& tile, int& bh) {
     int slice, level;
-    causal_order(linear, slices, by_batch ? B * tiles : tiles, slice, level, [](int j, int count) { return SNAKE ? snake_order(j, count) : j; });
+    causal_order(linear, by_batch ? H : B * H, by_batch ? B * tiles : tiles, slice, level, [](int j, int count) { return SNAKE ? snake_order(j, count) : j; });
     tile = by_batch ? level % tiles : level;
     bh = by_batch ? level / tiles * H + slice : slice;
-    return true;
 }
 
 }  // namespace fattn

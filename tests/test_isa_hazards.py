@@ -60,7 +60,7 @@ def test_hand_emitted_mfma_results_are_not_touched_too_early(text):
     """The result of a hand-emitted MFMA (architectural accumulator, or the big-head-dim forward's pinned accumulation
     tuples) may be touched only after two more MFMAs or 11 wait states of s_nop.  Followed along the control flow:
     an unconditional branch to its target, a conditional one both ways."""
-    kernels = re.findall(r"^(_ZN5fattn(?:15bwd_dkdv_kernel|18bwd_dq_wide_kernel|15fwd_wide_kernel|20sage_fwd_wide_kernel|15fwd_bigd_kernel)\w+):.*?\.end_amdhsa_kernel", text, re.S | re.M)
+    kernels = re.findall(r"^(_ZN5fattn(?:15bwd_dkdv_kernel|21bwd_dkdv_dealt_kernel|18bwd_dq_wide_kernel|24bwd_dq_wide_dealt_kernel|15fwd_wide_kernel|20sage_fwd_wide_kernel|15fwd_bigd_kernel)\w+):.*?\.end_amdhsa_kernel", text, re.S | re.M)
     assert len(kernels) >= 9
     checked = 0
     for name in kernels:

@@ -11,10 +11,12 @@ SRC = r"""
 #include <cstdlib>
 #include "xcd_order.hpp"
 int unit(int linear, int total, int tiles, int B, int H, bool falling, bool by_batch, bool snake) {
-    int tile, bh;
-    const bool dealt = snake ? fattn::dealt_unit<true>(linear, total, tiles, B, H, falling, by_batch, 1, tile, bh)
-                             : fattn::dealt_unit<false>(linear, total, tiles, B, H, falling, by_batch, 1, tile, bh);
-    if (dealt) return bh * tiles + tile;
+    if (fattn::deals_units(total, tiles, B, H, falling, by_batch, 1)) {
+        int tile, bh;
+        if (snake) fattn::dealt_unit<true>(linear, tiles, B, H, by_batch, tile, bh);
+        else fattn::dealt_unit<false>(linear, tiles, B, H, by_batch, tile, bh);
+        return bh * tiles + tile;
+    }
     if (by_batch) return snake ? fattn::xcd_remap_heads<true>(linear, total, tiles) : fattn::xcd_remap_heads<false>(linear, total, tiles);
     return fattn::xcd_remap(linear, total);
 }
