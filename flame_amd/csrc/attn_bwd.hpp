@@ -129,7 +129,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     } else if (block < p.n_whole) {
         wg = xcd_remap(block, p.n_whole);
     } else {          // the split key blocks come last in dispatch order and fill the final, partial round (or are all there is)
-        const int e = p.n_whole == 0 ? xcd_remap(block, nblocks) : block - p.n_whole;
+        const int e = p.n_whole == 0 ? xcd_remap_split(block, nblocks) : block - p.n_whole;
         nparts = p.split_parts;
         wg = p.n_whole + e / nparts;
         part = e % nparts;
@@ -938,7 +938,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams& p) {
     const int n_qt = (p.Sq + BM - 1) / BM;
     int wg, part = 0;
     if (p.dq_parts > 1) {
-        const int all = xcd_remap(blockIdx.x, gridDim.x);
+        const int all = xcd_remap_split(blockIdx.x, gridDim.x);
         part = all % p.dq_parts;
         wg = all / p.dq_parts;
     } else {

@@ -14,6 +14,9 @@ FATTN_HOST_DEVICE int xcd_remap(int linear, int total) {
     const int x = linear % kXcd;
     return x * (total / kXcd) + (x < total % kXcd ? x : total % kXcd) + linear / kXcd;
 }
+// Workgroups that share one walk: in turn where the total does not divide.  (Contiguous ranges there, dK/dV, us: 7 heads of 1500 D=64, 252 workgroups,
+// 16.6 -> 21.0, D=128 25.1 -> 27.7; 5 heads of 1100 D=96, 180 workgroups, 17.2 -> 19.5.  dQ 1 to 3 % at D=64 and 96.)
+FATTN_HOST_DEVICE int xcd_remap_split(int linear, int total) { return total % 8 == 0 ? xcd_remap(linear, total) : linear; }
 // Workgroups of which a compute unit holds two are dealt out one per unit, then a second one each.  Where (nearly) all fit at once
 // nothing is left to even out unequal walks: in the order of falling length the units with the longest walks would get the
 // longer ones of the second deal as well, so that one is turned round.  With more than three deals the order of falling length
@@ -37,7 +40,7 @@ template <bool SNAKE = false>
 FATTN_HOST_DEVICE int xcd_remap_heads(int linear, int total, int per_head) {
     constexpr int kXcd = 8;
     const int n_heads = total / per_head;
-    if (n_heads % kXcd != 0) return total % kXcd == 0 ? xcd_remap(linear, total) : linear;
+    if (n_heads % kXcd != 0) return xcd_remap_split(linear, total);
     const int x = linear % kXcd, j = SNAKE ? snake_order(linear / kXcd, total / kXcd) : linear / kXcd;
     return ((j / per_head) * kXcd + x) * per_head + j % per_head;
 }

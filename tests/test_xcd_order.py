@@ -23,8 +23,9 @@ int unit(int linear, int total, int tiles, int B, int H, bool falling, bool by_b
 int main(int, char** argv) {
     const int B = atoi(argv[1]), H = atoi(argv[2]), tiles = atoi(argv[3]), total = B * H * tiles;
     for (int i = 0; i < total; ++i)
-        printf("%d %d %d %d %d\n", unit(i, total, tiles, B, H, false, false, false), unit(i, total, tiles, B, H, true, false, false),
-               unit(i, total, tiles, B, H, true, false, true), unit(i, total, tiles, B, H, false, true, false), unit(i, total, tiles, B, H, false, true, true));
+        printf("%d %d %d %d %d %d\n", unit(i, total, tiles, B, H, false, false, false), unit(i, total, tiles, B, H, true, false, false),
+               unit(i, total, tiles, B, H, true, false, true), unit(i, total, tiles, B, H, false, true, false), unit(i, total, tiles, B, H, false, true, true),
+               fattn::xcd_remap_split(i, total));
 }
 """
 
@@ -41,10 +42,11 @@ def exe(tmp_path_factory):
                                                  (5, 15, 13), (13, 10, 5), (143, 7, 3), (2, 12, 40)])
 def test_every_unit_once(exe, batches, heads, tiles):
     out = subprocess.run([exe, str(batches), str(heads), str(tiles)], check=True, capture_output=True, text=True).stdout.split()
-    plain, falling, falling_snake, by_batch, by_batch_snake = ([int(v) for v in out[i::5]] for i in range(5))
+    plain, falling, falling_snake, by_batch, by_batch_snake, split = ([int(v) for v in out[i::6]] for i in range(6))
     total = batches * heads * tiles
     for ids in (plain, falling, falling_snake, by_batch, by_batch_snake):
         assert sorted(ids) == list(range(total))
+    assert split == (plain if total % 8 == 0 else list(range(total)))      # the workgroups that share walks: in turn where eight does not divide
     for x in range(8):
         mine = plain[x::8]
         assert mine == list(range(mine[0], mine[0] + len(mine))) if mine else True
