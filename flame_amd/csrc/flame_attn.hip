@@ -28,7 +28,7 @@
 #include "attn_fwd.hpp"
 #include "attn_fwd_bigd.hpp"
 #include "attn_fwd_keyshare.hpp"
-#include "last_round.hpp"
+#include "query_tile.hpp"
 #include "prep.hpp"
 #include "sage.hpp"
 #include "plan_cache.hpp"
@@ -468,29 +468,14 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
     const int64_t grid = n_kt * p.B * p.H;
     // 256-query workgroups (4 wavefronts of 64 queries) when they neither add padding rows nor leave compute units idle
     const int64_t n256 = (p.Sq + 255) / 256;
-    // (with key lengths the walks differ in length and the longest ones set the time: unless the units fill two
-    // rounds, twice as many workgroups of half the size finish sooner; so they do where the last round of the large ones is
-    // thin and cannot be cut (thin_last_round), and on short walks, where the start of a workgroup weighs most: up to 1024 keys past
-    // one round, from 2.25 rounds on, whose last is no longer cut for a few units, up to 1536 keys and at D = 64 up to 3072.
-    // Backward, equal walks, us, 256- -> 128-query workgroups, rounds of the former in brackets: D = 128, 512 keys [1] 85.8 -> 87.2,
-    // [2] 174.1 -> 157.8, [4] 333 -> 308; 1024 keys [1] 122.9 -> 122.9, [2] 251 -> 240, [4] 486 -> 464; 1536 keys [2] 335 -> 340, [2.5] 446 -> 434,
-    // [4] 685 -> 660; 2048 keys [2.5] 525 -> 508, [4] 814 -> 811; D = 64, 512 keys [2] 85.0 -> 76.1, [4] 166 -> 146; 1024 keys [2] 129.4 -> 124.3,
-    // [4] 259 -> 244; 1536 keys [2.5] 246 -> 236, [4] 378 -> 357; 2048 keys [1] 112.5 -> 118.0, [2.5] 291 -> 277, [4] 447 -> 436; 3072 keys [2.5] 410 -> 396,
-    // [4] 638 -> 623; 4096 keys [2.5] 529 -> 522, [4] 819 -> 817.
-    // Under the causal flag, four query tiles or more: D = 128, S = 1024 [1] 103 -> 91, [2] 184 -> 173; 2048 [1] 158 -> 142, [4] 538 -> 527; 3072 [3] 517 ->
-    // 509, [3.5] 630 -> 636; 4096 [1] 250 -> 227, [2] 425 -> 434; 8192 [2] 775 -> 809; D = 64, S = 1024 [1] 61.2 -> 50.6, [2] 105 -> 92; 2048 [2] 154 -> 148,
-    // [4] 294 -> 273; 4096 [2] 251.3 -> 252.7, [8] 971 -> 931; 8192 [2] 449 -> 457, [3.75] 814 -> 799.)
+    // and their rule says so (dq_takes_256); with key lengths only from two rounds on
     const int64_t total256 = n256 * p.B * p.H;
     const bool even = !p.m.causal && !p.m.kv_len;           // all walks equally long
     const bool wide_fits = !HASMASK && !p.key_mask && n256 * 256 <= ((int64_t)(p.Sq + 127) / 128) * 128 && total256 >= device_cu_count() &&
                            !(p.m.kv_len && total256 < 2 * device_cu_count()) && wg_waves_override() != 4;
     const int joint_mode = wide_fits ? bwd_schedule_override() : 0;
     const bool wide = wide_fits && (joint_mode != 0 ||      // (a schedule asked for by name has 256-query workgroups)
-                                    (!(thin_last_round(total256, device_cu_count(), 2) && (!even || total256 < 2 * device_cu_count())) &&
-                                     !(p.Sk <= 1024 && (even ? total256 > device_cu_count() : total256 % device_cu_count() != 0)) &&
-                                     !(p.m.causal && !p.m.kv_len && D != 96 && p.Sq > 768 && p.Sk == p.Sq &&
-                                       (p.Sk <= (D == 64 ? 4096 : 3072) || total256 <= device_cu_count())) &&
-                                     !(even && D != 96 && 4 * total256 >= 9 * device_cu_count() && p.Sk <= (D == 64 ? 3072 : 1536))));
+                                    dq_takes_256(total256, device_cu_count(), p.Sq, p.Sk, D, p.m.causal, p.m.kv_len != nullptr));
     const int64_t n_qt = wide ? n256 : (p.Sq + TQ::BM - 1) / TQ::BM;
     const int64_t grid_dq = n_qt * p.B * p.H;
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
@@ -1169,14 +1154,11 @@ int flame_sage_attn_fwd_bias_int8(const void* Qi8, const void* Ki8, const void* 
     // compute units without a workgroup, and nothing is excluded; else 128-query workgroups of four 32-query
     // wavefronts.  A last round that would occupy at most half of the compute units with 256-query workgroups is
     // cut into 128-query workgroups in a launch of its own: alone on its compute unit, such a workgroup takes little
-    // more than half the time of a 256-query one.  Up to 1024 keys the start of a second launch costs more than that gains (us, cut ->
-    // 128-query workgroups throughout, rounds in brackets: D = 128, 512 keys [1.12] 36.1 -> 32.9, [1.5] 38.2 -> 34.2, [2.5] 60.0 -> 55.6; 1024
-    // keys [1.12] 51.4 -> 48.9, [1.5] 56.2 -> 52.4, [2.5] 86.6 -> 83.3; 1536 keys [1.25] 68.2 -> 70.4; D = 64, 512 keys [1.25] 27.7 -> 24.5, 1024 keys [1.12]
-    // 38.3 -> 36.1, [2.5] 59.8 -> 60.0; 1536 keys [1.5] 51.7 -> 49.0, [2.5] 81.1 -> 86.0).
+    // more than half the time of a 256-query one.  (sage_takes_256)
     const int cus = device_cu_count();
     const int64_t n256 = (N_q + 255) / 256, total256 = n256 * B * H;
     const bool wide = n256 * 256 <= ((N_q + 127) / 128) * 128 && total256 >= cus && !causal && !kv_len && !bias &&
-                      N_kv % 64 == 0 && wg_waves_override() != 4 && !(total256 > cus && thin_last_round(total256, cus, 2) && N_kv <= 1024);
+                      N_kv % 64 == 0 && wg_waves_override() != 4 && sage_takes_256(total256, cus, N_kv);
     if (wide) {
         if (2 * total256 > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
         const LastRound r = cut_last_round(N_q, (int64_t)B * H, cus, false);
@@ -1238,37 +1220,11 @@ static bool fwd_fits_256(int B, int H, int N_q, bool has_mask_or_bias, bool has_
 // nothing is excluded at all: 4 wavefronts of 64 queries (launch_fwd_wide), else 8 of 32
 static bool fwd_plain(int N_kv, bool causal, bool has_kv_len) { return !causal && !has_kv_len && N_kv % 64 == 0; }
 
-// The rule for the forward's query tile, 256 rows per workgroup (true) or 128, of a call and of a launch plan; DP: padded head
-// dim, d96: the kernels of 96.  Ragged or causal calls up to D = 64 take 128, and so do thin last rounds (last_round.hpp, with the
-// figures); a plan may still ask for 256 there.
-// The 64-query wavefronts of launch_fwd_wide need 16 us from launch to result besides their steps (their first pass through
-// 40 KB of code among them), 128-query workgroups, two of which share a unit, 10, and those fill a last round more evenly.  Past
-// one round the shortest walks are therefore theirs, and longer ones where the last round is at most half full.  Measured
-// without exclusions, Sq = Sk, us, 256- -> 128-query workgroups, rounds of the former in brackets:
-//   D = 128   512 keys [1.12] 36.6 -> 32.2, [1.5] 40.9 -> 35.1, [2] 52.7 -> 48.4, [2.5] 70.1 -> 59.2, [4] 99.4 -> 90.0; 1024 keys [1.12] 54.6 -> 52.2,
-//             [1.5] 62.8 -> 57.4, [1.75] 68.9 -> 69.4, [2] 76.5 -> 76.4, [2.5] 102.5 -> 93.9, [4] 145.7 -> 145.7; 1536 keys [1.12] 64.6 -> 72.0,
-//             [1.5] 81.0 -> 78.8, [2] 104.6 -> 109.4; 2048 keys [1.5] 101.7 -> 102.5, [2] 127.3 -> 131.3, [2.5] 166.1 -> 161.7; 3072 keys [1.5] 143.9 -> 147.1
-//   D = 64    512 keys [1.12] 23.1 -> 21.2, [1.5] 26.4 -> 22.9, [2.5] 42.1 -> 36.1, [4] 61.2 -> 57.8; 1024 keys [1.12] 35.1 -> 33.4, [1.5] 42.5 -> 37.2,
-//             [1.75] 44.7 -> 42.9, [2] 47.0 -> 46.4, [4] 92.1 -> 91.2; 1536 keys [1.12] 41.4 -> 45.4, [1.5] 52.7 -> 48.0, [2] 68.0 -> 67.6,
-//             [4] 134.5 -> 138.8; 2048 keys [1.5] 65.2 -> 63.2, [2.5] 105.6 -> 98.8, [4] 156.5 -> 162.6; 3072 keys [1.5] 90.4 -> 91.5, [2.5] 150.9 -> 139.8,
-//             [3] 162.5 -> 166.7; 4096 keys [1.5] 114.3 -> 116.8, [2] 147.7 -> 149.9, [4] 279 -> 293
-// Under the causal flag (D = 128; four query tiles or more, so that the walks differ) they level better: S = 1024 [1] 31.2 -> 25.9,
-// [1.67] 54.6 -> 44.1, [2] 49.0 -> 47.3; 1536 [1.76] 68.2 -> 57.6, [3] 96.3 -> 88.2; 2048 [1] 52.5 -> 43.2, [2] 75.8 -> 77.1, [2.34] 101.2 -> 89.6, [4] 152.6 -> 147.0;
-// 3072 [1.5] 85.7 -> 82.2, [3] 159 -> 154, [6] 315 -> 325; 4096 [1] 96.4 -> 79.2, [2] 130.8 -> 140.9, [2.69] 186.8 -> 181.4; 8192 [2] 244 -> 265,
-// [2.62] 337.6 -> 332.5: the whole numbers of rounds are slices that divide by the eight XCDs, the others come in the order of causal_order.hpp.
-// (Not measured for the kernels of 96.)
+// The rule for the forward's query tile, 256 rows per workgroup (true) or 128, of a call and of a launch plan (which may still ask
+// for 256 where the rule does not); DP: padded head dim, d96: the kernels of 96.
 static bool fwd_rule_wide(int B, int H, int N_q, int N_kv, int DP, bool d96, bool causal, bool has_mask_or_bias, bool has_kv_len) {
-    const bool plain = fwd_plain(N_kv, causal, has_kv_len);
-    if (!fwd_fits_256(B, H, N_q, has_mask_or_bias, has_kv_len) || (!plain && DP == 64)) return false;
-    const int64_t total256 = (int64_t)((N_q + 255) / 256) * B * H, cus = device_cu_count();
-    const bool thin8 = thin_last_round(total256, cus, 8), half = thin_last_round(total256, cus, 2);
-    if (!d96 && !has_kv_len) {
-        const bool few = plain && thin_last_round(total256, cus, 32);         // (a handful more than whole rounds are cut cheaply)
-        if (!causal && !few && total256 > cus && N_kv <= (plain && thin8 ? 1024 : half ? (DP == 64 ? 3072 : 2048) : DP == 64 ? 1024 : 512)) return false;
-        if (causal && N_q > 768 && N_kv == N_q && (N_kv <= 3072 || total256 <= cus || B * H % 8 != 0)) return false;
-    }
-    // (without exclusions a last round on an eighth of the units is cut into 32-query workgroups, launch_fwd_wide)
-    return !thin_last_round(total256, cus, 3) || (plain && (total256 >= 2 * cus || thin8));
+    return fwd_fits_256(B, H, N_q, has_mask_or_bias, has_kv_len) &&
+           fwd_takes_256((int64_t)((N_q + 255) / 256) * B * H, device_cu_count(), (int64_t)B * H, N_q, N_kv, DP, d96, causal, has_kv_len);
 }
 
 static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, void* LSE,
