@@ -163,7 +163,7 @@ int launch_fwd(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
         if (rule_key_groups(grid, p.Sk)) return launch_fwd<D, EXCL, NW, DROP, 2>(p, s, wg_count);
     if constexpr ((EXCL == kExNone || EXCL == kExKeys || EXCL == kExBits) && DROP == kDropNone && KG == 1 && !DEALT) {
         const bool falling = p.m.causal && !p.m.kv_len;
-        if (!wg_count && deals_units(grid, (p.Sq + BM - 1) / BM, p.B, p.H, falling, !falling && (p.m.kv_len || EXCL != kExNone), 8))
+        if (!wg_count && deals_units(grid, (p.Sq + BM - 1) / BM, p.B, p.H, falling, !falling && (EXCL == kExBits || (p.B > 1 && (p.m.kv_len || EXCL == kExKeys))), 8))
             return launch_fwd<D, EXCL, NW, DROP, KG, AHEAD, true>(p, s);
     }
     static std::atomic<bool> lds_set{false};
@@ -384,7 +384,7 @@ int launch_bwd_bits(BwdParams p, hipStream_t s) {
     if (grid > 0x7fffffff || grid_dq > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     // (the causal flag goes into the bits: the walks of dQ differ by batch, those of dK/dV by the key lengths)
     const bool dealt_dq = deals_units(grid_dq, (int)n_qt, p.B, p.H, false, true, 1);
-    const bool dealt_kv = p.m.kv_len && deals_units(grid, (int)n_kt, p.B, p.H, false, true, 1);
+    const bool dealt_kv = deals_units(grid, (int)n_kt, p.B, p.H, false, p.B > 1 && p.m.kv_len, 1);
     static std::atomic<bool> dq_set[2], kv_set[2];
     auto kern_dq = dealt_dq ? bwd_dq_dealt_kernel<D, kExBits, 4> : bwd_dq_kernel<D, kExBits, 4>;
     auto kern_kv = dealt_kv ? bwd_dkdv_dealt_kernel<D, true> : bwd_dkdv_kernel<D, false, false, false, kDropNone, true>;
@@ -530,7 +530,7 @@ int launch_bwd(const BwdParams& p, hipStream_t s) {
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? FLAME_ATTN_OK : (int)e;
     }
-    const bool falling = p.m.causal && !p.m.kv_len && !p.key_mask, by_batch = p.m.kv_len || p.key_mask;
+    const bool falling = p.m.causal && !p.m.kv_len && !p.key_mask, by_batch = p.B > 1 && (p.m.kv_len || p.key_mask);
     // dQ first: besides dQ it leaves -delta = -rowsum(dO * O) and the rescaled LSE of every query row in the
     // workspace, which the dK/dV kernel stages per query tile.
     {
@@ -1068,7 +1068,7 @@ static int launch_sage_fwd(const SageFwdParams& p, hipStream_t s, int64_t wg_cou
     if constexpr (KG == 1)
         if (rule_key_groups(grid, p.Sk) && !p.bias) return launch_sage_fwd<D, NW, 2>(p, s, wg_count);
     if constexpr (KG == 1 && !DEALT)
-        if (!wg_count && deals_units(grid, (p.Sq + BM - 1) / BM, p.B, p.H, p.causal && !p.kv_len, p.kv_len != nullptr, 8))
+        if (!wg_count && deals_units(grid, (p.Sq + BM - 1) / BM, p.B, p.H, p.causal && !p.kv_len, p.B > 1 && p.kv_len, 8))
             return launch_sage_fwd<D, NW, KG, true>(p, s);
     static bool attr_done = false;
     auto kern = sage_fwd_kernel<D, NW, KG>;

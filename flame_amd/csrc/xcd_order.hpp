@@ -47,7 +47,10 @@ FATTN_HOST_DEVICE int xcd_remap_heads(int linear, int total, int per_head) {
 
 // Problems whose walks differ in length and whose slices do not divide by the XCDs: the units left over are dealt one by one
 // (causal_order.hpp).  Under the causal flag (falling): all B H slices, `tile` counted from the longest walk.  Where the batches differ
-// (by_batch): the H heads of every batch, batch after batch.
+// (by_batch: key lengths or key masks of several batches, masks as bits): the H heads of every batch, batch after batch, wherever H does not divide,
+// also where B H does and every XCD could keep whole slices: it would get long ones or short ones.  (That order -> this one, mean over 8 draws of key
+// lengths, forward / dK/dV / dQ, 4096 x 4096, D = 128: B=4 H=4 1.08 / 1.14 / 1.08 times as fast, B=8 H=4 1.06 / 1.10 / 0.99, B=8 H=2 1.13 / 1.13 / 1.15, B=8 H=12
+// 1.02 / 1.06 / 1.05; B=8 H=4 at D = 64 1.09 / 1.09 / 1.00.  One batch has nothing to level: B=1 H=12 4096 x 4096 D=128 with a key mask, backward 349 -> 353 us.)
 // deals_units: the host's choice between a kernel's two instances.  (As a condition within the kernels it was 200 to 270 instructions ahead of every
 // problem's first load: forward, us, B=4 H=16 S=1101 D=128 with a key mask 40.2 -> 40.6, B=4 H=16 S=1101 D=64 30.5 -> 30.8.)
 // least: the fewest tiles per slice under the causal flag.  (Forward with fewer than eight: 75 heads of 512 at D = 64 11.0 -> 12.1 us, 107 of 1024 with

@@ -73,9 +73,10 @@ def test_kernels(B, H, Sq, Sk, D, causal, lens, masked, rows, names):
     assert [x for x in got if x.startswith(("fwd_", "bwd_d"))] == list(names), got
 
 
-# slices that divide by eight, one workgroup per compute unit at most, no exclusion at all: the kernels without it
+# slices that divide by eight, one workgroup per compute unit at most, no exclusion at all, one sequence: the kernels without it
 @pytest.mark.parametrize("B,H,Sq,Sk,D,causal,lens,masked", [(1, 40, 1024, 1024, 64, True, None, False), (4, 16, 300, 400, 128, False, (400, 65, 0, 77), True),
-                                                            (1, 12, 1000, 1000, 128, True, None, False), (1, 37, 1024, 300, 64, False, None, False)])
+                                                            (1, 12, 1000, 1000, 128, True, None, False), (1, 37, 1024, 300, 64, False, None, False),
+                                                            (1, 12, 3000, 400, 64, False, (333,), False), (1, 12, 3000, 3100, 128, False, (3001,), True)])
 def test_other_problems(B, H, Sq, Sk, D, causal, lens, masked):
     got = check(B, H, Sq, Sk, D, causal, lens, masked)
     assert not any("dealt" in x for x in got), got
