@@ -324,7 +324,10 @@ __device__ __forceinline__ void sage_fwd_body(const SageFwdParams& p) {
     // (shortest first before: B=2 H=24 S=4608 D=128 causal 307 -> 276 us, B=1 H=24 S=2048 D=128 75.1 -> 61.8)
     if constexpr (DEALT) {
         int t, s;
-        dealt_unit<true>(blockIdx.x, n_qt, p.B, p.H, !falling, t, s);
+        if (falling) dealt_unit<true>(blockIdx.x, n_qt, p.B, p.H, false, t, s);
+        else dealt_unit(blockIdx.x, n_qt, p.B, p.H, true, t, s);         // (the batches do not come by length here: nothing to turn round, snake_order;
+        // turned round, as fast as without this order, least and most of 8 draws: B=6 H=4 S=2048 D=64 0.81 and 1.28, as here 1.01 and 1.06; B=4 H=12 S=2048
+        // D=64 0.90 and 1.00, here 0.92 and 1.07, D=128 0.94 and 1.11, here 0.96 and 1.10; B=4 H=4 S=4096 D=128 0.91 and 1.24, here 1.00 and 1.13)
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
