@@ -31,9 +31,11 @@ struct FwdKeyShareTile {
     static_assert(2 * TILE_ELEMS <= WAVE_ELEMS && BQ * O_STRIDE * 2 <= WAVE_ELEMS && WAVE_ELEMS * 2 % 512 == 0, "both fit");
 };
 
-// DROP (DropMode) as in fwd_kernel.
+// DROP (DropMode) as in fwd_kernel.  At D = 64 four wavefronts per SIMD, two workgroups of eight per unit; the draw by tiles takes 184 registers
+// and keeps to two: within 128 it spilled 56 bytes per lane (us, that -> this: 4 heads of 512 11.8 -> 10.1, 8 of 1024 19.5 -> 15.4, 16 of 1024 33.3 -> 26.4, 2 of 4096
+// 57.7 -> 45.7, 64 heads, 20 queries, 2000 keys 36.4 -> 25.3).
 template <int D, int NW_, int DROP>
-__global__ __launch_bounds__(64 * NW_, D == 64 ? 4 : 2) void fwd_keyshare_kernel(const FwdParams p) {
+__global__ __launch_bounds__(64 * NW_, D == 64 && DROP != kDropTiled ? 4 : 2) void fwd_keyshare_kernel(const FwdParams p) {
     using T = FwdKeyShareTile<D, NW_>;
     constexpr int BN = T::BN, NW = T::NW, RS = T::RS, DC = D / 16, DB = D / 32, GPR = RS / 8, NDMA = T::NDMA;
 

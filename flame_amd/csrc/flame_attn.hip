@@ -211,7 +211,8 @@ template <int D, int DROP>
 int launch_fwd_keyshare(const FwdParams& p, hipStream_t s, int64_t wg_count = 0) {
     const int64_t grid = (wg_count ? wg_count : (int64_t)((p.Sq + 31) / 32) * p.B * p.H) * p.key_splits;
     if (grid > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
-    return fwd_keyshare_waves(grid, D, p.Sk) == 4 ? launch_fwd_keyshare_nw<D, 4, DROP>(p, grid, s) : launch_fwd_keyshare_nw<D, 8, DROP>(p, grid, s);
+    const int fits_as = DROP == kDropTiled ? 128 : D;              // (a draw by tiles at D = 64 leaves two wavefronts per SIMD)
+    return fwd_keyshare_waves(grid, fits_as, p.Sk) == 4 ? launch_fwd_keyshare_nw<D, 4, DROP>(p, grid, s) : launch_fwd_keyshare_nw<D, 8, DROP>(p, grid, s);
 }
 
 // 256-query workgroups, one wavefront per SIMD (builds without keep-mask / bias only)

@@ -51,7 +51,7 @@ def test_wavefronts(oracle, B, H, Sq, Sk, D, causal, lens, compiled, waves):
 # rows that start on multiples of 64 elements, others, and a draw per 48 x 40 tile; more than 256 workgroups too
 @pytest.mark.parametrize("B,H,Sq,Sk,D,causal,chunk", [
     (1, 3, 70, 320, 64, False, None), (1, 2, 64, 192, 96, True, None), (1, 3, 70, 301, 128, True, None), (1, 2, 100, 90, 40, False, None),
-    (1, 2, 100, 90, 128, False, (48, 40)), (1, 258, 3, 128, 64, False, None)])
+    (1, 2, 100, 90, 128, False, (48, 40)), (1, 258, 3, 128, 64, False, None), (1, 2, 100, 90, 64, True, (48, 40)), (1, 258, 3, 128, 64, False, (2, 64))])
 def test_dropout(oracle, B, H, Sq, Sk, D, causal, chunk):
     from flame_amd import capi
     seed, sc = 0x2545F4914F6CDD1D, 1.0 / math.sqrt(D)

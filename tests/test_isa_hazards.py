@@ -250,8 +250,8 @@ def test_the_bias_counted_out_of_a_wait_is_younger_than_the_copies(text):
 def test_words_of_a_mask_are_not_waited_for_within_their_step(text):
     """The forward that walks by a mask's bits: loads return in order, so a step that waits for a word which it has requested itself waits
     for its tile copies as well.  The word is the next step's; the first wait behind it is the one in front of the barrier."""
-    for D, mfmas in ((64, 16), (96, 24), (128, 32)):          # half a step's or more are between
-        name = "_ZN5fattn10fwd_kernelILi%dELi6ELi4ELi0ELi1ELb0EEEvNS_9FwdParamsE" % D
+    for D, mfmas, form in [(*d, f) for d in ((64, 16), (96, 24), (128, 32)) for f in ("10fwd_kernelILi%dELi6ELi4ELi0ELi1ELb0EE", "16fwd_dealt_kernelILi%dELi6ELi4EE")]:
+        name = "_ZN5fattn" + form % D + "EvNS_9FwdParamsE"    # (half a step's MFMAs or more are between)
         body = re.search(r"^%s:.*?\.end_amdhsa_kernel" % name, text, re.S | re.M).group(0)
         ins = [l.strip() for l in body.split("\n") if re.match(r"^\s+[a-z]", l)]
         first = next(i for i, l in enumerate(ins) if l.startswith("v_mfma"))
@@ -261,3 +261,9 @@ def test_words_of_a_mask_are_not_waited_for_within_their_step(text):
             j = next(j for j in range(i, len(ins)) if ins[j].startswith("s_waitcnt") and "vmcnt" in ins[j])
             assert any(l.startswith("s_barrier") for l in ins[j:j + 8]), (name, ins[i:j + 1])
             assert sum(l.startswith("v_mfma") for l in ins[i:j]) >= mfmas, name
+
+
+def test_the_key_sharing_forward_keeps_its_state_in_registers(text):
+    """Every form of it, the draws of a dropout among them: none of a wavefront's running state in scratch memory."""
+    kernels = re.findall(r"^(_ZN5fattn19fwd_keyshare_kernel\w+):.*?\.amdhsa_private_segment_fixed_size (\d+)", text, re.S | re.M)
+    assert len(kernels) == 18 and all(int(size) == 0 for _, size in kernels), kernels
