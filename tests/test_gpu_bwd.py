@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from flame_amd import workloads as W
-from tests.gpu_util import assert_close_bf16, to_dev, to_f32
+from tests.gpu_util import assert_close_bf16, recorded_launches, to_dev, to_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -182,9 +182,15 @@ def test_split_last_round_matches_unsplit_walk():
 def test_wide_workgroups_with_exclusions(oracle, mode):
     """Enough query tiles that the forward and dQ kernels pick their 256-query (8-wavefront)
     workgroups, combined with a causal diagonal or ragged key lengths; oracle parity on a head subset."""
-    B, H, S, D = 2, 16, 2048, 128
-    t = [W.f32_to_bf16_bits(W.normal_f32(4242, s, B * H * S * D).reshape(B, H, S, D) * np.float32(0.7071)) for s in range(4)]
+    from flame_amd import capi
+    B, H, Sq, Sk, D = 4, 16, 2048, 2112, 128           # (as many keys as queries under the causal flag: 128-query dQ)
+    t = [W.f32_to_bf16_bits(W.normal_f32(4242, s, B * H * n * D).reshape(B, H, n, D) * np.float32(0.7071)) for s, n in enumerate((Sq, Sk, Sk, Sq))]
     w = W.Workload(f"wide_{mode}", t[0], t[1], t[2], t[3], 1.0 / math.sqrt(D), causal=(mode == "causal"),
-                   kv_len=np.array([S, 777], np.int32) if mode == "kvlen" else None)
+                   kv_len=np.array([Sk, 777, 64, 2000], np.int32) if mode == "kvlen" else None)
     _check_bwd(oracle, w, heads=(0, 1), tag="first head")
     _check_bwd(oracle, w, heads=(B * H - 1, B * H), tag="last head")
+    q, k, v, do = (to_dev(x) for x in t)
+    kw = dict(causal=w.causal, kv_len=None if w.kv_len is None else torch.from_numpy(w.kv_len).cuda())
+    o, lse = capi.attn_fwd(q, k, v, w.scale, **kw)
+    names = [x[0] for f in (lambda: capi.attn_fwd(q, k, v, w.scale, **kw), lambda: capi.attn_bwd(q, k, v, o, do, lse, w.scale, **kw)) for x in recorded_launches(f)]
+    assert names[0].startswith("fwd_kernel<128, 0, 8,") and names[1] == "bwd_dq_wide_kernel<128>", names

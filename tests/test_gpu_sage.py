@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from flame_amd import workloads as W
-from tests.gpu_util import TOL_LSE, assert_close_bf16, to_dev, to_f32
+from tests.gpu_util import TOL_LSE, assert_close_bf16, recorded_launches, to_dev, to_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -150,8 +150,10 @@ def test_sage_blocks_of_different_magnitude(oracle):
 
 
 @pytest.mark.parametrize("B,H,Sq,Sk,D", [(2, 16, 2048, 256, 64),      # 256 workgroups of 256 queries: whole rounds only
-                                          (1, 36, 2048, 192, 64),      # 288: the last 32 are cut into 64 of 128 queries
-                                          (1, 33, 2048, 320, 128),     # 264: the last 8 are cut into 16
+                                          (1, 36, 2048, 1088, 64),     # 288: the last 32 are cut into 64 of 128 queries
+                                          (1, 33, 2048, 1088, 128),    # 264: the last 8 are cut into 16
+                                          (1, 36, 2048, 192, 64),      # the same on a short walk: 128-query workgroups throughout
+                                          (1, 33, 2048, 320, 128),
                                           (2, 16, 2048, 64, 64),       # one key tile: prologue and a single step
                                           (2, 16, 1948, 128, 128),     # two key tiles; the last query tile is partly empty
                                           (1, 50, 1280, 576, 128)])    # 250 < compute units: 128-query workgroups only
@@ -173,6 +175,17 @@ def test_sage_large_problems_take_256_query_workgroups(oracle, B, H, Sq, Sk, D):
     qz, ref = _check_quant(oracle, w, smooth=True)
     o_bf16, _ = capi.attn_fwd(q, k, v, w.scale)
     _check_sage_fwd(oracle, w, qz, ref, v, o_bf16)
+    total = B * H * ((Sq + 255) // 256)
+    cut = total % 256 if Sk > 1024 else 0
+    wide = total >= 256 and (total % 256 == 0 or cut)
+    want = [(f"sage_fwd_wide_kernel<{D}>", total - cut)] if wide else [(f"sage_fwd_kernel<{D}, 4, 1>", 2 * total)]
+    assert _launched(qz, v, w.scale) == want + ([(f"sage_fwd_kernel<{D}, 4, 2>", 2 * cut)] if cut else [])
+
+
+def _launched(qz, v, scale):
+    """The kernels of the forward and their workgroups."""
+    from flame_amd import capi
+    return [(name, n) for name, n, _ in recorded_launches(lambda: capi.sage_fwd(qz, v, scale))]
 
 
 def _rows_with_padding(t, D):
@@ -223,7 +236,7 @@ def test_sage_head_dim_96_on_256_query_workgroups(oracle):
     """D = 96 on a problem that fills the chip (264 workgroups of 256 queries, the last 8 cut into 16): every head
     against the oracle."""
     from flame_amd import capi
-    B, H, Sq, Sk, D = 1, 33, 2048, 320, 96
+    B, H, Sq, Sk, D = 1, 33, 2048, 1088, 96
     w = W.Workload("sage_wide_d96", W.f32_to_bf16_bits(W.normal_f32(71, 0, B * H * Sq * D).reshape(B, H, Sq, D)),
                    W.f32_to_bf16_bits(W.normal_f32(71, 1, B * H * Sk * D).reshape(B, H, Sk, D)),
                    W.f32_to_bf16_bits(W.normal_f32(71, 2, B * H * Sk * D).reshape(B, H, Sk, D)), None, 1.0 / np.sqrt(D))
@@ -231,6 +244,7 @@ def test_sage_head_dim_96_on_256_query_workgroups(oracle):
     qz, ref = _check_quant(oracle, w, smooth=True)
     o_bf16, _ = capi.attn_fwd(q, k, v, w.scale)
     _check_sage_fwd(oracle, w, qz, ref, v, o_bf16)
+    assert _launched(qz, v, w.scale) == [("sage_fwd_wide_kernel<128>", 256), ("sage_fwd_kernel<128, 4, 2>", 16)]
 
 
 def test_sage_refuses_head_dims_it_cannot_pad():

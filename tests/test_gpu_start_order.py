@@ -17,7 +17,7 @@ def test_every_unit(B, H, Sq, Sk, D, causal, lens, masked):
 
 
 def check(B, H, Sq, Sk, D, causal, lens, masked, rows=False):
-    """masked: the lengths as a keep-mask of keys; rows: a keep-mask that differs by query on top.  Returns the kernels launched."""
+    """masked: the lengths as a keep-mask of keys; rows: a keep-mask that differs by query on top.  Returns the kernels launched and their workgroups."""
     from flame_amd import capi
     print(f"[start order] {B=} {H=} {Sq=} {Sk=} {D=} {causal=} {lens=} {masked=}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(Sq + Sk + D)
@@ -52,8 +52,8 @@ def check(B, H, Sq, Sk, D, causal, lens, masked, rows=False):
             # P and dS rounded to bf16 (2^-9 each) in sums of many, the result rounded to bf16; per head, so that none is left out
             diff, size = (x[b].float() - y).flatten(1).norm(dim=1), y.flatten(1).norm(dim=1)
             assert bool((diff <= 1e-2 * size).all()), (name, b, (diff / size).max())
-    forward = [x[0] for x in recorded_launches(lambda: capi.attn_fwd(q, k, v, sc, **kw))]
-    return forward + [x[0] for x in recorded_launches(lambda: capi.attn_bwd(q, k, v, o, do, lse, sc, **kw))]
+    launched = recorded_launches(lambda: capi.attn_fwd(q, k, v, sc, **kw)) + recorded_launches(lambda: capi.attn_bwd(q, k, v, o, do, lse, sc, **kw))
+    return [(name, workgroups) for name, workgroups, _ in launched]
 
 
 # The kernels compiled for that order, each launched by name: 256-query workgroups under the causal flag and with key lengths, key
@@ -70,7 +70,7 @@ def check(B, H, Sq, Sk, D, causal, lens, masked, rows=False):
     (3, 12, 1000, 1000, 128, False, (1000, 700, 990), False, True, ("fwd_dealt_kernel<128, 6, 4>", "bwd_dq_dealt_kernel<128, 6, 4>", "bwd_dkdv_dealt_kernel<128, true>"))])
 def test_kernels(B, H, Sq, Sk, D, causal, lens, masked, rows, names):
     got = check(B, H, Sq, Sk, D, causal, lens, masked, rows)
-    assert [x for x in got if x.startswith(("fwd_", "bwd_d"))] == list(names), got
+    assert [x for x, _ in got if x.startswith(("fwd_", "bwd_d"))] == list(names), got
 
 
 # slices that divide by eight, one workgroup per compute unit at most, no exclusion at all, one sequence: the kernels without it
@@ -79,7 +79,7 @@ def test_kernels(B, H, Sq, Sk, D, causal, lens, masked, rows, names):
                                                             (1, 12, 3000, 400, 64, False, (333,), False), (1, 12, 3000, 3100, 128, False, (3001,), True)])
 def test_other_problems(B, H, Sq, Sk, D, causal, lens, masked):
     got = check(B, H, Sq, Sk, D, causal, lens, masked)
-    assert not any("dealt" in x for x in got), got
+    assert not any("dealt" in x for x, _ in got), got
 
 
 @pytest.mark.parametrize("B,H,S,D,lens", [(1, 37, 1024, 64, None), (1, 37, 1024, 128, None), (3, 12, 1000, 128, (1000, 70, 600)), (5, 12, 640, 64, (640, 70, 600, 64, 333))])
