@@ -41,7 +41,7 @@ static __global__ __launch_bounds__(256, 2) void fwd_probs_kernel(const FwdProbs
 
     // bands of eight key tiles, query tiles across, as in bwd_wide_scores_kernel
     const int n_kt = p.sk_pad / kWideTile, n_qt = p.sq_pad / kWideTile;
-    const int wg = xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = xcd_remap_tiles(blockIdx.x, gridDim.x, p.causal);
     const int slice = wg / (n_kt * n_qt), in_slice = wg % (n_kt * n_qt);
     const int band = in_slice / (8 * n_qt), in_band = in_slice % (8 * n_qt), width = min(8, n_kt - 8 * band);
     const int kt = 8 * band + in_band % width, qt = in_band / width;
@@ -174,7 +174,7 @@ static __global__ __launch_bounds__(256, 2) void fwd_probs_pv_kernel(const FwdPr
     const int wd = wave & 1, wm = wave >> 1;          // this wavefront's 64 columns of the head dim and 64 queries
     const int n_kt = p.sk_pad / kWideTile, n_qt = p.sq_pad / kWideTile, n_dt = (p.d + kWideTile - 1) / kWideTile;
     // the column tiles of a query tile, which read the same P, side by side; then the query tiles, which read the same V
-    const int wg = xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = xcd_remap_split(blockIdx.x, gridDim.x);
     const int per = n_qt * n_dt, part_id = wg / per, split = part_id % p.key_splits, slice = part_id / p.key_splits;
     const int j = wg % per, dt = j % n_dt;
     const int mt = p.causal ? n_qt - 1 - j / n_dt : j / n_dt;              // causal: the longest walks first

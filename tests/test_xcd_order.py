@@ -23,9 +23,9 @@ int unit(int linear, int total, int tiles, int B, int H, bool falling, bool by_b
 int main(int, char** argv) {
     const int B = atoi(argv[1]), H = atoi(argv[2]), tiles = atoi(argv[3]), total = B * H * tiles;
     for (int i = 0; i < total; ++i)
-        printf("%d %d %d %d %d %d\n", unit(i, total, tiles, B, H, false, false, false), unit(i, total, tiles, B, H, true, false, false),
+        printf("%d %d %d %d %d %d %d %d\n", unit(i, total, tiles, B, H, false, false, false), unit(i, total, tiles, B, H, true, false, false),
                unit(i, total, tiles, B, H, true, false, true), unit(i, total, tiles, B, H, false, true, false), unit(i, total, tiles, B, H, false, true, true),
-               fattn::xcd_remap_split(i, total));
+               fattn::xcd_remap_split(i, total), fattn::xcd_remap_tiles(i, total, false), fattn::xcd_remap_tiles(i, total, true));
 }
 """
 
@@ -42,11 +42,12 @@ def exe(tmp_path_factory):
                                                  (5, 15, 13), (13, 10, 5), (143, 7, 3), (2, 12, 40)])
 def test_every_unit_once(exe, batches, heads, tiles):
     out = subprocess.run([exe, str(batches), str(heads), str(tiles)], check=True, capture_output=True, text=True).stdout.split()
-    plain, falling, falling_snake, by_batch, by_batch_snake, split = ([int(v) for v in out[i::6]] for i in range(6))
+    plain, falling, falling_snake, by_batch, by_batch_snake, split, even_tiles, causal_tiles = ([int(v) for v in out[i::8]] for i in range(8))
     total = batches * heads * tiles
     for ids in (plain, falling, falling_snake, by_batch, by_batch_snake):
         assert sorted(ids) == list(range(total))
     assert split == (plain if total % 8 == 0 else list(range(total)))      # the workgroups that share walks: in turn where eight does not divide
+    assert causal_tiles == split and even_tiles == (split if total <= 768 else plain)         # score tiles of wide heads
     for x in range(8):
         mine = plain[x::8]
         assert mine == list(range(mine[0], mine[0] + len(mine))) if mine else True
@@ -58,3 +59,18 @@ def test_every_unit_once(exe, batches, heads, tiles):
         for x in range(8):                        # in the order of the batches, within the eight units dealt at a time
             seq = [v // tiles // heads for v in by_batch[x::8]]
             assert all(seq[i] <= seq[i + heads] for i in range(len(seq) - heads))
+
+
+# Score tiles of wide heads under the causal flag, in bands of eight key tiles with the query tiles across: the XCDs' shares of those that are attended to differ by
+# no more than a band's eight columns do.  (In contiguous ranges an XCD has 0 to 28 of 15 x 15, 6 to 78 of 25 x 25, 15 to 120 of 31 x 31.)
+@pytest.mark.parametrize("side", [15, 25, 31])
+def test_causal_tiles_are_shared_out(exe, side):
+    out = subprocess.run([exe, "1", "1", str(side * side)], check=True, capture_output=True, text=True).stdout.split()
+
+    def attended(wg):
+        band, j = divmod(wg, 8 * side)
+        width = min(8, side - 8 * band)
+        return 8 * band + j % width <= j // width
+
+    share = [sum(attended(int(v)) for v in out[7::8][x::8]) for x in range(8)]
+    assert sum(share) == side * (side + 1) // 2 and max(share) - min(share) <= 8 * ((side + 7) // 8), share
