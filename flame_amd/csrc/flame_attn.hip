@@ -225,7 +225,8 @@ int launch_fwd_wide(FwdParams p, hipStream_t s) {
     if ((int64_t)((p.Sq + 255) / 256) * p.B * p.H * 8 > 0x7fffffff) return FLAME_ATTN_ERR_UNSUPPORTED;
     // A last round that would leave at least half of the compute units idle goes to smaller workgroups in a launch of its own:
     // 32-query ones that share the keys while these fit one per unit, else 128-query ones.  (B=2 H=24 S=1536 D=128: 288
-    // units of 256 queries, 92 us as two rounds, 79 us as one round and 256 small workgroups.)
+    // units of 256 queries, 92 us as two rounds, 79 us as one round and 256 small workgroups.)  At head dims 72 to 96
+    // the 32-query ones are the instance of 128; that of 96 was not timed here.
     static_assert(T::BM == 256, "cut_last_round counts in 256-query workgroups");
     const LastRound r = cut_last_round(p.Sq, (int64_t)p.B * p.H, device_cu_count(), true);
     {
@@ -1299,8 +1300,9 @@ static int attn_fwd_impl(const void* Q, const void* K, const void* V, void* O, v
     if (dropout_p != 0.f) {
         if (!set_dropout(p.m, dropout_p, dropout_seed, draw_cq, draw_ck, N_q, N_kv)) return FLAME_ATTN_ERR_INVALID;
         const int DP = std::max(padded_head_dim(D), padded_head_dim(Dv));
-        // the undropped call's choice between the kernels, without its split of the keys (this entry point has no workspace):
-        // the log-sum-exp is that of the undropped softmax, its sum joined in another order where that call splits
+        // the undropped call's choice between the kernels, without its split of the keys (this entry point has no workspace) and
+        // its instances of 96 (head dims 72 to 96 run zero-padded to 128; those with dropout were not built, nor timed): the
+        // log-sum-exp is that of the undropped softmax, its sum joined in another order where that call splits
         if (!hm && fwd_rule_keyshare((int64_t)B * H, N_q, DP))
             switch (drop_mode(p.m, N_kv)) {
                 case kDropRows64: return DP == 128 ? launch_fwd_keyshare<128, kDropRows64>(p, s) : launch_fwd_keyshare<64, kDropRows64>(p, s);

@@ -20,8 +20,8 @@ inline bool second_round_levels(int64_t total, int64_t cus, int N_q) {
 }
 
 // Forward.  Nothing is excluded at all (plain) or the last key tile is cut, the causal flag is set, or there are key lengths, which keep
-// 256-query workgroups wherever a last round allows it.  DP: padded head dim, d96: the kernels of 96, whose lines are those of
-// last_round.hpp alone.
+// 256-query workgroups wherever a last round allows it.  DP: padded head dim, d96: the kernels of 96.  These, and causal calls
+// with another number of keys than queries, were not measured on both sides: their lines are those of last_round.hpp alone.
 //
 // Plain, D = 128: 512 keys [1.12] 35.2 -> 32.4, [1.5] 43.2 -> 35.8, [2] 50.4 -> 45.0, [4] 96.5 -> 85.0; 768 keys [1.12] 43.0 -> 41.6; 1024 keys [1.06] 48.8 ->
 // 51.2, [1.12] 50.8 -> 51.8, [1.5] 61.2 -> 55.7, [2.25] 96.5 -> 85.1; 2048 keys [1.5] 101.2 -> 99.4, [1.75] 113.5 -> 119.9, [2.5] 164.8 -> 158.9; 3072 keys
