@@ -125,7 +125,7 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdParams& p, const int bloc
     const int n_kt = (p.Sk + BN - 1) / BN;
     int wg, part = 0, nparts = 1;
     if (p.n_whole < 0) {
-        wg = p.m.kv_len || p.key_mask ? xcd_remap_heads(block, nblocks, n_kt) : xcd_remap(block, nblocks);
+        wg = xcd_remap_heads(block, nblocks, n_kt, p.m.kv_len || p.key_mask, false);
     } else if (block < p.n_whole) {
         wg = xcd_remap(block, p.n_whole);
     } else {          // the split key blocks come last in dispatch order and fill the final, partial round (or are all there is)
@@ -936,23 +936,23 @@ __device__ __forceinline__ void bwd_dq_body(const BwdParams& p) {
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
+    const bool falling = !(EXCL == kExKeys) && p.m.causal && !p.m.kv_len;
     int wg, part = 0;
     if (p.dq_parts > 1) {
         const int all = xcd_remap_split(blockIdx.x, gridDim.x);
         part = all % p.dq_parts;
         wg = all / p.dq_parts;
     } else {
-        wg = p.m.kv_len || KEYS ? xcd_remap_heads<KG == 1 && !BITS>(blockIdx.x, gridDim.x, n_qt) : p.dq_base + xcd_remap(blockIdx.x, gridDim.x);
+        wg = p.dq_base + xcd_remap_heads<KG == 1 && !BITS>(blockIdx.x, gridDim.x, n_qt, p.m.kv_len || KEYS, falling);
     }
     int qt = wg % n_qt, bh = wg / n_qt;
-    const bool falling = !(EXCL == kExKeys) && p.m.causal && !p.m.kv_len;
     if constexpr (DEALT) {
         int t, s;
         dealt_unit<!BITS>(blockIdx.x, n_qt, p.B, p.H, !falling, t, s);
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling && p.dq_parts == 1) {
-        causal_longest_first<KG == 1>(blockIdx.x, wg, n_qt, gridDim.x, qt, bh);
+        causal_longest_first<KG == 1>(wg, n_qt, gridDim.x, qt, bh);
     }
     if (!BITS && (KEYS || p.m.kv_len) && p.dq_parts == 1) bh = longest_batches_first<KEYS>(bh, p.B, p.H, p.Sk, p.m);
     const int b = bh / p.H, hh = bh % p.H;
@@ -1399,16 +1399,16 @@ __device__ __forceinline__ void bwd_dq_wide_body(const BwdParams& p, const int b
     const int n = lane & 31, h = lane >> 5;
 
     const int n_qt = (p.Sq + BM - 1) / BM;
-    const int wg = p.m.kv_len ? xcd_remap_heads(block, nblocks, n_qt) : xcd_remap(block, nblocks);
-    int qt = wg % n_qt, bh = wg / n_qt;
     const bool falling = p.m.causal && !p.m.kv_len;
+    const int wg = xcd_remap_heads(block, nblocks, n_qt, p.m.kv_len != nullptr, falling);
+    int qt = wg % n_qt, bh = wg / n_qt;
     if constexpr (DEALT) {
         int t, s;
         dealt_unit(block, n_qt, p.B, p.H, !falling, t, s);
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
-        causal_longest_first(block, wg, n_qt, nblocks, qt, bh);
+        causal_longest_first(wg, n_qt, nblocks, qt, bh);
     }
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;

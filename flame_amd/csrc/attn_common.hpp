@@ -373,10 +373,10 @@ __device__ __forceinline__ void wait_vm() {
 // Causal problems: the key walk of query unit qt grows with qt, and workgroups start in id order, so the longest
 // walks must come first or they finish alone at the end.  Within the contiguous range of units that one XCD
 // works through (whole heads where the counts allow), the order becomes: last unit of every head, then the
-// units before them, and so on.  `wg`: unit id after xcd_remap, head-major, of workgroup `linear`; returns (qt, head) through refs.
+// units before them, and so on.  `wg`: unit id after xcd_remap, head-major, or, where eight does not divide the total, the
+// workgroup's own (all of them in one order, dealt to the XCDs in turn); returns (qt, head) through refs.
 template <bool SNAKE = false>
-__device__ __forceinline__ void causal_longest_first(int linear, int wg, int n_qt, int total, int& qt, int& bh) {
-    if (total % 8 != 0) wg = linear;               // all of them in one order, dealt to the XCDs in turn
+__device__ __forceinline__ void causal_longest_first(int wg, int n_qt, int total, int& qt, int& bh) {
     const int per_xcd = (total % 8 == 0) ? total / 8 : total;
     if (per_xcd % n_qt == 0) {
         const int heads = per_xcd / n_qt;

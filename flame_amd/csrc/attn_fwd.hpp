@@ -102,7 +102,7 @@ __device__ __forceinline__ void fwd_body(const FwdParams& p) {
     constexpr bool KNOWS_BIAS = EXCL == kExBiasF32 || EXCL == kExBiasBf16;       // no causal flag, no key lengths
     const bool falling = !KNOWS_BIAS && EXCL != kExKeys && p.m.causal && !p.m.kv_len;
     const bool by_batch = !KNOWS_BIAS && (p.m.kv_len || EXCL == kExKeys || EXCL == kExBits);
-    const int wg = by_batch ? xcd_remap_heads<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.wg_base + xcd_remap_heads<NW == 4 && KG == 1 && EXCL != kExBits>(blockIdx.x, gridDim.x, n_qt, by_batch, falling);
     int qt = wg % n_qt, bh = wg / n_qt;
     if constexpr (DEALT) {
         int t, s;
@@ -110,7 +110,7 @@ __device__ __forceinline__ void fwd_body(const FwdParams& p) {
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);         // (the compiler divides in vector registers)
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
-        causal_longest_first<NW == 4 && KG == 1>(blockIdx.x, wg, n_qt, gridDim.x, qt, bh);
+        causal_longest_first<NW == 4 && KG == 1>(wg, n_qt, gridDim.x, qt, bh);
     }
     if (EXCL == kExKeys || (p.m.kv_len && EXCL != kExBits)) bh = longest_batches_first<EXCL == kExKeys>(bh, p.B, p.H, p.Sk, p.m);
     // a bias that all batches share: its rows are read by the batches' workgroups one after the other on one XCD, from its L2

@@ -319,7 +319,7 @@ __device__ __forceinline__ void sage_fwd_body(const SageFwdParams& p) {
 
     const int n_qt = (p.Sq + BM - 1) / BM;
     const bool falling = p.causal && !p.kv_len;
-    const int wg = p.kv_len ? xcd_remap_heads(blockIdx.x, gridDim.x, n_qt) : p.wg_base + xcd_remap(blockIdx.x, gridDim.x);
+    const int wg = p.wg_base + xcd_remap_heads(blockIdx.x, gridDim.x, n_qt, p.kv_len != nullptr, falling);
     int qt = wg % n_qt, bh = wg / n_qt;
     // (shortest first before: B=2 H=24 S=4608 D=128 causal 307 -> 276 us, B=1 H=24 S=2048 D=128 75.1 -> 61.8)
     if constexpr (DEALT) {
@@ -331,7 +331,7 @@ __device__ __forceinline__ void sage_fwd_body(const SageFwdParams& p) {
         qt = __builtin_amdgcn_readfirstlane(falling ? n_qt - 1 - t : t);
         bh = __builtin_amdgcn_readfirstlane(s);
     } else if (falling) {
-        causal_longest_first<KG == 1>(blockIdx.x, wg, n_qt, gridDim.x, qt, bh);
+        causal_longest_first<KG == 1>(wg, n_qt, gridDim.x, qt, bh);
     }
     const int b = bh / p.H, hh = bh % p.H;
     const int q0 = qt * BM;

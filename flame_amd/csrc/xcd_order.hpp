@@ -10,13 +10,13 @@ namespace fattn {
 // (batch, head) then share one L2 and its K/V (forward) or Q/dO (backward) stay resident there.
 // Where the total does not divide, the first total % 8 ranges are one longer, as the shares of the XCDs are.
 FATTN_HOST_DEVICE int xcd_remap(int linear, int total) {
-    constexpr int kXcd = 8;
-    const int x = linear % kXcd;
-    return x * (total / kXcd) + (x < total % kXcd ? x : total % kXcd) + linear / kXcd;
+    constexpr unsigned kXcd = 8;
+    const unsigned l = (unsigned)linear, t = (unsigned)total, x = l % kXcd;
+    return (int)(x * (t / kXcd) + (x < t % kXcd ? x : t % kXcd) + l / kXcd);
 }
 // Workgroups that share one walk: in turn where the total does not divide.  (Contiguous ranges there, dK/dV, us: 7 heads of 1500 D=64, 252 workgroups,
 // 16.6 -> 21.0, D=128 25.1 -> 27.7; 5 heads of 1100 D=96, 180 workgroups, 17.2 -> 19.5.  dQ 1 to 3 % at D=64 and 96.)
-FATTN_HOST_DEVICE int xcd_remap_split(int linear, int total) { return total % 8 == 0 ? xcd_remap(linear, total) : linear; }
+FATTN_HOST_DEVICE int xcd_remap_split(int linear, int total, bool in_turn = true) { return in_turn && total % 8 != 0 ? linear : xcd_remap(linear, total); }
 // The same for P V of wide heads.  (Contiguous ranges there, us: one head of D = 512, S = 1200 19.2 -> 19.8, 2300 19.3 -> 19.9, 3200 24.9 -> 27.0; three heads of
 // D = 320, S = 2300 35.4 -> 37.7, causal 33.0 -> 32.1, S = 3968 75.5 -> 74.0, causal 54.7 -> 56.7.)
 // Tiles of the scores of wide heads: in turn under the causal flag, as ever fewer tiles of the later bands of keys are attended to and contiguous
@@ -26,7 +26,7 @@ FATTN_HOST_DEVICE int xcd_remap_split(int linear, int total) { return total % 8 
 // 13.6, 225 19.2 -> 19.5 / 12.7 -> 14.5, 324 23.9 -> 24.4 / 14.7 -> 15.6, 625 38.5 -> 39.0 / 22.9 -> 23.1, 961 53.9 -> 49.9 / 33.0 -> 29.4, 972 39.3 -> 40.7 / 25.0 -> 24.6, 2883
 // 112.7 -> 98.1 / 61.3 -> 59.0.  The products of the backward gain by contiguous ranges, 300 workgroups 53.2 -> 45.6, 837 160 -> 128, causal 120 -> 80.)
 FATTN_HOST_DEVICE int xcd_remap_tiles(int linear, int total, bool causal) {
-    return causal || total <= 768 ? xcd_remap_split(linear, total) : xcd_remap(linear, total);
+    return xcd_remap_split(linear, total, causal || total <= 768);
 }
 // Workgroups of which a compute unit holds two are dealt out one per unit, then a second one each.  Where (nearly) all fit at once
 // nothing is left to even out unequal walks: in the order of falling length the units with the longest walks would get the
@@ -47,11 +47,15 @@ FATTN_HOST_DEVICE int snake_order(int j, int total) {
 // slices x, x + 8, x + 16, ...: every slice still stays in one L2, and the heads of one batch are spread
 // over all XCDs.  `per_head`: tiles per (batch, head) slice; the id runs slice-major.
 // SNAKE: workgroups of which a compute unit holds two, the longest walks first: see snake_order.
+// by_heads: whether this order is wanted at all; in_turn: else, whether a total that does not divide goes in turn (under the causal flag all
+// workgroups are in one order then, from the longest walk to the shortest: causal_longest_first).  One call for all three orders, whose result alone is
+// divided: 40 to 60 instructions fewer ahead of a kernel's first load than with the choice in every kernel and a second division under the causal flag.
+// (Forward, us: 4 x 8 heads of 257, D = 72 8.64 -> 8.40, D = 128 9.85 -> 9.62, 2 x 16 of 577, D = 64 10.08 -> 9.86; forward and backward with dropout, B=2 H=16 S=1024
+// D=64 63.98 -> 63.31.)
 template <bool SNAKE = false>
-FATTN_HOST_DEVICE int xcd_remap_heads(int linear, int total, int per_head) {
+FATTN_HOST_DEVICE int xcd_remap_heads(int linear, int total, int per_head, bool by_heads = true, bool in_turn = true) {
     constexpr int kXcd = 8;
-    const int n_heads = total / per_head;
-    if (n_heads % kXcd != 0) return xcd_remap_split(linear, total);
+    if (!by_heads || total / per_head % kXcd != 0) return xcd_remap_split(linear, total, by_heads || in_turn);
     const int x = linear % kXcd, j = SNAKE ? snake_order(linear / kXcd, total / kXcd) : linear / kXcd;
     return ((j / per_head) * kXcd + x) * per_head + j % per_head;
 }

@@ -23,9 +23,10 @@ int unit(int linear, int total, int tiles, int B, int H, bool falling, bool by_b
 int main(int, char** argv) {
     const int B = atoi(argv[1]), H = atoi(argv[2]), tiles = atoi(argv[3]), total = B * H * tiles;
     for (int i = 0; i < total; ++i)
-        printf("%d %d %d %d %d %d %d %d\n", unit(i, total, tiles, B, H, false, false, false), unit(i, total, tiles, B, H, true, false, false),
+        printf("%d %d %d %d %d %d %d %d %d %d\n", unit(i, total, tiles, B, H, false, false, false), unit(i, total, tiles, B, H, true, false, false),
                unit(i, total, tiles, B, H, true, false, true), unit(i, total, tiles, B, H, false, true, false), unit(i, total, tiles, B, H, false, true, true),
-               fattn::xcd_remap_split(i, total), fattn::xcd_remap_tiles(i, total, false), fattn::xcd_remap_tiles(i, total, true));
+               fattn::xcd_remap_split(i, total), fattn::xcd_remap_tiles(i, total, false), fattn::xcd_remap_tiles(i, total, true),
+               fattn::xcd_remap_heads(i, total, tiles, false, false), fattn::xcd_remap_heads(i, total, tiles, false, true));
 }
 """
 
@@ -42,11 +43,12 @@ def exe(tmp_path_factory):
                                                  (5, 15, 13), (13, 10, 5), (143, 7, 3), (2, 12, 40)])
 def test_every_unit_once(exe, batches, heads, tiles):
     out = subprocess.run([exe, str(batches), str(heads), str(tiles)], check=True, capture_output=True, text=True).stdout.split()
-    plain, falling, falling_snake, by_batch, by_batch_snake, split, even_tiles, causal_tiles = ([int(v) for v in out[i::8]] for i in range(8))
+    plain, falling, falling_snake, by_batch, by_batch_snake, split, even_tiles, causal_tiles, no_heads, no_heads_in_turn = ([int(v) for v in out[i::10]] for i in range(10))
     total = batches * heads * tiles
     for ids in (plain, falling, falling_snake, by_batch, by_batch_snake):
         assert sorted(ids) == list(range(total))
     assert split == (plain if total % 8 == 0 else list(range(total)))      # the workgroups that share walks: in turn where eight does not divide
+    assert no_heads == plain and no_heads_in_turn == split
     assert causal_tiles == split and even_tiles == (split if total <= 768 else plain)         # score tiles of wide heads
     for x in range(8):
         mine = plain[x::8]
@@ -72,5 +74,5 @@ def test_causal_tiles_are_shared_out(exe, side):
         width = min(8, side - 8 * band)
         return 8 * band + j % width <= j // width
 
-    share = [sum(attended(int(v)) for v in out[7::8][x::8]) for x in range(8)]
+    share = [sum(attended(int(v)) for v in out[7::10][x::8]) for x in range(8)]
     assert sum(share) == side * (side + 1) // 2 and max(share) - min(share) <= 8 * ((side + 7) // 8), share
