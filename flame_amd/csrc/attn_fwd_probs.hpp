@@ -41,7 +41,7 @@ static __global__ __launch_bounds__(256, 2) void fwd_probs_kernel(const FwdProbs
 
     // bands of eight key tiles, query tiles across, as in bwd_wide_scores_kernel
     const int n_kt = p.sk_pad / kWideTile, n_qt = p.sq_pad / kWideTile;
-    const int wg = xcd_remap_tiles(blockIdx.x, gridDim.x, p.causal);
+    const int wg = xcd_remap_tiles(blockIdx.x, gridDim.x, n_kt * n_qt, p.causal);
     const int slice = wg / (n_kt * n_qt), in_slice = wg % (n_kt * n_qt);
     const int band = in_slice / (8 * n_qt), in_band = in_slice % (8 * n_qt), width = min(8, n_kt - 8 * band);
     const int kt = 8 * band + in_band % width, qt = in_band / width;

@@ -20,13 +20,14 @@ FATTN_HOST_DEVICE int xcd_remap_split(int linear, int total, bool in_turn = true
 // The same for P V of wide heads.  (Contiguous ranges there, us: one head of D = 512, S = 1200 19.2 -> 19.8, 2300 19.3 -> 19.9, 3200 24.9 -> 27.0; three heads of
 // D = 320, S = 2300 35.4 -> 37.7, causal 33.0 -> 32.1, S = 3968 75.5 -> 74.0, causal 54.7 -> 56.7.)
 // Tiles of the scores of wide heads: in turn under the causal flag, as ever fewer tiles of the later bands of keys are attended to and contiguous
-// ranges are unequal shares, and on small grids, whose rows all L2s hold; 768: one and a half rounds of two workgroups per compute unit.  (In
+// ranges are unequal shares, and on small grids of one slice, whose rows all L2s hold; 768: one and a half rounds of two workgroups per compute unit.  (In
 // turn -> contiguous, us, scores of the backward / probabilities of the forward: causal, one head of D = 512, S = 1800 17.9 -> 19.0 / 11.8 -> 13.2, S = 3200
 // 23.6 -> 36.0 / 14.7 -> 21.9, S = 3968 36.4 -> 42.8 / 22.7 -> 25.9, three of D = 320, S = 3968 60.7 -> 68.0 / 36.2 -> 42.7; without it 100 tiles 18.2 -> 18.9 / 13.7 ->
 // 13.6, 225 19.2 -> 19.5 / 12.7 -> 14.5, 324 23.9 -> 24.4 / 14.7 -> 15.6, 625 38.5 -> 39.0 / 22.9 -> 23.1, 961 53.9 -> 49.9 / 33.0 -> 29.4, 972 39.3 -> 40.7 / 25.0 -> 24.6, 2883
-// 112.7 -> 98.1 / 61.3 -> 59.0.  The products of the backward gain by contiguous ranges, 300 workgroups 53.2 -> 45.6, 837 160 -> 128, causal 120 -> 80.)
-FATTN_HOST_DEVICE int xcd_remap_tiles(int linear, int total, bool causal) {
-    return xcd_remap_split(linear, total, causal || total <= 768);
+// 112.7 -> 98.1 / 61.3 -> 59.0.  Of several slices an XCD
+// keeps its own: four of 81 tiles, D = 264 21.0 -> 19.4 / 13.7 -> 12.9, three of 100 23.5 -> 23.2 / 15.3 -> 15.3.  The products of the backward gain by contiguous ranges, 300 workgroups 53.2 -> 45.6, 837 160 -> 128, causal 120 -> 80.)
+FATTN_HOST_DEVICE int xcd_remap_tiles(int linear, int total, int per_slice, bool causal) {
+    return xcd_remap_split(linear, total, causal || (per_slice == total && total <= 768));
 }
 // Workgroups of which a compute unit holds two are dealt out one per unit, then a second one each.  Where (nearly) all fit at once
 // nothing is left to even out unequal walks: in the order of falling length the units with the longest walks would get the
